@@ -2,7 +2,8 @@
 
 Counterpart of the reference's setup.py:1-16, which JIT-builds its CUDA sources through
 torch.utils.cpp_extension; here the library has no torch or pybind dependency and is a
-plain `hipcc -shared`.  Run as `python build.py` (add `--incremental` to recompile only the
+plain `hipcc -shared`.  The operators on torch tensors (csrc/torch_ops.cpp, host code only) become an
+extension module beside it, which finds the library's functions at run time.  Run as `python build.py` (add `--incremental` to recompile only the
 sources that changed) or call build_library().
 """
 
@@ -16,6 +17,8 @@ import sys
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
 OBJ_DIR = os.path.join(PKG_DIR, "build")
+EXT_SOURCE = os.path.join(CSRC, "torch_ops.cpp")
+EXT_PATH = os.path.join(PKG_DIR, "custom_kernels", "_l3torch.so")
 LIB_PATH = os.path.join(PKG_DIR, "custom_kernels", "libl3kernels.so")
 SOURCES = ["l3_api.hip", "attn_decode.hip", "attn_mfma.hip", "attn_prefill.hip", "attn_prefill_tiled.hip",
            "linear_skinny.hip", "linear_splitk.hip", "attn_combine.hip", "rms_norm.hip", "rot_embed.hip",
@@ -45,8 +48,22 @@ def _newest_header() -> float:
     return max(os.path.getmtime(h) for h in hdrs)
 
 
+def _extension_command():
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    abi = int(torch.compiled_with_cxx11_abi())
+    return [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+            "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={abi}", *(f"-I{p}" for p in include_paths("cuda")),
+            f"-I{sysconfig.get_paths()['include']}", EXT_SOURCE, "-o", EXT_PATH, *(f"-L{p}" for p in library_paths("cuda")),
+            "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python"]
+
+
 def build_library(verbose: bool = True, extra_flags=(), incremental: bool = False, jobs: int = 8) -> str:
-    """Compile every source to an object file (in parallel) and link the shared library.  With
+    """Compile every source to an object file (in parallel), link the shared library and build the extension
+    module that runs its operators on torch tensors.  With
     `incremental` an object newer than its source and every header is kept."""
     os.makedirs(OBJ_DIR, exist_ok=True)
     base = [hipcc_path(), *HIPCC_FLAGS, *extra_flags, "-I", os.path.join(PKG_DIR, "..", "include")]
@@ -59,6 +76,8 @@ def build_library(verbose: bool = True, extra_flags=(), incremental: bool = Fals
         if incremental and os.path.exists(obj) and os.path.getmtime(obj) > max(os.path.getmtime(src), hdr_time):
             continue
         todo.append(base + ["-c", src, "-o", obj])
+    if not (incremental and os.path.exists(EXT_PATH) and os.path.getmtime(EXT_PATH) > max(os.path.getmtime(EXT_SOURCE), hdr_time)):
+        todo.append(_extension_command())
 
     def run(cmd):
         if verbose:

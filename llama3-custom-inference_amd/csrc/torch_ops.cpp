@@ -1,0 +1,720 @@
+// The operators on torch tensors: argument checks, output allocation, workspaces and the call into
+// libl3kernels.so, as a CPython extension module (custom_kernels/_l3torch.so).  It takes the place of
+// the pybind table of main.cpp:5-9 and of the tensor handling at the head of the host launchers
+// (custom_kernels.cu:233-338, 369-389, 418-442).
+//
+// Why it is native: a decode step calls small operators one after the other, and the calls, not the
+// kernels, set the pace.  The HIP runtime takes 2.4 us to enqueue a kernel; the same checks in Python with a
+// ctypes call took 6.5 us for rms_norm of one row, 7.9 us for rot_embed, 11.9 us for
+// flash_attention_decode over 256 tokens and 19.5 us for a split-K linear with its finishing pass.  Here
+// they take 3.9, 3.8, 4.5 and 13.5 us (the last is the kernels' own time).
+// Hence METH_FASTCALL functions with positional arguments, tensors unpacked in place, and outputs
+// taken from torch's caching allocator without a trip through the dispatcher.
+//
+// libl3kernels.so itself stays free of torch: its C functions are looked up by name (bind) in the
+// library that the Python side has loaded.
+#include <Python.h>
+#include <dlfcn.h>
+
+#include <ATen/core/Tensor.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <ATen/ops/empty_like.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <algorithm>
+#include <cmath>
+#include <utility>
+#include <vector>
+
+#include "../../include/l3_kernels.h"
+
+namespace {
+
+using at::Tensor;
+using at::TensorBase;
+
+#define L3_FUNCTIONS(X)                                                                                          \
+    X(l3_strerror) X(l3_attn_decode) X(l3_attn_decode_devlen) X(l3_attn_decode_workspace_bytes)                  \
+    X(l3_attn_workspace_init) X(l3_attn_prefill) X(l3_rms_norm) X(l3_add_rms_norm) X(l3_add_rms_norm_partials)   \
+    X(l3_rot_embed) X(l3_rot_embed_append_partials) X(l3_silu_mul) X(l3_silu_mul_rows) X(l3_linear_decode)       \
+    X(l3_linear_swiglu_decode) X(l3_linear_decode_fused) X(l3_linear_qkv_rope_append) X(l3_linear_splitk_plan)   \
+    X(l3_linear_splitk) X(l3_linear_splitk_finish)
+
+struct Library {
+#define X(name) decltype(&::name) name = nullptr;
+    L3_FUNCTIONS(X)
+#undef X
+} lib;
+
+// ------------------------------------------------------------------------------------------ arguments
+
+const Tensor& tensor(PyObject* o, const char* name) {
+    TORCH_CHECK_TYPE(THPVariable_Check(o), name, " must be a torch.Tensor");
+    return THPVariable_Unpack(o);
+}
+
+void require_gpu_bf16(const Tensor& t, const char* name) {
+    TORCH_CHECK(t.is_cuda(), name, " must be on the GPU (got ", t.device(), "); there is no CPU path");
+    // the reference's data_ptr<at::BFloat16>() raises the same way (custom_kernels.cu:274)
+    TORCH_CHECK(t.scalar_type() == at::kBFloat16, "expected scalar type BFloat16 for ", name, " but found ", t.scalar_type());
+}
+
+const Tensor& gpu_bf16(PyObject* o, const char* name) {
+    const Tensor& t = tensor(o, name);
+    require_gpu_bf16(t, name);
+    return t;
+}
+
+int integer(PyObject* o) {
+    const long v = PyLong_AsLong(o);
+    if (v == -1 && PyErr_Occurred()) throw python_error();
+    return int(v);
+}
+
+double number(PyObject* o) {
+    const double v = PyFloat_AsDouble(o);
+    if (v == -1.0 && PyErr_Occurred()) throw python_error();
+    return v;
+}
+
+const Tensor* optional_tensor(PyObject* o, const char* name) { return o == Py_None ? nullptr : &gpu_bf16(o, name); }
+
+// Raises for an error code of the library.
+template <typename... Detail>
+void check(int64_t rc, const Detail&... detail) {
+    TORCH_CHECK(rc >= 0, lib.l3_strerror(int(rc)), ": ", detail..., " (l3 error ", rc, ")");
+}
+
+int64_t size_at(const Tensor& t, int i) { return t.sizes()[i]; }
+int64_t stride_at(const Tensor& t, int i) { return t.strides()[i]; }
+void* ptr(const TensorBase& t) { return t.data_ptr(); }
+
+// A contiguous tensor with t's values; t itself (kept alive by the caller's arguments) where it is one.
+const Tensor& contiguous(const Tensor& t, Tensor& copy) {
+    if (t.is_contiguous()) return t;
+    copy = t.contiguous();
+    return copy;
+}
+
+Tensor new_empty(at::IntArrayRef sizes, const Tensor& like, at::ScalarType type = at::kBFloat16) {
+    return Tensor(at::detail::empty_cuda(sizes, type, like.device(), std::nullopt));
+}
+
+// torch.empty_like for a dense tensor: the same sizes and strides.
+Tensor empty_like_dense(const Tensor& t) {
+    return Tensor(at::detail::empty_strided_cuda(t.sizes(), t.strides(), t.scalar_type(), t.device()));
+}
+
+PyObject* wrap(Tensor&& t) { return THPVariable_Wrap(std::move(t)); }
+
+PyObject* wrap_pair(Tensor&& a, Tensor&& b) {
+    PyObject* pair = PyTuple_New(2);
+    if (!pair) throw python_error();
+    PyTuple_SET_ITEM(pair, 0, wrap(std::move(a)));
+    PyTuple_SET_ITEM(pair, 1, wrap(std::move(b)));
+    return pair;
+}
+
+// The tensor's device made current for the length of a call (nothing to do in a single-GPU process),
+// and torch's current stream there.
+struct OnDevice {
+    c10::DeviceIndex before = -1;
+    c10::DeviceIndex index;
+    hipStream_t stream;
+    explicit OnDevice(const Tensor& t) : index(t.device().index()) {
+        const c10::DeviceIndex now = c10::hip::current_device();
+        if (now != index) {
+            c10::hip::set_device(index);
+            before = now;
+        }
+        stream = c10::hip::getCurrentHIPStream(index).stream();
+    }
+    ~OnDevice() {
+        if (before >= 0) c10::hip::set_device(before);
+    }
+    OnDevice(const OnDevice&) = delete;
+    OnDevice& operator=(const OnDevice&) = delete;
+};
+
+// ------------------------------------------------------------------------------------- decode attention
+
+// Workspaces of decode attention: one per (device, stream), grown on demand, whose head holds the arrival
+// counters of the single-launch form.  Calls on one stream are ordered and can share one; another stream
+// gets its own.  The interpreter lock guards the list.  It is bounded: beyond kMaxWorkspaces streams the
+// one unused longest goes back to torch's allocator, which hands its memory only to later work of the
+// stream it was allocated on.
+struct Workspace {
+    c10::DeviceIndex device;
+    hipStream_t stream;
+    TensorBase memory;
+};
+constexpr size_t kMaxWorkspaces = 64;
+
+std::vector<Workspace>& workspaces() {
+    static auto* all = new std::vector<Workspace>();   // outlives the allocator's own teardown
+    return *all;
+}
+
+const TensorBase& attention_workspace(const OnDevice& on, const Tensor& like, size_t nbytes) {
+    auto& all = workspaces();
+    size_t i = 0;
+    while (i < all.size() && !(all[i].stream == on.stream && all[i].device == on.index)) ++i;
+    if (i == all.size() || size_t(all[i].memory.numel()) < nbytes) {
+        TensorBase memory = at::detail::empty_cuda({int64_t(std::max(nbytes, size_t(4) << 20))}, at::kByte, like.device(),
+                                                   std::nullopt);
+        check(lib.l3_attn_workspace_init(ptr(memory), size_t(memory.numel()), on.stream), "l3_attn_workspace_init");
+        if (i < all.size()) {
+            all[i].memory = std::move(memory);
+        } else {
+            if (all.size() >= kMaxWorkspaces) all.pop_back();
+            i = all.size();
+            all.push_back({on.index, on.stream, std::move(memory)});
+        }
+    }
+    if (i > 0) std::rotate(all.begin(), all.begin() + i, all.begin() + i + 1);   // most recently used first
+    return all[0].memory;
+}
+
+struct DecodeShape {
+    int B, QH, KVH, S, HD;
+};
+
+DecodeShape check_qkv(const Tensor& q, const Tensor& k, const Tensor& v) {
+    TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && v.dim() == 4, "expected 4-D query, keys and values");
+    const auto qs = q.sizes(), ks = k.sizes();
+    TORCH_CHECK(qs[0] == ks[0] && qs[2] == 1 && qs[3] == ks[3] && ks == v.sizes(), "shape mismatch: query ", qs, ", keys ",
+                ks, ", values ", v.sizes());
+    TORCH_CHECK(stride_at(q, 3) == 1 && stride_at(k, 3) == 1 && stride_at(v, 3) == 1,
+                "the head dimension of query, keys and values must be contiguous");
+    TORCH_CHECK(k.device() == q.device() && v.device() == q.device(), "query, keys and values must be on the same device");
+    return {int(ks[0]), int(qs[1]), int(ks[1]), int(ks[2]), int(ks[3])};
+}
+
+void check_heads(int QH, int KVH, int HD) {
+    if (HD != 64 && HD != 128) check(L3_ERR_HEAD_SIZE, HD);
+    const int R = KVH > 0 && QH % KVH == 0 ? QH / KVH : 0;
+    if (R != 1 && R != 2 && R != 3 && R != 4 && R != 8) check(L3_ERR_HEAD_RATIO, QH, "/", KVH);
+}
+
+// With kv_len the KV length is read from device memory and S only bounds it.
+void decode(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& out, const DecodeShape& s, int num_splits,
+            int flags, const int32_t* kv_len) {
+    const OnDevice on(q);
+    // Outside stream capture the workspace is the one kept for the stream.  Preparing a new one synchronises,
+    // which a capture does not allow, so a call under capture takes a plain buffer from the graph's memory pool
+    // and runs split kernel + combine.
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    TORCH_CHECK(hipStreamIsCapturing(on.stream, &capture) == hipSuccess, "hipStreamIsCapturing failed");
+    const bool capturing = capture != hipStreamCaptureStatusNone;
+    flags = capturing ? flags & ~L3_ATTN_FLAG_WS_COUNTERS : flags | L3_ATTN_FLAG_WS_COUNTERS;
+    const size_t nbytes = lib.l3_attn_decode_workspace_bytes(s.B, s.QH, s.KVH, s.S, s.HD, num_splits, flags);
+    TensorBase own;
+    void* ws = nullptr;
+    if (nbytes > 0 && capturing) {
+        own = at::detail::empty_cuda({int64_t(std::max(nbytes, size_t(256)))}, at::kByte, q.device(), std::nullopt);
+        ws = ptr(own);
+    } else if (nbytes > 0) {
+        ws = ptr(attention_workspace(on, q, nbytes));
+    }
+    const float scale = float(1.0 / std::sqrt(double(s.HD)));
+    const int64_t* qs = q.strides().data();
+    const int64_t* ks = k.strides().data();
+    const int64_t* vs = v.strides().data();
+    const int64_t* os = out.strides().data();
+    const int rc = kv_len ? lib.l3_attn_decode_devlen(ptr(q), ptr(k), ptr(v), ptr(out), ws, nbytes, s.B, s.QH, s.KVH, s.S,
+                                                      s.HD, qs, ks, vs, os, scale, num_splits, flags, kv_len, on.stream)
+                          : lib.l3_attn_decode(ptr(q), ptr(k), ptr(v), ptr(out), ws, nbytes, s.B, s.QH, s.KVH, s.S, s.HD,
+                                               qs, ks, vs, os, scale, num_splits, flags, on.stream);
+    check(rc, "B=", s.B, " QH=", s.QH, " KVH=", s.KVH, " S=", s.S, " HD=", s.HD);
+}
+
+Tensor empty_like_query(const Tensor& q) {
+    if (q.is_non_overlapping_and_dense()) return empty_like_dense(q);
+    Tensor out = at::empty_like(q);
+    return stride_at(out, 3) == 1 ? out : new_empty(q.sizes(), q);
+}
+
+// (query, keys, values, num_splits, flags)
+PyObject* flash_attention_decode(PyObject* const* a) {
+    const Tensor& q = gpu_bf16(a[0], "query");
+    const Tensor& k = gpu_bf16(a[1], "keys");
+    const Tensor& v = gpu_bf16(a[2], "values");
+    const DecodeShape s = check_qkv(q, k, v);
+    check_heads(s.QH, s.KVH, s.HD);
+    TORCH_CHECK(s.B > 0 && s.S > 0, "flash_attention_decode needs at least one sequence and one cached token");
+    Tensor out = empty_like_query(q);
+    decode(q, k, v, out, s, integer(a[3]), integer(a[4]), nullptr);
+    return wrap(std::move(out));
+}
+
+// (query, keys, values, kv_len, num_splits, out or None, flags)
+PyObject* flash_attention_decode_devlen(PyObject* const* a) {
+    const Tensor& q = gpu_bf16(a[0], "query");
+    const Tensor& k = gpu_bf16(a[1], "keys");
+    const Tensor& v = gpu_bf16(a[2], "values");
+    const DecodeShape s = check_qkv(q, k, v);
+    const Tensor& len = tensor(a[3], "kv_len");
+    TORCH_CHECK(len.is_cuda() && len.scalar_type() == at::kInt && len.numel() == 1 && len.device() == q.device(),
+                "kv_len must be a one-element int32 tensor on the query's GPU");
+    Tensor out = a[5] == Py_None ? empty_like_query(q) : tensor(a[5], "out");
+    decode(q, k, v, out, s, integer(a[4]), integer(a[6]), static_cast<const int32_t*>(ptr(len)));
+    return wrap(std::move(out));
+}
+
+// (query, keys, values, flags)
+PyObject* flash_attention_prefill(PyObject* const* a) {
+    const Tensor& q = gpu_bf16(a[0], "query");
+    const Tensor& k = gpu_bf16(a[1], "keys");
+    const Tensor& v = gpu_bf16(a[2], "values");
+    TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && k.sizes() == v.sizes(),
+                "flash_attention_prefill expects 4-D query, keys and values (keys and values alike)");
+    const auto qs = q.sizes(), ks = k.sizes();
+    const int64_t B = qs[0], QH = qs[1], T = qs[2], HD = qs[3], KVH = ks[1], S = ks[2];
+    TORCH_CHECK(ks[0] == B && ks[3] == HD && T <= S, "shape mismatch: query ", qs, ", keys ", ks);
+    TORCH_CHECK(stride_at(q, 3) == 1 && stride_at(k, 3) == 1 && stride_at(v, 3) == 1,
+                "the head dimension of query, keys and values must be contiguous");
+    check_heads(int(QH), int(KVH), int(HD));
+    // a (B, QH, T, HD) view of a contiguous (B, T, QH, HD) tensor
+    const int64_t sizes[4] = {B, QH, T, HD}, strides[4] = {T * QH * HD, HD, QH * HD, 1};
+    Tensor out(at::detail::empty_strided_cuda(sizes, strides, at::kBFloat16, q.device()));
+    if (out.numel() > 0) {
+        const OnDevice on(q);
+        const int rc = lib.l3_attn_prefill(ptr(q), ptr(k), ptr(v), ptr(out), int(B), int(QH), int(KVH), int(T), int(S), int(HD),
+                                           q.strides().data(), k.strides().data(), v.strides().data(), strides,
+                                           float(1.0 / std::sqrt(double(HD))), integer(a[3]), on.stream);
+        check(rc, "B=", B, " QH=", QH, " KVH=", KVH, " T=", T, " S=", S, " HD=", HD);
+    }
+    return wrap(std::move(out));
+}
+
+// ------------------------------------------------------------------------------------ row-wise operators
+
+// (input, weight, eps)
+PyObject* rms_norm(PyObject* const* a) {
+    const Tensor& input = gpu_bf16(a[0], "input");
+    const Tensor& weight = gpu_bf16(a[1], "weight");
+    TORCH_CHECK(input.dim() == 3, "rms_norm expects a 3-D (B, T, C) input");
+    const int64_t C = size_at(input, 2);
+    TORCH_CHECK(weight.numel() == C, "weight has ", weight.numel(), " elements, expected ", C);
+    Tensor xc, wc;
+    const Tensor& x = contiguous(input, xc);
+    const Tensor& w = contiguous(weight, wc);
+    Tensor out = empty_like_dense(x);
+    const int64_t rows = size_at(x, 0) * size_at(x, 1);
+    if (rows > 0) {
+        const OnDevice on(x);
+        check(lib.l3_rms_norm(ptr(x), ptr(w), ptr(out), rows, int(C), float(number(a[2])), on.stream), "rows=", rows, " C=", C);
+    }
+    return wrap(std::move(out));
+}
+
+// (input, residual, weight, eps)
+PyObject* add_rms_norm(PyObject* const* a) {
+    const Tensor& input = gpu_bf16(a[0], "input");
+    const Tensor& residual = gpu_bf16(a[1], "residual");
+    const Tensor& weight = gpu_bf16(a[2], "weight");
+    TORCH_CHECK(input.dim() == 3 && residual.sizes() == input.sizes(),
+                "add_rms_norm expects two (B, T, C) tensors of the same shape");
+    const int64_t C = size_at(input, 2);
+    TORCH_CHECK(weight.numel() == C, "weight has ", weight.numel(), " elements, expected ", C);
+    Tensor xc, rc_, wc;
+    const Tensor& x = contiguous(input, xc);
+    const Tensor& r = contiguous(residual, rc_);
+    const Tensor& w = contiguous(weight, wc);
+    Tensor s = new_empty(x.sizes(), x), y = new_empty(x.sizes(), x);
+    const int64_t rows = size_at(x, 0) * size_at(x, 1);
+    if (rows > 0) {
+        const OnDevice on(x);
+        check(lib.l3_add_rms_norm(ptr(x), ptr(r), ptr(w), ptr(s), ptr(y), rows, int(C), float(number(a[3])), on.stream), "rows=",
+              rows, " C=", C);
+    }
+    return wrap_pair(std::move(s), std::move(y));
+}
+
+const Tensor& partials(PyObject* o, const char* what) {
+    const Tensor& part = tensor(o, "part");
+    TORCH_CHECK(part.is_cuda() && part.scalar_type() == at::kFloat && part.dim() == 3 && part.is_contiguous(), what,
+                ": expected contiguous float32 (ksplit, rows, N) partials");
+    return part;
+}
+
+// (input, part, weight, eps)
+PyObject* add_rms_norm_partials(PyObject* const* a) {
+    const Tensor& input = gpu_bf16(a[0], "input");
+    const Tensor& weight = gpu_bf16(a[2], "weight");
+    const Tensor& part = partials(a[1], "add_rms_norm_partials");
+    const int64_t C = input.dim() > 0 ? input.sizes().back() : 0;
+    const int64_t rows = C > 0 ? input.numel() / C : 0;
+    TORCH_CHECK(size_at(part, 1) == rows && size_at(part, 2) == C, "add_rms_norm_partials: partials ", part.sizes(),
+                " do not fit input ", input.sizes());
+    TORCH_CHECK(weight.numel() == C && weight.is_contiguous(), "weight has ", weight.numel(), " elements, expected ", C);
+    Tensor xc;
+    const Tensor& x = contiguous(input, xc);
+    Tensor s = new_empty(x.sizes(), x), y = new_empty(x.sizes(), x);
+    const OnDevice on(x);
+    check(lib.l3_add_rms_norm_partials(ptr(x), ptr(part), int(size_at(part, 0)), ptr(weight), ptr(s), ptr(y), int(rows), int(C),
+                                       float(number(a[3])), on.stream),
+          "rows=", rows, " C=", C, " ksplit=", size_at(part, 0));
+    return wrap_pair(std::move(s), std::move(y));
+}
+
+// (a, b)
+PyObject* silu_mul(PyObject* const* args) {
+    const Tensor& a = gpu_bf16(args[0], "a");
+    const Tensor& b = gpu_bf16(args[1], "b");
+    TORCH_CHECK(a.sizes() == b.sizes(), "silu_mul: shapes differ: ", a.sizes(), " vs ", b.sizes());
+    Tensor y = new_empty(a.sizes(), a);
+    if (a.numel() == 0) return wrap(std::move(y));
+    const OnDevice on(a);
+    if (a.is_contiguous() && b.is_contiguous()) {
+        check(lib.l3_silu_mul(ptr(a), ptr(b), ptr(y), y.numel(), on.stream), "n=", y.numel());
+        return wrap(std::move(y));
+    }
+    const int64_t C = a.sizes().back(), rows = a.numel() / C;
+    if (C % 8 == 0 && a.strides().back() == 1 && b.strides().back() == 1) {
+        // rows with a stride (the two halves of a fused gate|up projection): no copies where the leading
+        // dimensions fold into one
+        const Tensor a2 = a.reshape({rows, C}), b2 = b.reshape({rows, C});
+        const auto row_ok = [](const Tensor& t2, const Tensor& t) {
+            return stride_at(t2, 1) == 1 && reinterpret_cast<uintptr_t>(ptr(t2)) % 16 == 0 && stride_at(t2, 0) % 8 == 0 &&
+                   ptr(t2) == ptr(t);
+        };
+        if (row_ok(a2, a) && row_ok(b2, b)) {
+            check(lib.l3_silu_mul_rows(ptr(a2), ptr(b2), ptr(y), rows, C, std::max(stride_at(a2, 0), C),
+                                       std::max(stride_at(b2, 0), C), on.stream),
+                  "rows=", rows, " cols=", C);
+            return wrap(std::move(y));
+        }
+    }
+    const Tensor ac = a.contiguous(), bc = b.contiguous();
+    check(lib.l3_silu_mul(ptr(ac), ptr(bc), ptr(y), y.numel(), on.stream), "n=", y.numel());
+    return wrap(std::move(y));
+}
+
+// (input, freq)
+PyObject* rot_embed(PyObject* const* a) {
+    const Tensor& x = gpu_bf16(a[0], "input");
+    const Tensor& freq = tensor(a[1], "freq");
+    TORCH_CHECK(freq.is_cuda() && freq.scalar_type() == at::kFloat, "expected a GPU float32 freq table but found ",
+                freq.scalar_type(), " on ", freq.device());
+    TORCH_CHECK(x.dim() == 4 && freq.dim() == 2, "rot_embed expects a 4-D (B, T, NH, HD) input and a 2-D (T, HD) freq table");
+    const auto xs = x.sizes();
+    TORCH_CHECK(size_at(freq, 0) == xs[1] && size_at(freq, 1) == xs[3], "freq is ", freq.sizes(), ", expected (", xs[1], ", ",
+                xs[3], ")");
+    TORCH_CHECK(stride_at(x, 3) == 1, "the head dimension of input must be contiguous");
+    Tensor fc;
+    const Tensor& f = contiguous(freq, fc);
+    Tensor out = new_empty(xs, x);
+    if (out.numel() > 0) {
+        const OnDevice on(x);
+        check(lib.l3_rot_embed(ptr(x), static_cast<const float*>(ptr(f)), ptr(out), int(xs[0]), int(xs[1]), int(xs[2]), int(xs[3]),
+                               x.strides().data(), on.stream),
+              "B=", xs[0], " T=", xs[1], " NH=", xs[2], " HD=", xs[3], " strides=", x.strides());
+    }
+    return wrap(std::move(out));
+}
+
+// ---------------------------------------------------------------------------------------------- linears
+
+// The activations of a linear as rows with a stride, and what is common to its argument checks.
+struct Rows {
+    const void* x;
+    int64_t stride, K, rows;
+    Tensor copy;   // keeps a rearranged copy alive
+};
+
+Rows linear_rows(const Tensor& x, int max_rows) {
+    Rows r;
+    r.K = x.dim() > 0 ? x.sizes().back() : 0;
+    r.rows = r.K > 0 ? x.numel() / r.K : 0;
+    TORCH_CHECK(r.rows >= 1 && r.rows <= max_rows, "linear_decode: 1..", max_rows, " activation rows expected, got ", x.sizes());
+    if (x.dim() == 2 && stride_at(x, 1) == 1) {
+        r.x = ptr(x);   // rows as they are (any row stride)
+        r.stride = stride_at(x, 0);
+    } else if (x.is_contiguous()) {
+        r.x = ptr(x);
+        r.stride = r.K;
+    } else {
+        r.copy = x.reshape({r.rows, r.K});
+        if (stride_at(r.copy, 1) != 1) r.copy = r.copy.contiguous();
+        r.x = ptr(r.copy);
+        r.stride = stride_at(r.copy, 0);
+    }
+    return r;
+}
+
+void check_weight(const Tensor& w, const Tensor& like, const Tensor& x, int64_t K) {
+    TORCH_CHECK(w.dim() == 2 && size_at(w, 1) == K && stride_at(w, 1) == 1 && size_at(w, 0) == size_at(like, 0) &&
+                    stride_at(w, 0) == stride_at(like, 0),
+                "linear_decode: weight ", w.sizes(), " does not fit x ", x.sizes());
+}
+
+// (How many rows of that width the fused norm takes, the library checks.)
+void check_norm_weight(const Tensor& norm, int64_t K, const char* what) {
+    TORCH_CHECK(norm.dim() == 1 && norm.numel() == K && norm.is_contiguous(), what, ": norm_weight ", norm.sizes(),
+                " does not fit K=", K);
+}
+
+// A contiguous output of x's leading shape with N columns.
+Tensor rows_out(const Tensor& x, int64_t N) {
+    c10::SmallVector<int64_t, 5> sizes(x.sizes().begin(), x.sizes().end());
+    sizes.back() = N;
+    return new_empty(sizes, x);
+}
+
+// 17..64 activation rows: the split-K kernel plus its finishing pass (one launch serves up to 16).
+bool use_splitk(const Tensor& x, const Tensor& w) {
+    const int64_t K = x.dim() > 0 ? x.sizes().back() : 0;
+    if (K <= 0 || w.dim() != 2 || !x.is_cuda()) return false;
+    const int64_t rows = x.numel() / K;
+    return rows > L3_LINEAR_MAX_ROWS && rows <= L3_LINEAR_SPLITK_MAX_ROWS;
+}
+
+// Float32 partial products (ksplit, rows, N); ksplit 0 = the library's choice.
+Tensor splitk(const Tensor& x, const Tensor& w, int ksplit) {
+    const Rows r = linear_rows(x, L3_LINEAR_SPLITK_MAX_ROWS);
+    check_weight(w, w, x, r.K);
+    const int64_t N = size_at(w, 0);
+    const OnDevice on(x);
+    if (ksplit <= 0) {
+        ksplit = lib.l3_linear_splitk_plan(int(N), int(r.K), 0);
+        check(ksplit, "N=", N, " K=", r.K);
+    }
+    Tensor part = new_empty({ksplit, r.rows, N}, x, at::kFloat);
+    check(lib.l3_linear_splitk(r.x, ptr(w), ptr(part), size_t(part.numel()) * 4, int(r.rows), int(N), int(r.K), r.stride,
+                               stride_at(w, 0), ksplit, on.stream),
+          "M=", r.rows, " N=", N, " K=", r.K, " ksplit=", ksplit);
+    return part;
+}
+
+const void* residual_rows(const Tensor* residual, int64_t rows, int64_t N, Tensor& copy, const char* what) {
+    if (!residual) return nullptr;
+    TORCH_CHECK(residual->numel() == rows * N && residual->dim() > 0 && residual->sizes().back() == N, what, ": residual ",
+                residual->sizes(), " does not fit (", rows, ", ", N, ")");
+    return ptr(contiguous(*residual, copy));
+}
+
+// bf16(sum of the partials) (+ residual) into y, contiguous with rows x N elements.
+void splitk_finish(const Tensor& part, const Tensor* residual, const Tensor& y) {
+    const int64_t rows = size_at(part, 1), N = size_at(part, 2);
+    Tensor copy;
+    const void* r = residual_rows(residual, rows, N, copy, "linear_splitk_finish");
+    const OnDevice on(part);
+    check(lib.l3_linear_splitk_finish(ptr(part), int(size_at(part, 0)), r, ptr(y), int(rows), int(N), N, on.stream), "rows=", rows,
+          " N=", N, " ksplit=", size_at(part, 0));
+}
+
+// (x, weight)
+PyObject* linear_decode(PyObject* const* a) {
+    const Tensor& x = gpu_bf16(a[0], "x");
+    const Tensor& w = gpu_bf16(a[1], "weight");
+    if (use_splitk(x, w)) {
+        const Tensor part = splitk(x, w, 0);
+        Tensor y = rows_out(x, size_at(w, 0));
+        splitk_finish(part, nullptr, y);
+        return wrap(std::move(y));
+    }
+    const Rows r = linear_rows(x, L3_LINEAR_MAX_ROWS);
+    check_weight(w, w, x, r.K);
+    const int64_t N = size_at(w, 0);
+    Tensor y = rows_out(x, N);
+    const OnDevice on(x);
+    check(lib.l3_linear_decode(r.x, ptr(w), ptr(y), int(r.rows), int(N), int(r.K), r.stride, stride_at(w, 0), N, on.stream), "M=",
+          r.rows, " N=", N, " K=", r.K);
+    return wrap(std::move(y));
+}
+
+// (x, w_gate, w_up)
+PyObject* linear_swiglu_decode(PyObject* const* a) {
+    const Tensor& x = gpu_bf16(a[0], "x");
+    const Tensor& wg = gpu_bf16(a[1], "weight");
+    const Tensor& wu = gpu_bf16(a[2], "weight");
+    const Rows r = linear_rows(x, L3_LINEAR_MAX_ROWS);
+    check_weight(wg, wg, x, r.K);
+    check_weight(wu, wg, x, r.K);
+    const int64_t N = size_at(wg, 0);
+    Tensor y = rows_out(x, N);
+    const OnDevice on(x);
+    check(lib.l3_linear_swiglu_decode(r.x, ptr(wg), ptr(wu), ptr(y), int(r.rows), int(N), int(r.K), r.stride, stride_at(wg, 0), N,
+                                      on.stream),
+          "M=", r.rows, " N=", N, " K=", r.K);
+    return wrap(std::move(y));
+}
+
+// (x, weight, norm_weight or None, eps, w_up or None, residual or None)
+PyObject* linear_decode_fused(PyObject* const* a) {
+    const Tensor& x = gpu_bf16(a[0], "x");
+    const Tensor& w = gpu_bf16(a[1], "weight");
+    const Tensor* norm = optional_tensor(a[2], "norm_weight");
+    const Tensor* up = optional_tensor(a[4], "weight");
+    const Tensor* residual = optional_tensor(a[5], "residual");
+    if (!norm && !up && use_splitk(x, w)) {
+        // the residual joins when the splits are added up
+        const Tensor part = splitk(x, w, 0);
+        Tensor y = rows_out(x, size_at(w, 0));
+        splitk_finish(part, residual, y);
+        return wrap(std::move(y));
+    }
+    const Rows r = linear_rows(x, L3_LINEAR_MAX_ROWS);
+    check_weight(w, w, x, r.K);
+    if (up) check_weight(*up, w, x, r.K);
+    const int64_t N = size_at(w, 0);
+    if (norm) check_norm_weight(*norm, r.K, "linear_decode_fused");
+    Tensor copy;
+    const void* res = residual_rows(residual, r.rows, N, copy, "linear_decode_fused");
+    Tensor y = rows_out(x, N);
+    const OnDevice on(x);
+    check(lib.l3_linear_decode_fused(r.x, norm ? ptr(*norm) : nullptr, float(number(a[3])), ptr(w), up ? ptr(*up) : nullptr, res,
+                                     ptr(y), int(r.rows), int(N), int(r.K), r.stride, stride_at(w, 0), N, on.stream),
+          "M=", r.rows, " N=", N, " K=", r.K);
+    return wrap(std::move(y));
+}
+
+// (x, weight, ksplit)
+PyObject* linear_splitk(PyObject* const* a) {
+    return wrap(splitk(gpu_bf16(a[0], "x"), gpu_bf16(a[1], "weight"), integer(a[2])));
+}
+
+// (part, residual or None)
+PyObject* linear_splitk_finish(PyObject* const* a) {
+    const Tensor& part = partials(a[0], "linear_splitk_finish");
+    Tensor y = new_empty({size_at(part, 1), size_at(part, 2)}, part);
+    splitk_finish(part, optional_tensor(a[1], "residual"), y);
+    return wrap(std::move(y));
+}
+
+// Rotary table, position and cache of the operators that append to the KV cache.
+struct Cache {
+    const Tensor *k, *v, *table, *pos;
+    int64_t maxB, L, KVH, HD;
+};
+
+Cache cache_args(PyObject* table, PyObject* cache_k, PyObject* cache_v, PyObject* pos) {
+    Cache c{&gpu_bf16(cache_k, "cache_k"), &gpu_bf16(cache_v, "cache_v"), &tensor(table, "freq_table"), &tensor(pos, "pos"),
+            0, 0, 0, 0};
+    TORCH_CHECK(c.k->dim() == 4 && c.k->sizes() == c.v->sizes() && c.k->strides() == c.v->strides(),
+                "cache_k and cache_v must be (maxB, L, KVH, HD) tensors of the same layout");
+    const auto s = c.k->sizes();
+    c.maxB = s[0], c.L = s[1], c.KVH = s[2], c.HD = s[3];
+    TORCH_CHECK(stride_at(*c.k, 3) == 1 && stride_at(*c.k, 2) == c.HD, "the (KVH, HD) dimensions of the cache must be contiguous");
+    TORCH_CHECK(c.table->is_cuda() && c.table->scalar_type() == at::kFloat && c.table->dim() == 2 &&
+                    size_at(*c.table, 1) == c.HD && c.table->is_contiguous(),
+                "freq_table must be a contiguous (rows, HD) float32 GPU tensor");
+    TORCH_CHECK(c.pos->is_cuda() && c.pos->scalar_type() == at::kInt && c.pos->numel() == 1,
+                "pos must be a one-element int32 GPU tensor");
+    return c;
+}
+
+// (x, w_qkv, freq_table, cache_k, cache_v, pos, n_head, norm_weight or None, eps)
+PyObject* linear_qkv_rope_append(PyObject* const* a) {
+    const Tensor& x = gpu_bf16(a[0], "x");
+    const Tensor& w = gpu_bf16(a[1], "weight");
+    const Rows r = linear_rows(x, L3_LINEAR_MAX_ROWS);
+    check_weight(w, w, x, r.K);
+    const Cache c = cache_args(a[2], a[3], a[4], a[5]);
+    const int64_t NH = integer(a[6]);
+    TORCH_CHECK(size_at(w, 0) == (NH + 2 * c.KVH) * c.HD && r.rows <= c.maxB, "w_qkv ", w.sizes(), " does not match n_head=", NH,
+                ", cache ", c.k->sizes());
+    const Tensor* norm = optional_tensor(a[7], "norm_weight");
+    if (norm) check_norm_weight(*norm, r.K, "linear_qkv_rope_append");
+    Tensor out = new_empty({r.rows, 1, NH, c.HD}, x);
+    const OnDevice on(x);
+    check(lib.l3_linear_qkv_rope_append(r.x, norm ? ptr(*norm) : nullptr, float(number(a[8])), ptr(w),
+                                        static_cast<const float*>(ptr(*c.table)), ptr(out), ptr(*c.k), ptr(*c.v),
+                                        static_cast<const int32_t*>(ptr(*c.pos)), int(r.rows), int(NH), int(c.KVH), int(c.HD),
+                                        int(r.K), r.stride, stride_at(w, 0), c.k->strides().data(), int(c.L),
+                                        int(size_at(*c.table, 0)), on.stream),
+          "B=", r.rows, " NH=", NH, " KVH=", c.KVH, " HD=", c.HD, " K=", r.K);
+    return wrap(std::move(out));
+}
+
+// (part, freq_table, cache_k, cache_v, pos, n_head)
+PyObject* rot_embed_append_partials(PyObject* const* a) {
+    const Tensor& part = partials(a[0], "rot_embed_append_partials");
+    const Cache c = cache_args(a[1], a[2], a[3], a[4]);
+    const int64_t NH = integer(a[5]), ksplit = size_at(part, 0), B = size_at(part, 1);
+    TORCH_CHECK(size_at(part, 2) == (NH + 2 * c.KVH) * c.HD && B <= c.maxB, "partials ", part.sizes(), " do not match n_head=", NH,
+                ", cache ", c.k->sizes());
+    Tensor out = new_empty({B, 1, NH, c.HD}, part);
+    const OnDevice on(part);
+    check(lib.l3_rot_embed_append_partials(static_cast<const float*>(ptr(part)), int(ksplit),
+                                           static_cast<const float*>(ptr(*c.table)), ptr(out), ptr(*c.k), ptr(*c.v),
+                                           static_cast<const int32_t*>(ptr(*c.pos)), int(B), int(NH), int(c.KVH), int(c.HD),
+                                           c.k->strides().data(), int(c.L), int(size_at(*c.table, 0)), on.stream),
+          "B=", B, " NH=", NH, " KVH=", c.KVH, " HD=", c.HD, " ksplit=", ksplit);
+    return wrap(std::move(out));
+}
+
+// --------------------------------------------------------------------------------------------- the module
+
+template <PyObject* (*F)(PyObject* const*), int N>
+PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    if (n != N) {
+        PyErr_Format(PyExc_TypeError, "%d arguments expected, got %zd", N, n);
+        return nullptr;
+    }
+    if (!lib.l3_strerror) {
+        PyErr_SetString(PyExc_RuntimeError, "bind() has not been called");
+        return nullptr;
+    }
+    try {
+        return F(args);
+    } catch (python_error& e) {
+        e.restore();
+    } catch (...) {
+        torch::translate_exception_to_python(std::current_exception());
+    }
+    return nullptr;
+}
+
+// bind(path): looks the library's functions up; the Python side has loaded it from the same path.
+PyObject* bind(PyObject*, PyObject* arg) {
+    const char* path = PyUnicode_AsUTF8(arg);
+    if (!path) return nullptr;
+    void* handle = dlopen(path, RTLD_NOW | RTLD_LOCAL);
+    if (!handle) {
+        PyErr_Format(PyExc_ImportError, "%s: %s", path, dlerror());
+        return nullptr;
+    }
+    Library found;
+#define X(name)                                                                       \
+    if (!(found.name = reinterpret_cast<decltype(found.name)>(dlsym(handle, #name)))) { \
+        PyErr_Format(PyExc_ImportError, "%s has no " #name, path);                    \
+        return nullptr;                                                               \
+    }
+    L3_FUNCTIONS(X)
+#undef X
+    lib = found;
+    Py_RETURN_NONE;
+}
+
+#define ENTRY(name, n) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<name, n>)), METH_FASTCALL, nullptr}
+
+PyMethodDef methods[] = {
+    {"bind", bind, METH_O, nullptr},
+    ENTRY(flash_attention_decode, 5),
+    ENTRY(flash_attention_decode_devlen, 7),
+    ENTRY(flash_attention_prefill, 4),
+    ENTRY(rms_norm, 3),
+    ENTRY(add_rms_norm, 4),
+    ENTRY(add_rms_norm_partials, 4),
+    ENTRY(silu_mul, 2),
+    ENTRY(rot_embed, 2),
+    ENTRY(linear_decode, 2),
+    ENTRY(linear_swiglu_decode, 3),
+    ENTRY(linear_decode_fused, 6),
+    ENTRY(linear_splitk, 3),
+    ENTRY(linear_splitk_finish, 2),
+    ENTRY(linear_qkv_rope_append, 9),
+    ENTRY(rot_embed_append_partials, 6),
+    {nullptr, nullptr, 0, nullptr},
+};
+
+PyModuleDef definition = {PyModuleDef_HEAD_INIT, "_l3torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__l3torch() { return PyModule_Create(&definition); }

@@ -209,6 +209,25 @@ def load():
     return lib
 
 
+_native = None   # (the ctypes library it is bound to, the extension module)
+
+
+def native():
+    """The extension module that runs the operators on torch tensors (csrc/torch_ops.cpp), bound to the
+    loaded library."""
+    global _native
+    if _native is None or _native[0] is not _lib:
+        lib = load()
+        try:
+            from . import _l3torch
+        except ImportError as e:
+            raise ImportError(f"{e}: build it with `python llama3-custom-inference_amd/build.py`. "
+                              "There is no fallback implementation.") from e
+        _l3torch.bind(library_path())
+        _native = (lib, _l3torch)
+    return _native[1]
+
+
 def strerror(code: int) -> str:
     return load().l3_strerror(int(code)).decode()
 

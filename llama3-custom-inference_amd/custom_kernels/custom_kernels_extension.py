@@ -25,7 +25,6 @@ __all__ = ["flash_attention_decode", "rms_norm", "rot_embed", "attention_num_spl
            "flash_attention_split", "flash_attention_combine", "flash_attention_decode_devlen",
            "rot_embed_append", "add_rms_norm", "silu_mul", "argmax", "flash_attention_prefill"]
 
-_cu_count = {}
 _workspaces = {}  # (device index, stream handle) -> uint8 tensor
 
 
@@ -66,18 +65,8 @@ def _on_device(device):
     return torch.cuda.device(idx)
 
 
-def _cus(device) -> int:
-    idx = device.index if device.index is not None else torch.cuda.current_device()
-    n = _cu_count.get(idx)
-    if n is None:
-        n = torch.cuda.get_device_properties(idx).multi_processor_count
-        _cu_count[idx] = n
-    return n
-
-
 def _workspace(device, stream_ptr: int, nbytes: int):
-    """Scratch for the kernels that need it (attention partials, argmax partials), kept per
-    (device, stream) and grown on demand so that a decode step does not allocate.  Calls on one
+    """Scratch for the argmax partials, kept per (device, stream) and grown on demand so that a decode step does not allocate.  Calls on one
     stream are ordered and can share it; another stream gets its own.  While a stream is being
     captured into a HIP graph the buffer comes from the graph's own memory pool instead (a plain
     allocation that lives and dies with the graph) and is not cached."""
@@ -89,34 +78,6 @@ def _workspace(device, stream_ptr: int, nbytes: int):
         ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
         _workspaces[key] = ws
     return ws
-
-
-_attn_workspaces = {}  # (device index, stream handle) -> uint8 tensor that starts with prepared arrival counters
-
-
-def _attn_workspace(lib, device, stream_ptr: int, flags: int, size_of):
-    """Workspace and flags for a decode-attention call.  Outside stream capture the workspace is one kept per
-    (device, stream) whose head holds the arrival counters of the single-launch form, prepared once by
-    l3_attn_workspace_init when the buffer is (re)allocated -- that call synchronises, which a capture
-    would not allow, so a call under capture takes a plain buffer from the graph's pool and runs split
-    kernel + combine.  ``size_of(flags)`` returns the bytes the call needs with those flags."""
-    if torch.cuda.is_current_stream_capturing():
-        flags &= ~_l3lib.L3_ATTN_FLAG_WS_COUNTERS
-        nbytes = size_of(flags)
-        return (_workspace(device, stream_ptr, nbytes) if nbytes else None), nbytes, flags
-    flags |= _l3lib.L3_ATTN_FLAG_WS_COUNTERS
-    nbytes = size_of(flags)
-    if nbytes == 0:
-        return None, 0, flags
-    key = (device.index if device.index is not None else torch.cuda.current_device(), stream_ptr)
-    ws = _attn_workspaces.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(max(nbytes, 4 << 20), dtype=torch.uint8, device=device)
-        rc = lib.l3_attn_workspace_init(ws.data_ptr(), ws.numel(), stream_ptr)
-        if rc != 0:
-            _fail(rc, "l3_attn_workspace_init")
-        _attn_workspaces[key] = ws
-    return ws, nbytes, flags
 
 
 # Flags the attention operators pass to the library when the caller gives none: a context-local
@@ -179,40 +140,7 @@ def flash_attention_decode(query, keys, values, num_splits: int = 0, flags=None)
     context, normally 0) are extensions for tests and sweeps; the reference signature is the three
     tensors.
     """
-    lib = _l3lib.load()
-    flags = _flags(flags)
-    B, QH, KVH, S, HD = _check_qkv(query, keys, values)
-    if keys.device != query.device or values.device != query.device:
-        raise RuntimeError("query, keys and values must be on the same device")
-    if HD not in (64, 128):
-        _fail(_l3lib.L3_ERR_HEAD_SIZE, str(HD))
-    if KVH == 0 or QH % KVH != 0 or (QH // KVH) not in (1, 2, 3, 4, 8):
-        _fail(_l3lib.L3_ERR_HEAD_RATIO, f"{QH}/{KVH}")
-
-    out = torch.empty_like(query)
-    if out.stride(3) != 1:
-        out = torch.empty(query.shape, dtype=query.dtype, device=query.device)
-    if B == 0 or S == 0:
-        raise RuntimeError("flash_attention_decode needs at least one sequence and one cached token")
-
-    with _on_device(query.device):
-        # num_splits == 0 lets the library plan for the current device (split count and kernel form)
-        stream_ptr = _stream_ptr(query.device)
-        ws, ws_bytes, flags = _attn_workspace(
-            lib, query.device, stream_ptr, flags,
-            lambda f: lib.l3_attn_decode_workspace_bytes(B, QH, KVH, S, HD, num_splits, f))
-        rc = lib.l3_attn_decode(
-            query.data_ptr(), keys.data_ptr(), values.data_ptr(), out.data_ptr(),
-            ws.data_ptr() if ws is not None else None, ws_bytes,
-            B, QH, KVH, S, HD,
-            _l3lib.i64_array((query.stride(0), query.stride(1))),
-            _l3lib.i64_array((keys.stride(0), keys.stride(1), keys.stride(2))),
-            _l3lib.i64_array((values.stride(0), values.stride(1), values.stride(2))),
-            _l3lib.i64_array((out.stride(0), out.stride(1))),
-            1.0 / math.sqrt(HD), num_splits, flags, stream_ptr)
-    if rc != 0:
-        _fail(rc, f"B={B} QH={QH} KVH={KVH} S={S} HD={HD}")
-    return out
+    return _l3lib.native().flash_attention_decode(query, keys, values, num_splits, _flags(flags))
 
 
 def flash_attention_decode_static(query, keys, values, out, num_splits: int = 0, flags=None):
@@ -260,36 +188,7 @@ def flash_attention_prefill(query, keys, values, flags=None):
     (B, QH, T, HD) view of a contiguous (B, T, QH, HD) tensor, so the model's
     ``y.transpose(1, 2).contiguous()`` (model.py:120) is free.  For S == T it computes what the
     reference asks of torch for this case (model.py:114-116).  An extension of the operator set."""
-    lib = _l3lib.load()
-    _require_gpu_bf16("query", query)
-    _require_gpu_bf16("keys", keys)
-    _require_gpu_bf16("values", values)
-    if query.dim() != 4 or keys.dim() != 4 or tuple(values.shape) != tuple(keys.shape):
-        raise RuntimeError("flash_attention_prefill expects 4-D query, keys and values (keys and values alike)")
-    B, QH, T, HD = query.shape
-    Bk, KVH, S, HDk = keys.shape
-    if Bk != B or HDk != HD or T > S:
-        raise RuntimeError(f"shape mismatch: query {tuple(query.shape)}, keys {tuple(keys.shape)}")
-    if query.stride(3) != 1 or keys.stride(3) != 1 or values.stride(3) != 1:
-        raise RuntimeError("the head dimension of query, keys and values must be contiguous")
-    if HD not in (64, 128):
-        _fail(_l3lib.L3_ERR_HEAD_SIZE, str(HD))
-    if KVH == 0 or QH % KVH != 0 or (QH // KVH) not in (1, 2, 3, 4, 8):
-        _fail(_l3lib.L3_ERR_HEAD_RATIO, f"{QH}/{KVH}")
-    out = torch.empty((B, T, QH, HD), dtype=query.dtype, device=query.device).transpose(1, 2)
-    if out.numel() == 0:
-        return out
-    with _on_device(query.device):
-        rc = lib.l3_attn_prefill(
-            query.data_ptr(), keys.data_ptr(), values.data_ptr(), out.data_ptr(), B, QH, KVH, T, S, HD,
-            _l3lib.i64_array((query.stride(0), query.stride(1), query.stride(2))),
-            _l3lib.i64_array((keys.stride(0), keys.stride(1), keys.stride(2))),
-            _l3lib.i64_array((values.stride(0), values.stride(1), values.stride(2))),
-            _l3lib.i64_array((out.stride(0), out.stride(1), out.stride(2))),
-            1.0 / math.sqrt(HD), _flags(flags), _stream_ptr(query.device))
-    if rc != 0:
-        _fail(rc, f"B={B} QH={QH} KVH={KVH} T={T} S={S} HD={HD}")
-    return out
+    return _l3lib.native().flash_attention_prefill(query, keys, values, _flags(flags))
 
 
 def flash_attention_split(query, keys, values, num_splits: int = 0, flags=None):
@@ -349,33 +248,9 @@ def flash_attention_decode_devlen(query, keys, values, kv_len, num_splits: int =
     captured once in a HIP graph and replayed while the cache grows (an extension; the reference
     takes the length from keys.size(2), custom_kernels.cu:246).  ``out`` may be supplied to keep
     the call allocation-free under capture."""
-    lib = _l3lib.load()
-    flags = _flags(flags)
-    B, QH, KVH, L, HD = _check_qkv(query, keys, values)
-    if keys.device != query.device or values.device != query.device:
-        raise RuntimeError("query, keys and values must be on the same device")
-    if not kv_len.is_cuda or kv_len.dtype != torch.int32 or kv_len.numel() != 1 or kv_len.device != query.device:
-        raise RuntimeError("kv_len must be a one-element int32 tensor on the query's GPU")
-    if out is None:
-        out = torch.empty_like(query)
-    else:
+    if out is not None:
         _check_out(out, query, "flash_attention_decode_devlen")
-    with _on_device(query.device):
-        stream_ptr = _stream_ptr(query.device)
-        ws, ws_bytes, flags = _attn_workspace(
-            lib, query.device, stream_ptr, flags,
-            lambda f: lib.l3_attn_decode_workspace_bytes(B, QH, KVH, L, HD, num_splits, f))
-        rc = lib.l3_attn_decode_devlen(
-            query.data_ptr(), keys.data_ptr(), values.data_ptr(), out.data_ptr(),
-            ws.data_ptr() if ws is not None else None, ws_bytes, B, QH, KVH, L, HD,
-            _l3lib.i64_array((query.stride(0), query.stride(1))),
-            _l3lib.i64_array((keys.stride(0), keys.stride(1), keys.stride(2))),
-            _l3lib.i64_array((values.stride(0), values.stride(1), values.stride(2))),
-            _l3lib.i64_array((out.stride(0), out.stride(1))),
-            1.0 / math.sqrt(HD), num_splits, flags, kv_len.data_ptr(), stream_ptr)
-    if rc != 0:
-        _fail(rc, f"B={B} QH={QH} KVH={KVH} L={L} HD={HD}")
-    return out
+    return _l3lib.native().flash_attention_decode_devlen(query, keys, values, kv_len, num_splits, out, _flags(flags))
 
 
 def rot_embed_append(qkv, freq_table, cache_k, cache_v, pos, n_head: int, out=None):
@@ -427,63 +302,12 @@ def linear_qkv_rope_append(x, w_qkv, freq_table, cache_k, cache_v, pos, n_head: 
     """linear_decode_fused(x, w_qkv, norm_weight) followed by rot_embed_append in one launch: the
     whole of model.py:95-106 for one new token per sequence.  x (B, 1, K); returns the rotated
     queries (B, 1, n_head, HD); keys and values are written into the caches at ``pos``."""
-    lib = _l3lib.load()
-    x2, rows, N, K = _linear_args(x, (w_qkv,))
-    _require_gpu_bf16("cache_k", cache_k)
-    _require_gpu_bf16("cache_v", cache_v)
-    if cache_k.dim() != 4 or cache_k.shape != cache_v.shape or cache_k.stride() != cache_v.stride():
-        raise RuntimeError("cache_k and cache_v must be (maxB, L, KVH, HD) tensors of the same layout")
-    maxB, L, KVH, HD = cache_k.shape
-    if N != (n_head + 2 * KVH) * HD or rows > maxB:
-        raise RuntimeError(f"w_qkv {tuple(w_qkv.shape)} does not match n_head={n_head}, cache {tuple(cache_k.shape)}")
-    if cache_k.stride(3) != 1 or cache_k.stride(2) != HD:
-        raise RuntimeError("the (KVH, HD) dimensions of the cache must be contiguous")
-    if not freq_table.is_cuda or freq_table.dtype != torch.float32 or freq_table.dim() != 2 \
-            or freq_table.size(1) != HD or not freq_table.is_contiguous():
-        raise RuntimeError("freq_table must be a contiguous (rows, HD) float32 GPU tensor")
-    if not pos.is_cuda or pos.dtype != torch.int32 or pos.numel() != 1:
-        raise RuntimeError("pos must be a one-element int32 GPU tensor")
-    if norm_weight is not None:
-        _require_gpu_bf16("norm_weight", norm_weight)
-        if tuple(norm_weight.shape) != (K,) or not norm_weight.is_contiguous() \
-                or rows > linear_decode_fused_max_rows(K):
-            raise RuntimeError(f"linear_qkv_rope_append: norm_weight {tuple(norm_weight.shape)} / {rows} rows "
-                               f"do not fit the fused input norm (K={K})")
-    out = torch.empty((rows, 1, n_head, HD), dtype=x.dtype, device=x.device)
-    with _on_device(x.device):
-        rc = lib.l3_linear_qkv_rope_append(x2.data_ptr(), None if norm_weight is None else norm_weight.data_ptr(),
-                                           float(eps), w_qkv.data_ptr(), freq_table.data_ptr(), out.data_ptr(),
-                                           cache_k.data_ptr(), cache_v.data_ptr(), pos.data_ptr(), rows, n_head, KVH,
-                                           HD, K, x2.stride(0), w_qkv.stride(0),
-                                           _l3lib.i64_array((cache_k.stride(0), cache_k.stride(1))), L,
-                                           freq_table.size(0), _stream_ptr(x.device))
-    if rc != 0:
-        _fail(rc, f"B={rows} NH={n_head} KVH={KVH} HD={HD} K={K}")
-    return out
+    return _l3lib.native().linear_qkv_rope_append(x, w_qkv, freq_table, cache_k, cache_v, pos, n_head, norm_weight, eps)
 
 
 def rms_norm(input, weight, eps):
     """input (B, T, C) bf16, weight (C,) bf16 -> (B, T, C) bf16 (model.py:70-72)."""
-    lib = _l3lib.load()
-    _require_gpu_bf16("input", input)
-    _require_gpu_bf16("weight", weight)
-    if input.dim() != 3:
-        raise RuntimeError("rms_norm expects a 3-D (B, T, C) input")
-    C = input.size(2)
-    if weight.numel() != C:
-        raise RuntimeError(f"weight has {weight.numel()} elements, expected {C}")
-    x = input if input.is_contiguous() else input.contiguous()
-    w = weight if weight.is_contiguous() else weight.contiguous()
-    out = torch.empty_like(x)
-    rows = x.size(0) * x.size(1)
-    if rows == 0:
-        return out
-    with _on_device(x.device):
-        rc = lib.l3_rms_norm(x.data_ptr(), w.data_ptr(), out.data_ptr(), rows, C, float(eps),
-                             _stream_ptr(x.device))
-    if rc != 0:
-        _fail(rc, f"rows={rows} C={C}")
-    return out
+    return _l3lib.native().rms_norm(input, weight, eps)
 
 
 def add_rms_norm(input, residual, weight, eps):
@@ -491,105 +315,13 @@ def add_rms_norm(input, residual, weight, eps):
     addition of model.py:147-148 fused with the norm that follows it.  Both outputs carry the same
     bits as ``s = input + residual`` (bf16) followed by ``rms_norm(s, weight, eps)``.  An extension
     of the reference's operator set."""
-    lib = _l3lib.load()
-    _require_gpu_bf16("input", input)
-    _require_gpu_bf16("residual", residual)
-    _require_gpu_bf16("weight", weight)
-    if input.dim() != 3 or tuple(residual.shape) != tuple(input.shape):
-        raise RuntimeError("add_rms_norm expects two (B, T, C) tensors of the same shape")
-    C = input.size(2)
-    if weight.numel() != C:
-        raise RuntimeError(f"weight has {weight.numel()} elements, expected {C}")
-    x = input if input.is_contiguous() else input.contiguous()
-    r = residual if residual.is_contiguous() else residual.contiguous()
-    w = weight if weight.is_contiguous() else weight.contiguous()
-    s = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    y = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    rows = x.size(0) * x.size(1)
-    if rows == 0:
-        return s, y
-    with _on_device(x.device):
-        rc = lib.l3_add_rms_norm(x.data_ptr(), r.data_ptr(), w.data_ptr(), s.data_ptr(), y.data_ptr(), rows, C,
-                                 float(eps), _stream_ptr(x.device))
-    if rc != 0:
-        _fail(rc, f"rows={rows} C={C}")
-    return s, y
+    return _l3lib.native().add_rms_norm(input, residual, weight, eps)
 
 
 def silu_mul(a, b):
     """F.silu(a) * b for two bf16 tensors of the same shape in one launch (model.py:134), with the
     two roundings of the two torch kernels, so the bits are the same.  An extension."""
-    lib = _l3lib.load()
-    _require_gpu_bf16("a", a)
-    _require_gpu_bf16("b", b)
-    if tuple(a.shape) != tuple(b.shape):
-        raise RuntimeError(f"silu_mul: shapes differ: {tuple(a.shape)} vs {tuple(b.shape)}")
-    C = a.shape[-1] if a.dim() else 1
-    rows = a.numel() // max(C, 1)
-    strided = (a.dim() >= 1 and a.numel() > 0 and C % 8 == 0 and a.stride(-1) == 1 and b.stride(-1) == 1
-               and not (a.is_contiguous() and b.is_contiguous()))
-    if strided:
-        # rows with a stride (the two halves of a fused gate|up projection): no copies
-        a2, b2 = a.reshape(rows, C), b.reshape(rows, C)
-        if a2.stride(1) == 1 and b2.stride(1) == 1 and a2.data_ptr() % 16 == 0 and b2.data_ptr() % 16 == 0 \
-                and a2.stride(0) % 8 == 0 and b2.stride(0) % 8 == 0 and a2.data_ptr() == a.data_ptr() \
-                and b2.data_ptr() == b.data_ptr():
-            y = torch.empty(a.shape, dtype=a.dtype, device=a.device)
-            with _on_device(a.device):
-                rc = lib.l3_silu_mul_rows(a2.data_ptr(), b2.data_ptr(), y.data_ptr(), rows, C, max(a2.stride(0), C),
-                                          max(b2.stride(0), C), _stream_ptr(a.device))
-            if rc != 0:
-                _fail(rc, f"rows={rows} cols={C}")
-            return y
-    ac = a if a.is_contiguous() else a.contiguous()
-    bc = b if b.is_contiguous() else b.contiguous()
-    y = torch.empty(ac.shape, dtype=ac.dtype, device=ac.device)
-    if y.numel() == 0:
-        return y
-    with _on_device(ac.device):
-        rc = lib.l3_silu_mul(ac.data_ptr(), bc.data_ptr(), y.data_ptr(), y.numel(), _stream_ptr(ac.device))
-    if rc != 0:
-        _fail(rc, f"n={y.numel()}")
-    return y
-
-
-def _linear_args(x, weights, max_rows=None):
-    _require_gpu_bf16("x", x)
-    K = x.shape[-1]
-    rows = x.numel() // max(K, 1)
-    max_rows = _l3lib.L3_LINEAR_MAX_ROWS if max_rows is None else max_rows
-    if x.dim() < 1 or rows < 1 or rows > max_rows:
-        raise RuntimeError(f"linear_decode: 1..{max_rows} activation rows expected, got {tuple(x.shape)}")
-    w0 = weights[0]
-    for w in weights:
-        _require_gpu_bf16("weight", w)
-        if w.dim() != 2 or w.shape[1] != K or w.stride(1) != 1 or \
-                (w is not w0 and (w.shape[0] != w0.shape[0] or w.stride(0) != w0.stride(0))):
-            raise RuntimeError(f"linear_decode: weight {tuple(w.shape)} does not fit x {tuple(x.shape)}")
-    if x.dim() == 2 and x.stride(1) == 1:
-        x2 = x                          # rows as they are (any row stride)
-    elif x.is_contiguous():
-        x2 = x.view(rows, K)
-    else:
-        x2 = x.reshape(rows, K)
-        if x2.stride(1) != 1:
-            x2 = x2.contiguous()
-    return x2, rows, w0.shape[0], K
-
-
-def _rows_out(x, rows: int, N: int):
-    """A contiguous output of x's leading shape with N columns, (rows, N) to the kernel."""
-    if x.dim() == 2:
-        return x.new_empty((rows, N))
-    return x.new_empty(x.shape[:-1] + (N,))
-
-
-def _use_splitk(x, weight) -> bool:
-    """17..64 activation rows: the split-K kernel plus its finishing pass (one launch serves up to 16)."""
-    K = x.shape[-1]
-    if K <= 0 or weight.dim() != 2 or not x.is_cuda:
-        return False
-    return _l3lib.L3_LINEAR_MAX_ROWS < x.numel() // K <= _l3lib.L3_LINEAR_SPLITK_MAX_ROWS
+    return _l3lib.native().silu_mul(a, b)
 
 
 def linear_decode(x, weight):
@@ -599,31 +331,13 @@ def linear_decode(x, weight):
     linear_splitk and linear_splitk_finish (N % 8 == 0, K % 128 == 0), which suits matrices of a
     few thousand rows -- a vocabulary projection at those batch sizes is a library GEMM's job.
     An extension."""
-    lib = _l3lib.load()
-    if _use_splitk(x, weight):
-        return linear_splitk_finish(linear_splitk(x, weight)).view(*x.shape[:-1], weight.shape[0])
-    x2, rows, N, K = _linear_args(x, (weight,))
-    y = _rows_out(x, rows, N)
-    with _on_device(x.device):
-        rc = lib.l3_linear_decode(x2.data_ptr(), weight.data_ptr(), y.data_ptr(), rows, N, K, x2.stride(0),
-                                  weight.stride(0), N, _stream_ptr(x.device))
-    if rc != 0:
-        _fail(rc, f"M={rows} N={N} K={K}")
-    return y
+    return _l3lib.native().linear_decode(x, weight)
 
 
 def linear_swiglu_decode(x, w_gate, w_up):
     """F.silu(F.linear(x, w_gate)) * F.linear(x, w_up) for at most 16 activation rows in one
     launch (model.py:134 with w_gate = c_fc2, w_up = c_fc), same rounding points.  An extension."""
-    lib = _l3lib.load()
-    x2, rows, N, K = _linear_args(x, (w_gate, w_up))
-    y = _rows_out(x, rows, N)
-    with _on_device(x.device):
-        rc = lib.l3_linear_swiglu_decode(x2.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(), y.data_ptr(), rows, N, K,
-                                         x2.stride(0), w_gate.stride(0), N, _stream_ptr(x.device))
-    if rc != 0:
-        _fail(rc, f"M={rows} N={N} K={K}")
-    return y
+    return _l3lib.native().linear_swiglu_decode(x, w_gate, w_up)
 
 
 def linear_decode_fused_max_rows(K: int) -> int:
@@ -636,33 +350,7 @@ def linear_decode_fused(x, weight, norm_weight=None, eps: float = 1e-5, w_up=Non
     rms_norm(x, norm_weight, eps) in front (model.py:70-72), the SwiGLU product with a second
     matrix w_up (weight is then the gate, model.py:134), and `residual + result` behind
     (model.py:147-148) -- all with the rounding points of the separate operators.  An extension."""
-    lib = _l3lib.load()
-    if norm_weight is None and w_up is None and _use_splitk(x, weight):
-        # 17..64 rows, small matrix: split-K, the residual joins when the splits are added up
-        return linear_splitk_finish(linear_splitk(x, weight), residual).view(*x.shape[:-1], weight.shape[0])
-    x2, rows, N, K = _linear_args(x, (weight,) if w_up is None else (weight, w_up))
-    if norm_weight is not None:
-        _require_gpu_bf16("norm_weight", norm_weight)
-        if tuple(norm_weight.shape) != (K,) or not norm_weight.is_contiguous():
-            raise RuntimeError(f"linear_decode_fused: norm_weight {tuple(norm_weight.shape)} does not fit K={K}")
-        if rows > linear_decode_fused_max_rows(K):
-            raise RuntimeError(f"linear_decode_fused: the input norm takes at most "
-                               f"{linear_decode_fused_max_rows(K)} rows of width {K}, got {rows}")
-    r2 = None
-    if residual is not None:
-        _require_gpu_bf16("residual", residual)
-        if residual.numel() != rows * N or residual.shape[-1] != N:
-            raise RuntimeError(f"linear_decode_fused: residual {tuple(residual.shape)} does not fit ({rows}, {N})")
-        r2 = residual if residual.is_contiguous() else residual.reshape(rows, N).contiguous()
-    y = _rows_out(x, rows, N)
-    with _on_device(x.device):
-        rc = lib.l3_linear_decode_fused(x2.data_ptr(), None if norm_weight is None else norm_weight.data_ptr(),
-                                        float(eps), weight.data_ptr(), None if w_up is None else w_up.data_ptr(),
-                                        None if r2 is None else r2.data_ptr(), y.data_ptr(), rows, N, K,
-                                        x2.stride(0), weight.stride(0), N, _stream_ptr(x.device))
-    if rc != 0:
-        _fail(rc, f"M={rows} N={N} K={K}")
-    return y
+    return _l3lib.native().linear_decode_fused(x, weight, norm_weight, eps, w_up, residual)
 
 
 def linear_splitk(x, weight, ksplit: int = 0):
@@ -671,101 +359,27 @@ def linear_splitk(x, weight, ksplit: int = 0):
     rot_embed_append_partials, which sum the splits on their way (or sum them yourself).
     ksplit 0 lets the library choose.  Stands for nn.Linear at batch sizes where the activations no
     longer fit one matrix-instruction column block (model.py:95,121,134).  An extension."""
-    lib = _l3lib.load()
-    x2, rows, N, K = _linear_args(x, (weight,), _l3lib.L3_LINEAR_SPLITK_MAX_ROWS)
-    with _on_device(x.device):
-        if ksplit <= 0:
-            ksplit = lib.l3_linear_splitk_plan(N, K, _cus(x.device))
-            if ksplit < 0:
-                _fail(ksplit, f"N={N} K={K}")
-        part = torch.empty((ksplit, rows, N), dtype=torch.float32, device=x.device)
-        rc = lib.l3_linear_splitk(x2.data_ptr(), weight.data_ptr(), part.data_ptr(), part.numel() * 4, rows, N, K,
-                                  x2.stride(0), weight.stride(0), ksplit, _stream_ptr(x.device))
-    if rc != 0:
-        _fail(rc, f"M={rows} N={N} K={K} ksplit={ksplit}")
-    return part
+    return _l3lib.native().linear_splitk(x, weight, ksplit)
 
 
 def linear_splitk_finish(part, residual=None):
     """bf16(part.sum(0)) for linear_splitk's partial products (ksplit, rows, N), summed in split
     order and rounded once -- what the unsplit linear would have returned -- plus ``residual``
     (rows x N, bf16) with the rounding of a separate addition if given.  Returns (rows, N)."""
-    lib = _l3lib.load()
-    if not part.is_cuda or part.dtype != torch.float32 or part.dim() != 3 or not part.is_contiguous():
-        raise RuntimeError("linear_splitk_finish: expected contiguous float32 (ksplit, rows, N) partials")
-    ksplit, rows, N = part.shape
-    r2 = None
-    if residual is not None:
-        _require_gpu_bf16("residual", residual)
-        if residual.numel() != rows * N or residual.shape[-1] != N:
-            raise RuntimeError(f"linear_splitk_finish: residual {tuple(residual.shape)} does not fit ({rows}, {N})")
-        r2 = residual.reshape(rows, N)
-        if not r2.is_contiguous():
-            r2 = r2.contiguous()
-    y = torch.empty((rows, N), dtype=torch.bfloat16, device=part.device)
-    with _on_device(part.device):
-        rc = lib.l3_linear_splitk_finish(part.data_ptr(), ksplit, None if r2 is None else r2.data_ptr(), y.data_ptr(),
-                                         rows, N, N, _stream_ptr(part.device))
-    if rc != 0:
-        _fail(rc, f"rows={rows} N={N} ksplit={ksplit}")
-    return y
+    return _l3lib.native().linear_splitk_finish(part, residual)
 
 
 def add_rms_norm_partials(input, part, weight, eps):
     """add_rms_norm(input, r, weight, eps) with r = bf16(part.sum(0)) formed inside the kernel:
     ``part`` is linear_splitk's output for the linear whose result is the residual branch
     (model.py:147-148).  Returns (input + r, rms_norm(input + r))."""
-    lib = _l3lib.load()
-    _require_gpu_bf16("input", input)
-    _require_gpu_bf16("weight", weight)
-    C = input.shape[-1]
-    rows = input.numel() // C
-    if not part.is_cuda or part.dtype != torch.float32 or part.dim() != 3 or not part.is_contiguous() \
-            or tuple(part.shape[1:]) != (rows, C):
-        raise RuntimeError(f"add_rms_norm_partials: partials {tuple(part.shape)} do not fit input {tuple(input.shape)}")
-    if weight.numel() != C or not weight.is_contiguous():
-        raise RuntimeError(f"weight has {weight.numel()} elements, expected {C}")
-    x = input if input.is_contiguous() else input.contiguous()
-    s = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    y = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    with _on_device(x.device):
-        rc = lib.l3_add_rms_norm_partials(x.data_ptr(), part.data_ptr(), part.shape[0], weight.data_ptr(),
-                                          s.data_ptr(), y.data_ptr(), rows, C, float(eps), _stream_ptr(x.device))
-    if rc != 0:
-        _fail(rc, f"rows={rows} C={C} ksplit={part.shape[0]}")
-    return s, y
+    return _l3lib.native().add_rms_norm_partials(input, part, weight, eps)
 
 
 def rot_embed_append_partials(part, freq_table, cache_k, cache_v, pos, n_head: int):
     """rot_embed_append on a fused qkv projection that is still in linear_splitk's partial
     products (ksplit, B, (n_head + 2*KVH)*HD): summed, rounded to bf16, rotated, appended."""
-    lib = _l3lib.load()
-    _require_gpu_bf16("cache_k", cache_k)
-    _require_gpu_bf16("cache_v", cache_v)
-    if cache_k.dim() != 4 or cache_k.shape != cache_v.shape or cache_k.stride() != cache_v.stride():
-        raise RuntimeError("cache_k and cache_v must be (maxB, L, KVH, HD) tensors of the same layout")
-    maxB, L, KVH, HD = cache_k.shape
-    if not part.is_cuda or part.dtype != torch.float32 or part.dim() != 3 or not part.is_contiguous():
-        raise RuntimeError("rot_embed_append_partials: expected contiguous float32 (ksplit, B, N) partials")
-    ksplit, B, N = part.shape
-    if N != (n_head + 2 * KVH) * HD or B > maxB:
-        raise RuntimeError(f"partials {tuple(part.shape)} do not match n_head={n_head}, cache {tuple(cache_k.shape)}")
-    if cache_k.stride(3) != 1 or cache_k.stride(2) != HD:
-        raise RuntimeError("the (KVH, HD) dimensions of the cache must be contiguous")
-    if not freq_table.is_cuda or freq_table.dtype != torch.float32 or freq_table.dim() != 2 \
-            or freq_table.size(1) != HD or not freq_table.is_contiguous():
-        raise RuntimeError("freq_table must be a contiguous (rows, HD) float32 GPU tensor")
-    if not pos.is_cuda or pos.dtype != torch.int32 or pos.numel() != 1:
-        raise RuntimeError("pos must be a one-element int32 GPU tensor")
-    out = torch.empty((B, 1, n_head, HD), dtype=cache_k.dtype, device=part.device)
-    with _on_device(part.device):
-        rc = lib.l3_rot_embed_append_partials(part.data_ptr(), ksplit, freq_table.data_ptr(), out.data_ptr(),
-                                              cache_k.data_ptr(), cache_v.data_ptr(), pos.data_ptr(), B, n_head, KVH,
-                                              HD, _l3lib.i64_array((cache_k.stride(0), cache_k.stride(1))), L,
-                                              freq_table.size(0), _stream_ptr(part.device))
-    if rc != 0:
-        _fail(rc, f"B={B} NH={n_head} KVH={KVH} HD={HD} ksplit={ksplit}")
-    return out
+    return _l3lib.native().rot_embed_append_partials(part, freq_table, cache_k, cache_v, pos, n_head)
 
 
 def argmax(logits):
@@ -827,25 +441,4 @@ def greedy_step(logits, tokens, text_mask, tok, pos, kv_len, eos, stop_tokens):
 def rot_embed(input, freq):
     """input (B, T, NH, HD) bf16 (any strides on the first three dims), freq (T, HD) float32
     interleaved cos/sin -> contiguous (B, T, NH, HD) bf16 (model.py:100-101)."""
-    lib = _l3lib.load()
-    _require_gpu_bf16("input", input)
-    if not freq.is_cuda or freq.dtype != torch.float32:
-        raise RuntimeError(f"expected a GPU float32 freq table but found {freq.dtype} on {freq.device}")
-    if input.dim() != 4 or freq.dim() != 2:
-        raise RuntimeError("rot_embed expects a 4-D (B, T, NH, HD) input and a 2-D (T, HD) freq table")
-    B, T, NH, HD = input.shape
-    if freq.size(0) != T or freq.size(1) != HD:
-        raise RuntimeError(f"freq is {tuple(freq.shape)}, expected {(T, HD)}")
-    if input.stride(3) != 1:
-        raise RuntimeError("the head dimension of input must be contiguous")
-    f = freq if freq.is_contiguous() else freq.contiguous()
-    out = input.new_empty((B, T, NH, HD))
-    if out.numel() == 0:
-        return out
-    with _on_device(input.device):
-        rc = lib.l3_rot_embed(input.data_ptr(), f.data_ptr(), out.data_ptr(), B, T, NH, HD,
-                              _l3lib.i64_array((input.stride(0), input.stride(1), input.stride(2))),
-                              _stream_ptr(input.device))
-    if rc != 0:
-        _fail(rc, f"B={B} T={T} NH={NH} HD={HD} strides={tuple(input.stride())}")
-    return out
+    return _l3lib.native().rot_embed(input, freq)
