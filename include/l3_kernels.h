@@ -343,28 +343,38 @@ int l3_linear_qkv_rope_append(const void* x, const void* norm_weight, float norm
                               void* stream);
 
 /*
- * Split-K form of l3_linear_decode for 17 .. 64 activation rows (hipBLASLt's territory in the
+ * Split-K form of l3_linear_decode for up to 64 activation rows (hipBLASLt's territory in the
  * reference: nn.Linear at batch 64, model.py:95,121,134).  Eight wavefronts of a workgroup share
- * the activations of one k range through LDS and take 128 weight rows (64, with the k range halved
- * among them, for small matrices); K is split `ksplit` ways across workgroups, each covering at
- * most 512 (1024) k, and split s writes its float32 partial products
+ * the activations of one k range through LDS and take 64 (32) weight rows; K is split `ksplit` ways
+ * across workgroups, and split s writes its float32 partial products
  * to part[s][m][n] (M x N floats per split, contiguous).  The splits are NOT added up here: the
  * elementwise operator that follows the linear in a decode step does that on its way
  * (l3_add_rms_norm_partials, l3_rot_embed_append_partials), in split order, without atomics;
  * l3_linear_splitk_finish does it where there is no such operator.
- * l3_linear_splitk_plan returns the split count for a device with num_cus compute units (<= 0: the
- * current device); l3_linear_splitk_workspace_bytes the size of `part`.  1 <= M <=
- * L3_LINEAR_SPLITK_MAX_ROWS, N % 8 == 0, K % 128 == 0, ceil((K / 128) / ksplit) <= 4 (<= 8 for a matrix
- * with fewer than 32 rows per compute unit, which gets 64-row workgroups); strides and
- * alignment as for l3_linear_decode.  Meant for matrices of a few thousand rows, where the split
- * count fills the device; for a matrix whose rows alone do (a vocabulary projection), every split
- * costs M x N floats of traffic and a library GEMM is the better tool.
+ * l3_linear_splitk_rows_plan returns the split count that suits M rows on a device with num_cus compute
+ * units (<= 0: the current device): as few splits as fill the device.  l3_linear_splitk_plan is the finer
+ * cut for a caller that does not know M; l3_linear_splitk_workspace_bytes the size of `part`.  1 <= M <=
+ * L3_LINEAR_SPLITK_MAX_ROWS, N % 8 == 0, K % 128 == 0, ceil((K / 128) / ksplit) no more than the coarser of
+ * the two plans takes, or 4 (8 for a matrix with fewer than 32 rows per compute unit); strides (below 2^28)
+ * and alignment as for l3_linear_decode.  Meant for matrices of a few thousand rows, where the split
+ * count fills the device; where the rows alone do (a vocabulary projection), see l3_linear_wide.
  */
 #define L3_LINEAR_SPLITK_MAX_ROWS 64
 int l3_linear_splitk_plan(int N, int K, int num_cus);
+int l3_linear_splitk_rows_plan(int M, int N, int K, int num_cus);
 size_t l3_linear_splitk_workspace_bytes(int M, int N, int ksplit);
 int l3_linear_splitk(const void* x, const void* w, void* part, size_t part_bytes, int M, int N, int K,
                      int64_t x_stride, int64_t w_stride, int ksplit, void* stream);
+
+/*
+ * y = x . w^T, or with w_up != NULL bf16(silu(x . w^T)) * bf16(x . w_up^T), plus the residual (M, N; y's row
+ * stride) with a rounding of its own if that is not NULL, for up to 64 activation rows in one
+ * launch without splits: for matrices whose rows alone fill the device (gate|up pair, vocabulary
+ * projection: model.py:134,225).  1 <= M <= L3_LINEAR_SPLITK_MAX_ROWS, K % 128 == 0, N % 8 == 0 (N % 4 with
+ * w_up); strides (below 2^28) and alignment as for l3_linear_decode, y 16-byte aligned without w_up.
+ */
+int l3_linear_wide(const void* x, const void* w, const void* w_up, const void* residual, void* y, int M, int N, int K,
+                   int64_t x_stride, int64_t w_stride, int64_t y_stride, void* stream);
 
 /*
  * y[m][n] = bf16(sum over the splits of part[s][m][n]), or bf16(residual + that) with the two

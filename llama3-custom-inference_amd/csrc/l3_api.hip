@@ -755,6 +755,29 @@ int l3_linear_splitk_plan(int N, int K, int num_cus) {
     return linear_splitk_plan(N, K, num_cus);
 }
 
+int l3_linear_splitk_rows_plan(int M, int N, int K, int num_cus) {
+    if (M <= 0 || M > L3_LINEAR_SPLITK_MAX_ROWS || N <= 0 || K <= 0 || K % 128 != 0) return L3_ERR_SHAPE;
+    if (num_cus <= 0) num_cus = current_device_cus();
+    return linear_splitk_rows_plan(N, K, num_cus);
+}
+
+int l3_linear_wide(const void* x, const void* w, const void* w_up, const void* residual, void* y, int M, int N, int K,
+                   int64_t x_stride, int64_t w_stride, int64_t y_stride, void* stream) {
+    if (!x || !w || !y) return L3_ERR_NULL_POINTER;
+    if (M <= 0 || M > L3_LINEAR_SPLITK_MAX_ROWS || N <= 0 || K <= 0 || N % (w_up ? 4 : 8) != 0 || K % 128 != 0)
+        return L3_ERR_SHAPE;
+    if (N > (1 << 24) || K > (1 << 24)) return L3_ERR_SHAPE;
+    if (x_stride < K || w_stride < K || y_stride < N || x_stride % 8 || w_stride % 8 || y_stride % (w_up ? 4 : 8) ||
+        x_stride > kLinearMaxPitch || w_stride > kLinearMaxPitch)
+        return L3_ERR_STRIDE;
+    if (!aligned(x, 16) || !aligned(w, 16) || (w_up && !aligned(w_up, 16)) || !aligned(y, w_up ? 8 : 16) ||
+        (residual && !aligned(residual, w_up ? 8 : 16)))
+        return L3_ERR_ALIGNMENT;
+    return launch_linear_wide(static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w),
+                              static_cast<const uint16_t*>(w_up), static_cast<const uint16_t*>(residual), static_cast<uint16_t*>(y), M, N, K, x_stride, w_stride,
+                              y_stride, current_device_cus(), static_cast<hipStream_t>(stream)) == 0 ? L3_OK : L3_ERR_HIP;
+}
+
 size_t l3_linear_splitk_workspace_bytes(int M, int N, int ksplit) {
     if (M <= 0 || N <= 0 || ksplit <= 0) return 0;
     return size_t(ksplit) * size_t(M) * size_t(N) * sizeof(float);
@@ -766,9 +789,10 @@ int l3_linear_splitk(const void* x, const void* w, void* part, size_t part_bytes
     if (M <= 0 || M > L3_LINEAR_SPLITK_MAX_ROWS || N <= 0 || K <= 0 || N % 8 != 0 || K % 128 != 0) return L3_ERR_SHAPE;
     if (N > (1 << 24) || K > (1 << 24)) return L3_ERR_SHAPE;
     if (ksplit <= 0 || ksplit > K / 128 ||
-        (K / 128 + ksplit - 1) / ksplit > linear_splitk_max_chunks(N, current_device_cus()))
+        (K / 128 + ksplit - 1) / ksplit > linear_splitk_max_chunks(N, K, current_device_cus()))
         return L3_ERR_SPLITS;
-    if (x_stride < K || w_stride < K || x_stride % 8 || w_stride % 8) return L3_ERR_STRIDE;
+    if (x_stride < K || w_stride < K || x_stride % 8 || w_stride % 8 || x_stride > kLinearMaxPitch || w_stride > kLinearMaxPitch)
+        return L3_ERR_STRIDE;
     if (!aligned(x, 16) || !aligned(w, 16) || !aligned(part, 16)) return L3_ERR_ALIGNMENT;
     if (part_bytes < l3_linear_splitk_workspace_bytes(M, N, ksplit)) return L3_ERR_WORKSPACE;
     return launch_linear_splitk(static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w),

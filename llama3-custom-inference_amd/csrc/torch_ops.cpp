@@ -39,9 +39,9 @@ using at::TensorBase;
 #define L3_FUNCTIONS(X)                                                                                          \
     X(l3_strerror) X(l3_attn_decode) X(l3_attn_decode_devlen) X(l3_attn_decode_workspace_bytes)                  \
     X(l3_attn_workspace_init) X(l3_attn_prefill) X(l3_rms_norm) X(l3_add_rms_norm) X(l3_add_rms_norm_partials)   \
-    X(l3_rot_embed) X(l3_rot_embed_append_partials) X(l3_silu_mul) X(l3_silu_mul_rows) X(l3_linear_decode)       \
-    X(l3_linear_swiglu_decode) X(l3_linear_decode_fused) X(l3_linear_qkv_rope_append) X(l3_linear_splitk_plan)   \
-    X(l3_linear_splitk) X(l3_linear_splitk_finish)
+    X(l3_rot_embed) X(l3_rot_embed_append_partials) X(l3_silu_mul) X(l3_silu_mul_rows)       \
+    X(l3_linear_decode_fused) X(l3_linear_qkv_rope_append) X(l3_linear_splitk_rows_plan)   \
+    X(l3_linear_splitk) X(l3_linear_splitk_finish) X(l3_linear_wide)
 
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
@@ -452,12 +452,6 @@ void check_weight(const Tensor& w, const Tensor& like, const Tensor& x, int64_t 
                 "linear_decode: weight ", w.sizes(), " does not fit x ", x.sizes());
 }
 
-// (How many rows of that width the fused norm takes, the library checks.)
-void check_norm_weight(const Tensor& norm, int64_t K, const char* what) {
-    TORCH_CHECK(norm.dim() == 1 && norm.numel() == K && norm.is_contiguous(), what, ": norm_weight ", norm.sizes(),
-                " does not fit K=", K);
-}
-
 // A contiguous output of x's leading shape with N columns.
 Tensor rows_out(const Tensor& x, int64_t N) {
     c10::SmallVector<int64_t, 5> sizes(x.sizes().begin(), x.sizes().end());
@@ -465,12 +459,38 @@ Tensor rows_out(const Tensor& x, int64_t N) {
     return new_empty(sizes, x);
 }
 
-// 17..64 activation rows: the split-K kernel plus its finishing pass (one launch serves up to 16).
-bool use_splitk(const Tensor& x, const Tensor& w) {
+// Which kernels a linear takes.  kSkinny streams weights past operands held in registers: up to 16 rows, anything
+// folded in, one launch.  kWide and kSplit share the activations through LDS (K % 128 == 0, N % 8 == 0): one launch
+// where the rows of the matrix fill the device, partial products plus a finishing pass where they do not.
+// Activations (rows padded by 8 elements) that the skinny kernel's input norm stages in LDS.
+constexpr int64_t kNormStageElements = 24576;
+
+enum class Route { kSkinny, kWide, kSplit };
+
+// From here on the rows of a matrix alone fill the device (64 to a workgroup; 32 of each of the SwiGLU pair).
+constexpr int64_t kWideRows = 12288, kWidePairRows = 6144;
+
+// Graph-timed over rotating weights, skinny against wide or split plus finish (us; + 2 with a norm in front, which
+// is then a launch of its own): vocabulary projection 128256 x 2048, 2 rows 81 / 86, 3 rows 88 / 86, 4 rows 96 / 85, 16
+// rows 139 / 87; gate|up pair 8192 x 2048, 3 rows 14.0 / 13.2, 4 rows 14.7 / 13.3, 16 rows 21.0 / 12.8; pair 14336 x
+// 4096 (235 MB), 1 row 47.9 / 39.2; 2048 x 8192, 4 rows 10.2 / 10.6, 5 rows 15.4 / 10.7; 4096 x 4096, 5 rows 10.1 / 10.4, 16
+// rows 12.3 / 10.6; 6144 x 4096, 2 rows 11.3 / 12.8, 5 rows 16.2 / 12.9; 4096 x 14336, 1 row 23.2 / 22.9; 2048 x 2048 and
+// 3072 x 2048, 12 rows 6.7 / 6.6 and 6.9 / 7.1.
+Route route_of(const Tensor& x, const Tensor& w, bool pair, bool residual) {
     const int64_t K = x.dim() > 0 ? x.sizes().back() : 0;
-    if (K <= 0 || w.dim() != 2 || !x.is_cuda()) return false;
-    const int64_t rows = x.numel() / K;
-    return rows > L3_LINEAR_MAX_ROWS && rows <= L3_LINEAR_SPLITK_MAX_ROWS;
+    if (K <= 0 || w.dim() != 2) return Route::kSkinny;   // (its checks say what is wrong)
+    const int64_t rows = x.numel() / K, N = size_at(w, 0);
+    if (rows > L3_LINEAR_SPLITK_MAX_ROWS) return Route::kSkinny;
+    const bool fits = K % 128 == 0 && N % 8 == 0;
+    if (pair) {
+        if (rows > L3_LINEAR_MAX_ROWS) return residual ? Route::kSkinny : Route::kWide;
+        const bool large = N * K >= int64_t(32) << 20;   // each of the two
+        return fits && N >= kWidePairRows && (rows >= 4 || large) ? Route::kWide : Route::kSkinny;
+    }
+    if (rows > L3_LINEAR_MAX_ROWS) return N >= kWideRows ? Route::kWide : Route::kSplit;
+    if (!fits) return Route::kSkinny;
+    if (N >= kWideRows) return rows >= 4 ? Route::kWide : Route::kSkinny;
+    return N * K >= int64_t(rows >= 5 ? 16 : 32) << 20 ? Route::kSplit : Route::kSkinny;
 }
 
 // Float32 partial products (ksplit, rows, N); ksplit 0 = the library's choice.
@@ -480,7 +500,7 @@ Tensor splitk(const Tensor& x, const Tensor& w, int ksplit) {
     const int64_t N = size_at(w, 0);
     const OnDevice on(x);
     if (ksplit <= 0) {
-        ksplit = lib.l3_linear_splitk_plan(int(N), int(r.K), 0);
+        ksplit = lib.l3_linear_splitk_rows_plan(int(r.rows), int(N), int(r.K), 0);
         check(ksplit, "N=", N, " K=", r.K);
     }
     Tensor part = new_empty({ksplit, r.rows, N}, x, at::kFloat);
@@ -507,70 +527,81 @@ void splitk_finish(const Tensor& part, const Tensor* residual, const Tensor& y) 
           " N=", N, " ksplit=", size_at(part, 0));
 }
 
-// (x, weight)
-PyObject* linear_decode(PyObject* const* a) {
-    const Tensor& x = gpu_bf16(a[0], "x");
-    const Tensor& w = gpu_bf16(a[1], "weight");
-    if (use_splitk(x, w)) {
-        const Tensor part = splitk(x, w, 0);
-        Tensor y = rows_out(x, size_at(w, 0));
-        splitk_finish(part, nullptr, y);
-        return wrap(std::move(y));
-    }
-    const Rows r = linear_rows(x, L3_LINEAR_MAX_ROWS);
-    check_weight(w, w, x, r.K);
-    const int64_t N = size_at(w, 0);
-    Tensor y = rows_out(x, N);
-    const OnDevice on(x);
-    check(lib.l3_linear_decode(r.x, ptr(w), ptr(y), int(r.rows), int(N), int(r.K), r.stride, stride_at(w, 0), N, on.stream), "M=",
-          r.rows, " N=", N, " K=", r.K);
-    return wrap(std::move(y));
-}
-
-// (x, w_gate, w_up)
-PyObject* linear_swiglu_decode(PyObject* const* a) {
-    const Tensor& x = gpu_bf16(a[0], "x");
-    const Tensor& wg = gpu_bf16(a[1], "weight");
-    const Tensor& wu = gpu_bf16(a[2], "weight");
-    const Rows r = linear_rows(x, L3_LINEAR_MAX_ROWS);
-    check_weight(wg, wg, x, r.K);
-    check_weight(wu, wg, x, r.K);
-    const int64_t N = size_at(wg, 0);
-    Tensor y = rows_out(x, N);
-    const OnDevice on(x);
-    check(lib.l3_linear_swiglu_decode(r.x, ptr(wg), ptr(wu), ptr(y), int(r.rows), int(N), int(r.K), r.stride, stride_at(wg, 0), N,
-                                      on.stream),
-          "M=", r.rows, " N=", N, " K=", r.K);
-    return wrap(std::move(y));
-}
-
-// (x, weight, norm_weight or None, eps, w_up or None, residual or None)
-PyObject* linear_decode_fused(PyObject* const* a) {
-    const Tensor& x = gpu_bf16(a[0], "x");
-    const Tensor& w = gpu_bf16(a[1], "weight");
-    const Tensor* norm = optional_tensor(a[2], "norm_weight");
-    const Tensor* up = optional_tensor(a[4], "weight");
-    const Tensor* residual = optional_tensor(a[5], "residual");
-    if (!norm && !up && use_splitk(x, w)) {
-        // the residual joins when the splits are added up
-        const Tensor part = splitk(x, w, 0);
-        Tensor y = rows_out(x, size_at(w, 0));
-        splitk_finish(part, residual, y);
-        return wrap(std::move(y));
-    }
-    const Rows r = linear_rows(x, L3_LINEAR_MAX_ROWS);
+// The whole product (or, with up, the SwiGLU product of two) of up to 64 rows in one launch.
+Tensor wide(const Tensor& x, const Tensor& w, const Tensor* up, const Tensor* residual) {
+    const Rows r = linear_rows(x, L3_LINEAR_SPLITK_MAX_ROWS);
     check_weight(w, w, x, r.K);
     if (up) check_weight(*up, w, x, r.K);
     const int64_t N = size_at(w, 0);
-    if (norm) check_norm_weight(*norm, r.K, "linear_decode_fused");
     Tensor copy;
     const void* res = residual_rows(residual, r.rows, N, copy, "linear_decode_fused");
     Tensor y = rows_out(x, N);
     const OnDevice on(x);
-    check(lib.l3_linear_decode_fused(r.x, norm ? ptr(*norm) : nullptr, float(number(a[3])), ptr(w), up ? ptr(*up) : nullptr, res,
-                                     ptr(y), int(r.rows), int(N), int(r.K), r.stride, stride_at(w, 0), N, on.stream),
+    check(lib.l3_linear_wide(r.x, ptr(w), up ? ptr(*up) : nullptr, res, ptr(y), int(r.rows), int(N), int(r.K), r.stride,
+                             stride_at(w, 0), N, on.stream),
           "M=", r.rows, " N=", N, " K=", r.K);
-    return wrap(std::move(y));
+    return y;
+}
+
+// (How many rows of that width the skinny kernel's norm takes; the same limit whatever the route.)
+void check_norm_weight(const Tensor& norm, int64_t rows, int64_t K, const char* what) {
+    TORCH_CHECK(norm.dim() == 1 && norm.numel() == K && norm.is_contiguous(), what, ": norm_weight ", norm.sizes(),
+                " does not fit K=", K);
+    const int64_t most = K % 512 == 0 ? std::min<int64_t>(16, kNormStageElements / (K + 8)) : 0;
+    TORCH_CHECK(rows <= most, what, ": the input norm takes at most ", most, " rows of width ", K, ", got ", rows);
+}
+
+// x (.. , K) normalised into a tensor of its own.
+Tensor normalised(const Tensor& x, const Tensor& norm, double eps) {
+    Tensor copy;
+    const Tensor& xc = contiguous(x, copy);
+    Tensor h = new_empty(x.sizes(), x);
+    const int64_t K = x.sizes().back(), rows = x.numel() / K;
+    const OnDevice on(x);
+    check(lib.l3_rms_norm(ptr(xc), ptr(norm), ptr(h), rows, int(K), float(eps), on.stream), "rows=", rows, " C=", K);
+    return h;
+}
+
+// The linear with what is folded into it.
+Tensor linear(const Tensor& x, const Tensor& w, const Tensor* norm, double eps, const Tensor* up, const Tensor* residual) {
+    const Route route = route_of(x, w, up != nullptr, residual != nullptr);
+    const Rows r = linear_rows(x, route == Route::kSkinny ? L3_LINEAR_MAX_ROWS : L3_LINEAR_SPLITK_MAX_ROWS);
+    check_weight(w, w, x, r.K);
+    if (up) check_weight(*up, w, x, r.K);
+    if (norm) check_norm_weight(*norm, r.rows, r.K, "linear_decode_fused");
+    if (route != Route::kSkinny) {
+        const Tensor h = norm ? normalised(x, *norm, eps) : x;
+        if (route == Route::kWide) return wide(h, w, up, residual);
+        const Tensor part = splitk(h, w, 0);
+        Tensor y = rows_out(x, size_at(w, 0));
+        splitk_finish(part, residual, y);   // the residual joins when the splits are added up
+        return y;
+    }
+    const int64_t N = size_at(w, 0);
+    Tensor copy;
+    const void* res = residual_rows(residual, r.rows, N, copy, "linear_decode_fused");
+    Tensor y = rows_out(x, N);
+    const OnDevice on(x);
+    check(lib.l3_linear_decode_fused(r.x, norm ? ptr(*norm) : nullptr, float(eps), ptr(w), up ? ptr(*up) : nullptr, res, ptr(y),
+                                     int(r.rows), int(N), int(r.K), r.stride, stride_at(w, 0), N, on.stream),
+          "M=", r.rows, " N=", N, " K=", r.K);
+    return y;
+}
+
+// (x, weight)
+PyObject* linear_decode(PyObject* const* a) {
+    return wrap(linear(gpu_bf16(a[0], "x"), gpu_bf16(a[1], "weight"), nullptr, 0.0, nullptr, nullptr));
+}
+
+// (x, w_gate, w_up)
+PyObject* linear_swiglu_decode(PyObject* const* a) {
+    return wrap(linear(gpu_bf16(a[0], "x"), gpu_bf16(a[1], "weight"), nullptr, 0.0, &gpu_bf16(a[2], "weight"), nullptr));
+}
+
+// (x, weight, norm_weight or None, eps, w_up or None, residual or None)
+PyObject* linear_decode_fused(PyObject* const* a) {
+    return wrap(linear(gpu_bf16(a[0], "x"), gpu_bf16(a[1], "weight"), optional_tensor(a[2], "norm_weight"), number(a[3]),
+                       optional_tensor(a[4], "weight"), optional_tensor(a[5], "residual")));
 }
 
 // (x, weight, ksplit)
@@ -619,7 +650,7 @@ PyObject* linear_qkv_rope_append(PyObject* const* a) {
     TORCH_CHECK(size_at(w, 0) == (NH + 2 * c.KVH) * c.HD && r.rows <= c.maxB, "w_qkv ", w.sizes(), " does not match n_head=", NH,
                 ", cache ", c.k->sizes());
     const Tensor* norm = optional_tensor(a[7], "norm_weight");
-    if (norm) check_norm_weight(*norm, r.K, "linear_qkv_rope_append");
+    if (norm) check_norm_weight(*norm, r.rows, r.K, "linear_qkv_rope_append");
     Tensor out = new_empty({r.rows, 1, NH, c.HD}, x);
     const OnDevice on(x);
     check(lib.l3_linear_qkv_rope_append(r.x, norm ? ptr(*norm) : nullptr, float(number(a[8])), ptr(w),

@@ -135,6 +135,12 @@ SIGNATURES = {
          ctypes.c_int64, ctypes.c_void_p],
     ),
     "l3_linear_splitk_plan": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int]),
+    "l3_linear_splitk_rows_plan": (ctypes.c_int, [ctypes.c_int] * 4),
+    "l3_linear_wide": (
+        ctypes.c_int,
+        [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+         ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_void_p],
+    ),
     "l3_linear_splitk_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int, ctypes.c_int, ctypes.c_int]),
     "l3_linear_splitk": (
         ctypes.c_int,

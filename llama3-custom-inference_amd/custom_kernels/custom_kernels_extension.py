@@ -66,9 +66,9 @@ def _on_device(device):
 
 
 def _workspace(device, stream_ptr: int, nbytes: int):
-    """Scratch for the argmax partials, kept per (device, stream) and grown on demand so that a decode step does not allocate.  Calls on one
-    stream are ordered and can share it; another stream gets its own.  While a stream is being
-    captured into a HIP graph the buffer comes from the graph's own memory pool instead (a plain
+    """Scratch for the argmax partials, kept per (device, stream) and grown on demand so that a decode
+    step does not allocate.  Calls on one stream are ordered and can share it; another stream gets its
+    own.  While a stream is being captured into a HIP graph the buffer comes from the graph's own memory pool instead (a plain
     allocation that lives and dies with the graph) and is not cached."""
     if torch.cuda.is_current_stream_capturing():
         return torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
@@ -327,16 +327,16 @@ def silu_mul(a, b):
 def linear_decode(x, weight):
     """F.linear(x, weight) for at most 64 activation rows (model.py:95,121,134,225 when T == 1):
     one pass over the weight matrix at HBM speed instead of a GEMM.  x (..., K), weight (N, K)
-    -> (..., N).  Up to 16 rows are one launch whatever the matrix; 17..64 rows go through
-    linear_splitk and linear_splitk_finish (N % 8 == 0, K % 128 == 0), which suits matrices of a
-    few thousand rows -- a vocabulary projection at those batch sizes is a library GEMM's job.
-    An extension."""
+    -> (..., N).  Up to 16 rows are one launch whatever the matrix; 17..64 rows (N % 8 == 0,
+    K % 128 == 0) are one launch where the rows of the matrix fill the device (a vocabulary
+    projection), else linear_splitk and linear_splitk_finish.  An extension."""
     return _l3lib.native().linear_decode(x, weight)
 
 
 def linear_swiglu_decode(x, w_gate, w_up):
-    """F.silu(F.linear(x, w_gate)) * F.linear(x, w_up) for at most 16 activation rows in one
-    launch (model.py:134 with w_gate = c_fc2, w_up = c_fc), same rounding points.  An extension."""
+    """F.silu(F.linear(x, w_gate)) * F.linear(x, w_up) for at most 64 activation rows in one
+    launch (model.py:134 with w_gate = c_fc2, w_up = c_fc), same rounding points; from 17 rows on
+    K % 128 == 0.  An extension."""
     return _l3lib.native().linear_swiglu_decode(x, w_gate, w_up)
 
 
@@ -354,7 +354,7 @@ def linear_decode_fused(x, weight, norm_weight=None, eps: float = 1e-5, w_up=Non
 
 
 def linear_splitk(x, weight, ksplit: int = 0):
-    """x (..., K) with 17..64 rows times weight (N, K)^T as float32 partial products
+    """x (..., K) with up to 64 rows times weight (N, K)^T as float32 partial products
     (ksplit, rows, N) -- NOT added up: hand them to add_rms_norm_partials or
     rot_embed_append_partials, which sum the splits on their way (or sum them yourself).
     ksplit 0 lets the library choose.  Stands for nn.Linear at batch sizes where the activations no

@@ -165,7 +165,6 @@ class LlamaDecoder:
 
     FUSED_MAX_ROWS = 4   # rows up to which the fused single-launch linears carry the whole decode step
     QKV_FUSED_MAX_ROWS = 16   # rows up to which the split-K route takes the single-launch qkv + rope + append linear (+2..6 %)
-    SWIGLU_MAX_ROWS = 14  # rows up to which the split-K route takes the single-launch gate|up + SwiGLU linear (+3 % at 7..10 rows, level at 16)
 
     def _splitk(self, rows: int) -> bool:
         """5..64 activation rows: the split-K linears (activations shared through LDS, splits added
@@ -175,30 +174,19 @@ class LlamaDecoder:
         those re-reads the activations of its k range, which the 8192-wide down projection feels first."""
         return self.decode_linear_rows > 0 and self.FUSED_MAX_ROWS < rows <= 64 and hasattr(self.ops, "linear_splitk")
 
-    def _gate_up(self, L):
-        """c_fc2 and c_fc stacked into one (2 * hidden, C) matrix: one GEMM instead of two."""
-        if "c_fc_cat" not in L:
-            L["c_fc_cat"] = torch.cat([L["c_fc2"], L["c_fc"]], dim=0)
-        return L["c_fc_cat"]
-
     def _decode_layers_splitk(self, x, append_and_attend, project_and_attend=None):
         """The layers of one decode step (T == 1) at 5..64 rows; returns the final hidden state.
         append_and_attend(L, qkv partial products) -> attention output (B, 1, C);
         project_and_attend(L, normalised input) -> the same from the single-launch qkv projection
         (rotary embedding and cache append inside), taken while the rows are few enough for it."""
         c, ops = self.config, self.ops
-        H = c.hidden_dim
         rows = x.numel() // x.shape[-1]
         qkv_fused = project_and_attend is not None and rows <= self.QKV_FUSED_MAX_ROWS
         h = ops.rms_norm(x, self.layers[0]["ln_1"], c.norm_eps)
         for i, L in enumerate(self.layers):
             y = project_and_attend(L, h) if qkv_fused else append_and_attend(L, ops.linear_splitk(h, L["c_attn"]))
             x, h = ops.add_rms_norm_partials(x, ops.linear_splitk(y, L["c_proj"]), L["ln_2"], c.norm_eps)
-            if rows <= self.SWIGLU_MAX_ROWS:
-                t = ops.linear_swiglu_decode(h, L["c_fc2"], L["c_fc"])     # one launch for the pair and the product
-            else:
-                gu = F.linear(h, self._gate_up(L))
-                t = ops.silu_mul(gu[..., :H], gu[..., H:])
+            t = ops.linear_swiglu_decode(h, L["c_fc2"], L["c_fc"])     # one launch for the pair and the product
             next_norm = self.layers[i + 1]["ln_1"] if i + 1 < len(self.layers) else self.ln_f
             x, h = ops.add_rms_norm_partials(x, ops.linear_splitk(t, L["mlp_proj"]), next_norm, c.norm_eps)
         return h
@@ -253,7 +241,7 @@ class LlamaDecoder:
                 return y.transpose(1, 2).reshape(B, 1, c.n_embd)
 
             h = self._decode_layers_splitk(x, append_and_attend, project_and_attend)
-            return F.linear(h, self.wte).float()
+            return self.ops.linear_decode(h, self.wte).float()
         for L in self.layers:
             x = x + self._attention(L, self.ops.rms_norm(x, L["ln_1"], c.norm_eps), freqs_cis, start_pos)
             h = self.ops.rms_norm(x, L["ln_2"], c.norm_eps)
@@ -416,7 +404,7 @@ class GraphedDecodeLoop:
                                                       L["cache_v"][:B].transpose(1, 2), self.kv_len)
                 return y.transpose(1, 2).reshape(B, 1, c.n_embd)
 
-            logits = F.linear(m._decode_layers_splitk(x, append_and_attend, project_and_attend)[:, -1], m.wte)
+            logits = ops.linear_decode(m._decode_layers_splitk(x, append_and_attend, project_and_attend)[:, -1], m.wte)
         else:
             h = ops.rms_norm(x, m.layers[0]["ln_1"], c.norm_eps)
             for i, L in enumerate(m.layers):
@@ -625,7 +613,7 @@ def bench_e2e(args, torch_mod, dev, cpu_ops=None):
         # ... then the library's weight-streaming linear kernels where they apply (up to 16 rows)
         model.set_decode_linear_rows(16)
         rec["decode_linear"] = ("l3_linear_decode (fused)" if 0 < batch <= model.decode_linear_rows else
-                                "l3_linear_splitk for c_attn / c_proj / mlp c_proj, F.linear for gate|up and lm_head"
+                                "l3_linear_splitk for c_attn / c_proj / mlp c_proj, l3_linear_wide for gate|up and lm_head"
                                 if model._splitk(batch) else "torch F.linear")
         for mode in ("eager", "graphed"):
             graphed = mode == "graphed"
