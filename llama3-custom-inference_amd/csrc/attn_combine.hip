@@ -164,31 +164,29 @@ int launch_attn_combine(const AttnParams& p, int HD, int producer_groups, hipStr
         const int G = producer_groups;
         const int xg = (G > 0 && p.QH % (4 * G) == 0 && (int64_t(G) * p.B) % 8 == 0) ? G : 0;
         if (HD == 64) {
-            hipLaunchKernelGGL((attn_combine_rows_kernel<64>), rgrid, rblock, 0, stream, p.part_o, p.part_ml, p.out,
-                               p.QH, p.num_splits, pairs, p.o_sb, p.o_sh, p.seqlen_dev, p.tokens_per_split, xg);
+            return enqueue(attn_combine_rows_kernel<64>, rgrid, rblock, 0, stream, p.part_o, p.part_ml, p.out,
+                           p.QH, p.num_splits, pairs, p.o_sb, p.o_sh, p.seqlen_dev, p.tokens_per_split, xg);
         } else {
-            hipLaunchKernelGGL((attn_combine_rows_kernel<128>), rgrid, rblock, 0, stream, p.part_o, p.part_ml, p.out,
-                               p.QH, p.num_splits, pairs, p.o_sb, p.o_sh, p.seqlen_dev, p.tokens_per_split, xg);
+            return enqueue(attn_combine_rows_kernel<128>, rgrid, rblock, 0, stream, p.part_o, p.part_ml, p.out,
+                           p.QH, p.num_splits, pairs, p.o_sb, p.o_sh, p.seqlen_dev, p.tokens_per_split, xg);
         }
-        return int(hipGetLastError());
     }
     const bool few = int64_t(p.B) * p.QH <= 64 && p.num_splits > kCombineRows;   // few heads, many rows each
     const dim3 grid(unsigned(p.B) * unsigned(p.QH), few ? 4u : 1u);
     const dim3 block(kCombineWaves * kWaveSize);
     if (HD == 64 && few) {
-        hipLaunchKernelGGL((attn_combine_kernel<64, 4>), grid, block, 0, stream, p.part_o, p.part_ml, p.out, p.QH,
-                           p.num_splits, p.o_sb, p.o_sh, p.seqlen_dev, p.tokens_per_split);
+        return enqueue(attn_combine_kernel<64, 4>, grid, block, 0, stream, p.part_o, p.part_ml, p.out, p.QH,
+                       p.num_splits, p.o_sb, p.o_sh, p.seqlen_dev, p.tokens_per_split);
     } else if (HD == 64) {
-        hipLaunchKernelGGL((attn_combine_kernel<64, 1>), grid, block, 0, stream, p.part_o, p.part_ml, p.out, p.QH,
-                           p.num_splits, p.o_sb, p.o_sh, p.seqlen_dev, p.tokens_per_split);
+        return enqueue(attn_combine_kernel<64, 1>, grid, block, 0, stream, p.part_o, p.part_ml, p.out, p.QH,
+                       p.num_splits, p.o_sb, p.o_sh, p.seqlen_dev, p.tokens_per_split);
     } else if (few) {
-        hipLaunchKernelGGL((attn_combine_kernel<128, 4>), grid, block, 0, stream, p.part_o, p.part_ml, p.out, p.QH,
-                           p.num_splits, p.o_sb, p.o_sh, p.seqlen_dev, p.tokens_per_split);
+        return enqueue(attn_combine_kernel<128, 4>, grid, block, 0, stream, p.part_o, p.part_ml, p.out, p.QH,
+                       p.num_splits, p.o_sb, p.o_sh, p.seqlen_dev, p.tokens_per_split);
     } else {
-        hipLaunchKernelGGL((attn_combine_kernel<128, 1>), grid, block, 0, stream, p.part_o, p.part_ml, p.out, p.QH,
-                           p.num_splits, p.o_sb, p.o_sh, p.seqlen_dev, p.tokens_per_split);
+        return enqueue(attn_combine_kernel<128, 1>, grid, block, 0, stream, p.part_o, p.part_ml, p.out, p.QH,
+                       p.num_splits, p.o_sb, p.o_sh, p.seqlen_dev, p.tokens_per_split);
     }
-    return int(hipGetLastError());
 }
 
 }  // namespace l3

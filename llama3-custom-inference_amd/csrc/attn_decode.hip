@@ -221,8 +221,7 @@ attn_splitkv_fma_kernel(const AttnParams p) {
 template <int HD, int R>
 int launch_split(const AttnParams& p, hipStream_t stream) {
     const dim3 grid(unsigned(p.B) * unsigned(p.KVH) * unsigned(p.num_splits));
-    hipLaunchKernelGGL((attn_splitkv_fma_kernel<HD, R>), grid, dim3(kAttnWaves * kWaveSize), 0, stream, p);
-    return int(hipGetLastError());
+    return enqueue(attn_splitkv_fma_kernel<HD, R>, grid, dim3(kAttnWaves * kWaveSize), 0, stream, p);
 }
 
 template <int HD>

@@ -211,13 +211,11 @@ __global__ void fill_zero_u32_kernel(unsigned* dst, size_t n) {
 }  // namespace
 
 int launch_xcd_probe(unsigned* where, int n, int stride_words, hipStream_t stream) {
-    hipLaunchKernelGGL(xcd_probe_kernel, dim3(unsigned(n)), dim3(kWaveSize), 0, stream, where, stride_words);
-    return int(hipGetLastError());
+    return enqueue(xcd_probe_kernel, dim3(unsigned(n)), dim3(kWaveSize), 0, stream, where, stride_words);
 }
 
 int launch_fill_zero_u32(unsigned* dst, size_t n, hipStream_t stream) {
-    hipLaunchKernelGGL(fill_zero_u32_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, stream, dst, n);
-    return int(hipGetLastError());
+    return enqueue(fill_zero_u32_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, stream, dst, n);
 }
 
 bool attn_mfma_can_merge_in_launch(int B, int KVH, bool coop, int num_splits) {
@@ -259,24 +257,25 @@ int launch_attn_splitkv_mfma(const AttnParams& params, int HD, int R, bool coop,
             p.part_o += row0 * HD;
             p.part_ml += row0;
         }
+        int rc;
         if (coop) {
             const dim3 grid(unsigned(p.KVH), unsigned(p.B), unsigned(p.num_splits));
             if (HD == 64 && p.tokens_per_split <= 2 * kMfmaWaves * 32) {
-                hipLaunchKernelGGL((attn_splitkv_mfma_kernel<64, true, 4>), grid, block, 0, stream, R, 0, p);
+                rc = enqueue(attn_splitkv_mfma_kernel<64, true, 4>, grid, block, 0, stream, R, 0, p);
             } else if (HD == 64) {
-                hipLaunchKernelGGL((attn_splitkv_mfma_kernel<64, true>), grid, block, 0, stream, R, 0, p);
+                rc = enqueue(attn_splitkv_mfma_kernel<64, true>, grid, block, 0, stream, R, 0, p);
             } else {
-                hipLaunchKernelGGL((attn_splitkv_mfma_kernel<128, true>), grid, block, 0, stream, R, 0, p);
+                rc = enqueue(attn_splitkv_mfma_kernel<128, true>, grid, block, 0, stream, R, 0, p);
             }
         } else {
             const dim3 grid(unsigned(p.KVH / hpw), unsigned(p.B), unsigned((p.num_splits + spw - 1) / spw));
             if (HD == 64) {
-                hipLaunchKernelGGL((attn_splitkv_mfma_kernel<64, false>), grid, block, 0, stream, R, hpw_log2, p);
+                rc = enqueue(attn_splitkv_mfma_kernel<64, false>, grid, block, 0, stream, R, hpw_log2, p);
             } else {
-                hipLaunchKernelGGL((attn_splitkv_mfma_kernel<128, false>), grid, block, 0, stream, R, hpw_log2, p);
+                rc = enqueue(attn_splitkv_mfma_kernel<128, false>, grid, block, 0, stream, R, hpw_log2, p);
             }
         }
-        if (const hipError_t e = hipGetLastError(); e != hipSuccess) return int(e);
+        if (rc != 0) return rc;
     }
     return 0;
 }

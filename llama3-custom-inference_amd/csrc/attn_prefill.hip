@@ -95,11 +95,10 @@ int launch_attn_prefill(const PrefillParams& p, int HD, hipStream_t stream) {
     const dim3 grid(unsigned(p.B) * unsigned(p.KVH) * unsigned(wgs_per_head));
     const dim3 block(kMfmaWaves * kWaveSize);
     if (HD == 64) {
-        hipLaunchKernelGGL((attn_prefill_mfma_kernel<64>), grid, block, 0, stream, p);
+        return enqueue(attn_prefill_mfma_kernel<64>, grid, block, 0, stream, p);
     } else {
-        hipLaunchKernelGGL((attn_prefill_mfma_kernel<128>), grid, block, 0, stream, p);
+        return enqueue(attn_prefill_mfma_kernel<128>, grid, block, 0, stream, p);
     }
-    return int(hipGetLastError());
 }
 
 }  // namespace l3

@@ -660,8 +660,7 @@ int launch_blocks(Kernel kernel, const PrefillParams& p, int waves, int col_bloc
     PrefillParams q = p;
     const int cus = current_device_cus();
     q.snake = (int64_t(grid.x) <= 4 * int64_t(cus)) ? cus : 0;
-    hipLaunchKernelGGL(kernel, grid, dim3(waves * kWaveSize), 0, stream, q);
-    return int(hipGetLastError());
+    return enqueue(kernel, grid, dim3(waves * kWaveSize), 0, stream, q);
 }
 
 }  // namespace

@@ -172,32 +172,29 @@ int launch_greedy_step(const uint16_t* logits, int64_t row_stride, int rows, int
                        int64_t* tokens, const uint8_t* text_mask, int64_t total_len, int64_t* tok, int* pos,
                        int* kv_len, uint8_t* eos, const int64_t* stop, int n_stop, hipStream_t stream) {
     const int parts = argmax_parts(V);
-    hipLaunchKernelGGL(argmax_partial_kernel, dim3(unsigned(parts), unsigned(rows)), dim3(kMiscThreads), 0, stream,
-                       logits, row_stride, V, kArgmaxChunk, part_val, part_idx);
-    hipLaunchKernelGGL(greedy_step_kernel, dim3(1), dim3(kGreedyThreads), 0, stream, part_val, part_idx, parts, rows,
-                       tokens, text_mask, total_len, tok, pos, kv_len, eos, stop, n_stop);
-    return int(hipGetLastError());
+    if (const int rc = enqueue(argmax_partial_kernel, dim3(unsigned(parts), unsigned(rows)), dim3(kMiscThreads), 0, stream,
+                               logits, row_stride, V, kArgmaxChunk, part_val, part_idx); rc != 0) return rc;
+    return enqueue(greedy_step_kernel, dim3(1), dim3(kGreedyThreads), 0, stream, part_val, part_idx, parts, rows,
+                   tokens, text_mask, total_len, tok, pos, kv_len, eos, stop, n_stop);
 }
 
 int launch_silu_mul_rows(const uint16_t* a, const uint16_t* b, uint16_t* y, int64_t rows, int64_t cols,
                          int64_t a_row_stride, int64_t b_row_stride, hipStream_t stream) {
     const int64_t vpr = cols / 8;
     const dim3 grid(unsigned((vpr + kMiscThreads - 1) / kMiscThreads), unsigned(std::min<int64_t>(rows, 65535)));
-    hipLaunchKernelGGL(silu_mul_kernel, grid, dim3(kMiscThreads), 0, stream, a, b, y, rows, vpr, a_row_stride,
-                       b_row_stride);
-    return int(hipGetLastError());
+    return enqueue(silu_mul_kernel, grid, dim3(kMiscThreads), 0, stream, a, b, y, rows, vpr, a_row_stride,
+                   b_row_stride);
 }
 
 int launch_silu_mul(const uint16_t* a, const uint16_t* b, uint16_t* y, int64_t n, bool vec_ok, hipStream_t stream) {
     if (vec_ok) {
         const int64_t nvec = n / 8;
-        hipLaunchKernelGGL(silu_mul_kernel, dim3(unsigned((nvec + kMiscThreads - 1) / kMiscThreads)),
-                           dim3(kMiscThreads), 0, stream, a, b, y, int64_t(1), nvec, int64_t(0), int64_t(0));
+        return enqueue(silu_mul_kernel, dim3(unsigned((nvec + kMiscThreads - 1) / kMiscThreads)),
+                       dim3(kMiscThreads), 0, stream, a, b, y, int64_t(1), nvec, int64_t(0), int64_t(0));
     } else {
-        hipLaunchKernelGGL(silu_mul_scalar_kernel, dim3(unsigned((n + kMiscThreads - 1) / kMiscThreads)),
-                           dim3(kMiscThreads), 0, stream, a, b, y, n);
+        return enqueue(silu_mul_scalar_kernel, dim3(unsigned((n + kMiscThreads - 1) / kMiscThreads)),
+                       dim3(kMiscThreads), 0, stream, a, b, y, n);
     }
-    return int(hipGetLastError());
 }
 
 int argmax_parts(int V) { return (V + kArgmaxChunk - 1) / kArgmaxChunk; }
@@ -205,11 +202,10 @@ int argmax_parts(int V) { return (V + kArgmaxChunk - 1) / kArgmaxChunk; }
 int launch_argmax(const uint16_t* logits, int64_t row_stride, int rows, int V, float* part_val, int* part_idx,
                   int64_t* out, hipStream_t stream) {
     const int parts = argmax_parts(V);
-    hipLaunchKernelGGL(argmax_partial_kernel, dim3(unsigned(parts), unsigned(rows)), dim3(kMiscThreads), 0, stream,
-                       logits, row_stride, V, kArgmaxChunk, part_val, part_idx);
-    hipLaunchKernelGGL(argmax_final_kernel, dim3(unsigned(rows)), dim3(kWaveSize), 0, stream, part_val, part_idx,
-                       parts, out);
-    return int(hipGetLastError());
+    if (const int rc = enqueue(argmax_partial_kernel, dim3(unsigned(parts), unsigned(rows)), dim3(kMiscThreads), 0, stream,
+                               logits, row_stride, V, kArgmaxChunk, part_val, part_idx); rc != 0) return rc;
+    return enqueue(argmax_final_kernel, dim3(unsigned(rows)), dim3(kWaveSize), 0, stream, part_val, part_idx,
+                   parts, out);
 }
 
 }  // namespace l3

@@ -61,17 +61,15 @@ int launch_hbm_rw_stream(const void* src, void* dst, size_t bytes, int workgroup
     uint4* d4 = static_cast<uint4*>(dst);
     const int64_t n16 = int64_t(bytes / 16);
     // a workgroup's trip moves kStreamThreads * 16 bytes per load in flight: 8, 16, 32 or 64 KiB
-    if (block_kib == 8) hipLaunchKernelGGL(hbm_rw_stream_kernel<1>, g, b, 0, stream, s4, d4, n16);
-    else if (block_kib == 16) hipLaunchKernelGGL(hbm_rw_stream_kernel<2>, g, b, 0, stream, s4, d4, n16);
-    else if (block_kib == 32) hipLaunchKernelGGL(hbm_rw_stream_kernel<4>, g, b, 0, stream, s4, d4, n16);
-    else hipLaunchKernelGGL(hbm_rw_stream_kernel<8>, g, b, 0, stream, s4, d4, n16);
-    return int(hipGetLastError());
+    if (block_kib == 8) return enqueue(hbm_rw_stream_kernel<1>, g, b, 0, stream, s4, d4, n16);
+    else if (block_kib == 16) return enqueue(hbm_rw_stream_kernel<2>, g, b, 0, stream, s4, d4, n16);
+    else if (block_kib == 32) return enqueue(hbm_rw_stream_kernel<4>, g, b, 0, stream, s4, d4, n16);
+    else return enqueue(hbm_rw_stream_kernel<8>, g, b, 0, stream, s4, d4, n16);
 }
 
 int launch_hbm_read_stream(const void* src, size_t bytes, void* sink, int workgroups, hipStream_t stream) {
-    hipLaunchKernelGGL(hbm_read_stream_kernel, dim3(unsigned(workgroups)), dim3(kStreamThreads), 0, stream,
-                       static_cast<const uint4*>(src), int64_t(bytes / 16), static_cast<uint32_t*>(sink));
-    return int(hipGetLastError());
+    return enqueue(hbm_read_stream_kernel, dim3(unsigned(workgroups)), dim3(kStreamThreads), 0, stream,
+                   static_cast<const uint4*>(src), int64_t(bytes / 16), static_cast<uint32_t*>(sink));
 }
 
 }  // namespace l3

@@ -324,9 +324,8 @@ int launch_variant(const LinearParams& p, hipStream_t stream) {
     const int rb_per_wg = NW / p.sk;
     const dim3 grid(unsigned((row_blocks + rb_per_wg - 1) / rb_per_wg));
     const size_t lds = XLDS ? size_t(p.M) * size_t(p.K + 8) * sizeof(uint16_t) : 0;
-    hipLaunchKernelGGL((linear_skinny_kernel<NW, CBLK, U, SWIGLU, XLDS, RW>), grid, dim3(NW * kWaveSize), lds, stream,
-                       p);
-    return int(hipGetLastError());
+    return enqueue(linear_skinny_kernel<NW, CBLK, U, SWIGLU, XLDS, RW>, grid, dim3(NW * kWaveSize), lds, stream,
+                   p);
 }
 
 }  // namespace

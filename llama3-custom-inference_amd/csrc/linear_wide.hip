@@ -298,9 +298,8 @@ int launch_variant(WideParams p, int ksplit, hipStream_t stream) {
     constexpr int N_WG = 16 * RF * WR / (OUT == WideOut::kSwiglu ? 2 : 1);
     p.row_groups = (p.N + N_WG - 1) / N_WG;
     p.chunks_per_split = (p.K / kWideChunk + ksplit - 1) / ksplit;
-    hipLaunchKernelGGL((linear_wide_kernel<CB, RF, WR, WC, WK, ST, OUT>), dim3(unsigned(p.row_groups) * unsigned(ksplit)),
-                       dim3(kWideWaves * kWaveSize), 0, stream, p);
-    return int(hipGetLastError());
+    return enqueue(linear_wide_kernel<CB, RF, WR, WC, WK, ST, OUT>, dim3(unsigned(p.row_groups) * unsigned(ksplit)),
+                   dim3(kWideWaves * kWaveSize), 0, stream, p);
 }
 
 // Blocks of 16 activation rows -> the kernel for them.
@@ -370,9 +369,8 @@ WideParams wide_params(const uint16_t* x, const uint16_t* w, int M, int N, int K
 
 int launch_linear_splitk_finish(const float* part, int ksplit, const uint16_t* res, uint16_t* y, int M, int N,
                                 int64_t y_stride, hipStream_t stream) {
-    hipLaunchKernelGGL(linear_splitk_finish_kernel, dim3(unsigned((N / 8 + 255) / 256), unsigned(M)), dim3(256), 0,
-                       stream, part, ksplit, int64_t(M) * N, res, y, N, y_stride);
-    return int(hipGetLastError());
+    return enqueue(linear_splitk_finish_kernel, dim3(unsigned((N / 8 + 255) / 256), unsigned(M)), dim3(256), 0,
+                   stream, part, ksplit, int64_t(M) * N, res, y, N, y_stride);
 }
 
 // Splits of K without regard to the activation rows: 128, 256, 512 k per split (1024 for matrices of few rows), the

@@ -268,9 +268,8 @@ add_rms_norm_partials_kernel(const uint16_t* __restrict__ x, const float* __rest
 int launch_add_rms_norm_partials(const uint16_t* x, const float* part, int ksplit, int64_t split_stride,
                                  const uint16_t* w, uint16_t* sum_out, uint16_t* y, int rows, int C, float eps,
                                  hipStream_t stream) {
-    hipLaunchKernelGGL(add_rms_norm_partials_kernel, dim3(unsigned(rows)), dim3(kRmsThreads), 0, stream, x, part,
-                       ksplit, split_stride, w, sum_out, y, C, eps);
-    return int(hipGetLastError());
+    return enqueue(add_rms_norm_partials_kernel, dim3(unsigned(rows)), dim3(kRmsThreads), 0, stream, x, part,
+                   ksplit, split_stride, w, sum_out, y, C, eps);
 }
 
 namespace {
@@ -285,30 +284,29 @@ int launch_rms_norm_impl(const uint16_t* x, const uint16_t* res, const uint16_t*
         const int64_t waves = std::min<int64_t>(rows / 2, int64_t(current_device_cus()) * 8);
         const dim3 grid(unsigned((waves + 3) / 4));
         if (nvec <= 64 * 4) {
-            hipLaunchKernelGGL((rms_norm_stream_kernel<4, ADD>), grid, block, 0, stream, x, res, w, sum_out, y, rows, C,
-                               eps);
+            return enqueue(rms_norm_stream_kernel<4, ADD>, grid, block, 0, stream, x, res, w, sum_out, y, rows, C,
+                           eps);
         } else {
-            hipLaunchKernelGGL((rms_norm_stream_kernel<8, ADD>), grid, block, 0, stream, x, res, w, sum_out, y, rows,
-                               C, eps);
+            return enqueue(rms_norm_stream_kernel<8, ADD>, grid, block, 0, stream, x, res, w, sum_out, y, rows,
+                           C, eps);
         }
     } else if (vec_ok && nvec <= 256 * 4) {
         // few rows (decode): the whole workgroup on one row keeps the latency short
         const dim3 grid{unsigned(rows)};
         if (nvec <= 256) {
-            hipLaunchKernelGGL((rms_norm_rows_kernel<256, 1, ADD>), grid, block, 0, stream, x, res, w, sum_out, y,
-                               rows, C, eps);
+            return enqueue(rms_norm_rows_kernel<256, 1, ADD>, grid, block, 0, stream, x, res, w, sum_out, y,
+                           rows, C, eps);
         } else if (nvec <= 512) {
-            hipLaunchKernelGGL((rms_norm_rows_kernel<256, 2, ADD>), grid, block, 0, stream, x, res, w, sum_out, y,
-                               rows, C, eps);
+            return enqueue(rms_norm_rows_kernel<256, 2, ADD>, grid, block, 0, stream, x, res, w, sum_out, y,
+                           rows, C, eps);
         } else {
-            hipLaunchKernelGGL((rms_norm_rows_kernel<256, 4, ADD>), grid, block, 0, stream, x, res, w, sum_out, y,
-                               rows, C, eps);
+            return enqueue(rms_norm_rows_kernel<256, 4, ADD>, grid, block, 0, stream, x, res, w, sum_out, y,
+                           rows, C, eps);
         }
     } else {
-        hipLaunchKernelGGL((rms_norm_generic_kernel<ADD>), dim3(unsigned(rows)), block, 0, stream, x, res, w, sum_out,
-                           y, C, eps);
+        return enqueue(rms_norm_generic_kernel<ADD>, dim3(unsigned(rows)), block, 0, stream, x, res, w, sum_out,
+                       y, C, eps);
     }
-    return int(hipGetLastError());
 }
 
 }  // namespace

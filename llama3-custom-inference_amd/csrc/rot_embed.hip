@@ -160,10 +160,9 @@ int launch_rot_embed_append(const uint16_t* qkv, const float* table, uint16_t* q
                             int64_t c_sb, int64_t c_st, int cache_len, int table_rows, hipStream_t stream) {
     const int items = B * (NH + 2 * KVH) * (HD / 8);
     const unsigned blocks = unsigned((items + kRopeThreads - 1) / kRopeThreads);
-    hipLaunchKernelGGL(rot_embed_append_kernel<false>, dim3(blocks), dim3(kRopeThreads), 0, stream, qkv, nullptr, 1,
-                       int64_t(0), table, q_out, cache_k, cache_v, pos_dev, items, NH, KVH, HD, qkv_sb, c_sb, c_st,
-                       cache_len, table_rows);
-    return int(hipGetLastError());
+    return enqueue(rot_embed_append_kernel<false>, dim3(blocks), dim3(kRopeThreads), 0, stream, qkv, nullptr, 1,
+                   int64_t(0), table, q_out, cache_k, cache_v, pos_dev, items, NH, KVH, HD, qkv_sb, c_sb, c_st,
+                   cache_len, table_rows);
 }
 
 int launch_rot_embed_append_partials(const float* part, int ksplit, int64_t split_stride, const float* table,
@@ -172,10 +171,9 @@ int launch_rot_embed_append_partials(const float* part, int ksplit, int64_t spli
                                      int table_rows, hipStream_t stream) {
     const int items = B * (NH + 2 * KVH) * (HD / 8);
     const unsigned blocks = unsigned((items + kRopeThreads - 1) / kRopeThreads);
-    hipLaunchKernelGGL(rot_embed_append_kernel<true>, dim3(blocks), dim3(kRopeThreads), 0, stream, nullptr, part,
-                       ksplit, split_stride, table, q_out, cache_k, cache_v, pos_dev, items, NH, KVH, HD,
-                       int64_t(NH + 2 * KVH) * HD, c_sb, c_st, cache_len, table_rows);
-    return int(hipGetLastError());
+    return enqueue(rot_embed_append_kernel<true>, dim3(blocks), dim3(kRopeThreads), 0, stream, nullptr, part,
+                   ksplit, split_stride, table, q_out, cache_k, cache_v, pos_dev, items, NH, KVH, HD,
+                   int64_t(NH + 2 * KVH) * HD, c_sb, c_st, cache_len, table_rows);
 }
 
 int launch_rot_embed(const uint16_t* x, const float* freq, uint16_t* y, int B, int T, int NH, int HD,
@@ -191,9 +189,9 @@ int launch_rot_embed(const uint16_t* x, const float* freq, uint16_t* y, int B, i
         const int vpr_shift = pow2 ? __builtin_ctz(unsigned(vpr)) : 0;
         const dim3 grid(unsigned((T + rpw - 1) / rpw), unsigned(B));
         const dim3 block(kRopeThreads);
-#define L3_ROPE_ROWS(HG, POW2)                                                                                       \
-    hipLaunchKernelGGL((rot_embed_rows_kernel<HG, POW2>), grid, block, 0, stream, x, freq, y, T, NH, HD, sb, st, sh, \
-                       tpr, vpr, rpw, tpr_shift, vpr_shift)
+#define L3_ROPE_ROWS(HG, POW2)                                                                                   \
+    return enqueue(rot_embed_rows_kernel<HG, POW2>, grid, block, 0, stream, x, freq, y, T, NH, HD, sb, st, sh, \
+                   tpr, vpr, rpw, tpr_shift, vpr_shift)
         if (hg == 4) {
             if (pow2) L3_ROPE_ROWS(4, true); else L3_ROPE_ROWS(4, false);
         } else if (hg == 2) {
@@ -205,15 +203,14 @@ int launch_rot_embed(const uint16_t* x, const float* freq, uint16_t* y, int B, i
     } else if (vec_ok) {
         const int64_t items = rows * (HD / 8);
         const unsigned blocks = unsigned((items + kRopeThreads - 1) / kRopeThreads);
-        hipLaunchKernelGGL(rot_embed_vec_kernel, dim3(blocks), dim3(kRopeThreads), 0, stream, x, freq, y, items, T,
-                           NH, HD, sb, st, sh);
+        return enqueue(rot_embed_vec_kernel, dim3(blocks), dim3(kRopeThreads), 0, stream, x, freq, y, items, T,
+                       NH, HD, sb, st, sh);
     } else {
         const int64_t items = rows * (HD / 2);
         const unsigned blocks = unsigned((items + kRopeThreads - 1) / kRopeThreads);
-        hipLaunchKernelGGL(rot_embed_pair_kernel, dim3(blocks), dim3(kRopeThreads), 0, stream, x, freq, y, items, T,
-                           NH, HD, sb, st, sh);
+        return enqueue(rot_embed_pair_kernel, dim3(blocks), dim3(kRopeThreads), 0, stream, x, freq, y, items, T,
+                       NH, HD, sb, st, sh);
     }
-    return int(hipGetLastError());
 }
 
 }  // namespace l3
