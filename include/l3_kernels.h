@@ -404,6 +404,26 @@ int l3_rot_embed_append_partials(const void* part, int ksplit, const float* freq
                                  const int64_t cache_strides[2], int cache_len, int table_rows, void* stream);
 
 /*
+ * All transformer layers of one decode step (model.py:143-150 for T == 1) for M <= 4 sequences in one launch: input
+ * norms, fused qkv projection with rotary embedding and cache append at *pos_dev, attention over the first
+ * *pos_dev + 1 cached tokens, output projection, SwiGLU MLP, residual additions, with the rounding points of the
+ * separate operators.  x, out: (M, C) bf16.  layers_dev: n_layer records of nine device pointers in device memory -- ln_1,
+ * c_attn, c_proj, ln_2, gate, up and down weights, key cache, value cache -- all 16-byte aligned and dense, caches
+ * (>= M, cache_len, KVH, HD) with strides {batch, token} and contiguous (KVH, HD).
+ * Built for the 1B architecture on a device of 256 compute units (l3_decode_layers_supported says so for the current
+ * one, L3_ERR_SHAPE elsewhere); every workgroup attends for itself, so meant for caches of a few hundred tokens.
+ * workspace: l3_decode_layers_workspace_bytes bytes, 256-byte aligned, zeroed once before the first launch and handed
+ * to one launch at a time.  The workgroups of a launch wait for each other; all waits are bounded.  If one runs out
+ * -- the device did not hold the whole launch at once, because something else occupied part of it -- the first
+ * word of the workspace is non-zero afterwards: results are void then, as are those of later launches with this workspace.
+ */
+int l3_decode_layers_supported(int M, int C, int H, int QH, int KVH, int HD);
+size_t l3_decode_layers_workspace_bytes(int M, int n_layer);
+int l3_decode_layers(const void* layers_dev, int n_layer, const void* x, void* out, int M, const float* freq_table,
+                     int table_rows, const int32_t* pos_dev, const int64_t cache_strides[2], int cache_len, float eps,
+                     void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * out[r] = index of the first maximum of the bf16 row logits[r*row_stride : r*row_stride + V]
  * (int64; a NaN counts as the maximum and the first one wins, as in torch.argmax): the greedy pick of model.py:371.  Two small
  * launches (per-chunk maxima into the caller's workspace of l3_argmax_workspace_bytes(rows, V)

@@ -21,7 +21,7 @@ EXT_SOURCE = os.path.join(CSRC, "torch_ops.cpp")
 EXT_PATH = os.path.join(PKG_DIR, "custom_kernels", "_l3torch.so")
 LIB_PATH = os.path.join(PKG_DIR, "custom_kernels", "libl3kernels.so")
 SOURCES = ["l3_api.hip", "attn_decode.hip", "attn_mfma.hip", "attn_prefill.hip", "attn_prefill_tiled.hip",
-           "linear_skinny.hip", "linear_wide.hip", "attn_combine.hip", "rms_norm.hip", "rot_embed.hip",
+           "linear_skinny.hip", "linear_wide.hip", "decode_layers.hip", "attn_combine.hip", "rms_norm.hip", "rot_embed.hip",
            "decode_misc.hip", "hbm_stream.hip"]
 
 HIPCC_FLAGS = [

@@ -847,6 +847,34 @@ int l3_rot_embed_append_partials(const void* part, int ksplit, const float* freq
                                             static_cast<hipStream_t>(stream)) == 0 ? L3_OK : L3_ERR_HIP;
 }
 
+int l3_decode_layers_supported(int M, int C, int H, int QH, int KVH, int HD) {
+    return decode_layers_supported(M, C, H, QH, KVH, HD, current_device_cus());
+}
+
+size_t l3_decode_layers_workspace_bytes(int M, int n_layer) {
+    if (M <= 0 || M > 4 || n_layer <= 0) return 0;
+    return decode_layers_workspace_bytes(M, n_layer);
+}
+
+int l3_decode_layers(const void* layers_dev, int n_layer, const void* x, void* out, int M, const float* freq_table,
+                     int table_rows, const int32_t* pos_dev, const int64_t cache_strides[2], int cache_len, float eps,
+                     void* workspace, size_t workspace_bytes, void* stream) {
+    if (!layers_dev || !x || !out || !freq_table || !pos_dev || !cache_strides || !workspace) return L3_ERR_NULL_POINTER;
+    if (M <= 0 || M > 4 || n_layer <= 0 || n_layer > 4096 || table_rows <= 0 || cache_len <= 0) return L3_ERR_SHAPE;
+    if (cache_strides[0] < 0 || cache_strides[0] % 8 || cache_strides[1] <= 0 || cache_strides[1] % 8 ||
+        cache_strides[1] >= kAttnMaxTokenStride)
+        return L3_ERR_STRIDE;
+    if (!aligned(layers_dev, 8) || !aligned(x, 16) || !aligned(out, 16) || !aligned(freq_table, 16) || !aligned(pos_dev, 4) ||
+        !aligned(workspace, kWorkspaceAlign))
+        return L3_ERR_ALIGNMENT;
+    if (workspace_bytes < decode_layers_workspace_bytes(M, n_layer)) return L3_ERR_WORKSPACE;
+    if (!decode_layers_supported(M, 2048, 8192, 32, 8, 64, current_device_cus())) return L3_ERR_SHAPE;
+    return launch_decode_layers(static_cast<const DecodeLayerPointers*>(layers_dev), n_layer, static_cast<const uint16_t*>(x),
+                                static_cast<uint16_t*>(out), M, freq_table, table_rows, pos_dev, cache_strides[0],
+                                cache_strides[1], cache_len, eps, 0.125f, workspace,
+                                static_cast<hipStream_t>(stream)) == 0 ? L3_OK : L3_ERR_HIP;
+}
+
 size_t l3_argmax_workspace_bytes(int rows, int V) {
     if (rows <= 0 || V <= 0) return 0;
     return size_t(rows) * size_t(argmax_parts(V)) * (sizeof(float) + sizeof(int));

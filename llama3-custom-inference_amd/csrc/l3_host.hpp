@@ -150,6 +150,17 @@ int launch_linear_splitk(const uint16_t* x, const uint16_t* w, float* part, int 
 int launch_linear_splitk_finish(const float* part, int ksplit, const uint16_t* res, uint16_t* y, int M, int N,
                                 int64_t y_stride, hipStream_t stream);
 int launch_linear_skinny(LinearParams p, bool swiglu, int num_cus, hipStream_t stream);
+// One transformer layer as the whole-step kernel takes it (all device pointers; row-major (rows, k) weights).
+struct DecodeLayerPointers {
+    const uint16_t *ln_1, *c_attn, *c_proj, *ln_2, *w_gate, *w_up, *w_down;
+    uint16_t *cache_k, *cache_v;
+};
+constexpr size_t kDecodeLayersControlBytes = 8192;
+bool decode_layers_supported(int M, int C, int H, int QH, int KVH, int HD, int num_cus);
+size_t decode_layers_workspace_bytes(int M, int n_layer);
+int launch_decode_layers(const DecodeLayerPointers* layers, int n_layer, const uint16_t* x, uint16_t* out, int M,
+                         const float* rope_table, int table_rows, const int* pos, int64_t c_sb, int64_t c_st, int cache_len,
+                         float eps, float scale, void* ws, hipStream_t stream);
 int launch_attn_prefill(const PrefillParams& p, int HD, hipStream_t stream);        // a wavefront per column group
 // Workgroups of the tiled prefill kernel: 16-column blocks per wavefront, wavefronts per workgroup
 // (small workgroups, several per compute unit).

@@ -20,7 +20,7 @@
 // 7.0 -> 6.5 us; vocabulary projection 128256 x 2048 107 (library GEMM) -> 95 us.
 #include <algorithm>
 
-#include "attn_mfma_core.hpp"
+#include "lds_loads.hpp"
 
 namespace l3 {
 
@@ -44,39 +44,6 @@ struct WideParams {
 };
 
 enum class WideOut { kPartials, kSwiglu, kRows };
-
-typedef uint32_t srd_t __attribute__((ext_vector_type(4)));   // a buffer resource: base, no range limit, raw
-
-__device__ __forceinline__ srd_t make_srd(const void* base) {
-    const uint64_t a = reinterpret_cast<uint64_t>(base);
-    srd_t r;
-    r.x = uint32_t(wave_uniform(int(uint32_t(a))));
-    r.y = uint32_t(wave_uniform(int(uint32_t(a >> 32) & 0xffffu)));
-    r.z = 0xffffffffu;
-    r.w = 0x00020000u;
-    return r;
-}
-
-// 16 bytes per lane from base + lane_off + uniform_off to LDS address lds + lane * 16 (lds is wave-uniform).
-// The compiler does not see the load: whoever reads that LDS waits for it with wait_loads().
-template <bool STREAM>
-__device__ __forceinline__ void load_to_lds(const srd_t& base, uint32_t lds, uint32_t lane_off, int uniform_off) {
-    if constexpr (STREAM) {
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
-                     ::"s"(lds), "v"(lane_off), "s"(base), "s"(uniform_off) : "memory");
-    } else {
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                     ::"s"(lds), "v"(lane_off), "s"(base), "s"(uniform_off) : "memory");
-    }
-}
-
-// Until at most NEWER of this wavefront's vector memory operations are outstanding.
-template <int NEWER>
-__device__ __forceinline__ void wait_loads() {
-    static_assert(NEWER < 64, "six bits");
-    __builtin_amdgcn_s_waitcnt((NEWER & 15) | ((NEWER >> 4) << 14) | 0x0F70);
-}
-__device__ __forceinline__ void barrier() { asm volatile("s_barrier" ::: "memory"); }
 
 // CB: blocks of 16 activation rows.  RF: blocks of 16 weight rows per wavefront (SwiGLU: half of them of each
 // matrix).  The eight wavefronts are WR (weight rows) x WC (activation rows) x WK (k steps of a stage); WK
@@ -106,7 +73,7 @@ linear_wide_kernel(const WideParams p) {
     const int n_chunks = min(p.K / kWideChunk, c0 + p.chunks_per_split) - c0;   // at least 1
 
     // loads: lane l of a load covers row l / 16 of its four rows, chunk position l % 16
-    const uint32_t ring = uint32_t(reinterpret_cast<uintptr_t>(L3_LDS_PTR(unsigned char, s_ring)));
+    const uint32_t ring = lds_address(s_ring);
     // (row groups of four are all inside N or all outside: those outside re-read the last one and are never stored;
     // one resource per load keeps the lane offsets below four row pitches)
     const int ld_row = lane >> 4;

@@ -382,6 +382,73 @@ def rot_embed_append_partials(part, freq_table, cache_k, cache_v, pos, n_head: i
     return _l3lib.native().rot_embed_append_partials(part, freq_table, cache_k, cache_v, pos, n_head)
 
 
+class DecodeLayers:
+    """All transformer layers of one decode step in one launch (l3_decode_layers), for up to four sequences of the
+    1B architecture.  ``layers``: dicts with ln_1, c_attn, c_proj, ln_2, c_fc2 (gate), c_fc (up), mlp_proj, cache_k and
+    cache_v.  The workgroups of a launch wait for each other, with bounds; ``failed()`` (it synchronises) says
+    whether a wait has run out: every result since then is void and the object of no more use, the operators one by
+    one do the same work.  One launch of an object at a time.  An extension."""
+
+    NAMES = ("ln_1", "c_attn", "c_proj", "ln_2", "c_fc2", "c_fc", "mlp_proj", "cache_k", "cache_v")
+
+    def __init__(self, layers, rows: int):
+        self.rows, self.n_layer = rows, len(layers)
+        self.tensors = [[L[n] for n in self.NAMES] for L in layers]     # kept alive
+        cache = layers[0]["cache_k"]
+        for L in layers:
+            for name in self.NAMES:
+                _require_gpu_bf16(name, L[name])
+                if not L[name].is_contiguous() or L[name].data_ptr() % 16 or L[name].shape != layers[0][name].shape \
+                        or L[name].device != cache.device:
+                    raise RuntimeError(f"DecodeLayers: {name} must be contiguous and alike in all layers")
+        maxB, self.cache_len, KVH, HD = cache.shape
+        H, C = layers[0]["c_fc"].shape
+        QH = layers[0]["c_attn"].shape[0] // HD - 2 * KVH
+        want = dict(ln_1=(C,), ln_2=(C,), c_attn=((QH + 2 * KVH) * HD, C), c_proj=(C, QH * HD), c_fc=(H, C), c_fc2=(H, C),
+                    mlp_proj=(C, H), cache_v=tuple(cache.shape))
+        wrong = [n for n, shape in want.items() if tuple(layers[0][n].shape) != shape]
+        with _on_device(cache.device):
+            if rows > maxB or wrong or not self.supported(rows, C, H, QH, KVH, HD):
+                raise RuntimeError(f"DecodeLayers: rows={rows} C={C} H={H} QH={QH} KVH={KVH} HD={HD} is not served {wrong}")
+            nbytes = _l3lib.load().l3_decode_layers_workspace_bytes(rows, self.n_layer)
+        self.table = torch.tensor([[t.data_ptr() for t in row] for row in self.tensors], dtype=torch.int64, device=cache.device)
+        self.workspace = torch.zeros(nbytes, dtype=torch.uint8, device=cache.device)
+        self.strides, self.C, self.HD = (cache.stride(0), cache.stride(1)), C, HD
+
+    def holds(self, layers) -> bool:
+        """Whether ``layers`` are still the tensors that this object was made for."""
+        return len(layers) == self.n_layer and all(L[n] is t for L, row in zip(layers, self.tensors)
+                                                   for n, t in zip(self.NAMES, row))
+
+    @staticmethod
+    def supported(rows: int, C: int, H: int, QH: int, KVH: int, HD: int) -> bool:
+        return bool(_l3lib.load().l3_decode_layers_supported(rows, C, H, QH, KVH, HD))
+
+    def __call__(self, x, freq_table, pos, eps: float):
+        """x (rows, 1, C) -> the hidden state behind the last layer, (rows, 1, C); keys and values are appended to the
+        caches at the device-side position ``pos``."""
+        _require_gpu_bf16("x", x)
+        if tuple(x.shape) != (self.rows, 1, self.C) or not x.is_contiguous() or x.device != self.table.device:
+            raise RuntimeError(f"DecodeLayers: x {tuple(x.shape)} does not fit ({self.rows}, 1, {self.C})")
+        if not freq_table.is_cuda or freq_table.dtype != torch.float32 or freq_table.dim() != 2 \
+                or freq_table.size(1) != self.HD or not freq_table.is_contiguous():
+            raise RuntimeError("freq_table must be a contiguous (rows, HD) float32 GPU tensor")
+        if not pos.is_cuda or pos.dtype != torch.int32 or pos.numel() != 1:
+            raise RuntimeError("pos must be a one-element int32 GPU tensor")
+        out = torch.empty_like(x)
+        with _on_device(x.device):
+            rc = _l3lib.load().l3_decode_layers(self.table.data_ptr(), self.n_layer, x.data_ptr(), out.data_ptr(), self.rows,
+                                                freq_table.data_ptr(), freq_table.size(0), pos.data_ptr(),
+                                                _l3lib.i64_array(self.strides), self.cache_len, float(eps),
+                                                self.workspace.data_ptr(), self.workspace.numel(), _stream_ptr(x.device))
+        if rc != 0:
+            _fail(rc, f"rows={self.rows} n_layer={self.n_layer}")
+        return out
+
+    def failed(self) -> bool:
+        return bool(self.workspace[:4].any().item())
+
+
 def argmax(logits):
     """Index of the first maximum along the last dimension of a 2-D bf16 tensor (rows, V), as
     int64 -- torch.argmax(logits.float(), dim=-1) for the greedy pick of model.py:371 (the float

@@ -103,6 +103,8 @@ class LlamaDecoder:
                                               scale_factor=c.rope_scale_factor, device=self.device)
         self.prefill_backend = "unset"
         self._graphs = {}
+        self._layer_launches = {}        # rows -> ops.DecodeLayers
+        self._layers_in_one_launch = hasattr(ops, "DecodeLayers")
         # nn.Linear calls with at most this many activation rows (the decode step) go through the
         # library's weight-streaming kernels when the operator module has them; 0 = always F.linear
         self.decode_linear_rows = 16 if hasattr(ops, "linear_decode") else 0
@@ -196,6 +198,31 @@ class LlamaDecoder:
         folded into the linears); 0 when the operator module has no such operator."""
         f = getattr(self.ops, "linear_decode_fused_max_rows", None)
         return min(self.decode_linear_rows, f(self.config.n_embd), self.FUSED_MAX_ROWS) if f else 0
+
+    # Positions (rows x length) up to which a decode step takes all layers in one launch: its workgroups each attend for
+    # themselves, which at 4096 positions has used up what it gains (us per 16 layers, against the operators: 1 row 256
+    # tokens 391 : 581, 2048 492 : 589, 4096 595 : 605; 2 rows 2048 616 : 636; 4 rows 256 504 : 740, 1024 654 : 739, 2048 866 : 764).
+    ONE_LAUNCH_MAX_POSITIONS = 4096
+
+    def _one_launch(self, rows: int, total_len: int):
+        """The single launch of all layers for a decode step of these rows, or None where the operators one by one take
+        it.  Who uses it looks at failed() before handing out results, and does the work again without it
+        (_give_up_one_launch) should it be true."""
+        c = self.config
+        if not self._layers_in_one_launch or not 0 < rows <= self._fused_rows() or rows * total_len > self.ONE_LAUNCH_MAX_POSITIONS:
+            return None
+        made = self._layer_launches.get(rows)
+        if made is None or not made.holds(self.layers):
+            with torch.cuda.device(self.device):
+                if not self.ops.DecodeLayers.supported(rows, c.n_embd, c.hidden_dim, c.n_head, c.n_kv_head, self.hd):
+                    return None
+            made = self._layer_launches[rows] = self.ops.DecodeLayers(self.layers, rows)
+        return made
+
+    def _give_up_one_launch(self):
+        self._layers_in_one_launch = False
+        self._layer_launches.clear()
+        self._graphs.clear()   # recorded decode steps contain it
 
     def _prefill_attention(self, q, k, v):
         """Causal GQA attention for T > 1.  The reference hands this case to torch
@@ -292,8 +319,12 @@ class LlamaDecoder:
             loop.graph.replay()
             if not ignore_eos and (cur_pos - min_prompt_len) % 16 == 0 and bool(loop.eos.all()):
                 break
+        rows = loop.tokens.tolist()
+        if loop.layers is not None and loop.layers.failed():
+            self._give_up_one_launch()
+            return self.generate_graphed(prompt_tokens, max_gen_len, echo, ignore_eos)
         out = []
-        for i, toks in enumerate(loop.tokens.tolist()):
+        for i, toks in enumerate(rows):
             start = 0 if echo else len(prompt_tokens[i])
             toks = toks[start:len(prompt_tokens[i]) + max_gen_len]
             for s_ in self.tokenizer.stop_tokens:
@@ -324,8 +355,15 @@ class LlamaDecoder:
         stop_tokens = torch.tensor(list(self.tokenizer.stop_tokens), device=self.device)
         eos_reached = torch.zeros(bsz, dtype=torch.bool, device=self.device)
         prev_pos = 0
+        layers = self._one_launch(bsz, total_len)
+        pos = torch.full((1,), min_prompt_len, dtype=torch.int32, device=self.device)
         for cur_pos in range(min_prompt_len, total_len):
-            logits = self.forward(tokens[:, prev_pos:cur_pos], start_pos=prev_pos)
+            if prev_pos == 0 or layers is None:
+                logits = self.forward(tokens[:, prev_pos:cur_pos], start_pos=prev_pos)
+            else:
+                x = layers(F.embedding(tokens[:, prev_pos:cur_pos], self.wte), self.freqs_cis, pos, c.norm_eps)
+                logits = self.ops.linear_decode_fused(x, self.wte, norm_weight=self.ln_f, eps=c.norm_eps).float()
+                pos += 1
             next_token = torch.argmax(logits[:, -1], dim=-1).reshape(-1)
             next_token = torch.where(input_text_mask[:, cur_pos], tokens[:, cur_pos], next_token)
             tokens[:, cur_pos] = next_token
@@ -333,8 +371,12 @@ class LlamaDecoder:
             prev_pos = cur_pos
             if not ignore_eos and bool(eos_reached.all()):
                 break
+        rows = tokens.tolist()
+        if layers is not None and layers.failed():
+            self._give_up_one_launch()
+            return self.generate(prompt_tokens, max_gen_len, temperature, echo, ignore_eos)
         out = []
-        for i, toks in enumerate(tokens.tolist()):
+        for i, toks in enumerate(rows):
             start = 0 if echo else len(prompt_tokens[i])
             toks = toks[start:len(prompt_tokens[i]) + max_gen_len]
             for s in self.tokenizer.stop_tokens:
@@ -370,6 +412,7 @@ class GraphedDecodeLoop:
         self.kv_len = _t.ones(1, dtype=_t.int32, device=dev)           # pos + 1
         self.eos = _t.zeros(batch, dtype=_t.bool, device=dev)
         self.stop = _t.tensor(list(model.tokenizer.stop_tokens), device=dev)
+        self.layers = model._one_launch(batch, total_len)
         self.graph = None
         self.prefill_graphs = {}   # prompt length -> (recorded prefill or None when it failed its check, logits)
 
@@ -377,7 +420,10 @@ class GraphedDecodeLoop:
         c, B = m.config, self.B
         ops = m.ops
         x = F.embedding(self.tok, m.wte)
-        if 0 < B <= m._fused_rows():
+        if self.layers is not None:
+            x = self.layers(x, m.freqs_cis, self.pos, c.norm_eps)
+            logits = ops.linear_decode_fused(x[:, -1], m.wte, norm_weight=m.ln_f, eps=c.norm_eps)
+        elif 0 < B <= m._fused_rows():
             # five launches per layer: norms, rotary embedding, cache append and residual additions ride
             # with the linears
             lin = ops.linear_decode_fused

@@ -1,0 +1,94 @@
+"""GPU parity: all layers of a decode step in one launch (l3_decode_layers) against float32 arithmetic on the same bf16
+weights, for every number of rows and at positions around the edges of its attention tiles (32 tokens, 256 per round of
+a row's wavefronts), and the way back to the operators when a launch has reported a wait that ran out."""
+
+import pytest
+import torch
+
+from helpers import randn_bf16
+
+pytestmark = pytest.mark.gpu
+
+C, H, QH, KVH, HD, EPS = 2048, 8192, 32, 8, 64, 1e-5
+
+
+def _layers(gpu, n, batch, length):
+    def w(seed, *shape):
+        return randn_bf16(shape, seed, scale=0.02).to(gpu)
+
+    return [dict(ln_1=(1 + w(i, C)), ln_2=(1 + w(i + 1, C)), c_attn=w(i + 2, (QH + 2 * KVH) * HD, C), c_proj=w(i + 3, C, C),
+                 c_fc2=w(i + 4, H, C), c_fc=w(i + 5, H, C), mlp_proj=w(i + 6, C, H),
+                 cache_k=randn_bf16((batch, length, KVH, HD), i + 7).to(gpu),
+                 cache_v=randn_bf16((batch, length, KVH, HD), i + 8).to(gpu)) for i in range(0, 10 * n, 10)]
+
+
+def _rotate(t, table):
+    a, b = t[..., 0::2], t[..., 1::2]
+    cos, sin = table[0::2], table[1::2]
+    return torch.stack((a * cos - b * sin, a * sin + b * cos), -1).flatten(-2)
+
+
+def _float32_step(x, layers, table, pos):
+    """Hidden state behind the layers and the appended (key, value) rows, without any intermediate rounding."""
+    x = x[:, 0].float()
+    B, rows = x.shape[0], []
+    for L in layers:
+        def norm(t, w):
+            return t * torch.rsqrt((t * t).mean(-1, keepdim=True) + EPS) * w.float()
+
+        q, k, v = (norm(x, L["ln_1"]) @ L["c_attn"].float().t()).split([QH * HD, KVH * HD, KVH * HD], -1)
+        q, k, v = _rotate(q.view(B, QH, HD), table[pos]), _rotate(k.view(B, KVH, HD), table[pos]), v.view(B, KVH, HD)
+        rows.append((k, v))
+        keys = torch.cat((L["cache_k"][:B, :pos].float(), k[:, None]), 1)
+        values = torch.cat((L["cache_v"][:B, :pos].float(), v[:, None]), 1)
+        score = (q.view(B, 1, KVH, QH // KVH, HD) * keys[:, :, :, None]).sum(-1) / HD ** 0.5
+        y = (torch.softmax(score, 1)[..., None] * values[:, :, :, None]).sum(1).reshape(B, C)
+        x = x + y @ L["c_proj"].float().t()
+        h = norm(x, L["ln_2"])
+        x = x + (torch.nn.functional.silu(h @ L["c_fc2"].float().t()) * (h @ L["c_fc"].float().t())) @ L["mlp_proj"].float().t()
+    return x, rows
+
+
+@pytest.mark.parametrize("B", [1, 2, 3, 4])
+def test_decode_layers_against_float32(gpu, B):
+    from custom_kernels import custom_kernels_extension as ops
+    from llama_arch import precompute_freqs_cis
+
+    layers = _layers(gpu, 2, B, 600)
+    one_launch = ops.DecodeLayers(layers, B)
+    table = precompute_freqs_cis(HD, 640, 500000.0, True, scale_factor=32.0, device=gpu)
+    for pos in (0, 31, 32, 127, 256, 599):
+        print(f"decode_layers B={B} pos={pos}", flush=True)
+        x = randn_bf16((B, 1, C), 900 + pos).to(gpu)
+        before = [(L["cache_k"].clone(), L["cache_v"].clone()) for L in layers]
+        want, rows = _float32_step(x, layers, table, pos)
+        y = one_launch(x, table, torch.tensor([pos], dtype=torch.int32, device=gpu), EPS)
+        assert not one_launch.failed()
+        # Per layer ten roundings to bf16 lie on the way (input norm, qkv, rotated q, attention weights and output, the two
+        # products with their additions, second norm, gate, silu and up with their product), each off by at most
+        # 2^-9 of its value and 2^-9 / sqrt(3) in the mean: sqrt(20) of those in two layers, 5.1e-3 of the result.
+        tol = 3 * 20 ** 0.5 * 2.0 ** -9 / 3 ** 0.5
+        assert (y[:, 0].float() - want).norm() <= tol * want.norm()
+        for L, (k0, v0), (k, v) in zip(layers, before, rows):
+            for cache, old, new in ((L["cache_k"], k0, k), (L["cache_v"], v0, v)):
+                assert (cache[:, pos].float() - new).norm() <= tol * new.norm()
+                cache[:, pos] = old[:, pos]
+                assert torch.equal(cache, old)      # nothing but the appended row has changed
+
+
+def test_generation_without_the_one_launch_after_a_wait_ran_out(gpu):
+    from custom_kernels import custom_kernels_extension as ops
+    from llama_arch import LlamaConfig, LlamaDecoder, random_prompts
+
+    m = LlamaDecoder(LlamaConfig(n_layer=2, vocab_size=4096, max_model_len=48, max_gen_batch_size=2), ops, gpu)
+    prompts = random_prompts(2, 16, 4096, 5)
+    for generate in (m.generate, m.generate_graphed):
+        m._layers_in_one_launch = True
+        first = generate(prompts, 16, ignore_eos=True)
+        assert m._layers_in_one_launch and not m._layer_launches[2].failed()
+        with torch.inference_mode():
+            m._layer_launches[2].workspace[0] = 1       # what a launch leaves when a wait has run out
+        again = generate(prompts, 16, ignore_eos=True)
+        assert not m._layers_in_one_launch
+        assert again == generate(prompts, 16, ignore_eos=True)
+        assert len(first[0]) == len(again[0]) == 16
