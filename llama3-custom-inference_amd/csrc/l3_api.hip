@@ -877,7 +877,7 @@ int l3_decode_layers(const void* layers_dev, int n_layer, const void* x, void* o
 
 size_t l3_argmax_workspace_bytes(int rows, int V) {
     if (rows <= 0 || V <= 0) return 0;
-    return size_t(rows) * size_t(argmax_parts(V)) * (sizeof(float) + sizeof(int));
+    return size_t(rows) * size_t(argmax_parts(V)) * sizeof(uint64_t);
 }
 
 int l3_argmax(const void* logits, int64_t row_stride, int rows, int V, void* workspace, size_t workspace_bytes,
@@ -887,10 +887,7 @@ int l3_argmax(const void* logits, int64_t row_stride, int rows, int V, void* wor
     if (row_stride < V) return L3_ERR_STRIDE;
     if (!aligned(logits, 2) || !aligned(out, 8) || !aligned(workspace, 8)) return L3_ERR_ALIGNMENT;
     if (workspace_bytes < l3_argmax_workspace_bytes(rows, V)) return L3_ERR_WORKSPACE;
-    const size_t parts = size_t(rows) * size_t(argmax_parts(V));
-    float* pv = static_cast<float*>(workspace);
-    int* pi = reinterpret_cast<int*>(pv + parts);
-    return launch_argmax(static_cast<const uint16_t*>(logits), row_stride, rows, V, pv, pi, out,
+    return launch_argmax(static_cast<const uint16_t*>(logits), row_stride, rows, V, static_cast<uint64_t*>(workspace), out,
                          static_cast<hipStream_t>(stream)) == 0 ? L3_OK : L3_ERR_HIP;
 }
 
@@ -905,11 +902,8 @@ int l3_greedy_step(const void* logits, int64_t row_stride, int rows, int V, void
         !aligned(kv_len, 4) || (stop_tokens && !aligned(stop_tokens, 8)))
         return L3_ERR_ALIGNMENT;
     if (workspace_bytes < l3_argmax_workspace_bytes(rows, V)) return L3_ERR_WORKSPACE;
-    const size_t parts = size_t(rows) * size_t(argmax_parts(V));
-    float* pv = static_cast<float*>(workspace);
-    int* pi = reinterpret_cast<int*>(pv + parts);
-    return launch_greedy_step(static_cast<const uint16_t*>(logits), row_stride, rows, V, pv, pi, tokens, text_mask,
-                              total_len, tok, pos, kv_len, eos, stop_tokens, n_stop,
+    return launch_greedy_step(static_cast<const uint16_t*>(logits), row_stride, rows, V, static_cast<uint64_t*>(workspace),
+                              tokens, text_mask, total_len, tok, pos, kv_len, eos, stop_tokens, n_stop,
                               static_cast<hipStream_t>(stream)) == 0 ? L3_OK : L3_ERR_HIP;
 }
 

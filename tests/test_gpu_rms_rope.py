@@ -313,6 +313,24 @@ def test_argmax_treats_nan_as_the_maximum_like_torch(gpu):
     np.testing.assert_array_equal(out.numpy(), np.array([4000, 17, 0, 7, 0, V - 1]))
 
 
+@pytest.mark.parametrize("rows,V,offset", [(1, 2047, 0), (2, 2056, 0), (300, 16385, 0), (256, 16392, 0), (257, 16384, 1), (3, 9, 5)])
+def test_argmax_edges_of_the_chunks(gpu, rows, V, offset):
+    """The largest logit first, last and around the places where a workgroup's or a load's logits end, for 2048 and 8192
+    logits per workgroup, with and without 16-byte alignment; and rows of both zeros, which are equal."""
+    from custom_kernels import custom_kernels_extension as cke
+
+    flat = torch.zeros(rows * V + offset, dtype=torch.bfloat16)
+    x = flat[offset:].view(rows, V)
+    x[:] = -randn_bf16((rows, V), 95).abs() - 1
+    places = [p for p in (0, 7, 8, V // 8 * 8 - 1, V // 8 * 8, 2047, 2048, 8191, 8192, V - 1) if p < V]
+    for r in range(rows):
+        p = places[r % len(places)]
+        x[r, p] = -0.0
+        x[r, p + 1:p + 2] = 0.0
+    got = cke.argmax(flat.to(gpu)[offset:].view(rows, V)).cpu()
+    np.testing.assert_array_equal(got.numpy(), [places[r % len(places)] for r in range(rows)])
+
+
 @pytest.mark.parametrize("rows,V,L,pos0", [(1, 128256, 256, 127), (64, 128256, 256, 200), (5, 1000, 20, 7), (3, 50, 9, 8)])
 def test_greedy_step_matches_generate_bookkeeping(gpu, rows, V, L, pos0):
     """argmax + the per-token bookkeeping of generate() (model.py:371-378) in place on the device,
