@@ -367,6 +367,14 @@ int l3_linear_splitk(const void* x, const void* w, void* part, size_t part_bytes
                      int64_t x_stride, int64_t w_stride, int ksplit, void* stream);
 
 /*
+ * l3_linear_qkv_rope_append without a norm for up to 64 activation rows: 1 <= B <= L3_LINEAR_SPLITK_MAX_ROWS,
+ * K % 128 == 0, strides and alignment as for l3_linear_splitk; the same rounding points, sums in another order.
+ */
+int l3_linear_qkv_rope_append_rows(const void* x, const void* w_qkv, const float* freq_table, void* q_out, void* cache_k,
+                                   void* cache_v, const int32_t* pos_dev, int B, int NH, int KVH, int HD, int K, int64_t x_stride,
+                                   int64_t w_stride, const int64_t cache_strides[2], int cache_len, int table_rows, void* stream);
+
+/*
  * y = x . w^T, or with w_up != NULL bf16(silu(x . w^T)) * bf16(x . w_up^T), plus the residual (M, N; y's row
  * stride) with a rounding of its own if that is not NULL, for up to 64 activation rows in one
  * launch without splits: for matrices whose rows alone fill the device (gate|up pair, vocabulary

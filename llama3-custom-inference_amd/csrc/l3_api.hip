@@ -647,14 +647,6 @@ int l3_silu_mul(const void* a, const void* b, void* y, int64_t n, void* stream) 
 
 namespace {
 
-struct QkvTarget {
-    const float* table;
-    const int* pos;
-    uint16_t *q_out, *cache_k, *cache_v;
-    int NH, KVH, HD, cache_len, table_rows;
-    int64_t c_sb, c_st;
-};
-
 int linear_decode_impl(const void* x, const void* norm_w, float norm_eps, const void* w0, const void* w1,
                        const void* res, void* y, int M, int N, int K, int64_t x_stride, int64_t w_stride,
                        int64_t y_stride, bool swiglu, void* stream, const QkvTarget* qkv = nullptr) {
@@ -713,11 +705,9 @@ int l3_linear_decode_fused(const void* x, const void* norm_weight, float norm_ep
                               w_up != nullptr, stream);
 }
 
-int l3_linear_qkv_rope_append(const void* x, const void* norm_weight, float norm_eps, const void* w_qkv,
-                              const float* freq_table, void* q_out, void* cache_k, void* cache_v,
-                              const int32_t* pos_dev, int B, int NH, int KVH, int HD, int K, int64_t x_stride,
-                              int64_t w_stride, const int64_t cache_strides[2], int cache_len, int table_rows,
-                              void* stream) {
+static int check_qkv_target(const float* freq_table, const void* q_out, const void* cache_k, const void* cache_v,
+                            const int32_t* pos_dev, int B, int NH, int KVH, int HD, const int64_t cache_strides[2], int cache_len,
+                            int table_rows) {
     if (!freq_table || !q_out || !cache_k || !cache_v || !pos_dev || !cache_strides) return L3_ERR_NULL_POINTER;
     if (NH <= 0 || KVH <= 0 || HD <= 0 || HD % 8 != 0 || cache_len <= 0 || table_rows <= 0) return L3_ERR_SHAPE;
     if (int64_t(NH + 2 * KVH) * HD > (1 << 24)) return L3_ERR_SHAPE;
@@ -726,16 +716,37 @@ int l3_linear_qkv_rope_append(const void* x, const void* norm_weight, float norm
     if (!aligned(q_out, 16) || !aligned(cache_k, 16) || !aligned(cache_v, 16) || !aligned(freq_table, 16) ||
         !aligned(pos_dev, 4))
         return L3_ERR_ALIGNMENT;
-    QkvTarget t;
-    t.table = freq_table; t.pos = pos_dev;
-    t.q_out = static_cast<uint16_t*>(q_out);
-    t.cache_k = static_cast<uint16_t*>(cache_k);
-    t.cache_v = static_cast<uint16_t*>(cache_v);
-    t.NH = NH; t.KVH = KVH; t.HD = HD; t.cache_len = cache_len; t.table_rows = table_rows;
-    t.c_sb = cache_strides[0]; t.c_st = cache_strides[1];
+    return L3_OK;
+}
+
+int l3_linear_qkv_rope_append(const void* x, const void* norm_weight, float norm_eps, const void* w_qkv,
+                              const float* freq_table, void* q_out, void* cache_k, void* cache_v,
+                              const int32_t* pos_dev, int B, int NH, int KVH, int HD, int K, int64_t x_stride,
+                              int64_t w_stride, const int64_t cache_strides[2], int cache_len, int table_rows,
+                              void* stream) {
+    if (const int rc = check_qkv_target(freq_table, q_out, cache_k, cache_v, pos_dev, B, NH, KVH, HD, cache_strides, cache_len,
+                                        table_rows); rc != L3_OK) return rc;
+    const QkvTarget t = {freq_table, pos_dev, static_cast<uint16_t*>(q_out), static_cast<uint16_t*>(cache_k),
+                         static_cast<uint16_t*>(cache_v), NH, KVH, HD, cache_len, table_rows, cache_strides[0], cache_strides[1]};
     const int N = (NH + 2 * KVH) * HD;
     return linear_decode_impl(x, norm_weight, norm_eps, w_qkv, nullptr, nullptr, nullptr, B, N, K, x_stride, w_stride,
                               N, false, stream, &t);
+}
+
+int l3_linear_qkv_rope_append_rows(const void* x, const void* w_qkv, const float* freq_table, void* q_out, void* cache_k,
+                                   void* cache_v, const int32_t* pos_dev, int B, int NH, int KVH, int HD, int K, int64_t x_stride,
+                                   int64_t w_stride, const int64_t cache_strides[2], int cache_len, int table_rows, void* stream) {
+    if (const int rc = check_qkv_target(freq_table, q_out, cache_k, cache_v, pos_dev, B, NH, KVH, HD, cache_strides, cache_len,
+                                        table_rows); rc != L3_OK) return rc;
+    if (!x || !w_qkv) return L3_ERR_NULL_POINTER;
+    if (B <= 0 || B > L3_LINEAR_SPLITK_MAX_ROWS || K <= 0 || K % 128 != 0 || K > (1 << 24)) return L3_ERR_SHAPE;
+    if (x_stride < K || w_stride < K || x_stride % 8 || w_stride % 8 || x_stride > kLinearMaxPitch || w_stride > kLinearMaxPitch)
+        return L3_ERR_STRIDE;
+    if (!aligned(x, 16) || !aligned(w_qkv, 16)) return L3_ERR_ALIGNMENT;
+    const QkvTarget t = {freq_table, pos_dev, static_cast<uint16_t*>(q_out), static_cast<uint16_t*>(cache_k),
+                         static_cast<uint16_t*>(cache_v), NH, KVH, HD, cache_len, table_rows, cache_strides[0], cache_strides[1]};
+    return launch_linear_wide_qkv(static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w_qkv), t, B, (NH + 2 * KVH) * HD, K,
+                                  x_stride, w_stride, current_device_cus(), static_cast<hipStream_t>(stream)) == 0 ? L3_OK : L3_ERR_HIP;
 }
 
 int l3_silu_mul_rows(const void* a, const void* b, void* y, int64_t rows, int64_t cols, int64_t a_row_stride,

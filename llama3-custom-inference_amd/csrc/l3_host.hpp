@@ -145,6 +145,16 @@ int linear_splitk_max_chunks(int N, int K, int num_cus);
 constexpr int64_t kLinearMaxPitch = int64_t(1) << 28;   // elements between two rows of the wide kernel's operands
 int launch_linear_wide(const uint16_t* x, const uint16_t* w, const uint16_t* w_up, const uint16_t* res, uint16_t* y, int M,
                        int N, int K, int64_t x_stride, int64_t w_stride, int64_t y_stride, int num_cus, hipStream_t stream);
+// Where the outputs of a qkv projection go: rotary table and position, rotated queries, key and value cache.
+struct QkvTarget {
+    const float* table;
+    const int* pos;
+    uint16_t *q_out, *cache_k, *cache_v;
+    int NH, KVH, HD, cache_len, table_rows;
+    int64_t c_sb, c_st;
+};
+int launch_linear_wide_qkv(const uint16_t* x, const uint16_t* w, const QkvTarget& target, int M, int N, int K, int64_t x_stride,
+                           int64_t w_stride, int num_cus, hipStream_t stream);
 int launch_linear_splitk(const uint16_t* x, const uint16_t* w, float* part, int M, int N, int K, int64_t x_stride,
                          int64_t w_stride, int ksplit, int num_cus, hipStream_t stream);
 int launch_linear_splitk_finish(const float* part, int ksplit, const uint16_t* res, uint16_t* y, int M, int N,

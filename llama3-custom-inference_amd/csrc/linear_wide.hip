@@ -41,13 +41,34 @@ struct WideParams {
     uint32_t x_pitch, w_pitch;   // bytes from a row to the next
     int64_t y_stride;
     int row_groups, chunks_per_split;
+    QkvTarget qkv;
 };
 
-enum class WideOut { kPartials, kSwiglu, kRows };
+enum class WideOut { kPartials, kSwiglu, kRows, kQkv };
+
+// Features n .. n + 3 (n % 4 == 0) of activation row m of a qkv projection, rounded to bf16: query and key pairs are
+// rotated at the device-side position, keys and values go into the cache row of that position (model.py:100-106).
+__device__ __forceinline__ void store_qkv(const QkvTarget& t, int m, int n, const f32x4_t& s) {
+    const int pos = *t.pos;
+    if (pos < 0 || pos >= t.cache_len || pos >= t.table_rows) return;   // never write outside the cache
+    const int slot = n / t.HD, d = n % t.HD;
+    uint2 v = make_uint2(pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3]));
+    uint16_t* to = t.q_out + (int64_t(m) * t.NH + slot) * t.HD + d;
+    if (slot < t.NH + t.KVH) {
+        const float4 cs = *reinterpret_cast<const float4*>(t.table + int64_t(pos) * t.HD + d);
+        v.x = rotate_pair(v.x, cs.x, cs.y);
+        v.y = rotate_pair(v.y, cs.z, cs.w);
+        if (slot >= t.NH) to = t.cache_k + m * t.c_sb + pos * t.c_st + (slot - t.NH) * t.HD + d;
+    } else {
+        to = t.cache_v + m * t.c_sb + pos * t.c_st + (slot - t.NH - t.KVH) * t.HD + d;
+    }
+    *reinterpret_cast<uint2*>(to) = v;
+}
 
 // CB: blocks of 16 activation rows.  RF: blocks of 16 weight rows per wavefront (SwiGLU: half of them of each
 // matrix).  The eight wavefronts are WR (weight rows) x WC (activation rows) x WK (k steps of a stage); WK
-// of them meet in LDS at the end.  A workgroup is one (row group, k range).
+// of them meet in LDS at the end.  A workgroup is one (row group, k range), or with kQkv one (row group, 16 CB of the
+// activation rows).
 template <int CB, int RF, int WR, int WC, int WK, int ST, WideOut OUT>
 __global__ void __launch_bounds__(kWideWaves * kWaveSize)
 linear_wide_kernel(const WideParams p) {
@@ -67,7 +88,8 @@ linear_wide_kernel(const WideParams p) {
     const int wave = wave_uniform(int(threadIdx.x) / kWaveSize);
     const int fn = lane & 15, fg = lane >> 4;
     const int wr = wave % WR, wc = (wave / WR) % WC, wk = wave / (WR * WC);
-    const int group = int(blockIdx.x) % p.row_groups, split = int(blockIdx.x) / p.row_groups;
+    const int group = int(blockIdx.x) % p.row_groups, part = int(blockIdx.x) / p.row_groups;
+    const int split = OUT == WideOut::kQkv ? 0 : part, m0 = OUT == WideOut::kQkv ? part * (CB * 16) : 0;
     const int n0 = group * N_WG;
     const int c0 = split * p.chunks_per_split;
     const int n_chunks = min(p.K / kWideChunk, c0 + p.chunks_per_split) - c0;   // at least 1
@@ -90,7 +112,7 @@ linear_wide_kernel(const WideParams p) {
 #pragma unroll
     for (int j = 0; j < XI; ++j) {
         const int first = ((wave * XI + j) % (CB * 4)) * 4;
-        const int row = min(first, p.M - 1);
+        const int row = min(m0 + first, p.M - 1);
         bx[j] = make_srd(reinterpret_cast<const char*>(p.x) + int64_t(row) * p.x_pitch);
         xoff[j] = uint32_t(min(ld_row, p.M - 1 - row)) * p.x_pitch + uint32_t(((lane & 15) ^ ((first + ld_row) & 15)) * 16);
     }
@@ -163,10 +185,12 @@ linear_wide_kernel(const WideParams p) {
 
     // acc[r][c][i]: weight row 16 block + 4 fg + i against activation row 16 (wc CBW + c) + fn
     auto store = [&](int block, int cblock, int l, const f32x4_t& s, const f32x4_t& u) __attribute__((always_inline)) {
-        const int m = cblock * 16 + (l & 15), n = n0 + block * 16 + 4 * (l >> 4);
+        const int m = m0 + cblock * 16 + (l & 15), n = n0 + block * 16 + 4 * (l >> 4);
         if (m >= p.M || n >= p.N) return;
         if constexpr (OUT == WideOut::kPartials) {
             *reinterpret_cast<f32x4_t*>(p.part + (int64_t(split) * p.M + m) * p.N + n) = s;
+        } else if constexpr (OUT == WideOut::kQkv) {
+            store_qkv(p.qkv, m, n, s);
         } else {
             float o[4];
 #pragma unroll
@@ -261,10 +285,10 @@ linear_wide_kernel(const WideParams p) {
 }
 
 template <int CB, int RF, int WR, int WC, int WK, int ST, WideOut OUT>
-int launch_variant(WideParams p, int ksplit, hipStream_t stream) {
+int launch_variant(WideParams p, int ksplit, hipStream_t stream) {   // (kQkv: groups of activation rows)
     constexpr int N_WG = 16 * RF * WR / (OUT == WideOut::kSwiglu ? 2 : 1);
     p.row_groups = (p.N + N_WG - 1) / N_WG;
-    p.chunks_per_split = (p.K / kWideChunk + ksplit - 1) / ksplit;
+    p.chunks_per_split = OUT == WideOut::kQkv ? p.K / kWideChunk : (p.K / kWideChunk + ksplit - 1) / ksplit;
     return enqueue(linear_wide_kernel<CB, RF, WR, WC, WK, ST, OUT>, dim3(unsigned(p.row_groups) * unsigned(ksplit)),
                    dim3(kWideWaves * kWaveSize), 0, stream, p);
 }
@@ -329,6 +353,7 @@ WideParams wide_params(const uint16_t* x, const uint16_t* w, int M, int N, int K
     p.x_pitch = uint32_t(x_stride * 2);
     p.w_pitch = uint32_t(w_stride * 2);
     p.y_stride = N;
+    p.qkv = QkvTarget{};
     return p;
 }
 
@@ -369,6 +394,26 @@ int launch_linear_splitk(const uint16_t* x, const uint16_t* w, float* part, int 
     // more than one workgroup per unit: rings of two stages, so that two fit
     if (wgs64 > num_cus) return launch_by_rows<2, 2, WideOut::kPartials>(p, ksplit, stream);
     return launch_by_rows<2, 4, WideOut::kPartials>(p, ksplit, stream);
+}
+
+// The qkv projection of a decode step with rotary embedding and cache append behind it: no splits, so that the sums
+// are whole where they are rotated.  32 weight rows per workgroup leave most units idle at one workgroup per row
+// group, and the activations, not the weights, are most of what such a workgroup loads: so the activation rows are dealt
+// to 16, 32 or 64 per workgroup, as few as the units have room for (the groups of a weight row share an XCD's L2).
+// A second round of workgroups costs more than it saves.  Split-K linear and the append that adds it up, one launch with
+// 64 / 32 / 16 rows per workgroup, us: 3072 x 2048, 17 rows 7.9, 7.2 / 7.2 / 6.4, 32 rows 8.2, 8.0 / 7.7 / 7.2, 64 rows 9.6,
+// 9.9 / 7.8 / 11.0; 6144 x 4096, 32 rows 14.7, - / 13.5 / 21.1, 64 rows 17.9, 17.5 / 22.6 / 30.6.  Up to 16 rows (against the
+// skinny kernel's epilogue): 3072 x 2048, 5 rows 6.7, 6.4, 16 rows 7.8, 7.4; 6144 x 4096, 16.4, 10.9 and 20.7, 12.6.
+int launch_linear_wide_qkv(const uint16_t* x, const uint16_t* w, const QkvTarget& target, int M, int N, int K, int64_t x_stride,
+                           int64_t w_stride, int num_cus, hipStream_t stream) {
+    WideParams p = wide_params(x, w, M, N, K, x_stride, w_stride);
+    p.qkv = target;
+    const int row_groups = (N + 31) / 32;
+    auto room = [&](int rows) { return M <= rows || row_groups * ((M + rows - 1) / rows) <= num_cus; };
+    if (room(16)) return launch_variant<1, 1, 2, 1, 4, 6, WideOut::kQkv>(p, (M + 15) / 16, stream);
+    if (room(32)) return launch_variant<2, 1, 2, 1, 4, 4, WideOut::kQkv>(p, (M + 31) / 32, stream);
+    if (M <= 48) return launch_variant<3, 1, 2, 1, 4, 6, WideOut::kQkv>(p, 1, stream);
+    return launch_variant<4, 1, 2, 1, 4, 6, WideOut::kQkv>(p, 1, stream);
 }
 
 // The whole sums in one launch: y, or with w_up the SwiGLU product, plus the residual if there is one.

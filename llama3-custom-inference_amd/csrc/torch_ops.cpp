@@ -41,7 +41,7 @@ using at::TensorBase;
     X(l3_attn_workspace_init) X(l3_attn_prefill) X(l3_rms_norm) X(l3_add_rms_norm) X(l3_add_rms_norm_partials)   \
     X(l3_rot_embed) X(l3_rot_embed_append_partials) X(l3_silu_mul) X(l3_silu_mul_rows)       \
     X(l3_linear_decode_fused) X(l3_linear_qkv_rope_append) X(l3_linear_splitk_rows_plan)   \
-    X(l3_linear_splitk) X(l3_linear_splitk_finish) X(l3_linear_wide)
+    X(l3_linear_splitk) X(l3_linear_splitk_finish) X(l3_linear_wide) X(l3_linear_qkv_rope_append_rows)
 
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
@@ -662,6 +662,26 @@ PyObject* linear_qkv_rope_append(PyObject* const* a) {
     return wrap(std::move(out));
 }
 
+// (x, w_qkv, freq_table, cache_k, cache_v, pos, n_head)
+PyObject* linear_qkv_rope_append_rows(PyObject* const* a) {
+    const Tensor& x = gpu_bf16(a[0], "x");
+    const Tensor& w = gpu_bf16(a[1], "weight");
+    const Rows r = linear_rows(x, L3_LINEAR_SPLITK_MAX_ROWS);
+    check_weight(w, w, x, r.K);
+    const Cache c = cache_args(a[2], a[3], a[4], a[5]);
+    const int64_t NH = integer(a[6]);
+    TORCH_CHECK(size_at(w, 0) == (NH + 2 * c.KVH) * c.HD && r.rows <= c.maxB, "w_qkv ", w.sizes(), " does not match n_head=", NH,
+                ", cache ", c.k->sizes());
+    Tensor out = new_empty({r.rows, 1, NH, c.HD}, x);
+    const OnDevice on(x);
+    check(lib.l3_linear_qkv_rope_append_rows(r.x, ptr(w), static_cast<const float*>(ptr(*c.table)), ptr(out), ptr(*c.k), ptr(*c.v),
+                                             static_cast<const int32_t*>(ptr(*c.pos)), int(r.rows), int(NH), int(c.KVH), int(c.HD),
+                                             int(r.K), r.stride, stride_at(w, 0), c.k->strides().data(), int(c.L),
+                                             int(size_at(*c.table, 0)), on.stream),
+          "B=", r.rows, " NH=", NH, " KVH=", c.KVH, " HD=", c.HD, " K=", r.K);
+    return wrap(std::move(out));
+}
+
 // (part, freq_table, cache_k, cache_v, pos, n_head)
 PyObject* rot_embed_append_partials(PyObject* const* a) {
     const Tensor& part = partials(a[0], "rot_embed_append_partials");
@@ -740,6 +760,7 @@ PyMethodDef methods[] = {
     ENTRY(linear_splitk, 3),
     ENTRY(linear_splitk_finish, 2),
     ENTRY(linear_qkv_rope_append, 9),
+    ENTRY(linear_qkv_rope_append_rows, 7),
     ENTRY(rot_embed_append_partials, 6),
     {nullptr, nullptr, 0, nullptr},
 };

@@ -305,6 +305,11 @@ def linear_qkv_rope_append(x, w_qkv, freq_table, cache_k, cache_v, pos, n_head: 
     return _l3lib.native().linear_qkv_rope_append(x, w_qkv, freq_table, cache_k, cache_v, pos, n_head, norm_weight, eps)
 
 
+def linear_qkv_rope_append_rows(x, w_qkv, freq_table, cache_k, cache_v, pos, n_head: int):
+    """linear_qkv_rope_append without a norm for up to 64 sequences: x (B, 1, K), K a multiple of 128.  An extension."""
+    return _l3lib.native().linear_qkv_rope_append_rows(x, w_qkv, freq_table, cache_k, cache_v, pos, n_head)
+
+
 def rms_norm(input, weight, eps):
     """input (B, T, C) bf16, weight (C,) bf16 -> (B, T, C) bf16 (model.py:70-72)."""
     return _l3lib.native().rms_norm(input, weight, eps)

@@ -166,27 +166,26 @@ class LlamaDecoder:
         return y.transpose(1, 2).contiguous().view(B, T, c.n_embd)
 
     FUSED_MAX_ROWS = 4   # rows up to which the fused single-launch linears carry the whole decode step
-    QKV_FUSED_MAX_ROWS = 16   # rows up to which the split-K route takes the single-launch qkv + rope + append linear (+2..6 %)
+    QKV_FUSED_MAX_ROWS = 64   # rows the single-launch qkv + rope + append linear takes
 
     def _splitk(self, rows: int) -> bool:
         """5..64 activation rows: the split-K linears (activations shared through LDS, splits added
-        up by the operator that follows) stand for F.linear on the output and down projections, and
-        from 17 rows on for the qkv projection too.  Measured end to end, this route overtakes the
-        fused single-launch linears at 5 rows (+6 % at 5, +8 % at 6, more beyond): every workgroup of
-        those re-reads the activations of its k range, which the 8192-wide down projection feels first."""
-        return self.decode_linear_rows > 0 and self.FUSED_MAX_ROWS < rows <= 64 and hasattr(self.ops, "linear_splitk")
+        up by the operator that follows) stand for F.linear on the output and down projections.  Measured
+        end to end, this route overtakes the fused single-launch linears at 5 rows (+6 % at 5, +8 % at 6, more
+        beyond): every workgroup of those re-reads the activations of its k range, which the 8192-wide down
+        projection feels first."""
+        return self.decode_linear_rows > 0 and self.FUSED_MAX_ROWS < rows <= self.QKV_FUSED_MAX_ROWS \
+            and hasattr(self.ops, "linear_splitk")
 
-    def _decode_layers_splitk(self, x, append_and_attend, project_and_attend=None):
-        """The layers of one decode step (T == 1) at 5..64 rows; returns the final hidden state.
-        append_and_attend(L, qkv partial products) -> attention output (B, 1, C);
-        project_and_attend(L, normalised input) -> the same from the single-launch qkv projection
-        (rotary embedding and cache append inside), taken while the rows are few enough for it."""
+    def _decode_layers_splitk(self, x, pos, attend):
+        """The layers of one decode step (T == 1) at 5..64 rows, at the device-side position pos; returns the final hidden
+        state.  attend(L, q) -> attention output of the rotated queries (B, 1, n_head, hd)."""
         c, ops = self.config, self.ops
-        rows = x.numel() // x.shape[-1]
-        qkv_fused = project_and_attend is not None and rows <= self.QKV_FUSED_MAX_ROWS
+        B = x.shape[0]
         h = ops.rms_norm(x, self.layers[0]["ln_1"], c.norm_eps)
         for i, L in enumerate(self.layers):
-            y = project_and_attend(L, h) if qkv_fused else append_and_attend(L, ops.linear_splitk(h, L["c_attn"]))
+            q = ops.linear_qkv_rope_append_rows(h, L["c_attn"], self.freqs_cis, L["cache_k"], L["cache_v"], pos, c.n_head)
+            y = attend(L, q.transpose(1, 2)).transpose(1, 2).reshape(B, 1, c.n_embd)
             x, h = ops.add_rms_norm_partials(x, ops.linear_splitk(y, L["c_proj"]), L["ln_2"], c.norm_eps)
             t = ops.linear_swiglu_decode(h, L["c_fc2"], L["c_fc"])     # one launch for the pair and the product
             next_norm = self.layers[i + 1]["ln_1"] if i + 1 < len(self.layers) else self.ln_f
@@ -254,20 +253,11 @@ class LlamaDecoder:
         if T == 1 and self._splitk(B):
             pos = torch.tensor([start_pos], dtype=torch.int32, device=self.device)
 
-            def append_and_attend(L, part):
-                q = self.ops.rot_embed_append_partials(part, self.freqs_cis, L["cache_k"], L["cache_v"], pos, c.n_head)
-                y = self.ops.flash_attention_decode(q.transpose(1, 2), L["cache_k"][:B, :start_pos + 1].transpose(1, 2),
-                                                    L["cache_v"][:B, :start_pos + 1].transpose(1, 2))
-                return y.transpose(1, 2).reshape(B, 1, c.n_embd)
+            def attend(L, q):
+                return self.ops.flash_attention_decode(q, L["cache_k"][:B, :start_pos + 1].transpose(1, 2),
+                                                       L["cache_v"][:B, :start_pos + 1].transpose(1, 2))
 
-            def project_and_attend(L, hn):
-                q = self.ops.linear_qkv_rope_append(hn, L["c_attn"], self.freqs_cis, L["cache_k"], L["cache_v"], pos,
-                                                    c.n_head)
-                y = self.ops.flash_attention_decode(q.transpose(1, 2), L["cache_k"][:B, :start_pos + 1].transpose(1, 2),
-                                                    L["cache_v"][:B, :start_pos + 1].transpose(1, 2))
-                return y.transpose(1, 2).reshape(B, 1, c.n_embd)
-
-            h = self._decode_layers_splitk(x, append_and_attend, project_and_attend)
+            h = self._decode_layers_splitk(x, pos, attend)
             return self.ops.linear_decode(h, self.wte).float()
         for L in self.layers:
             x = x + self._attention(L, self.ops.rms_norm(x, L["ln_1"], c.norm_eps), freqs_cis, start_pos)
@@ -437,20 +427,11 @@ class GraphedDecodeLoop:
                 x = lin(t, L["mlp_proj"], residual=x)
             logits = lin(x[:, -1], m.wte, norm_weight=m.ln_f, eps=c.norm_eps)
         elif m._splitk(B):
-            def append_and_attend(L, part):
-                q = ops.rot_embed_append_partials(part, m.freqs_cis, L["cache_k"], L["cache_v"], self.pos, c.n_head)
-                y = ops.flash_attention_decode_devlen(q.transpose(1, 2), L["cache_k"][:B].transpose(1, 2),
-                                                      L["cache_v"][:B].transpose(1, 2), self.kv_len)
-                return y.transpose(1, 2).reshape(B, 1, c.n_embd)
+            def attend(L, q):
+                return ops.flash_attention_decode_devlen(q, L["cache_k"][:B].transpose(1, 2), L["cache_v"][:B].transpose(1, 2),
+                                                         self.kv_len)
 
-            def project_and_attend(L, hn):
-                q = ops.linear_qkv_rope_append(hn, L["c_attn"], m.freqs_cis, L["cache_k"], L["cache_v"], self.pos,
-                                               c.n_head)
-                y = ops.flash_attention_decode_devlen(q.transpose(1, 2), L["cache_k"][:B].transpose(1, 2),
-                                                      L["cache_v"][:B].transpose(1, 2), self.kv_len)
-                return y.transpose(1, 2).reshape(B, 1, c.n_embd)
-
-            logits = ops.linear_decode(m._decode_layers_splitk(x, append_and_attend, project_and_attend)[:, -1], m.wte)
+            logits = ops.linear_decode(m._decode_layers_splitk(x, self.pos, attend)[:, -1], m.wte)
         else:
             h = ops.rms_norm(x, m.layers[0]["ln_1"], c.norm_eps)
             for i, L in enumerate(m.layers):

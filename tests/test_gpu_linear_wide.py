@@ -56,3 +56,35 @@ def test_linear_wide_swiglu_against_oracle(gpu, M, N, K):
     assert (err <= 3.5 * 2.0 ** -7 * ref.abs() + 2.0 ** -18 * ref.abs().max()).all(), err.max().item()
     res = randn_bf16((M, N), 214, scale=3.0).to(gpu)
     assert torch.equal(_wide(x, wg, wu, res), res + y)
+
+
+@pytest.mark.parametrize("B,NH,KVH,HD,K", [(1, 4, 1, 8, 128), (16, 32, 8, 64, 2048), (17, 6, 2, 72, 1152), (33, 8, 2, 128, 640),
+                                           (48, 4, 4, 64, 384), (49, 32, 8, 64, 1024), (64, 32, 8, 64, 2048)])
+def test_linear_qkv_rope_append_rows_against_oracle(gpu, B, NH, KVH, HD, K):
+    from custom_kernels import custom_kernels_extension as cke
+    from custom_kernels import precompute_freqs_cis
+
+    print(f"linear_qkv_rope_append_rows B={B} NH={NH} KVH={KVH} HD={HD} K={K}", flush=True)
+    L, at = 40, 17
+    x = randn_bf16((B, K), 221).to(gpu)
+    w = randn_bf16(((NH + 2 * KVH) * HD, K + 8), 222, scale=0.05).to(gpu)[:, :K]
+    table = precompute_freqs_cis(HD, 64, 500000.0, True, scale_factor=32.0, device=gpu)
+    before_k, before_v = randn_bf16((B + 1, L, KVH, HD), 223).to(gpu), randn_bf16((B + 1, L, KVH, HD), 224).to(gpu)
+    k, v = before_k.clone(), before_v.clone()
+    q = cke.linear_qkv_rope_append_rows(x.view(B, 1, K), w, table, k, v, torch.tensor([at], dtype=torch.int32, device=gpu), NH)
+    assert q.shape == (B, 1, NH, HD)
+    ref = linear_ref(t2f32(x), t2f32(w)).reshape(B, NH + 2 * KVH, HD)
+    assert_linear_close(v[:B, at].reshape(B, -1), ref[:, NH + KVH:].reshape(B, -1), "values")
+    # A sum that straddles a bf16 boundary may round the other way, one ulp (2^-7 at most) of each of the two values that a
+    # rotation adds up, and the result is rounded once (2^-8); sums that cancel as in assert_linear_close.
+    c, s = (table[at, i::2].double().cpu().numpy() for i in (0, 1))
+    r = ref[:, :NH + KVH].astype("float64")
+    a, b = r[..., 0::2], r[..., 1::2]
+    got = torch.cat((q[:, 0], k[:B, at]), 1).double().cpu().numpy()
+    slack = 2.0 ** -17 * abs(ref).max()
+    for y, want, size in ((got[..., 0::2], a * c - b * s, abs(a * c) + abs(b * s)), (got[..., 1::2], a * s + b * c, abs(a * s) + abs(b * c))):
+        assert (abs(y - want) <= (2.0 ** -7 + 2.0 ** -8) * size + slack).all()
+    # nothing else is written, and nothing at all at a position outside the cache
+    k[:B, at], v[:B, at] = before_k[:B, at], before_v[:B, at]
+    cke.linear_qkv_rope_append_rows(x.view(B, 1, K), w, table, k, v, torch.tensor([L], dtype=torch.int32, device=gpu), NH)
+    assert torch.equal(k, before_k) and torch.equal(v, before_v)
