@@ -221,12 +221,13 @@ add_rms_norm_partials_kernel(const uint16_t* __restrict__ x, const float* __rest
     const int tid = threadIdx.x;
     const int64_t row = blockIdx.x;
     const int nvec = C / 8;
-    uint4 xv[MAXV];
+    uint4 xv[MAXV], wv[MAXV];
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < MAXV; ++j) {
         const int vi = tid + j * kRmsThreads;
         if (vi < nvec) {
+            wv[j] = load16(w + vi * 8);
             float f[8], r[8];
             unpack8(load16(x + row * C + vi * 8), f);
             unpack8(sum_splits_bf16x8(part + row * C + vi * 8, ksplit, split_stride), r);
@@ -252,7 +253,7 @@ add_rms_norm_partials_kernel(const uint16_t* __restrict__ x, const float* __rest
         if (vi < nvec) {
             float f[8], g[8];
             unpack8(xv[j], f);
-            unpack8(load16(w + vi * 8), g);
+            unpack8(wv[j], g);
             uint4 o;
             o.x = pack_bf16x2(f[0] * inv * g[0], f[1] * inv * g[1]);
             o.y = pack_bf16x2(f[2] * inv * g[2], f[3] * inv * g[3]);
