@@ -430,6 +430,12 @@ size_t l3_decode_layers_workspace_bytes(int M, int n_layer);
 int l3_decode_layers(const void* layers_dev, int n_layer, const void* x, void* out, int M, const float* freq_table,
                      int table_rows, const int32_t* pos_dev, const int64_t cache_strides[2], int cache_len, float eps,
                      void* workspace, size_t workspace_bytes, void* stream);
+/* The same with the rows of x picked from an embedding (vocab, C): row m is that of tokens[m * token_stride] (a token
+ * outside [0, vocab) counts as the nearest inside). */
+int l3_decode_layers_tokens(const void* layers_dev, int n_layer, const int64_t* tokens, int64_t token_stride, const void* embedding,
+                            int64_t vocab, void* out, int M, const float* freq_table, int table_rows, const int32_t* pos_dev,
+                            const int64_t cache_strides[2], int cache_len, float eps, void* workspace, size_t workspace_bytes,
+                            void* stream);
 
 /*
  * out[r] = index of the first maximum of the bf16 row logits[r*row_stride : r*row_stride + V]

@@ -54,7 +54,9 @@ static_assert(kQkvRows % 4 == 0 && kHD % 4 == 0 && kC / kSlots == 64 && kH / kXc
 
 struct LayersParams {
     const DecodeLayerPointers* layers;
-    const uint16_t* x;          // (M, C)
+    const uint16_t* x;          // (M, C), or with tokens the embedding (vocab, C) they pick the rows from
+    const int64_t* tokens;
+    int64_t token_stride, vocab;
     uint16_t* out;              // (M, C)
     const float* rope_table;
     const int* pos;
@@ -82,6 +84,12 @@ __device__ __forceinline__ void store_device(uint64_t* p, uint64_t v) {
 }
 __device__ __forceinline__ uint64_t load_device(const uint64_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Row m of the input.
+__device__ __forceinline__ const uint16_t* input_row(const LayersParams& p, int m) {
+    int64_t row = m;
+    if (p.tokens) row = max(int64_t(0), min(p.tokens[m * p.token_stride], p.vocab - 1));
+    return p.x + row * kC;
 }
 __device__ __forceinline__ void wait_own_accesses() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 // two tagged bf16 values
@@ -328,7 +336,7 @@ decode_layers_kernel(const LayersParams p) {
         if (first) {
 #pragma unroll
             for (int m = 0; m < M; ++m) {
-                const uint2 v = *reinterpret_cast<const uint2*>(p.x + m * kC + col);
+                const uint2 v = *reinterpret_cast<const uint2*>(input_row(p, m) + col);
                 f[m][0] = __uint_as_float(v.x << 16);
                 f[m][1] = __uint_as_float(v.x & 0xffff0000u);
                 f[m][2] = __uint_as_float(v.y << 16);
@@ -383,7 +391,7 @@ decode_layers_kernel(const LayersParams p) {
     const int kv_len = max(1, min(pos + 1, p.cache_len));
     const bool pos_ok = pos >= 0 && pos < p.cache_len && pos < p.table_rows;
     // wavefront m < M: column 64 s + lane of row m of the residual stream (a bf16 value)
-    float xcol = wave < M ? bf16_to_f32(p.x[wave * kC + s * 64 + lane]) : 0.f;
+    float xcol = wave < M ? bf16_to_f32(input_row(p, wave)[s * 64 + lane]) : 0.f;
     // The XCDs' partial sums of row m = wave join it; every XCD gets the new row (dst, its own copy).
     auto join = [&](uint64_t* rows, uint32_t layer_tag, uint32_t* dst) __attribute__((always_inline)) {
         uint64_t* const at = rows + wave * kC + s * 64 + lane;
@@ -644,12 +652,15 @@ size_t decode_layers_workspace_bytes(int M, int n_layer) {
     return kDecodeLayersControlBytes + part + local;
 }
 
-int launch_decode_layers(const DecodeLayerPointers* layers, int n_layer, const uint16_t* x, uint16_t* out, int M,
-                         const float* rope_table, int table_rows, const int* pos, int64_t c_sb, int64_t c_st, int cache_len,
+int launch_decode_layers(const DecodeLayerPointers* layers, int n_layer, const uint16_t* x, const int64_t* tokens,
+                         int64_t token_stride, int64_t vocab, uint16_t* out, int M, const float* rope_table, int table_rows, const int* pos, int64_t c_sb, int64_t c_st, int cache_len,
                          float eps, float scale, void* ws, hipStream_t stream) {
     LayersParams p;
     p.layers = layers;
     p.x = x;
+    p.tokens = tokens;
+    p.token_stride = token_stride;
+    p.vocab = vocab;
     p.out = out;
     p.rope_table = rope_table;
     p.pos = pos;

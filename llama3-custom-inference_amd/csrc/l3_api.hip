@@ -867,9 +867,10 @@ size_t l3_decode_layers_workspace_bytes(int M, int n_layer) {
     return decode_layers_workspace_bytes(M, n_layer);
 }
 
-int l3_decode_layers(const void* layers_dev, int n_layer, const void* x, void* out, int M, const float* freq_table,
-                     int table_rows, const int32_t* pos_dev, const int64_t cache_strides[2], int cache_len, float eps,
-                     void* workspace, size_t workspace_bytes, void* stream) {
+static int decode_layers_impl(const void* layers_dev, int n_layer, const void* x, const int64_t* tokens, int64_t token_stride,
+                              int64_t vocab, void* out, int M, const float* freq_table, int table_rows, const int32_t* pos_dev,
+                              const int64_t cache_strides[2], int cache_len, float eps, void* workspace, size_t workspace_bytes,
+                              void* stream) {
     if (!layers_dev || !x || !out || !freq_table || !pos_dev || !cache_strides || !workspace) return L3_ERR_NULL_POINTER;
     if (M <= 0 || M > 4 || n_layer <= 0 || n_layer > 4096 || table_rows <= 0 || cache_len <= 0) return L3_ERR_SHAPE;
     if (cache_strides[0] < 0 || cache_strides[0] % 8 || cache_strides[1] <= 0 || cache_strides[1] % 8 ||
@@ -881,9 +882,28 @@ int l3_decode_layers(const void* layers_dev, int n_layer, const void* x, void* o
     if (workspace_bytes < decode_layers_workspace_bytes(M, n_layer)) return L3_ERR_WORKSPACE;
     if (!decode_layers_supported(M, 2048, 8192, 32, 8, 64, current_device_cus())) return L3_ERR_SHAPE;
     return launch_decode_layers(static_cast<const DecodeLayerPointers*>(layers_dev), n_layer, static_cast<const uint16_t*>(x),
-                                static_cast<uint16_t*>(out), M, freq_table, table_rows, pos_dev, cache_strides[0],
-                                cache_strides[1], cache_len, eps, 0.125f, workspace,
+                                tokens, token_stride, vocab, static_cast<uint16_t*>(out), M, freq_table, table_rows, pos_dev,
+                                cache_strides[0], cache_strides[1], cache_len, eps, 0.125f, workspace,
                                 static_cast<hipStream_t>(stream)) == 0 ? L3_OK : L3_ERR_HIP;
+}
+
+int l3_decode_layers(const void* layers_dev, int n_layer, const void* x, void* out, int M, const float* freq_table,
+                     int table_rows, const int32_t* pos_dev, const int64_t cache_strides[2], int cache_len, float eps,
+                     void* workspace, size_t workspace_bytes, void* stream) {
+    return decode_layers_impl(layers_dev, n_layer, x, nullptr, 0, 0, out, M, freq_table, table_rows, pos_dev, cache_strides,
+                              cache_len, eps, workspace, workspace_bytes, stream);
+}
+
+int l3_decode_layers_tokens(const void* layers_dev, int n_layer, const int64_t* tokens, int64_t token_stride, const void* embedding,
+                            int64_t vocab, void* out, int M, const float* freq_table, int table_rows, const int32_t* pos_dev,
+                            const int64_t cache_strides[2], int cache_len, float eps, void* workspace, size_t workspace_bytes,
+                            void* stream) {
+    if (!tokens) return L3_ERR_NULL_POINTER;
+    if (vocab <= 0 || vocab > (1 << 24)) return L3_ERR_SHAPE;
+    if (token_stride < 0) return L3_ERR_STRIDE;
+    if (!aligned(tokens, 8)) return L3_ERR_ALIGNMENT;
+    return decode_layers_impl(layers_dev, n_layer, embedding, tokens, token_stride, vocab, out, M, freq_table, table_rows, pos_dev,
+                              cache_strides, cache_len, eps, workspace, workspace_bytes, stream);
 }
 
 size_t l3_argmax_workspace_bytes(int rows, int V) {

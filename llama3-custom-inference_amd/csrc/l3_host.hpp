@@ -168,8 +168,8 @@ struct DecodeLayerPointers {
 constexpr size_t kDecodeLayersControlBytes = 8192;
 bool decode_layers_supported(int M, int C, int H, int QH, int KVH, int HD, int num_cus);
 size_t decode_layers_workspace_bytes(int M, int n_layer);
-int launch_decode_layers(const DecodeLayerPointers* layers, int n_layer, const uint16_t* x, uint16_t* out, int M,
-                         const float* rope_table, int table_rows, const int* pos, int64_t c_sb, int64_t c_st, int cache_len,
+int launch_decode_layers(const DecodeLayerPointers* layers, int n_layer, const uint16_t* x, const int64_t* tokens,
+                         int64_t token_stride, int64_t vocab, uint16_t* out, int M, const float* rope_table, int table_rows, const int* pos, int64_t c_sb, int64_t c_st, int cache_len,
                          float eps, float scale, void* ws, hipStream_t stream);
 int launch_attn_prefill(const PrefillParams& p, int HD, hipStream_t stream);        // a wavefront per column group
 // Workgroups of the tiled prefill kernel: 16-column blocks per wavefront, wavefronts per workgroup

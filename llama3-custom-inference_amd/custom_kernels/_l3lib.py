@@ -182,6 +182,12 @@ SIGNATURES = {
         [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_int,
          ctypes.c_void_p, _c_i64p, ctypes.c_int, ctypes.c_float, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p],
     ),
+    "l3_decode_layers_tokens": (
+        ctypes.c_int,
+        [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
+         ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, _c_i64p, ctypes.c_int, ctypes.c_float, ctypes.c_void_p,
+         ctypes.c_size_t, ctypes.c_void_p],
+    ),
     "l3_argmax_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int, ctypes.c_int]),
     "l3_argmax": (
         ctypes.c_int,

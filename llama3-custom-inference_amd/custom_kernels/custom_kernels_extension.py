@@ -399,6 +399,7 @@ class DecodeLayers:
     def __init__(self, layers, rows: int):
         self.rows, self.n_layer = rows, len(layers)
         self.tensors = [[L[n] for n in self.NAMES] for L in layers]     # kept alive
+        self.pointers = [[t.data_ptr() for t in row] for row in self.tensors]
         cache = layers[0]["cache_k"]
         for L in layers:
             for name in self.NAMES:
@@ -416,14 +417,15 @@ class DecodeLayers:
             if rows > maxB or wrong or not self.supported(rows, C, H, QH, KVH, HD):
                 raise RuntimeError(f"DecodeLayers: rows={rows} C={C} H={H} QH={QH} KVH={KVH} HD={HD} is not served {wrong}")
             nbytes = _l3lib.load().l3_decode_layers_workspace_bytes(rows, self.n_layer)
-        self.table = torch.tensor([[t.data_ptr() for t in row] for row in self.tensors], dtype=torch.int64, device=cache.device)
+        self.table = torch.tensor(self.pointers, dtype=torch.int64, device=cache.device)
         self.workspace = torch.zeros(nbytes, dtype=torch.uint8, device=cache.device)
         self.strides, self.C, self.HD = (cache.stride(0), cache.stride(1)), C, HD
 
     def holds(self, layers) -> bool:
-        """Whether ``layers`` are still the tensors that this object was made for."""
-        return len(layers) == self.n_layer and all(L[n] is t for L, row in zip(layers, self.tensors)
-                                                   for n, t in zip(self.NAMES, row))
+        """Whether ``layers`` are still the tensors, in the memory, that this object was made for."""
+        return len(layers) == self.n_layer and all(L[n] is t and t.data_ptr() == at
+                                                   for L, row, ptrs in zip(layers, self.tensors, self.pointers)
+                                                   for n, t, at in zip(self.NAMES, row, ptrs))
 
     @staticmethod
     def supported(rows: int, C: int, H: int, QH: int, KVH: int, HD: int) -> bool:
@@ -435,17 +437,31 @@ class DecodeLayers:
         _require_gpu_bf16("x", x)
         if tuple(x.shape) != (self.rows, 1, self.C) or not x.is_contiguous() or x.device != self.table.device:
             raise RuntimeError(f"DecodeLayers: x {tuple(x.shape)} does not fit ({self.rows}, 1, {self.C})")
+        return self._launch("l3_decode_layers", (x.data_ptr(),), freq_table, pos, eps)
+
+    def from_tokens(self, tokens, embedding, freq_table, pos, eps: float):
+        """The same with x = embedding[tokens]: tokens (rows, 1) int64 with any row stride, embedding (vocab, C)."""
+        _require_gpu_bf16("embedding", embedding)
+        if embedding.dim() != 2 or embedding.size(1) != self.C or not embedding.is_contiguous() or embedding.device != self.table.device:
+            raise RuntimeError(f"DecodeLayers: embedding {tuple(embedding.shape)} does not fit (vocab, {self.C})")
+        if tuple(tokens.shape) != (self.rows, 1) or tokens.dtype != torch.int64 or tokens.device != self.table.device:
+            raise RuntimeError(f"DecodeLayers: tokens must be ({self.rows}, 1) int64 on the GPU of the layers")
+        return self._launch("l3_decode_layers_tokens", (tokens.data_ptr(), tokens.stride(0), embedding.data_ptr(), embedding.size(0)),
+                            freq_table, pos, eps)
+
+    def _launch(self, function, source, freq_table, pos, eps):
         if not freq_table.is_cuda or freq_table.dtype != torch.float32 or freq_table.dim() != 2 \
                 or freq_table.size(1) != self.HD or not freq_table.is_contiguous():
             raise RuntimeError("freq_table must be a contiguous (rows, HD) float32 GPU tensor")
         if not pos.is_cuda or pos.dtype != torch.int32 or pos.numel() != 1:
             raise RuntimeError("pos must be a one-element int32 GPU tensor")
-        out = torch.empty_like(x)
-        with _on_device(x.device):
-            rc = _l3lib.load().l3_decode_layers(self.table.data_ptr(), self.n_layer, x.data_ptr(), out.data_ptr(), self.rows,
-                                                freq_table.data_ptr(), freq_table.size(0), pos.data_ptr(),
-                                                _l3lib.i64_array(self.strides), self.cache_len, float(eps),
-                                                self.workspace.data_ptr(), self.workspace.numel(), _stream_ptr(x.device))
+        device = self.table.device
+        out = torch.empty((self.rows, 1, self.C), dtype=torch.bfloat16, device=device)
+        with _on_device(device):
+            rc = getattr(_l3lib.load(), function)(self.table.data_ptr(), self.n_layer, *source, out.data_ptr(), self.rows,
+                                                  freq_table.data_ptr(), freq_table.size(0), pos.data_ptr(),
+                                                  _l3lib.i64_array(self.strides), self.cache_len, float(eps),
+                                                  self.workspace.data_ptr(), self.workspace.numel(), _stream_ptr(device))
         if rc != 0:
             _fail(rc, f"rows={self.rows} n_layer={self.n_layer}")
         return out

@@ -361,7 +361,7 @@ class LlamaDecoder:
             if prev_pos == 0 or layers is None:
                 logits = self.forward(tokens[:, prev_pos:cur_pos], start_pos=prev_pos)
             else:
-                x = layers(F.embedding(tokens[:, prev_pos:cur_pos], self.wte), self.freqs_cis, pos, c.norm_eps)
+                x = layers.from_tokens(tokens[:, prev_pos:cur_pos], self.wte, self.freqs_cis, pos, c.norm_eps)
                 logits = self.ops.linear_decode_fused(x, self.wte, norm_weight=self.ln_f, eps=c.norm_eps).float()
                 pos += 1
             next_token = torch.argmax(logits[:, -1], dim=-1).reshape(-1)
@@ -419,9 +419,9 @@ class GraphedDecodeLoop:
     def step(self, m: "LlamaDecoder"):
         c, B = m.config, self.B
         ops = m.ops
-        x = F.embedding(self.tok, m.wte)
+        x = F.embedding(self.tok, m.wte) if self.layers is None else None
         if self.layers is not None:
-            x = self.layers(x, m.freqs_cis, self.pos, c.norm_eps)
+            x = self.layers.from_tokens(self.tok, m.wte, m.freqs_cis, self.pos, c.norm_eps)
             logits = ops.linear_decode_fused(x[:, -1], m.wte, norm_weight=m.ln_f, eps=c.norm_eps)
         elif 0 < B <= m._fused_rows():
             # five launches per layer: norms, rotary embedding, cache append and residual additions ride

@@ -74,6 +74,14 @@ def test_decode_layers_against_float32(gpu, B):
                 assert (cache[:, pos].float() - new).norm() <= tol * new.norm()
                 cache[:, pos] = old[:, pos]
                 assert torch.equal(cache, old)      # nothing but the appended row has changed
+        # the same from an embedding whose rows tokens with a stride pick, the first and the last row among them
+        rows = 27 - 9 * torch.arange(B, device=gpu)
+        embedding = randn_bf16((28, C), 901).to(gpu)
+        embedding[rows] = x[:, 0]
+        tokens = torch.full((B, 5), 10 ** 9, device=gpu)
+        tokens[:, 2] = rows
+        assert torch.equal(one_launch.from_tokens(tokens[:, 2:3], embedding, table, torch.tensor([pos], dtype=torch.int32, device=gpu),
+                                                  EPS), y)
 
 
 def test_generation_without_the_one_launch_after_a_wait_ran_out(gpu):
