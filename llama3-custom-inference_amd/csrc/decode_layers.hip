@@ -286,10 +286,7 @@ decode_layers_kernel(const LayersParams p) {
         load_into_ring(p, RingLoader(lds_address(s_ring), g, s, wave - kComputeWaves));
         return;
     }
-    auto sync = []() __attribute__((always_inline)) {
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        barrier();
-    };
+    auto sync = []() __attribute__((always_inline)) { barrier_after_lds(); };
 
     // ---- waiting for other workgroups: poll() until it says that everything it reads is there
     const uint32_t launch = uint32_t(wave_uniform(int(ctl->launches[0]))) + 1;

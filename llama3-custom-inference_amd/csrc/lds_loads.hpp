@@ -42,6 +42,10 @@ __device__ __forceinline__ void wait_loads() {
     static_assert(NEWER < 64, "six bits");
     __builtin_amdgcn_s_waitcnt((NEWER & 15) | ((NEWER >> 4) << 14) | 0x0F70);
 }
+// The bare barrier, for wavefronts that read no LDS.
 __device__ __forceinline__ void barrier() { asm volatile("s_barrier" ::: "memory"); }
+// For wavefronts that do: behind it a stage may be loaded over, so what they have asked of LDS has to have arrived.  (The
+// compiler waits where the values are used, and may move that use behind a barrier; it costs nothing where it did not.)
+__device__ __forceinline__ void barrier_after_lds() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 }  // namespace l3

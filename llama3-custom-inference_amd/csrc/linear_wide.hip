@@ -176,7 +176,7 @@ linear_wide_kernel(const WideParams p) {
                 // this wavefront's part of the stage has landed, then everybody's; the stage that is requested next was
                 // last read before this barrier
                 if (t + d + ST - 2 < n_chunks) wait_loads<NI*(ST - 2)>(); else wait_loads<0>();
-                barrier();
+                barrier_after_lds();
                 if (t + d + ST - 1 < n_chunks) request((d + ST - 1) % ST);
                 multiply(s_ring + d * STAGE);
             }
