@@ -18,8 +18,8 @@
 // sums over everything (behind c_proj and behind the down projection) cross XCDs, as float32 partial rows that every
 // XCD adds up in the same order; all other hand-overs stay behind one L2.
 // What one workgroup hands to others carries its own tag, so that nobody waits for an acknowledgement, a counter and a
-// flag one after the other: inside an XCD 32-bit words of a bf16 value and the launch's number, plain stores, polled past the
-// L1 (0.6 us for a row of 2048 to all 32 workgroups; a counter in the L2 and then the data 1.5 us); across XCDs 64-bit words
+// flag one after the other: inside an XCD 32-bit words of a bf16 value, the launch's number and the writer's XCD, plain stores,
+// polled past the L1 (0.6 us for a row of 2048 to all 32 workgroups; a counter in the L2 and then the data 1.5 us); across XCDs 64-bit words
 // of a float32 value and the launch's and the layer's number, device-scope stores and polls (1.3 us; a flag per XCD behind
 // an L2 counter and then the data 2.3 us, one counter 3.5 us).  Every place is written once per launch, or per layer and
 // again only after all its readers have handed in something later.
@@ -290,7 +290,9 @@ decode_layers_kernel(const LayersParams p) {
 
     // ---- waiting for other workgroups: poll() until it says that everything it reads is there
     const uint32_t launch = uint32_t(wave_uniform(int(ctl->launches[0]))) + 1;
-    const uint32_t tag = launch & 0xffffu;
+    // A word handed over inside the XCD names its launch and the XCD that wrote it, and is awaited with the reader's own: from
+    // a workgroup that runs elsewhere than its number says nothing is taken, its K/V row (no tag of its own) included.
+    const uint32_t tag = (launch & 0xfffu) << 4 | xcc_id();
     bool alone = wave_uniform(int(load_device(&ctl->error[0]))) != 0;   // a wait has run out: go on without waiting
     auto wait_for = [&](auto poll) __attribute__((always_inline)) {
         for (int polls = 1; __builtin_amdgcn_ballot_w64(!poll()) != 0 && !alone; ++polls) {

@@ -84,6 +84,35 @@ def test_decode_layers_against_float32(gpu, B):
                                                   EPS), y)
 
 
+def _handed_over(one_launch, rows, n_layer):
+    """The words that the workgroups of an XCD have handed each other, (layer, XCD, word), from the workspace: residual rows
+    (written from the second layer on), rows behind c_proj, q | k | v, hidden units."""
+    words = one_launch.workspace.view(torch.int32)[8192 // 4 + 2 * 8 * rows * C * 2:].cpu()
+    return words.view(n_layer, 8, rows * (2 * C + (QH // KVH + 2) * HD + H // 8))
+
+
+@pytest.mark.parametrize("B", [1, 4])
+def test_handed_over_words_name_their_launch_and_the_xcd_that_wrote_them(gpu, B):
+    """... so that what a workgroup behind another L2 wrote is never taken (its K/V row among it, whose arrival only these words
+    tell); also where the launch number leaves its bits of the tag."""
+    from custom_kernels import custom_kernels_extension as ops
+    from llama_arch import precompute_freqs_cis
+
+    layers = _layers(gpu, 2, B, 64)
+    one_launch = ops.DecodeLayers(layers, B)
+    table = precompute_freqs_cis(HD, 64, 500000.0, True, scale_factor=32.0, device=gpu)
+    x, pos = randn_bf16((B, 1, C), 910).to(gpu), torch.tensor([40], dtype=torch.int32, device=gpu)
+    first = one_launch(x, table, pos, EPS)
+    for before in (1, 4094, 4095, 4096, 65534, 65535, 65536):
+        one_launch.workspace.view(torch.int32)[64] = before              # launches so far
+        print(f"decode_layers B={B} launch {before + 1}", flush=True)
+        assert torch.equal(one_launch(x, table, pos, EPS), first) and not one_launch.failed()
+        tags = _handed_over(one_launch, B, 2) & 0xffff
+        assert torch.equal(tags[1], tags[1, :, :1].expand_as(tags[1])) and torch.equal(tags[0, :, B * C:], tags[1, :, B * C:])
+        assert (tags[1] >> 4 == (before + 1) % 4096).all()
+        assert sorted((tags[1, :, 0] & 15).tolist()) == list(range(8))
+
+
 def test_generation_without_the_one_launch_after_a_wait_ran_out(gpu):
     from custom_kernels import custom_kernels_extension as ops
     from llama_arch import LlamaConfig, LlamaDecoder, random_prompts
