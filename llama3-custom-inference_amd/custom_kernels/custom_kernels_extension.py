@@ -397,29 +397,44 @@ class DecodeLayers:
     NAMES = ("ln_1", "c_attn", "c_proj", "ln_2", "c_fc2", "c_fc", "mlp_proj", "cache_k", "cache_v")
 
     def __init__(self, layers, rows: int):
+        if (why := self.unserved(layers, rows)) is not None:
+            raise RuntimeError(f"DecodeLayers: {why}")
         self.rows, self.n_layer = rows, len(layers)
         self.tensors = [[L[n] for n in self.NAMES] for L in layers]     # kept alive
         self.pointers = [[t.data_ptr() for t in row] for row in self.tensors]
         cache = layers[0]["cache_k"]
-        for L in layers:
-            for name in self.NAMES:
-                _require_gpu_bf16(name, L[name])
-                if not L[name].is_contiguous() or L[name].data_ptr() % 16 or L[name].shape != layers[0][name].shape \
-                        or L[name].device != cache.device:
-                    raise RuntimeError(f"DecodeLayers: {name} must be contiguous and alike in all layers")
-        maxB, self.cache_len, KVH, HD = cache.shape
-        H, C = layers[0]["c_fc"].shape
-        QH = layers[0]["c_attn"].shape[0] // HD - 2 * KVH
-        want = dict(ln_1=(C,), ln_2=(C,), c_attn=((QH + 2 * KVH) * HD, C), c_proj=(C, QH * HD), c_fc=(H, C), c_fc2=(H, C),
-                    mlp_proj=(C, H), cache_v=tuple(cache.shape))
-        wrong = [n for n, shape in want.items() if tuple(layers[0][n].shape) != shape]
+        _, self.cache_len, _, HD = cache.shape
+        C = layers[0]["c_fc"].shape[1]
         with _on_device(cache.device):
-            if rows > maxB or wrong or not self.supported(rows, C, H, QH, KVH, HD):
-                raise RuntimeError(f"DecodeLayers: rows={rows} C={C} H={H} QH={QH} KVH={KVH} HD={HD} is not served {wrong}")
             nbytes = _l3lib.load().l3_decode_layers_workspace_bytes(rows, self.n_layer)
         self.table = torch.tensor(self.pointers, dtype=torch.int64, device=cache.device)
         self.workspace = torch.zeros(nbytes, dtype=torch.uint8, device=cache.device)
         self.strides, self.C, self.HD = (cache.stride(0), cache.stride(1)), C, HD
+
+    @staticmethod
+    def unserved(layers, rows: int):
+        """Why the launch does not take these layers (rows with a padded stride, another architecture ...), or None where it does.
+        The operators one by one take more."""
+        first = layers[0]
+        cache = first["cache_k"]
+        for L in layers:
+            for name in DecodeLayers.NAMES:
+                t = L[name]
+                _require_gpu_bf16(name, t)
+                if not t.is_contiguous() or t.data_ptr() % 16 or t.shape != first[name].shape or t.device != cache.device:
+                    return f"{name} must be contiguous and alike in all layers"
+        if cache.dim() != 4 or first["c_fc"].dim() != 2:
+            return f"cache {tuple(cache.shape)}, c_fc {tuple(first['c_fc'].shape)}"
+        maxB, _, KVH, HD = cache.shape
+        H, C = first["c_fc"].shape
+        QH = first["c_attn"].shape[0] // HD - 2 * KVH
+        want = dict(ln_1=(C,), ln_2=(C,), c_attn=((QH + 2 * KVH) * HD, C), c_proj=(C, QH * HD), c_fc=(H, C), c_fc2=(H, C),
+                    mlp_proj=(C, H), cache_v=tuple(cache.shape))
+        wrong = [n for n, shape in want.items() if tuple(first[n].shape) != shape]
+        with _on_device(cache.device):
+            if rows > maxB or wrong or not DecodeLayers.supported(rows, C, H, QH, KVH, HD):
+                return f"rows={rows} C={C} H={H} QH={QH} KVH={KVH} HD={HD} is not served {wrong}"
+        return None
 
     def holds(self, layers) -> bool:
         """Whether ``layers`` are still the tensors, in the memory, that this object was made for."""

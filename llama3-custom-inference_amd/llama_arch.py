@@ -220,11 +220,16 @@ class LlamaDecoder:
         c = self.config
         if not self._layers_in_one_launch or not 0 < rows <= self._fused_rows() or rows * total_len > self.ONE_LAUNCH_MAX_POSITIONS:
             return None
+        if not self.wte.is_contiguous() or self.wte.data_ptr() % 16:
+            return None
         made = self._layer_launches.get(rows)
         if made is None or not made.holds(self.layers):
             with torch.cuda.device(self.device):
                 if not self.ops.DecodeLayers.supported(rows, c.n_embd, c.hidden_dim, c.n_head, c.n_kv_head, self.hd):
                     return None
+            # what the operators take and the launch does not, rows with a padded stride among them, is theirs
+            if self.ops.DecodeLayers.unserved(self.layers, rows) is not None:
+                return None
             made = self._layer_launches[rows] = self.ops.DecodeLayers(self.layers, rows)
         return made
 
