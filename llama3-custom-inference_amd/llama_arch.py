@@ -197,10 +197,29 @@ class LlamaDecoder:
             q = ops.linear_qkv_rope_append_rows(h, L["c_attn"], self.freqs_cis, L["cache_k"], L["cache_v"], pos, c.n_head)
             y = attend(L, q.transpose(1, 2)).transpose(1, 2).reshape(B, 1, c.n_embd)
             x, h = ops.add_rms_norm_partials(x, ops.linear_splitk(y, L["c_proj"]), L["ln_2"], c.norm_eps)
-            t = ops.linear_swiglu_decode(h, L["c_fc2"], L["c_fc"])     # one launch for the pair and the product
+            t = self._swiglu(h, L["c_fc2"], L["c_fc"])
             next_norm = self.layers[i + 1]["ln_1"] if i + 1 < len(self.layers) else self.ln_f
             x, h = ops.add_rms_norm_partials(x, ops.linear_splitk(t, L["mlp_proj"]), next_norm, c.norm_eps)
         return h
+
+    # What the streaming linears need of a weight beside its width: dense 16-byte rows, and more than 16 activation rows want
+    # the vocabulary in whole eights (the SwiGLU pair in fours, which a hidden size that the down projection takes always is).
+    # F.linear takes any, so it has the rest.
+    def _vocabulary(self, h):
+        """Logits of a decode step at 5..64 rows."""
+        w = self.wte
+        if w.shape[0] % 8 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0:
+            return self.ops.linear_decode(h, w)
+        return F.linear(h, w)
+
+    def _swiglu(self, h, gate, up):
+        """The SwiGLU product of a decode step at 5..64 rows: one launch for the pair and the product."""
+        if h.shape[0] > self.PAIR_MAX_ROWS_STRIDED and not (gate.is_contiguous() and up.is_contiguous() and
+                                                            gate.data_ptr() % 16 == 0 and up.data_ptr() % 16 == 0):
+            return self.ops.silu_mul(F.linear(h, gate), F.linear(h, up))
+        return self.ops.linear_swiglu_decode(h, gate, up)
+
+    PAIR_MAX_ROWS_STRIDED = 14   # rows up to which a padded pair is the streaming linear's too (as dense pairs always are)
 
     def _fused_rows(self) -> int:
         """Rows up to which the decode step uses linear_decode_fused (norms and residual additions
@@ -272,8 +291,7 @@ class LlamaDecoder:
                 return self.ops.flash_attention_decode(q, L["cache_k"][:B, :start_pos + 1].transpose(1, 2),
                                                        L["cache_v"][:B, :start_pos + 1].transpose(1, 2))
 
-            h = self._decode_layers_splitk(x, pos, attend)
-            return self.ops.linear_decode(h, self.wte).float()
+            return self._vocabulary(self._decode_layers_splitk(x, pos, attend)).float()
         h = self.ops.rms_norm(x, self.layers[0]["ln_1"], c.norm_eps)
         for i, L in enumerate(self.layers):
             x, h = self._add_norm(x, self._attention(L, h, freqs_cis, start_pos), L["ln_2"])
@@ -446,7 +464,7 @@ class GraphedDecodeLoop:
                 return ops.flash_attention_decode_devlen(q, L["cache_k"][:B].transpose(1, 2), L["cache_v"][:B].transpose(1, 2),
                                                          self.kv_len)
 
-            logits = ops.linear_decode(m._decode_layers_splitk(x, self.pos, attend)[:, -1], m.wte)
+            logits = m._vocabulary(m._decode_layers_splitk(x, self.pos, attend)[:, -1])
         else:
             h = ops.rms_norm(x, m.layers[0]["ln_1"], c.norm_eps)
             for i, L in enumerate(m.layers):

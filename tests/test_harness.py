@@ -115,6 +115,47 @@ def test_split_k_decode_path_matches_cpu_logits(gpu, rows):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows,vocab,strided", [(5, 1004, False), (16, 1004, False), (17, 1004, False), (17, 1001, False), (64, 1001, False),
+                                                (5, 1000, True), (15, 1000, True), (16, 1000, True), (64, 1000, True)])
+def test_decode_steps_with_weights_that_only_the_library_gemm_takes(gpu, rows, vocab, strided):
+    """A vocabulary that is no multiple of eight (from 17 rows on, where the prompt pass has the library GEMM too, of four), and gate / up / embedding weights with strides of their own: the
+    decode step of 5..64 sequences, eager and as the graph loop runs it, against the float32 CPU model."""
+    from custom_kernels import custom_kernels_extension as cke
+
+    cfg = tiny_config(n_head=8, n_kv_head=2, n_embd=512, hidden_dim=1024, max_gen_batch_size=rows, vocab_size=vocab)
+    ref = la.LlamaDecoder(cfg, CpuOps, "cpu", dtype=torch.float32, seed=9)
+    dut = la.LlamaDecoder(cfg, cke, gpu, dtype=torch.bfloat16, seed=9)
+    ref.wte = dut.wte.float().cpu()
+    for Lr, Ld in zip(ref.layers, dut.layers):
+        for key in ("c_attn", "c_proj", "c_fc", "c_fc2", "mlp_proj"):
+            Lr[key] = Ld[key].float().cpu()
+    if strided:
+        def padded(t, by):
+            return torch.zeros(t.shape[0], t.shape[1] + by, dtype=t.dtype, device=gpu)[:, :t.shape[1]].copy_(t)
+        dut.wte = padded(dut.wte, 3 if rows > 16 else 8)
+        for Ld in dut.layers if rows > 14 else []:
+            Ld["c_fc"], Ld["c_fc2"] = padded(Ld["c_fc"], 8), Ld["c_fc2"].t().contiguous().t()
+    ids = torch.tensor(la.random_prompts(rows, 10, 900, 13))
+    with torch.inference_mode():
+        ref.forward(ids[:, :9], start_pos=0)
+        dut.forward(ids[:, :9].to(gpu), start_pos=0)
+        print(f"library GEMM weights: rows={rows} vocab={vocab} strided={strided}", flush=True)
+        want = ref.forward(ids[:, 9:], start_pos=9)
+        loop = la.GraphedDecodeLoop(dut, rows, 12)
+        loop.tok.copy_(ids[:, 9:])
+        loop.pos.fill_(9)
+        loop.kv_len.fill_(10)
+        steps, vocabulary = [], dut._vocabulary
+        dut._vocabulary = lambda h: steps.append(vocabulary(h)) or steps[-1]
+        eager = dut.forward(ids[:, 9:].to(gpu), start_pos=9).cpu()
+        loop.step(dut)
+    assert len(steps) == 2
+    scale = want.abs().max().item()
+    for got in (eager[:, -1], steps[1].float().cpu()):
+        assert (got - want[:, -1]).abs().max().item() <= 0.04 * scale
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("batch", [1, 3, 4, 5, 9, 16, 20])
 def test_graphed_decode_loop_matches_eager(gpu, batch):
     """The HIP-graph replay of the decode step against the eager loop, replay by replay: same
