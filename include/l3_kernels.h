@@ -355,11 +355,12 @@ int l3_linear_qkv_rope_append(const void* x, const void* norm_weight, float norm
  * units (<= 0: the current device): as few splits as fill the device.  l3_linear_splitk_plan is the finer
  * cut for a caller that does not know M; l3_linear_splitk_workspace_bytes the size of `part`.  1 <= M <=
  * L3_LINEAR_SPLITK_MAX_ROWS, N % 8 == 0, K % 128 == 0, ceil((K / 128) / ksplit) no more than the coarser of
- * the two plans takes, or 4 (8 for a matrix with fewer than 32 rows per compute unit); strides (below 2^28)
- * and alignment as for l3_linear_decode.  Meant for matrices of a few thousand rows, where the split
+ * the two plans takes, or 4 (8 for a matrix with fewer than 32 rows per compute unit); strides and alignment
+ * as for l3_linear_decode (rows further than L3_LINEAR_WIDE_MAX_STRIDE apart are read one by one, slowly).  Meant for matrices of a few thousand rows, where the split
  * count fills the device; where the rows alone do (a vocabulary projection), see l3_linear_wide.
  */
 #define L3_LINEAR_SPLITK_MAX_ROWS 64
+#define L3_LINEAR_WIDE_MAX_STRIDE ((int64_t)1 << 28)   /* elements between two rows, of l3_linear_wide's operands too */
 int l3_linear_splitk_plan(int N, int K, int num_cus);
 int l3_linear_splitk_rows_plan(int M, int N, int K, int num_cus);
 size_t l3_linear_splitk_workspace_bytes(int M, int N, int ksplit);
@@ -368,7 +369,7 @@ int l3_linear_splitk(const void* x, const void* w, void* part, size_t part_bytes
 
 /*
  * l3_linear_qkv_rope_append without a norm for up to 64 activation rows: 1 <= B <= L3_LINEAR_SPLITK_MAX_ROWS,
- * K % 128 == 0, strides and alignment as for l3_linear_splitk; the same rounding points, sums in another order.
+ * K % 128 == 0, strides (up to L3_LINEAR_WIDE_MAX_STRIDE) and alignment as for l3_linear_decode; the same rounding points, sums in another order.
  */
 int l3_linear_qkv_rope_append_rows(const void* x, const void* w_qkv, const float* freq_table, void* q_out, void* cache_k,
                                    void* cache_v, const int32_t* pos_dev, int B, int NH, int KVH, int HD, int K, int64_t x_stride,
@@ -379,7 +380,7 @@ int l3_linear_qkv_rope_append_rows(const void* x, const void* w_qkv, const float
  * stride) with a rounding of its own if that is not NULL, for up to 64 activation rows in one
  * launch without splits: for matrices whose rows alone fill the device (gate|up pair, vocabulary
  * projection: model.py:134,225).  1 <= M <= L3_LINEAR_SPLITK_MAX_ROWS, K % 128 == 0, N % 8 == 0 (N % 4 with
- * w_up); strides (below 2^28) and alignment as for l3_linear_decode, y 16-byte aligned without w_up.
+ * w_up); strides (up to L3_LINEAR_WIDE_MAX_STRIDE) and alignment as for l3_linear_decode, y 16-byte aligned without w_up.
  */
 int l3_linear_wide(const void* x, const void* w, const void* w_up, const void* residual, void* y, int M, int N, int K,
                    int64_t x_stride, int64_t w_stride, int64_t y_stride, void* stream);

@@ -740,7 +740,8 @@ int l3_linear_qkv_rope_append_rows(const void* x, const void* w_qkv, const float
                                         table_rows); rc != L3_OK) return rc;
     if (!x || !w_qkv) return L3_ERR_NULL_POINTER;
     if (B <= 0 || B > L3_LINEAR_SPLITK_MAX_ROWS || K <= 0 || K % 128 != 0 || K > (1 << 24)) return L3_ERR_SHAPE;
-    if (x_stride < K || w_stride < K || x_stride % 8 || w_stride % 8 || x_stride > kLinearMaxPitch || w_stride > kLinearMaxPitch)
+    if (x_stride < K || w_stride < K || x_stride % 8 || w_stride % 8 || x_stride > L3_LINEAR_WIDE_MAX_STRIDE ||
+        w_stride > L3_LINEAR_WIDE_MAX_STRIDE)
         return L3_ERR_STRIDE;
     if (!aligned(x, 16) || !aligned(w_qkv, 16)) return L3_ERR_ALIGNMENT;
     const QkvTarget t = {freq_table, pos_dev, static_cast<uint16_t*>(q_out), static_cast<uint16_t*>(cache_k),
@@ -779,7 +780,7 @@ int l3_linear_wide(const void* x, const void* w, const void* w_up, const void* r
         return L3_ERR_SHAPE;
     if (N > (1 << 24) || K > (1 << 24)) return L3_ERR_SHAPE;
     if (x_stride < K || w_stride < K || y_stride < N || x_stride % 8 || w_stride % 8 || y_stride % (w_up ? 4 : 8) ||
-        x_stride > kLinearMaxPitch || w_stride > kLinearMaxPitch)
+        x_stride > L3_LINEAR_WIDE_MAX_STRIDE || w_stride > L3_LINEAR_WIDE_MAX_STRIDE)
         return L3_ERR_STRIDE;
     if (!aligned(x, 16) || !aligned(w, 16) || (w_up && !aligned(w_up, 16)) || !aligned(y, w_up ? 8 : 16) ||
         (residual && !aligned(residual, w_up ? 8 : 16)))
@@ -802,8 +803,7 @@ int l3_linear_splitk(const void* x, const void* w, void* part, size_t part_bytes
     if (ksplit <= 0 || ksplit > K / 128 ||
         (K / 128 + ksplit - 1) / ksplit > linear_splitk_max_chunks(N, K, current_device_cus()))
         return L3_ERR_SPLITS;
-    if (x_stride < K || w_stride < K || x_stride % 8 || w_stride % 8 || x_stride > kLinearMaxPitch || w_stride > kLinearMaxPitch)
-        return L3_ERR_STRIDE;
+    if (x_stride < K || w_stride < K || x_stride % 8 || w_stride % 8) return L3_ERR_STRIDE;
     if (!aligned(x, 16) || !aligned(w, 16) || !aligned(part, 16)) return L3_ERR_ALIGNMENT;
     if (part_bytes < l3_linear_splitk_workspace_bytes(M, N, ksplit)) return L3_ERR_WORKSPACE;
     return launch_linear_splitk(static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w),

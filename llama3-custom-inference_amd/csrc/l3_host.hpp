@@ -142,7 +142,6 @@ int launch_rot_embed_append_partials(const float* part, int ksplit, int64_t spli
                                      int table_rows, hipStream_t stream);
 int linear_splitk_rows_plan(int N, int K, int num_cus);
 int linear_splitk_max_chunks(int N, int K, int num_cus);
-constexpr int64_t kLinearMaxPitch = int64_t(1) << 28;   // elements between two rows of the wide kernel's operands
 int launch_linear_wide(const uint16_t* x, const uint16_t* w, const uint16_t* w_up, const uint16_t* res, uint16_t* y, int M,
                        int N, int K, int64_t x_stride, int64_t w_stride, int64_t y_stride, int num_cus, hipStream_t stream);
 // Where the outputs of a qkv projection go: rotary table and position, rotated queries, key and value cache.

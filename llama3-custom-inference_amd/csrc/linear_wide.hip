@@ -327,6 +327,29 @@ linear_splitk_finish_kernel(const float* __restrict__ part, int ksplit, int64_t 
     store16(y + int64_t(m) * y_stride + n, o);
 }
 
+// Partial products of operands whose rows lie too far apart for the 32-bit offsets of the loads above (a column of a
+// tensor of tens of gigabytes): a wavefront per output, split after split.
+__global__ void __launch_bounds__(kWaveSize)
+linear_splitk_far_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, float* __restrict__ part, int K,
+                         int64_t x_stride, int64_t w_stride, int ksplit, int chunks_per_split) {
+    const int n = int(blockIdx.x), m = int(blockIdx.y), N = int(gridDim.x), M = int(gridDim.y);
+    x += m * x_stride;
+    w += n * w_stride;
+    for (int s = 0; s < ksplit; ++s) {
+        const int64_t end = min(int64_t(K), int64_t(s + 1) * chunks_per_split * kWideChunk);
+        float sum = 0.f;
+        for (int64_t k = int64_t(s) * chunks_per_split * kWideChunk + int(threadIdx.x) * 8; k < end; k += kWaveSize * 8) {
+            float a[8], b[8];
+            unpack8(load16(x + k), a);
+            unpack8(load16(w + k), b);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) sum = fmaf(a[i], b[i], sum);
+        }
+        sum = wave_sum(sum);
+        if (threadIdx.x == 0) part[(int64_t(s) * M + m) * N + n] = sum;
+    }
+}
+
 int chunks_of(int K) { return K / kWideChunk; }
 
 // Splits of K of the partial-product form (which imply the weight rows per workgroup, launch_linear_splitk).  One workgroup per compute unit at most:
@@ -387,6 +410,11 @@ int linear_splitk_max_chunks(int N, int K, int num_cus) {
 
 int launch_linear_splitk(const uint16_t* x, const uint16_t* w, float* part, int M, int N, int K, int64_t x_stride,
                          int64_t w_stride, int ksplit, int num_cus, hipStream_t stream) {
+    if (M == 1) x_stride = K;   // (a single row has no next one)
+    if (x_stride > L3_LINEAR_WIDE_MAX_STRIDE || w_stride > L3_LINEAR_WIDE_MAX_STRIDE) {
+        return enqueue(linear_splitk_far_kernel, dim3(unsigned(N), unsigned(M)), dim3(kWaveSize), 0, stream, x, w, part, K, x_stride,
+                       w_stride, ksplit, (chunks_of(K) + ksplit - 1) / ksplit);
+    }
     WideParams p = wide_params(x, w, M, N, K, x_stride, w_stride);
     p.part = part;
     const int64_t wgs64 = int64_t((N + 63) / 64) * ksplit;

@@ -426,7 +426,8 @@ struct Rows {
     Tensor copy;   // keeps a rearranged copy alive
 };
 
-Rows linear_rows(const Tensor& x, int max_rows) {
+// `near_each_other`: for the kernels that share activations through LDS, which address a few rows with 32 bits.
+Rows linear_rows(const Tensor& x, int max_rows, bool near_each_other) {
     Rows r;
     r.K = x.dim() > 0 ? x.sizes().back() : 0;
     r.rows = r.K > 0 ? x.numel() / r.K : 0;
@@ -442,6 +443,13 @@ Rows linear_rows(const Tensor& x, int max_rows) {
         if (stride_at(r.copy, 1) != 1) r.copy = r.copy.contiguous();
         r.x = ptr(r.copy);
         r.stride = stride_at(r.copy, 0);
+    }
+    if (near_each_other && r.stride > L3_LINEAR_WIDE_MAX_STRIDE) {
+        if (r.rows > 1) {
+            r.copy = x.contiguous();
+            r.x = ptr(r.copy);
+        }
+        r.stride = r.K;
     }
     return r;
 }
@@ -495,7 +503,7 @@ Route route_of(const Tensor& x, const Tensor& w, bool pair, bool residual) {
 
 // Float32 partial products (ksplit, rows, N); ksplit 0 = the library's choice.
 Tensor splitk(const Tensor& x, const Tensor& w, int ksplit) {
-    const Rows r = linear_rows(x, L3_LINEAR_SPLITK_MAX_ROWS);
+    const Rows r = linear_rows(x, L3_LINEAR_SPLITK_MAX_ROWS, true);
     check_weight(w, w, x, r.K);
     const int64_t N = size_at(w, 0);
     const OnDevice on(x);
@@ -529,7 +537,7 @@ void splitk_finish(const Tensor& part, const Tensor* residual, const Tensor& y) 
 
 // The whole product (or, with up, the SwiGLU product of two) of up to 64 rows in one launch.
 Tensor wide(const Tensor& x, const Tensor& w, const Tensor* up, const Tensor* residual) {
-    const Rows r = linear_rows(x, L3_LINEAR_SPLITK_MAX_ROWS);
+    const Rows r = linear_rows(x, L3_LINEAR_SPLITK_MAX_ROWS, true);
     check_weight(w, w, x, r.K);
     if (up) check_weight(*up, w, x, r.K);
     const int64_t N = size_at(w, 0);
@@ -565,7 +573,7 @@ Tensor normalised(const Tensor& x, const Tensor& norm, double eps) {
 // The linear with what is folded into it.
 Tensor linear(const Tensor& x, const Tensor& w, const Tensor* norm, double eps, const Tensor* up, const Tensor* residual) {
     const Route route = route_of(x, w, up != nullptr, residual != nullptr);
-    const Rows r = linear_rows(x, route == Route::kSkinny ? L3_LINEAR_MAX_ROWS : L3_LINEAR_SPLITK_MAX_ROWS);
+    const Rows r = linear_rows(x, route == Route::kSkinny ? L3_LINEAR_MAX_ROWS : L3_LINEAR_SPLITK_MAX_ROWS, false);
     check_weight(w, w, x, r.K);
     if (up) check_weight(*up, w, x, r.K);
     if (norm) check_norm_weight(*norm, r.rows, r.K, "linear_decode_fused");
@@ -643,7 +651,7 @@ Cache cache_args(PyObject* table, PyObject* cache_k, PyObject* cache_v, PyObject
 PyObject* linear_qkv_rope_append(PyObject* const* a) {
     const Tensor& x = gpu_bf16(a[0], "x");
     const Tensor& w = gpu_bf16(a[1], "weight");
-    const Rows r = linear_rows(x, L3_LINEAR_MAX_ROWS);
+    const Rows r = linear_rows(x, L3_LINEAR_MAX_ROWS, false);
     check_weight(w, w, x, r.K);
     const Cache c = cache_args(a[2], a[3], a[4], a[5]);
     const int64_t NH = integer(a[6]);
@@ -666,7 +674,7 @@ PyObject* linear_qkv_rope_append(PyObject* const* a) {
 PyObject* linear_qkv_rope_append_rows(PyObject* const* a) {
     const Tensor& x = gpu_bf16(a[0], "x");
     const Tensor& w = gpu_bf16(a[1], "weight");
-    const Rows r = linear_rows(x, L3_LINEAR_SPLITK_MAX_ROWS);
+    const Rows r = linear_rows(x, L3_LINEAR_SPLITK_MAX_ROWS, true);
     check_weight(w, w, x, r.K);
     const Cache c = cache_args(a[2], a[3], a[4], a[5]);
     const int64_t NH = integer(a[6]);

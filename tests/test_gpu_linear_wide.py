@@ -88,3 +88,33 @@ def test_linear_qkv_rope_append_rows_against_oracle(gpu, B, NH, KVH, HD, K):
     k[:B, at], v[:B, at] = before_k[:B, at], before_v[:B, at]
     cke.linear_qkv_rope_append_rows(x.view(B, 1, K), w, table, k, v, torch.tensor([L], dtype=torch.int32, device=gpu), NH)
     assert torch.equal(k, before_k) and torch.equal(v, before_v)
+
+
+@pytest.mark.parametrize("M,N,K,ksplit", [(1, 8, 128, 1), (3, 24, 1152, 3), (17, 8, 640, 2), (2, 8, 1280, 8)])
+@pytest.mark.parametrize("far", ["x", "w", "both"])
+def test_linear_splitk_of_rows_far_apart(gpu, M, N, K, ksplit, far):
+    """Rows more than 2^28 elements apart (activations picked out of a long context, say): the library's entry point takes
+    them, with splits that get no k among them, and so do the operators."""
+    from custom_kernels import _l3lib
+    from custom_kernels import custom_kernels_extension as cke
+
+    print(f"linear_splitk far={far} M={M} N={N} K={K} ksplit={ksplit}", flush=True)
+
+    def rows(values, apart):
+        t = torch.empty((values.shape[0] - 1) * apart + K, dtype=torch.bfloat16, device=gpu)
+        return t.as_strided(values.shape, (apart, 1)).copy_(values)
+
+    xv, wv = randn_bf16((M, K), 231), randn_bf16((N, K), 232, scale=0.05)
+    x = rows(xv, (1 << 28) + 8) if far != "w" else xv.to(gpu)
+    w = rows(wv, (1 << 28) + 8) if far != "x" else wv.to(gpu)
+    part = torch.full((ksplit, M, N), float("nan"), device=gpu)
+    rc = _l3lib.load().l3_linear_splitk(x.data_ptr(), w.data_ptr(), part.data_ptr(), part.numel() * 4, M, N, K, (1 << 28) + 8 if far != "w" else K,
+                                        w.stride(0), ksplit, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, rc
+    per = -(-(K // 128) // ksplit) * 128
+    for s in range(ksplit):
+        want = xv[:, s * per:(s + 1) * per].double() @ wv[:, s * per:(s + 1) * per].double().t()
+        # 32-bit sums of at most 1280 products of these sizes
+        assert ((part[s].cpu().double() - want).abs() <= 2.0 ** -20 * (xv.double().abs() @ wv.double().abs().t())).all()
+    if ksplit == 1 or M == 17:      # (the operator chooses its own splits)
+        assert_linear_close(cke.linear_splitk_finish(cke.linear_splitk(x, w)), linear_ref(t2f32(xv), t2f32(wv)), "far rows")
