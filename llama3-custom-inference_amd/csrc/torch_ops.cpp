@@ -426,12 +426,16 @@ struct Rows {
     Tensor copy;   // keeps a rearranged copy alive
 };
 
+void check_rows(int64_t rows, int max_rows, const Tensor& x) {
+    TORCH_CHECK(rows >= 1 && rows <= max_rows, "linear_decode: 1..", max_rows, " activation rows expected, got ", x.sizes());
+}
+
 // `near_each_other`: for the kernels that share activations through LDS, which address a few rows with 32 bits.
 Rows linear_rows(const Tensor& x, int max_rows, bool near_each_other) {
     Rows r;
     r.K = x.dim() > 0 ? x.sizes().back() : 0;
     r.rows = r.K > 0 ? x.numel() / r.K : 0;
-    TORCH_CHECK(r.rows >= 1 && r.rows <= max_rows, "linear_decode: 1..", max_rows, " activation rows expected, got ", x.sizes());
+    check_rows(r.rows, max_rows, x);
     if (x.dim() == 2 && stride_at(x, 1) == 1) {
         r.x = ptr(x);   // rows as they are (any row stride)
         r.stride = stride_at(x, 0);
@@ -484,21 +488,25 @@ constexpr int64_t kWideRows = 12288, kWidePairRows = 6144;
 // 4096 (235 MB), 1 row 47.9 / 39.2; 2048 x 8192, 4 rows 10.2 / 10.6, 5 rows 15.4 / 10.7; 4096 x 4096, 5 rows 10.1 / 10.4, 16
 // rows 12.3 / 10.6; 6144 x 4096, 2 rows 11.3 / 12.8, 5 rows 16.2 / 12.9; 4096 x 14336, 1 row 23.2 / 22.9; 2048 x 2048 and
 // 3072 x 2048, 12 rows 6.7 / 6.6 and 6.9 / 7.1.
-Route route_of(const Tensor& x, const Tensor& w, bool pair, bool residual) {
-    const int64_t K = x.dim() > 0 ? x.sizes().back() : 0;
-    if (K <= 0 || w.dim() != 2) return Route::kSkinny;   // (its checks say what is wrong)
-    const int64_t rows = x.numel() / K, N = size_at(w, 0);
-    if (rows > L3_LINEAR_SPLITK_MAX_ROWS) return Route::kSkinny;
-    const bool fits = K % 128 == 0 && N % 8 == 0;
-    if (pair) {
-        if (rows > L3_LINEAR_MAX_ROWS) return residual ? Route::kSkinny : Route::kWide;
-        const bool large = N * K >= int64_t(32) << 20;   // each of the two
-        return fits && N >= kWidePairRows && (rows >= 4 || large) ? Route::kWide : Route::kSkinny;
+//
+// Up to 16 rows the skinny kernel says what is taken and what is refused: operands that it takes and the others do not stay
+// with it, and so do those that it refuses.
+Route route_of(const Rows& r, const Tensor& w, bool pair, const Tensor* residual) {
+    const int64_t K = r.K, N = size_at(w, 0);
+    const bool near_rows = stride_at(w, 0) <= L3_LINEAR_WIDE_MAX_STRIDE;
+    if (r.rows > L3_LINEAR_MAX_ROWS) {
+        if (pair) return residual ? Route::kSkinny : Route::kWide;
+        return N >= kWideRows && near_rows ? Route::kWide : Route::kSplit;
     }
-    if (rows > L3_LINEAR_MAX_ROWS) return N >= kWideRows ? Route::kWide : Route::kSplit;
-    if (!fits) return Route::kSkinny;
-    if (N >= kWideRows) return rows >= 4 ? Route::kWide : Route::kSkinny;
-    return N * K >= int64_t(rows >= 5 ? 16 : 32) << 20 ? Route::kSplit : Route::kSkinny;
+    const auto misaligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 != 0; };
+    if (K % 128 != 0 || N % 8 != 0 || !near_rows || misaligned(r.x) || r.stride < K || r.stride % 8 != 0) return Route::kSkinny;
+    if (pair) {
+        const bool large = N * K >= int64_t(32) << 20;   // each of the two
+        return N >= kWidePairRows && (r.rows >= 4 || large) ? Route::kWide : Route::kSkinny;
+    }
+    if (residual && residual->is_contiguous() && misaligned(ptr(*residual))) return Route::kSkinny;
+    if (N >= kWideRows) return r.rows >= 4 ? Route::kWide : Route::kSkinny;
+    return N * K >= int64_t(r.rows >= 5 ? 16 : 32) << 20 ? Route::kSplit : Route::kSkinny;
 }
 
 // Float32 partial products (ksplit, rows, N); ksplit 0 = the library's choice.
@@ -572,10 +580,11 @@ Tensor normalised(const Tensor& x, const Tensor& norm, double eps) {
 
 // The linear with what is folded into it.
 Tensor linear(const Tensor& x, const Tensor& w, const Tensor* norm, double eps, const Tensor* up, const Tensor* residual) {
-    const Route route = route_of(x, w, up != nullptr, residual != nullptr);
-    const Rows r = linear_rows(x, route == Route::kSkinny ? L3_LINEAR_MAX_ROWS : L3_LINEAR_SPLITK_MAX_ROWS, false);
+    const Rows r = linear_rows(x, L3_LINEAR_SPLITK_MAX_ROWS, false);
     check_weight(w, w, x, r.K);
     if (up) check_weight(*up, w, x, r.K);
+    const Route route = route_of(r, w, up != nullptr, residual);
+    if (route == Route::kSkinny) check_rows(r.rows, L3_LINEAR_MAX_ROWS, x);
     if (norm) check_norm_weight(*norm, r.rows, r.K, "linear_decode_fused");
     if (route != Route::kSkinny) {
         const Tensor h = norm ? normalised(x, *norm, eps) : x;

@@ -118,3 +118,46 @@ def test_linear_splitk_of_rows_far_apart(gpu, M, N, K, ksplit, far):
         assert ((part[s].cpu().double() - want).abs() <= 2.0 ** -20 * (xv.double().abs() @ wv.double().abs().t())).all()
     if ksplit == 1 or M == 17:      # (the operator chooses its own splits)
         assert_linear_close(cke.linear_splitk_finish(cke.linear_splitk(x, w)), linear_ref(t2f32(xv), t2f32(wv)), "far rows")
+
+
+# one shape per route: wide, split from 5 rows on, split from 1 row on, pair
+ROUTES = [(4, 16384, 2048, False), (5, 2048, 8192, False), (1, 4096, 8192, False), (4, 8192, 2048, True)]
+
+
+@pytest.mark.parametrize("M,N,K,pair", ROUTES)
+def test_a_residual_aligned_to_eight_bytes_is_taken_whatever_the_route(gpu, M, N, K, pair):
+    from custom_kernels import custom_kernels_extension as cke
+
+    print(f"linear_decode_fused residual M={M} N={N} K={K} pair={pair}", flush=True)
+    x = randn_bf16((M, 1, K), 241).to(gpu)
+    w, up = randn_bf16((N, K), 242, scale=0.05).to(gpu), randn_bf16((N, K), 243, scale=0.05).to(gpu) if pair else None
+    product = cke.linear_decode_fused(x, w, w_up=up)
+    res = randn_bf16((M * N + 4,), 244, scale=3.0).to(gpu)
+    shifted = res[4:].view(M, 1, N)
+    assert shifted.data_ptr() % 16 == 8
+    y = cke.linear_decode_fused(x, w, w_up=up, residual=shifted)
+    if pair:
+        assert torch.equal(y, shifted + product)
+    else:
+        # another kernel's sum may round the other way, one ulp of the product, and the addition rounds once more
+        assert ((y - (shifted + product)).float().abs() <= 2.0 ** -7 * (product.float().abs() + y.float().abs())
+                + 2.0 ** -17 * product.float().abs().max()).all()
+    aligned = shifted.clone()
+    assert torch.equal(cke.linear_decode_fused(x, w, w_up=up, residual=aligned), aligned + product)
+
+
+@pytest.mark.parametrize("M,N,K,pair", ROUTES)
+def test_activations_that_the_skinny_kernel_refuses_are_refused_whatever_the_route(gpu, M, N, K, pair):
+    """Rows on top of each other and rows off 16 bytes, also where a norm in front would make a dense copy of them."""
+    from custom_kernels import custom_kernels_extension as cke
+
+    w = randn_bf16((N, K), 242, scale=0.05).to(gpu)
+    up = w if pair else None
+    rows = min(M, cke.linear_decode_fused_max_rows(K))
+    norm = torch.ones(K, dtype=torch.bfloat16, device=gpu)
+    off = randn_bf16((rows * K + 1,), 245).to(gpu)[1:].view(rows, K)
+    one = randn_bf16((1, K), 246).to(gpu).as_strided((rows, K), (0, 1))
+    for x in (off, one):
+        for kw in (dict(), dict(norm_weight=norm)):
+            with pytest.raises(RuntimeError):
+                cke.linear_decode_fused(x, w, w_up=up, **kw)
