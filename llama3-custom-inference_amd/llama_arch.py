@@ -300,6 +300,22 @@ class LlamaDecoder:
         return self._linear(h[:, -1:, :].contiguous(), self.wte).float()
 
     # ------------------------------------------------------------------------- generate
+    def _prompt_rows(self, prompt_tokens, total_len, looked_up):
+        """The prompts as rows of a (sequences, total_len) host tensor, padded.  Ids among the first `looked_up` positions that
+        are none of the vocabulary raise here, whichever way the embedding is read later (on the GPU F.embedding stops the
+        process, the one launch of a decode step takes the nearest row)."""
+        pad_id = self.tokenizer.pad_id
+        rows = torch.full((len(prompt_tokens), total_len), pad_id, dtype=torch.long)
+        for i, t in enumerate(prompt_tokens):
+            rows[i, :len(t)] = torch.tensor(t, dtype=torch.long)
+        if not all(len(t) == 0 or (min(t) >= 0 and max(t) < self.config.vocab_size) for t in prompt_tokens):
+            common = min(len(t) for t in prompt_tokens)
+            wrong = (rows < 0) | (rows >= self.config.vocab_size)
+            wrong[:, common:] &= rows[:, common:] != pad_id      # (behind the common prefix the pad id is no token)
+            if bool(wrong[:, :looked_up].any()):
+                raise IndexError(f"token id outside the vocabulary of {self.config.vocab_size}")
+        return rows
+
     @torch.inference_mode()
     def generate_graphed(self, prompt_tokens, max_gen_len, echo=False, ignore_eos=False):
         """generate() with the per-token loop replayed from a HIP graph: the prefill of the common
@@ -311,6 +327,7 @@ class LlamaDecoder:
         max_prompt_len = max(len(t) for t in prompt_tokens)
         total_len = min(c.block_size, max_gen_len + max_prompt_len)
         assert bsz <= c.max_gen_batch_size and total_len <= c.max_model_len
+        host = self._prompt_rows(prompt_tokens, total_len, max(total_len - 1, min_prompt_len))
         key = (bsz, total_len)
         loop = self._graphs.get(key)
         if loop is None:
@@ -318,12 +335,8 @@ class LlamaDecoder:
                 self._graphs.pop(next(iter(self._graphs)))
             loop = GraphedDecodeLoop(self, bsz, total_len)
             self._graphs[key] = loop
-        pad_id = self.tokenizer.pad_id
-        host = torch.full((bsz, total_len), pad_id, dtype=torch.long)
-        for i, t in enumerate(prompt_tokens):
-            host[i, :len(t)] = torch.tensor(t, dtype=torch.long)
         loop.tokens.copy_(host)
-        loop.text_mask.copy_(host != pad_id)
+        loop.text_mask.copy_(host != self.tokenizer.pad_id)
         loop.eos.zero_()
         # position min_prompt_len: prefill (recorded once per prompt length) + the usual bookkeeping
         logits = loop.prefill(self, min_prompt_len)
@@ -370,11 +383,8 @@ class LlamaDecoder:
         assert max_prompt_len <= c.block_size
         total_len = min(c.block_size, max_gen_len + max_prompt_len)
         assert total_len <= c.max_model_len, "KV cache too short for prompt + generation"
-        pad_id = self.tokenizer.pad_id
-        tokens = torch.full((bsz, total_len), pad_id, dtype=torch.long, device=self.device)
-        for i, t in enumerate(prompt_tokens):
-            tokens[i, :len(t)] = torch.tensor(t, dtype=torch.long, device=self.device)
-        input_text_mask = tokens != pad_id
+        tokens = self._prompt_rows(prompt_tokens, total_len, total_len - 1 if min_prompt_len < total_len else 0).to(self.device)
+        input_text_mask = tokens != self.tokenizer.pad_id
         stop_tokens = torch.tensor(list(self.tokenizer.stop_tokens), device=self.device)
         eos_reached = torch.zeros(bsz, dtype=torch.bool, device=self.device)
         prev_pos = 0

@@ -164,3 +164,18 @@ def test_weights_that_only_the_operators_take_are_left_to_them(gpu, name):
     graphed = m.generate_graphed(prompts, 16, ignore_eos=True)
     # (the loops plan the attention splits differently, a near tie may fork a stream)
     assert all(a[:8] == b[:8] for a, b in zip(graphed, want))
+
+
+def test_a_token_outside_the_vocabulary_is_refused(gpu):
+    """In a prompt that reaches past the common prefix the decode step looks it up, not the prompt pass."""
+    from custom_kernels import custom_kernels_extension as ops
+    from llama_arch import LlamaConfig, LlamaDecoder, random_prompts
+
+    m = LlamaDecoder(LlamaConfig(n_layer=2, vocab_size=4096, max_model_len=48, max_gen_batch_size=2), ops, gpu)
+    good = random_prompts(2, 16, 4096, 5)
+    assert m._one_launch(2, 33) is not None
+    for generate in (m.generate, m.generate_graphed):
+        for bad in (4096, -1):
+            with pytest.raises(IndexError):
+                generate([good[0], good[1] + [bad]], 16, ignore_eos=True)
+        assert len(generate([good[0], good[1] + [4095]], 16, ignore_eos=True)[1]) == 16      # (padded with 128004)
