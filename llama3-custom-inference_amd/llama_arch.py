@@ -25,6 +25,7 @@ or any object with the same three functions (the CPU baseline passes torch resta
 
 import math
 import time
+import warnings
 from dataclasses import dataclass
 
 import torch
@@ -105,6 +106,8 @@ class LlamaDecoder:
         self._graphs = {}
         self._layer_launches = {}        # rows -> ops.DecodeLayers
         self._layers_in_one_launch = hasattr(ops, "DecodeLayers")
+        self._one_launch_failures = 0    # in a row
+        self._one_launch_rests = 0       # generations until it is tried again
         # nn.Linear calls with at most this many activation rows (the decode step) go through the
         # library's weight-streaming kernels when the operator module has them; 0 = always F.linear
         self.decode_linear_rows = 16 if hasattr(ops, "linear_decode") else 0
@@ -252,10 +255,27 @@ class LlamaDecoder:
             made = self._layer_launches[rows] = self.ops.DecodeLayers(self.layers, rows)
         return made
 
+    ONE_LAUNCH_MAX_REST = 64
+
     def _give_up_one_launch(self):
+        """After a failed() launch: what shared the device with it (a long kernel on another stream, another model's launch) may
+        be gone soon or come back with every generation, so the operators have the repeated generation and the next one,
+        after further failures in a row the next 2, 4, ... 64."""
         self._layers_in_one_launch = False
         self._layer_launches.clear()
         self._graphs.clear()   # recorded decode steps contain it
+        self._one_launch_rests = 1 + min(2 ** self._one_launch_failures, self.ONE_LAUNCH_MAX_REST)
+        self._one_launch_failures += 1
+        warnings.warn("a one-launch decode step waited in vain for the rest of the device; this generation is repeated, and the next "
+                      f"{self._one_launch_rests - 1} made, with the operators one by one", RuntimeWarning, stacklevel=3)
+
+    def _one_launch_done(self, layers):
+        """At the end of a generation whose decode steps were `layers` (None: the operators)."""
+        if layers is not None:
+            self._one_launch_failures = 0
+        elif self._one_launch_rests > 0:
+            self._one_launch_rests -= 1
+            self._layers_in_one_launch = self._layers_in_one_launch or self._one_launch_rests == 0
 
     def _prefill_attention(self, q, k, v):
         """Causal GQA attention for T > 1.  The reference hands this case to torch
@@ -330,7 +350,8 @@ class LlamaDecoder:
         host = self._prompt_rows(prompt_tokens, total_len, max(total_len - 1, min_prompt_len))
         key = (bsz, total_len)
         loop = self._graphs.get(key)
-        if loop is None:
+        if loop is None or loop.layers is not self._one_launch(bsz, total_len):      # (recorded while it rested, say)
+            self._graphs.pop(key, None)
             while len(self._graphs) >= self.MAX_DECODE_LOOPS:      # recorded loops hold device memory
                 self._graphs.pop(next(iter(self._graphs)))
             loop = GraphedDecodeLoop(self, bsz, total_len)
@@ -359,6 +380,7 @@ class LlamaDecoder:
         if loop.layers is not None and loop.layers.failed():
             self._give_up_one_launch()
             return self.generate_graphed(prompt_tokens, max_gen_len, echo, ignore_eos)
+        self._one_launch_done(loop.layers)
         out = []
         for i, toks in enumerate(rows):
             start = 0 if echo else len(prompt_tokens[i])
@@ -408,6 +430,7 @@ class LlamaDecoder:
         if layers is not None and layers.failed():
             self._give_up_one_launch()
             return self.generate(prompt_tokens, max_gen_len, temperature, echo, ignore_eos)
+        self._one_launch_done(layers)
         out = []
         for i, toks in enumerate(rows):
             start = 0 if echo else len(prompt_tokens[i])

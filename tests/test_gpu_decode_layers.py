@@ -179,3 +179,33 @@ def test_a_token_outside_the_vocabulary_is_refused(gpu):
             with pytest.raises(IndexError):
                 generate([good[0], good[1] + [bad]], 16, ignore_eos=True)
         assert len(generate([good[0], good[1] + [4095]], 16, ignore_eos=True)[1]) == 16      # (padded with 128004)
+
+
+def test_the_one_launch_comes_back_after_a_wait_ran_out(gpu):
+    """A failure is told, costs the generation after it the launch, and each further one in a row twice as many."""
+    from custom_kernels import custom_kernels_extension as ops
+    from llama_arch import LlamaConfig, LlamaDecoder, random_prompts
+
+    m = LlamaDecoder(LlamaConfig(n_layer=2, vocab_size=4096, max_model_len=48, max_gen_batch_size=2), ops, gpu)
+    prompts = random_prompts(2, 16, 4096, 5)
+
+    def failing(generate):
+        launch = m._one_launch(2, 32)
+        with torch.inference_mode():
+            launch.workspace[0] = 1
+        with pytest.warns(RuntimeWarning, match="one by one"):
+            return generate(prompts, 16, ignore_eos=True)
+
+    for generate in (m.generate, m.generate_graphed):
+        first = generate(prompts, 16, ignore_eos=True)
+        assert 2 in m._layer_launches
+        for rests in (1, 2, 4):
+            by_operators = failing(generate)
+            for _ in range(rests):
+                assert m._one_launch(2, 32) is None
+                assert generate(prompts, 16, ignore_eos=True) == by_operators
+            assert m._one_launch(2, 32) is not None
+        assert generate(prompts, 16, ignore_eos=True) == first and 2 in m._layer_launches
+        assert m._one_launch_failures == 0
+    key, loop = next(iter(m._graphs.items()))
+    assert key == (2, 32) and loop.layers is m._layer_launches[2]
