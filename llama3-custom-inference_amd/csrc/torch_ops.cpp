@@ -26,6 +26,8 @@
 
 #include <algorithm>
 #include <cmath>
+#include <memory>
+#include <mutex>
 #include <utility>
 #include <vector>
 
@@ -108,13 +110,25 @@ Tensor empty_like_dense(const Tensor& t) {
     return Tensor(at::detail::empty_strided_cuda(t.sizes(), t.strides(), t.scalar_type(), t.device()));
 }
 
+// The work of a call with the interpreter lock released, so that other Python threads go on meanwhile (a launch waits while
+// the queue is full, an allocation may go to the driver, the first decode attention on a device synchronises).  Arguments are
+// unpacked before and results wrapped after it.
+template <typename F>
+auto unlocked(F&& work) {
+    struct Release {
+        PyThreadState* const state = PyEval_SaveThread();
+        ~Release() { PyEval_RestoreThread(state); }
+    } released;
+    return work();
+}
+
 PyObject* wrap(Tensor&& t) { return THPVariable_Wrap(std::move(t)); }
 
-PyObject* wrap_pair(Tensor&& a, Tensor&& b) {
+PyObject* wrap(std::pair<Tensor, Tensor>&& t) {
     PyObject* pair = PyTuple_New(2);
     if (!pair) throw python_error();
-    PyTuple_SET_ITEM(pair, 0, wrap(std::move(a)));
-    PyTuple_SET_ITEM(pair, 1, wrap(std::move(b)));
+    PyTuple_SET_ITEM(pair, 0, wrap(std::move(t.first)));
+    PyTuple_SET_ITEM(pair, 1, wrap(std::move(t.second)));
     return pair;
 }
 
@@ -143,39 +157,43 @@ struct OnDevice {
 
 // Workspaces of decode attention: one per (device, stream), grown on demand, whose head holds the arrival
 // counters of the single-launch form.  Calls on one stream are ordered and can share one; another stream
-// gets its own.  The interpreter lock guards the list.  It is bounded: beyond kMaxWorkspaces streams the
+// gets its own.  `in_use` keeps the launches of a call together where several threads call on one stream (the interpreter lock
+// is released by then).  The list is bounded: beyond kMaxWorkspaces streams the
 // one unused longest goes back to torch's allocator, which hands its memory only to later work of the
 // stream it was allocated on.
 struct Workspace {
     c10::DeviceIndex device;
     hipStream_t stream;
-    TensorBase memory;
+    std::mutex in_use;
+    TensorBase memory;   // guarded by in_use
+    Workspace(c10::DeviceIndex d, hipStream_t s) : device(d), stream(s) {}
 };
 constexpr size_t kMaxWorkspaces = 64;
 
-std::vector<Workspace>& workspaces() {
-    static auto* all = new std::vector<Workspace>();   // outlives the allocator's own teardown
-    return *all;
-}
-
-const TensorBase& attention_workspace(const OnDevice& on, const Tensor& like, size_t nbytes) {
-    auto& all = workspaces();
+std::shared_ptr<Workspace> attention_workspace(const OnDevice& on) {
+    static auto& all = *new std::vector<std::shared_ptr<Workspace>>();   // outlives the allocator's own teardown
+    static auto& all_mutex = *new std::mutex();
+    const std::lock_guard<std::mutex> lock(all_mutex);
     size_t i = 0;
-    while (i < all.size() && !(all[i].stream == on.stream && all[i].device == on.index)) ++i;
-    if (i == all.size() || size_t(all[i].memory.numel()) < nbytes) {
-        TensorBase memory = at::detail::empty_cuda({int64_t(std::max(nbytes, size_t(4) << 20))}, at::kByte, like.device(),
-                                                   std::nullopt);
-        check(lib.l3_attn_workspace_init(ptr(memory), size_t(memory.numel()), on.stream), "l3_attn_workspace_init");
-        if (i < all.size()) {
-            all[i].memory = std::move(memory);
-        } else {
-            if (all.size() >= kMaxWorkspaces) all.pop_back();
-            i = all.size();
-            all.push_back({on.index, on.stream, std::move(memory)});
-        }
+    while (i < all.size() && !(all[i]->stream == on.stream && all[i]->device == on.index)) ++i;
+    if (i == all.size()) {
+        if (all.size() >= kMaxWorkspaces) all.pop_back();
+        i = all.size();
+        all.push_back(std::make_shared<Workspace>(on.index, on.stream));
     }
     if (i > 0) std::rotate(all.begin(), all.begin() + i, all.begin() + i + 1);   // most recently used first
-    return all[0].memory;
+    return all[0];
+}
+
+// At least nbytes, prepared.  (With in_use held.)
+void* grown(Workspace& w, const Tensor& like, size_t nbytes) {
+    if (!w.memory.defined() || size_t(w.memory.numel()) < nbytes) {
+        TensorBase memory = at::detail::empty_cuda({int64_t(std::max(nbytes, size_t(4) << 20))}, at::kByte, like.device(),
+                                                   std::nullopt);
+        check(lib.l3_attn_workspace_init(ptr(memory), size_t(memory.numel()), w.stream), "l3_attn_workspace_init");
+        w.memory = std::move(memory);
+    }
+    return ptr(w.memory);
 }
 
 struct DecodeShape {
@@ -213,11 +231,15 @@ void decode(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& out
     const size_t nbytes = lib.l3_attn_decode_workspace_bytes(s.B, s.QH, s.KVH, s.S, s.HD, num_splits, flags);
     TensorBase own;
     void* ws = nullptr;
+    std::shared_ptr<Workspace> kept;
+    std::unique_lock<std::mutex> in_use;
     if (nbytes > 0 && capturing) {
         own = at::detail::empty_cuda({int64_t(std::max(nbytes, size_t(256)))}, at::kByte, q.device(), std::nullopt);
         ws = ptr(own);
     } else if (nbytes > 0) {
-        ws = ptr(attention_workspace(on, q, nbytes));
+        kept = attention_workspace(on);
+        in_use = std::unique_lock<std::mutex>(kept->in_use);
+        ws = grown(*kept, q, nbytes);
     }
     const float scale = float(1.0 / std::sqrt(double(s.HD)));
     const int64_t* qs = q.strides().data();
@@ -245,9 +267,12 @@ PyObject* flash_attention_decode(PyObject* const* a) {
     const DecodeShape s = check_qkv(q, k, v);
     check_heads(s.QH, s.KVH, s.HD);
     TORCH_CHECK(s.B > 0 && s.S > 0, "flash_attention_decode needs at least one sequence and one cached token");
-    Tensor out = empty_like_query(q);
-    decode(q, k, v, out, s, integer(a[3]), integer(a[4]), nullptr);
-    return wrap(std::move(out));
+    const int num_splits = integer(a[3]), flags = integer(a[4]);
+    return wrap(unlocked([&] {
+        Tensor out = empty_like_query(q);
+        decode(q, k, v, out, s, num_splits, flags, nullptr);
+        return out;
+    }));
 }
 
 // (query, keys, values, kv_len, num_splits, out or None, flags)
@@ -259,9 +284,13 @@ PyObject* flash_attention_decode_devlen(PyObject* const* a) {
     const Tensor& len = tensor(a[3], "kv_len");
     TORCH_CHECK(len.is_cuda() && len.scalar_type() == at::kInt && len.numel() == 1 && len.device() == q.device(),
                 "kv_len must be a one-element int32 tensor on the query's GPU");
-    Tensor out = a[5] == Py_None ? empty_like_query(q) : tensor(a[5], "out");
-    decode(q, k, v, out, s, integer(a[4]), integer(a[6]), static_cast<const int32_t*>(ptr(len)));
-    return wrap(std::move(out));
+    const int num_splits = integer(a[4]), flags = integer(a[6]);
+    Tensor given = a[5] == Py_None ? Tensor() : tensor(a[5], "out");
+    return wrap(unlocked([&] {
+        Tensor out = given.defined() ? std::move(given) : empty_like_query(q);
+        decode(q, k, v, out, s, num_splits, flags, static_cast<const int32_t*>(ptr(len)));
+        return out;
+    }));
 }
 
 // (query, keys, values, flags)
@@ -277,17 +306,20 @@ PyObject* flash_attention_prefill(PyObject* const* a) {
     TORCH_CHECK(stride_at(q, 3) == 1 && stride_at(k, 3) == 1 && stride_at(v, 3) == 1,
                 "the head dimension of query, keys and values must be contiguous");
     check_heads(int(QH), int(KVH), int(HD));
-    // a (B, QH, T, HD) view of a contiguous (B, T, QH, HD) tensor
-    const int64_t sizes[4] = {B, QH, T, HD}, strides[4] = {T * QH * HD, HD, QH * HD, 1};
-    Tensor out(at::detail::empty_strided_cuda(sizes, strides, at::kBFloat16, q.device()));
-    if (out.numel() > 0) {
-        const OnDevice on(q);
-        const int rc = lib.l3_attn_prefill(ptr(q), ptr(k), ptr(v), ptr(out), int(B), int(QH), int(KVH), int(T), int(S), int(HD),
-                                           q.strides().data(), k.strides().data(), v.strides().data(), strides,
-                                           float(1.0 / std::sqrt(double(HD))), integer(a[3]), on.stream);
-        check(rc, "B=", B, " QH=", QH, " KVH=", KVH, " T=", T, " S=", S, " HD=", HD);
-    }
-    return wrap(std::move(out));
+    const int flags = integer(a[3]);
+    return wrap(unlocked([&] {
+        // a (B, QH, T, HD) view of a contiguous (B, T, QH, HD) tensor
+        const int64_t sizes[4] = {B, QH, T, HD}, strides[4] = {T * QH * HD, HD, QH * HD, 1};
+        Tensor out(at::detail::empty_strided_cuda(sizes, strides, at::kBFloat16, q.device()));
+        if (out.numel() > 0) {
+            const OnDevice on(q);
+            const int rc = lib.l3_attn_prefill(ptr(q), ptr(k), ptr(v), ptr(out), int(B), int(QH), int(KVH), int(T), int(S), int(HD),
+                                               q.strides().data(), k.strides().data(), v.strides().data(), strides,
+                                               float(1.0 / std::sqrt(double(HD))), flags, on.stream);
+            check(rc, "B=", B, " QH=", QH, " KVH=", KVH, " T=", T, " S=", S, " HD=", HD);
+        }
+        return out;
+    }));
 }
 
 // ------------------------------------------------------------------------------------ row-wise operators
@@ -299,16 +331,19 @@ PyObject* rms_norm(PyObject* const* a) {
     TORCH_CHECK(input.dim() == 3, "rms_norm expects a 3-D (B, T, C) input");
     const int64_t C = size_at(input, 2);
     TORCH_CHECK(weight.numel() == C, "weight has ", weight.numel(), " elements, expected ", C);
-    Tensor xc, wc;
-    const Tensor& x = contiguous(input, xc);
-    const Tensor& w = contiguous(weight, wc);
-    Tensor out = empty_like_dense(x);
-    const int64_t rows = size_at(x, 0) * size_at(x, 1);
-    if (rows > 0) {
-        const OnDevice on(x);
-        check(lib.l3_rms_norm(ptr(x), ptr(w), ptr(out), rows, int(C), float(number(a[2])), on.stream), "rows=", rows, " C=", C);
-    }
-    return wrap(std::move(out));
+    const float eps = float(number(a[2]));
+    return wrap(unlocked([&] {
+        Tensor xc, wc;
+        const Tensor& x = contiguous(input, xc);
+        const Tensor& w = contiguous(weight, wc);
+        Tensor out = empty_like_dense(x);
+        const int64_t rows = size_at(x, 0) * size_at(x, 1);
+        if (rows > 0) {
+            const OnDevice on(x);
+            check(lib.l3_rms_norm(ptr(x), ptr(w), ptr(out), rows, int(C), eps, on.stream), "rows=", rows, " C=", C);
+        }
+        return out;
+    }));
 }
 
 // (input, residual, weight, eps)
@@ -320,18 +355,20 @@ PyObject* add_rms_norm(PyObject* const* a) {
                 "add_rms_norm expects two (B, T, C) tensors of the same shape");
     const int64_t C = size_at(input, 2);
     TORCH_CHECK(weight.numel() == C, "weight has ", weight.numel(), " elements, expected ", C);
-    Tensor xc, rc_, wc;
-    const Tensor& x = contiguous(input, xc);
-    const Tensor& r = contiguous(residual, rc_);
-    const Tensor& w = contiguous(weight, wc);
-    Tensor s = new_empty(x.sizes(), x), y = new_empty(x.sizes(), x);
-    const int64_t rows = size_at(x, 0) * size_at(x, 1);
-    if (rows > 0) {
-        const OnDevice on(x);
-        check(lib.l3_add_rms_norm(ptr(x), ptr(r), ptr(w), ptr(s), ptr(y), rows, int(C), float(number(a[3])), on.stream), "rows=",
-              rows, " C=", C);
-    }
-    return wrap_pair(std::move(s), std::move(y));
+    const float eps = float(number(a[3]));
+    return wrap(unlocked([&] {
+        Tensor xc, rc_, wc;
+        const Tensor& x = contiguous(input, xc);
+        const Tensor& r = contiguous(residual, rc_);
+        const Tensor& w = contiguous(weight, wc);
+        Tensor s = new_empty(x.sizes(), x), y = new_empty(x.sizes(), x);
+        const int64_t rows = size_at(x, 0) * size_at(x, 1);
+        if (rows > 0) {
+            const OnDevice on(x);
+            check(lib.l3_add_rms_norm(ptr(x), ptr(r), ptr(w), ptr(s), ptr(y), rows, int(C), eps, on.stream), "rows=", rows, " C=", C);
+        }
+        return std::pair(std::move(s), std::move(y));
+    }));
 }
 
 const Tensor& partials(PyObject* o, const char* what) {
@@ -351,27 +388,26 @@ PyObject* add_rms_norm_partials(PyObject* const* a) {
     TORCH_CHECK(size_at(part, 1) == rows && size_at(part, 2) == C, "add_rms_norm_partials: partials ", part.sizes(),
                 " do not fit input ", input.sizes());
     TORCH_CHECK(weight.numel() == C && weight.is_contiguous(), "weight has ", weight.numel(), " elements, expected ", C);
-    Tensor xc;
-    const Tensor& x = contiguous(input, xc);
-    Tensor s = new_empty(x.sizes(), x), y = new_empty(x.sizes(), x);
-    const OnDevice on(x);
-    check(lib.l3_add_rms_norm_partials(ptr(x), ptr(part), int(size_at(part, 0)), ptr(weight), ptr(s), ptr(y), int(rows), int(C),
-                                       float(number(a[3])), on.stream),
-          "rows=", rows, " C=", C, " ksplit=", size_at(part, 0));
-    return wrap_pair(std::move(s), std::move(y));
+    const float eps = float(number(a[3]));
+    return wrap(unlocked([&] {
+        Tensor xc;
+        const Tensor& x = contiguous(input, xc);
+        Tensor s = new_empty(x.sizes(), x), y = new_empty(x.sizes(), x);
+        const OnDevice on(x);
+        check(lib.l3_add_rms_norm_partials(ptr(x), ptr(part), int(size_at(part, 0)), ptr(weight), ptr(s), ptr(y), int(rows), int(C),
+                                           eps, on.stream),
+              "rows=", rows, " C=", C, " ksplit=", size_at(part, 0));
+        return std::pair(std::move(s), std::move(y));
+    }));
 }
 
-// (a, b)
-PyObject* silu_mul(PyObject* const* args) {
-    const Tensor& a = gpu_bf16(args[0], "a");
-    const Tensor& b = gpu_bf16(args[1], "b");
-    TORCH_CHECK(a.sizes() == b.sizes(), "silu_mul: shapes differ: ", a.sizes(), " vs ", b.sizes());
+Tensor silu_mul_of(const Tensor& a, const Tensor& b) {
     Tensor y = new_empty(a.sizes(), a);
-    if (a.numel() == 0) return wrap(std::move(y));
+    if (a.numel() == 0) return y;
     const OnDevice on(a);
     if (a.is_contiguous() && b.is_contiguous()) {
         check(lib.l3_silu_mul(ptr(a), ptr(b), ptr(y), y.numel(), on.stream), "n=", y.numel());
-        return wrap(std::move(y));
+        return y;
     }
     const int64_t C = a.sizes().back(), rows = a.numel() / C;
     if (C % 8 == 0 && a.strides().back() == 1 && b.strides().back() == 1) {
@@ -386,12 +422,20 @@ PyObject* silu_mul(PyObject* const* args) {
             check(lib.l3_silu_mul_rows(ptr(a2), ptr(b2), ptr(y), rows, C, std::max(stride_at(a2, 0), C),
                                        std::max(stride_at(b2, 0), C), on.stream),
                   "rows=", rows, " cols=", C);
-            return wrap(std::move(y));
+            return y;
         }
     }
     const Tensor ac = a.contiguous(), bc = b.contiguous();
     check(lib.l3_silu_mul(ptr(ac), ptr(bc), ptr(y), y.numel(), on.stream), "n=", y.numel());
-    return wrap(std::move(y));
+    return y;
+}
+
+// (a, b)
+PyObject* silu_mul(PyObject* const* args) {
+    const Tensor& a = gpu_bf16(args[0], "a");
+    const Tensor& b = gpu_bf16(args[1], "b");
+    TORCH_CHECK(a.sizes() == b.sizes(), "silu_mul: shapes differ: ", a.sizes(), " vs ", b.sizes());
+    return wrap(unlocked([&] { return silu_mul_of(a, b); }));
 }
 
 // (input, freq)
@@ -405,16 +449,18 @@ PyObject* rot_embed(PyObject* const* a) {
     TORCH_CHECK(size_at(freq, 0) == xs[1] && size_at(freq, 1) == xs[3], "freq is ", freq.sizes(), ", expected (", xs[1], ", ",
                 xs[3], ")");
     TORCH_CHECK(stride_at(x, 3) == 1, "the head dimension of input must be contiguous");
-    Tensor fc;
-    const Tensor& f = contiguous(freq, fc);
-    Tensor out = new_empty(xs, x);
-    if (out.numel() > 0) {
-        const OnDevice on(x);
-        check(lib.l3_rot_embed(ptr(x), static_cast<const float*>(ptr(f)), ptr(out), int(xs[0]), int(xs[1]), int(xs[2]), int(xs[3]),
-                               x.strides().data(), on.stream),
-              "B=", xs[0], " T=", xs[1], " NH=", xs[2], " HD=", xs[3], " strides=", x.strides());
-    }
-    return wrap(std::move(out));
+    return wrap(unlocked([&] {
+        Tensor fc;
+        const Tensor& f = contiguous(freq, fc);
+        Tensor out = new_empty(xs, x);
+        if (out.numel() > 0) {
+            const OnDevice on(x);
+            check(lib.l3_rot_embed(ptr(x), static_cast<const float*>(ptr(f)), ptr(out), int(xs[0]), int(xs[1]), int(xs[2]),
+                                   int(xs[3]), x.strides().data(), on.stream),
+                  "B=", xs[0], " T=", xs[1], " NH=", xs[2], " HD=", xs[3], " strides=", x.strides());
+        }
+        return out;
+    }));
 }
 
 // ---------------------------------------------------------------------------------------------- linears
@@ -607,31 +653,41 @@ Tensor linear(const Tensor& x, const Tensor& w, const Tensor* norm, double eps, 
 
 // (x, weight)
 PyObject* linear_decode(PyObject* const* a) {
-    return wrap(linear(gpu_bf16(a[0], "x"), gpu_bf16(a[1], "weight"), nullptr, 0.0, nullptr, nullptr));
+    const Tensor &x = gpu_bf16(a[0], "x"), &w = gpu_bf16(a[1], "weight");
+    return wrap(unlocked([&] { return linear(x, w, nullptr, 0.0, nullptr, nullptr); }));
 }
 
 // (x, w_gate, w_up)
 PyObject* linear_swiglu_decode(PyObject* const* a) {
-    return wrap(linear(gpu_bf16(a[0], "x"), gpu_bf16(a[1], "weight"), nullptr, 0.0, &gpu_bf16(a[2], "weight"), nullptr));
+    const Tensor &x = gpu_bf16(a[0], "x"), &w = gpu_bf16(a[1], "weight"), &up = gpu_bf16(a[2], "weight");
+    return wrap(unlocked([&] { return linear(x, w, nullptr, 0.0, &up, nullptr); }));
 }
 
 // (x, weight, norm_weight or None, eps, w_up or None, residual or None)
 PyObject* linear_decode_fused(PyObject* const* a) {
-    return wrap(linear(gpu_bf16(a[0], "x"), gpu_bf16(a[1], "weight"), optional_tensor(a[2], "norm_weight"), number(a[3]),
-                       optional_tensor(a[4], "weight"), optional_tensor(a[5], "residual")));
+    const Tensor &x = gpu_bf16(a[0], "x"), &w = gpu_bf16(a[1], "weight");
+    const Tensor *norm = optional_tensor(a[2], "norm_weight"), *up = optional_tensor(a[4], "weight");
+    const Tensor* residual = optional_tensor(a[5], "residual");
+    const double eps = number(a[3]);
+    return wrap(unlocked([&] { return linear(x, w, norm, eps, up, residual); }));
 }
 
 // (x, weight, ksplit)
 PyObject* linear_splitk(PyObject* const* a) {
-    return wrap(splitk(gpu_bf16(a[0], "x"), gpu_bf16(a[1], "weight"), integer(a[2])));
+    const Tensor &x = gpu_bf16(a[0], "x"), &w = gpu_bf16(a[1], "weight");
+    const int ksplit = integer(a[2]);
+    return wrap(unlocked([&] { return splitk(x, w, ksplit); }));
 }
 
 // (part, residual or None)
 PyObject* linear_splitk_finish(PyObject* const* a) {
     const Tensor& part = partials(a[0], "linear_splitk_finish");
-    Tensor y = new_empty({size_at(part, 1), size_at(part, 2)}, part);
-    splitk_finish(part, optional_tensor(a[1], "residual"), y);
-    return wrap(std::move(y));
+    const Tensor* residual = optional_tensor(a[1], "residual");
+    return wrap(unlocked([&] {
+        Tensor y = new_empty({size_at(part, 1), size_at(part, 2)}, part);
+        splitk_finish(part, residual, y);
+        return y;
+    }));
 }
 
 // Rotary table, position and cache of the operators that append to the KV cache.
@@ -660,43 +716,48 @@ Cache cache_args(PyObject* table, PyObject* cache_k, PyObject* cache_v, PyObject
 PyObject* linear_qkv_rope_append(PyObject* const* a) {
     const Tensor& x = gpu_bf16(a[0], "x");
     const Tensor& w = gpu_bf16(a[1], "weight");
-    const Rows r = linear_rows(x, L3_LINEAR_MAX_ROWS, false);
-    check_weight(w, w, x, r.K);
     const Cache c = cache_args(a[2], a[3], a[4], a[5]);
     const int64_t NH = integer(a[6]);
-    TORCH_CHECK(size_at(w, 0) == (NH + 2 * c.KVH) * c.HD && r.rows <= c.maxB, "w_qkv ", w.sizes(), " does not match n_head=", NH,
-                ", cache ", c.k->sizes());
     const Tensor* norm = optional_tensor(a[7], "norm_weight");
-    if (norm) check_norm_weight(*norm, r.rows, r.K, "linear_qkv_rope_append");
-    Tensor out = new_empty({r.rows, 1, NH, c.HD}, x);
-    const OnDevice on(x);
-    check(lib.l3_linear_qkv_rope_append(r.x, norm ? ptr(*norm) : nullptr, float(number(a[8])), ptr(w),
-                                        static_cast<const float*>(ptr(*c.table)), ptr(out), ptr(*c.k), ptr(*c.v),
-                                        static_cast<const int32_t*>(ptr(*c.pos)), int(r.rows), int(NH), int(c.KVH), int(c.HD),
-                                        int(r.K), r.stride, stride_at(w, 0), c.k->strides().data(), int(c.L),
-                                        int(size_at(*c.table, 0)), on.stream),
-          "B=", r.rows, " NH=", NH, " KVH=", c.KVH, " HD=", c.HD, " K=", r.K);
-    return wrap(std::move(out));
+    const float eps = float(number(a[8]));
+    return wrap(unlocked([&] {
+        const Rows r = linear_rows(x, L3_LINEAR_MAX_ROWS, false);
+        check_weight(w, w, x, r.K);
+        TORCH_CHECK(size_at(w, 0) == (NH + 2 * c.KVH) * c.HD && r.rows <= c.maxB, "w_qkv ", w.sizes(), " does not match n_head=",
+                    NH, ", cache ", c.k->sizes());
+        if (norm) check_norm_weight(*norm, r.rows, r.K, "linear_qkv_rope_append");
+        Tensor out = new_empty({r.rows, 1, NH, c.HD}, x);
+        const OnDevice on(x);
+        check(lib.l3_linear_qkv_rope_append(r.x, norm ? ptr(*norm) : nullptr, eps, ptr(w),
+                                            static_cast<const float*>(ptr(*c.table)), ptr(out), ptr(*c.k), ptr(*c.v),
+                                            static_cast<const int32_t*>(ptr(*c.pos)), int(r.rows), int(NH), int(c.KVH),
+                                            int(c.HD), int(r.K), r.stride, stride_at(w, 0), c.k->strides().data(), int(c.L),
+                                            int(size_at(*c.table, 0)), on.stream),
+              "B=", r.rows, " NH=", NH, " KVH=", c.KVH, " HD=", c.HD, " K=", r.K);
+        return out;
+    }));
 }
 
 // (x, w_qkv, freq_table, cache_k, cache_v, pos, n_head)
 PyObject* linear_qkv_rope_append_rows(PyObject* const* a) {
     const Tensor& x = gpu_bf16(a[0], "x");
     const Tensor& w = gpu_bf16(a[1], "weight");
-    const Rows r = linear_rows(x, L3_LINEAR_SPLITK_MAX_ROWS, true);
-    check_weight(w, w, x, r.K);
     const Cache c = cache_args(a[2], a[3], a[4], a[5]);
     const int64_t NH = integer(a[6]);
-    TORCH_CHECK(size_at(w, 0) == (NH + 2 * c.KVH) * c.HD && r.rows <= c.maxB, "w_qkv ", w.sizes(), " does not match n_head=", NH,
-                ", cache ", c.k->sizes());
-    Tensor out = new_empty({r.rows, 1, NH, c.HD}, x);
-    const OnDevice on(x);
-    check(lib.l3_linear_qkv_rope_append_rows(r.x, ptr(w), static_cast<const float*>(ptr(*c.table)), ptr(out), ptr(*c.k), ptr(*c.v),
-                                             static_cast<const int32_t*>(ptr(*c.pos)), int(r.rows), int(NH), int(c.KVH), int(c.HD),
-                                             int(r.K), r.stride, stride_at(w, 0), c.k->strides().data(), int(c.L),
-                                             int(size_at(*c.table, 0)), on.stream),
-          "B=", r.rows, " NH=", NH, " KVH=", c.KVH, " HD=", c.HD, " K=", r.K);
-    return wrap(std::move(out));
+    return wrap(unlocked([&] {
+        const Rows r = linear_rows(x, L3_LINEAR_SPLITK_MAX_ROWS, true);
+        check_weight(w, w, x, r.K);
+        TORCH_CHECK(size_at(w, 0) == (NH + 2 * c.KVH) * c.HD && r.rows <= c.maxB, "w_qkv ", w.sizes(), " does not match n_head=",
+                    NH, ", cache ", c.k->sizes());
+        Tensor out = new_empty({r.rows, 1, NH, c.HD}, x);
+        const OnDevice on(x);
+        check(lib.l3_linear_qkv_rope_append_rows(r.x, ptr(w), static_cast<const float*>(ptr(*c.table)), ptr(out), ptr(*c.k),
+                                                 ptr(*c.v), static_cast<const int32_t*>(ptr(*c.pos)), int(r.rows), int(NH),
+                                                 int(c.KVH), int(c.HD), int(r.K), r.stride, stride_at(w, 0),
+                                                 c.k->strides().data(), int(c.L), int(size_at(*c.table, 0)), on.stream),
+              "B=", r.rows, " NH=", NH, " KVH=", c.KVH, " HD=", c.HD, " K=", r.K);
+        return out;
+    }));
 }
 
 // (part, freq_table, cache_k, cache_v, pos, n_head)
@@ -706,14 +767,16 @@ PyObject* rot_embed_append_partials(PyObject* const* a) {
     const int64_t NH = integer(a[5]), ksplit = size_at(part, 0), B = size_at(part, 1);
     TORCH_CHECK(size_at(part, 2) == (NH + 2 * c.KVH) * c.HD && B <= c.maxB, "partials ", part.sizes(), " do not match n_head=", NH,
                 ", cache ", c.k->sizes());
-    Tensor out = new_empty({B, 1, NH, c.HD}, part);
-    const OnDevice on(part);
-    check(lib.l3_rot_embed_append_partials(static_cast<const float*>(ptr(part)), int(ksplit),
-                                           static_cast<const float*>(ptr(*c.table)), ptr(out), ptr(*c.k), ptr(*c.v),
-                                           static_cast<const int32_t*>(ptr(*c.pos)), int(B), int(NH), int(c.KVH), int(c.HD),
-                                           c.k->strides().data(), int(c.L), int(size_at(*c.table, 0)), on.stream),
-          "B=", B, " NH=", NH, " KVH=", c.KVH, " HD=", c.HD, " ksplit=", ksplit);
-    return wrap(std::move(out));
+    return wrap(unlocked([&] {
+        Tensor out = new_empty({B, 1, NH, c.HD}, part);
+        const OnDevice on(part);
+        check(lib.l3_rot_embed_append_partials(static_cast<const float*>(ptr(part)), int(ksplit),
+                                               static_cast<const float*>(ptr(*c.table)), ptr(out), ptr(*c.k), ptr(*c.v),
+                                               static_cast<const int32_t*>(ptr(*c.pos)), int(B), int(NH), int(c.KVH), int(c.HD),
+                                               c.k->strides().data(), int(c.L), int(size_at(*c.table, 0)), on.stream),
+              "B=", B, " NH=", NH, " KVH=", c.KVH, " HD=", c.HD, " ksplit=", ksplit);
+        return out;
+    }));
 }
 
 // --------------------------------------------------------------------------------------------- the module
