@@ -696,7 +696,8 @@ struct Cache {
     int64_t maxB, L, KVH, HD;
 };
 
-Cache cache_args(PyObject* table, PyObject* cache_k, PyObject* cache_v, PyObject* pos) {
+// `like`: the activations, whose GPU all of it has to be on.
+Cache cache_args(const Tensor& like, PyObject* table, PyObject* cache_k, PyObject* cache_v, PyObject* pos) {
     Cache c{&gpu_bf16(cache_k, "cache_k"), &gpu_bf16(cache_v, "cache_v"), &tensor(table, "freq_table"), &tensor(pos, "pos"),
             0, 0, 0, 0};
     TORCH_CHECK(c.k->dim() == 4 && c.k->sizes() == c.v->sizes() && c.k->strides() == c.v->strides(),
@@ -709,6 +710,9 @@ Cache cache_args(PyObject* table, PyObject* cache_k, PyObject* cache_v, PyObject
                 "freq_table must be a contiguous (rows, HD) float32 GPU tensor");
     TORCH_CHECK(c.pos->is_cuda() && c.pos->scalar_type() == at::kInt && c.pos->numel() == 1,
                 "pos must be a one-element int32 GPU tensor");
+    for (const Tensor* t : {c.k, c.v, c.table, c.pos}) {
+        TORCH_CHECK(t->device() == like.device(), "activations, freq_table, pos and the caches must be on the same device");
+    }
     return c;
 }
 
@@ -716,7 +720,7 @@ Cache cache_args(PyObject* table, PyObject* cache_k, PyObject* cache_v, PyObject
 PyObject* linear_qkv_rope_append(PyObject* const* a) {
     const Tensor& x = gpu_bf16(a[0], "x");
     const Tensor& w = gpu_bf16(a[1], "weight");
-    const Cache c = cache_args(a[2], a[3], a[4], a[5]);
+    const Cache c = cache_args(x, a[2], a[3], a[4], a[5]);
     const int64_t NH = integer(a[6]);
     const Tensor* norm = optional_tensor(a[7], "norm_weight");
     const float eps = float(number(a[8]));
@@ -742,7 +746,7 @@ PyObject* linear_qkv_rope_append(PyObject* const* a) {
 PyObject* linear_qkv_rope_append_rows(PyObject* const* a) {
     const Tensor& x = gpu_bf16(a[0], "x");
     const Tensor& w = gpu_bf16(a[1], "weight");
-    const Cache c = cache_args(a[2], a[3], a[4], a[5]);
+    const Cache c = cache_args(x, a[2], a[3], a[4], a[5]);
     const int64_t NH = integer(a[6]);
     return wrap(unlocked([&] {
         const Rows r = linear_rows(x, L3_LINEAR_SPLITK_MAX_ROWS, true);
@@ -763,7 +767,7 @@ PyObject* linear_qkv_rope_append_rows(PyObject* const* a) {
 // (part, freq_table, cache_k, cache_v, pos, n_head)
 PyObject* rot_embed_append_partials(PyObject* const* a) {
     const Tensor& part = partials(a[0], "rot_embed_append_partials");
-    const Cache c = cache_args(a[1], a[2], a[3], a[4]);
+    const Cache c = cache_args(part, a[1], a[2], a[3], a[4]);
     const int64_t NH = integer(a[5]), ksplit = size_at(part, 0), B = size_at(part, 1);
     TORCH_CHECK(size_at(part, 2) == (NH + 2 * c.KVH) * c.HD && B <= c.maxB, "partials ", part.sizes(), " do not match n_head=", NH,
                 ", cache ", c.k->sizes());

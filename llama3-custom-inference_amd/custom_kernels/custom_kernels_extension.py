@@ -471,6 +471,8 @@ class DecodeLayers:
         if not pos.is_cuda or pos.dtype != torch.int32 or pos.numel() != 1:
             raise RuntimeError("pos must be a one-element int32 GPU tensor")
         device = self.table.device
+        if freq_table.device != device or pos.device != device:
+            raise RuntimeError("DecodeLayers: freq_table and pos must be on the GPU of the layers")
         out = torch.empty((self.rows, 1, self.C), dtype=torch.bfloat16, device=device)
         with _on_device(device):
             rc = getattr(_l3lib.load(), function)(self.table.data_ptr(), self.n_layer, *source, out.data_ptr(), self.rows,
