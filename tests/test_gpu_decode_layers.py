@@ -84,6 +84,80 @@ def test_decode_layers_against_float32(gpu, B):
                                                   EPS), y)
 
 
+# (rows, position): around the tiles of 32 tokens and the rounds of a row's wavefronts, and the last position of the longest
+# cache for which the decode step is used (rows x length = 4096)
+@pytest.mark.parametrize("B,pos", [(1, 31), (1, 32), (1, 255), (1, 256), (1, 4095), (2, 130), (2, 2047), (3, 96), (3, 1364), (4, 65), (4, 1023)])
+def test_every_edge_token_counts(gpu, B, pos):
+    """Attention of the one launch with a handful of tokens, at every kind of edge, that share nearly all of the weight and
+    carry large values of their own: attending to one of them less (checked in the float32 reference) moves the result by far
+    more than the bound.  The appended token is one of them."""
+    from custom_kernels import custom_kernels_extension as ops
+    from llama_arch import LlamaDecoder, precompute_freqs_cis
+
+    assert B * (pos + 1) <= LlamaDecoder.ONE_LAUNCH_MAX_POSITIONS
+    L = _layers(gpu, 1, B, pos + 1)[0]
+    table = precompute_freqs_cis(HD, pos + 1, 500000.0, True, scale_factor=32.0, device=gpu)
+    x = randn_bf16((B, 1, C), 950 + pos).to(gpu)
+    # a key head's weights are those of its query heads together, so that the appended key points where the queries point
+    rep = QH // KVH
+    w_q = L["c_attn"][:QH * HD].float().view(KVH, rep, HD, C)
+    L["c_attn"][QH * HD:(QH + KVH) * HD] = w_q.sum(1).reshape(KVH * HD, C).to(torch.bfloat16)
+    h = x[:, 0].float()
+    h = h * torch.rsqrt((h * h).mean(-1, keepdim=True) + EPS) * L["ln_1"].float()
+    key = _rotate((h @ L["c_attn"][QH * HD:(QH + KVH) * HD].float().t()).view(B, KVH, HD), table[pos])
+    edges = sorted({t for t in (0, 31, 32, 127, 128, 255, 256, pos // 2, pos - 1) if 0 <= t < pos})
+    L["cache_k"][:, edges] = (key[:, None] + 0.05 * randn_bf16((B, len(edges), KVH, HD), 951).to(gpu)).to(torch.bfloat16)
+    L["cache_v"][:, edges] = randn_bf16((B, len(edges), KVH, HD), 952, scale=6.0).to(gpu)
+    # The appended value joins them: its weights are larger too.
+    L["c_attn"][(QH + KVH) * HD:] *= 6
+    # all keys larger, so that those few tokens have the weight of thousands
+    gain = 2.0
+    L["c_attn"][QH * HD:(QH + KVH) * HD] *= gain
+    L["cache_k"][:, edges] *= gain
+    want, _ = _float32_step(x, [L], table, pos)
+
+    # Ten roundings lie on the way in a layer (as above), each off by 2^-9 / sqrt(3) in the mean.  A score is the sum of HD
+    # products of a query and a key that have been rounded twice each, four such roundings of its terms, whose root sum of
+    # squares is `spread`; the weights of the few tokens are off by as much, and attention's part of the result with them.
+    # All of it independent, and rows differ: twice the mean.
+    q = _rotate((h @ L["c_attn"][:QH * HD].float().t()).view(B, KVH, rep, HD), table[pos])
+    spread2 = (q * (gain * key)[:, :, None]).pow(2).sum(-1).mean().item() / HD
+    tol = 2 * 2.0 ** -9 / 3 ** 0.5 * (10 + 4 * spread2) ** 0.5
+    scale = want.norm(dim=-1)
+
+    def without(t, head):
+        """The reference with no weight on token t for the query heads of one key head: what one XCD could get wrong."""
+        kept = dict(L)
+        if t == pos:
+            rows = slice((QH + head) * HD, (QH + head + 1) * HD)
+            kept["c_attn"] = L["c_attn"].clone()
+            kept["c_attn"][rows] *= -1
+        else:
+            kept["cache_k"] = L["cache_k"].clone()
+            kept["cache_k"][:, t, head] *= -1
+        return _float32_step(x, [kept], table, pos)[0]
+
+    print(f"decode_layers edges B={B} pos={pos} tol={tol:.4f}", flush=True)
+    for t in edges + [pos]:
+        assert ((without(t, t % KVH) - want).norm(dim=-1) > 1.5 * tol * scale).all(), t
+    one_launch = ops.DecodeLayers([L], B)
+    y = one_launch(x, table, torch.tensor([pos], dtype=torch.int32, device=gpu), EPS)
+    assert not one_launch.failed()
+    off = ((y[:, 0].float() - want).norm(dim=-1) / scale).max().item()
+    print(f"  off by {off:.4f}", flush=True)
+    assert off <= tol
+
+
+def test_one_launch_up_to_its_last_position_and_no_further(gpu):
+    from custom_kernels import custom_kernels_extension as ops
+    from llama_arch import LlamaConfig, LlamaDecoder
+
+    m = LlamaDecoder(LlamaConfig(n_layer=1, vocab_size=512, max_model_len=4200, max_gen_batch_size=5), ops, gpu)
+    for rows, most in ((1, 4096), (2, 2048), (3, 1365), (4, 1024)):
+        assert m._one_launch(rows, most) is not None and m._one_launch(rows, most + 1) is None
+    assert m._one_launch(5, 8) is None
+
+
 def _handed_over(one_launch, rows, n_layer):
     """The words that the workgroups of an XCD have handed each other, (layer, XCD, word), from the workspace: residual rows
     (written from the second layer on), rows behind c_proj, q | k | v, hidden units."""
@@ -111,6 +185,32 @@ def test_handed_over_words_name_their_launch_and_the_xcd_that_wrote_them(gpu, B)
         assert torch.equal(tags[1], tags[1, :, :1].expand_as(tags[1])) and torch.equal(tags[0, :, B * C:], tags[1, :, B * C:])
         assert (tags[1] >> 4 == (before + 1) % 4096).all()
         assert sorted((tags[1, :, 0] & 15).tolist()) == list(range(8))
+
+
+@pytest.mark.parametrize("B", [1, 2, 4])
+def test_generation_by_the_one_launch_and_by_the_operators(gpu, B):
+    """The same tokens, and keys and values as near as two orders of the sums leave them.  The embedding is wide, so that the
+    pick does not hang on the last bit of a logit."""
+    from custom_kernels import custom_kernels_extension as ops
+    from llama_arch import LlamaConfig, LlamaDecoder, random_prompts
+
+    m = LlamaDecoder(LlamaConfig(n_layer=4, vocab_size=4096, max_model_len=48, max_gen_batch_size=B), ops, gpu)
+    m.wte = randn_bf16((4096, C), 77).to(gpu)
+    prompts = random_prompts(B, 16, 4096, 5)
+    if B > 1:
+        prompts[1] = prompts[1][:9]       # (prompt tokens through the decode step)
+    for generate in (m.generate, m.generate_graphed):
+        results = []
+        for m._layers_in_one_launch in (True, False):
+            m._graphs.clear()
+            tokens = generate(prompts, 16, ignore_eos=True)
+            results.append((tokens, [L[n][:, :31].float() for L in m.layers for n in ("cache_k", "cache_v")]))
+        (tokens, one), (tokens_op, by_operators) = results
+        assert tokens == tokens_op and B in m._layer_launches and not m._layer_launches[B].failed()
+        # ten roundings per layer on either side, up to the layer in question
+        for i, (a, b) in enumerate(zip(one, by_operators)):
+            tol = 3 * (2 * 10 * (i // 2 + 1)) ** 0.5 * 2.0 ** -9 / 3 ** 0.5
+            assert ((a - b).norm(dim=(-1, -2)) <= tol * b.norm(dim=(-1, -2))).all(), (i, tol)
 
 
 def test_generation_without_the_one_launch_after_a_wait_ran_out(gpu):

@@ -161,3 +161,18 @@ def test_activations_that_the_skinny_kernel_refuses_are_refused_whatever_the_rou
         for kw in (dict(), dict(norm_weight=norm)):
             with pytest.raises(RuntimeError):
                 cke.linear_decode_fused(x, w, w_up=up, **kw)
+
+
+@pytest.mark.parametrize("M", [4, 7, 11])
+def test_a_norm_in_front_of_a_linear_that_fills_the_device(gpu, M):
+    """More than three rows of a vocabulary projection: the norm is a launch of its own and rounds where it would inside."""
+    from custom_kernels import custom_kernels_extension as cke
+
+    N, K, eps = 12288, 2048, 1e-5
+    print(f"norm and wide linear M={M}", flush=True)
+    x, norm = randn_bf16((M, 1, K), 251).to(gpu), randn_bf16((K,), 252, scale=0.02, mean=1.0).to(gpu)
+    w = randn_bf16((N, K), 253, scale=0.05).to(gpu)
+    y = cke.linear_decode_fused(x, w, norm_weight=norm, eps=eps)
+    h = cke.rms_norm(x, norm, eps)
+    assert_linear_close(y.view(M, N), linear_ref(t2f32(h.view(M, K)), t2f32(w)), f"norm and wide {M}")
+    assert torch.equal(y, cke.linear_decode(h, w))

@@ -322,3 +322,40 @@ def test_full_size_graphed_loop_matches_eager(gpu, full_size_model, batch):
         agree += common
         total += len(a)
     assert agree >= 0.98 * total, f"only {agree} of {total} tokens lie in common prefixes"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch", [1, 4])
+def test_full_size_one_launch_step_matches_the_operators(gpu, full_size_model, batch):
+    """Decode steps of all 16 layers in one launch against forward(), which runs the operators one by one, on the same tokens:
+    logits, and the appended keys and values of every layer."""
+    from custom_kernels import custom_kernels_extension as cke
+
+    m = full_size_model
+    launch = cke.DecodeLayers(m.layers, batch)
+    ids = torch.tensor(la.random_prompts(batch, 131, m.config.vocab_size, 41), device=gpu)
+    with torch.inference_mode():
+        m.forward(ids[:, :128], start_pos=0)
+        for at in (128, 129, 130):
+            print(f"full-size one launch: batch {batch} position {at}", flush=True)
+            want = m.forward(ids[:, at:at + 1], start_pos=at)[:, -1]
+            rows = [L[n][:batch, at].float() for L in m.layers for n in ("cache_k", "cache_v")]
+            for L in m.layers:
+                L["cache_k"][:batch, at] = L["cache_v"][:batch, at] = 0
+            pos = torch.tensor([at], dtype=torch.int32, device=gpu)
+            h = launch.from_tokens(ids[:, at:at + 1], m.wte, m.freqs_cis, pos, m.config.norm_eps)
+            got = cke.linear_decode_fused(h[:, -1], m.wte, norm_weight=m.ln_f, eps=m.config.norm_eps).float()
+            assert not launch.failed()
+            # Two orders of the sums, and ten roundings to bf16 per layer and side that they may send either way, in the mean
+            # by 2^-9 / 3 ** 0.5 each: (2 x 10 x layers) ** 0.5 of these up to a layer, 2.0e-2 behind all sixteen (each side
+            # alone is 1.9e-2 off float64 there).  Rows differ in it: twice the mean.
+            tol = [2 * (20 * (i + 1)) ** 0.5 * 2.0 ** -9 / 3 ** 0.5 for i in range(m.config.n_layer)]
+            worst = 0.0
+            for i, L in enumerate(m.layers):
+                for n, row in (("cache_k", rows[2 * i]), ("cache_v", rows[2 * i + 1])):
+                    off = ((L[n][:batch, at].float() - row).norm(dim=(1, 2)) / row.norm(dim=(1, 2))).max().item()
+                    worst = max(worst, off / tol[i])
+                    assert off <= tol[i], (i, n)
+            off = ((got - want).norm(dim=-1) / want.norm(dim=-1)).max().item()
+            print(f"  logits off by {off:.4f}, keys and values by at most {worst:.2f} of their bound", flush=True)
+            assert off <= tol[-1]
