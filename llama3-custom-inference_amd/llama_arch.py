@@ -16,9 +16,9 @@ the same tensor layouts and views -- without its checkpoint loading:
                                                        stop-token bookkeeping with one device-side .all()
                                                        (the reference iterates the tensor in Python, :380)
 
-Embedding, sampling and every nn.Linear with more than a few activation rows stay stock PyTorch,
-as in the reference; the linears of the decode step (T == 1) use ops.linear_decode /
-ops.linear_swiglu_decode when the operator module has them.  `ops` is the
+Embedding, sampling and the nn.Linear calls of a prompt pass stay stock PyTorch, as in the reference; so do those of a
+decode step (T == 1) above 64 sequences.  Up to four sequences all layers of a step are one launch where the model and the
+length suit it (ops.DecodeLayers), and up to 64 its linears are the operator module's, when it has them.  `ops` is the
 module that provides the three operators: custom_kernels.custom_kernels_extension on the GPU,
 or any object with the same three functions (the CPU baseline passes torch restatements).
 """
@@ -108,6 +108,7 @@ class LlamaDecoder:
         self._layers_in_one_launch = hasattr(ops, "DecodeLayers")
         self._one_launch_failures = 0    # in a row
         self._one_launch_rests = 0       # generations until it is tried again
+        self._one_launch_given_up = 0    # in all
         # nn.Linear calls with at most this many activation rows (the decode step) go through the
         # library's weight-streaming kernels when the operator module has them; 0 = always F.linear
         self.decode_linear_rows = 16 if hasattr(ops, "linear_decode") else 0
@@ -266,8 +267,21 @@ class LlamaDecoder:
         self._graphs.clear()   # recorded decode steps contain it
         self._one_launch_rests = 1 + min(2 ** self._one_launch_failures, self.ONE_LAUNCH_MAX_REST)
         self._one_launch_failures += 1
+        self._one_launch_given_up += 1
         warnings.warn("a one-launch decode step waited in vain for the rest of the device; this generation is repeated, and the next "
                       f"{self._one_launch_rests - 1} made, with the operators one by one", RuntimeWarning, stacklevel=3)
+
+    def decode_route(self, rows: int, total_len: int) -> str:
+        """What a decode step of these rows runs, for reports: as things stand now, and how often the one launch was given up."""
+        if self._one_launch(rows, total_len) is not None:
+            route = "l3_decode_layers (all layers in one launch), l3_linear_decode_fused for lm_head"
+        elif 0 < rows <= self._fused_rows():
+            route = "l3_linear_decode_fused throughout"
+        elif self._splitk(rows):
+            route = "l3_linear_qkv_rope_append_rows, l3_linear_splitk for c_proj / mlp c_proj, linear_swiglu_decode and linear_decode for gate|up and lm_head"
+        else:
+            route = "linear_decode" if 0 < rows <= self.decode_linear_rows else "torch F.linear"
+        return route + (f"; one launch given up {self._one_launch_given_up} times" if self._one_launch_given_up else "")
 
     def _one_launch_done(self, layers):
         """At the end of a generation whose decode steps were `layers` (None: the operators)."""
@@ -534,7 +548,7 @@ class GraphedDecodeLoop:
 
     def prefill(self, m: "LlamaDecoder", T: int):
         """Logits of the prompt's first T positions (model.py:365 with start_pos 0) for the tokens in
-        self.tokens.  The eager pass costs ~260 launches from Python (3.3 ms at batch 1, against 0.64 ms
+        self.tokens.  The eager pass costs ~260 launches from Python (3.3 ms at batch 1, against 0.48 ms
         for a decode step), so it is recorded too, once per prompt length.  A recorded pass is used only
         after it has reproduced the eager logits bit for bit on two replays with eager work in between
         (library GEMMs may record nodes that misbehave on later replays); otherwise the eager pass stays."""
@@ -703,11 +717,8 @@ def bench_e2e(args, torch_mod, dev, cpu_ops=None):
         best = max(timed_generate(model, batch, input_len, gen_len, sync=torch_mod.cuda.synchronize, graphed=True)[0]
                    for _ in range(3))
         rec["graphed_torch_linear"] = {"tok_per_s": round(best, 1)}
-        # ... then the library's weight-streaming linear kernels where they apply (up to 16 rows)
+        # ... then the library's decode step (decode_route says afterwards which)
         model.set_decode_linear_rows(16)
-        rec["decode_linear"] = ("l3_linear_decode (fused)" if 0 < batch <= model.decode_linear_rows else
-                                "l3_linear_splitk for c_attn / c_proj / mlp c_proj, l3_linear_wide for gate|up and lm_head"
-                                if model._splitk(batch) else "torch F.linear")
         for mode in ("eager", "graphed"):
             graphed = mode == "graphed"
             # warm-up generate, as llama3_inference.py:31-36 does (for the graphed loop it also records the graph)
@@ -722,6 +733,7 @@ def bench_e2e(args, torch_mod, dev, cpu_ops=None):
             rec[mode + "_tokens"] = toks
         same = sum(a == b for ra, rb in zip(rec.pop("eager_tokens"), rec.pop("graphed_tokens")) for a, b in zip(ra, rb))
         rec["graphed_vs_eager_same_tokens"] = f"{same}/{batch * gen_len}"
+        rec["decode_linear"] = model.decode_route(batch, input_len + gen_len)
         rec["prefill"] = model.prefill_backend
         rec["prefill_pass"] = model.prefill_pass_mode()
         results[batch] = rec

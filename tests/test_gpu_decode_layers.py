@@ -307,5 +307,7 @@ def test_the_one_launch_comes_back_after_a_wait_ran_out(gpu):
             assert m._one_launch(2, 32) is not None
         assert generate(prompts, 16, ignore_eos=True) == first and 2 in m._layer_launches
         assert m._one_launch_failures == 0
+    assert "l3_decode_layers" in m.decode_route(2, 32) and "given up 6 times" in m.decode_route(2, 32)
+    assert "l3_decode_layers" not in m.decode_route(2, 2049)
     key, loop = next(iter(m._graphs.items()))
     assert key == (2, 32) and loop.layers is m._layer_launches[2]
