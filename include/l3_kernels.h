@@ -318,9 +318,10 @@ int l3_linear_swiglu_decode(const void* x, const void* w_gate, const void* w_up,
  *   t = w_up ? bf16(silu(bf16(h.w^T))) * bf16(h.w_up^T) : h.w^T                   (model.py:134)
  *   y = residual ? bf16(residual + bf16(t)) : bf16(t)                             (model.py:147-148)
  * with the rounding points of the separate operators.  residual has y's shape and row stride and
- * may be y itself.  The input norm stages x in LDS and needs K % 512 == 0 and M * (K + 8) <= 24576
+ * may be y itself.  The input norm stages x in LDS and needs K % 512 == 0 and M * (K + 8) <= L3_LINEAR_NORM_STAGE_ELEMENTS
  * (L3_ERR_SHAPE otherwise); everything else as for l3_linear_decode.
  */
+#define L3_LINEAR_NORM_STAGE_ELEMENTS 24576
 int l3_linear_decode_fused(const void* x, const void* norm_weight, float norm_eps, const void* w, const void* w_up,
                            const void* residual, void* y, int M, int N, int K, int64_t x_stride, int64_t w_stride,
                            int64_t y_stride, void* stream);

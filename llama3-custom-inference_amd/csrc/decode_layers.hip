@@ -27,7 +27,7 @@
 // Every wait is bounded.  A wavefront whose wait runs out (the launch shares the device with something that keeps
 // part of it from becoming resident, or workgroups are not placed on XCDs in turn) raises the error word of the
 // control block and goes on without waiting, so that the launch always ends; the caller looks at the word when it
-// reads results, discards them and takes the launches per operator from then on.
+// reads results, discards them and does the work again with the launches per operator.
 //
 // Rounding points are those of the separate operators.
 #include "attn_merge.hpp"

@@ -46,7 +46,7 @@ __device__ __forceinline__ void store_qkv_pair(const LinearParams& p, int m, int
 }
 
 // Elements of LDS the staged activations may take (rows are padded by 8 elements).
-constexpr int kXldsMaxElems = 24576;
+constexpr int kXldsMaxElems = L3_LINEAR_NORM_STAGE_ELEMENTS;
 
 // RW = weight rows per wavefront.  16: the plain mapping above.  4 (at most 4 activation rows):
 // the 16 rows and the 16 columns of a matrix instruction are both split into four k

@@ -16,8 +16,8 @@
 //   * Rows are not padded in LDS: the 16-byte chunk c of row r sits at position c ^ (r & 15), which spreads the
 //     rows of an operand read over all banks.
 // Measured against what ran before (a library GEMM plus the SwiGLU product: 21.2 us): gate|up 14.4 us; down
-// projection 2048 x 8192 in 8 splits 11.8 -> 9.5 us; out projection 2048 x 2048 5.5 -> 5.2 us; qkv 3072 x 2048
-// 7.0 -> 6.5 us; vocabulary projection 128256 x 2048 107 (library GEMM) -> 95 us.
+// projection 2048 x 8192 in 8 splits 11.8 -> 9.9 us; out projection 2048 x 2048 5.5 -> 5.0 us; qkv 3072 x 2048
+// 7.0 -> 6.6 us; vocabulary projection 128256 x 2048 107 (library GEMM) -> 95 us.
 #include <algorithm>
 
 #include "lds_loads.hpp"
@@ -92,7 +92,7 @@ linear_wide_kernel(const WideParams p) {
     const int split = OUT == WideOut::kQkv ? 0 : part, m0 = OUT == WideOut::kQkv ? part * (CB * 16) : 0;
     const int n0 = group * N_WG;
     const int c0 = split * p.chunks_per_split;
-    const int n_chunks = min(p.K / kWideChunk, c0 + p.chunks_per_split) - c0;   // at least 1
+    const int n_chunks = min(p.K / kWideChunk, c0 + p.chunks_per_split) - c0;   // (none: the split's products are zeros)
 
     // loads: lane l of a load covers row l / 16 of its four rows, chunk position l % 16
     const uint32_t ring = lds_address(s_ring);
@@ -355,7 +355,7 @@ int chunks_of(int K) { return K / kWideChunk; }
 // Splits of K of the partial-product form (which imply the weight rows per workgroup, launch_linear_splitk).  One workgroup per compute unit at most:
 // with deep rings only one fits a unit, and a second round of a few workgroups costs as much as the first (4096 x
 // 14336: 14 splits, 896 workgroups 33 us; 4 splits, 256 workgroups 24 us).  64 rows share an activation tile
-// better (2048 x 8192: 9.5 us against 11.3 with 32); with a short K half the splits are worth more, to
+// better (2048 x 8192: 9.9 us against 11.3 with 32); with a short K half the splits are worth more, to
 // the operator that adds them up as well (2048 x 2048: 32 rows in 4 splits 5.0 us, 64 rows in 8 splits 5.6 us).
 int rows_plan(int N, int K, int num_cus) {
     const int rows = chunks_of(K) <= 16 ? 32 : 64;

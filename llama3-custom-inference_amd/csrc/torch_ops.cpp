@@ -520,9 +520,6 @@ Tensor rows_out(const Tensor& x, int64_t N) {
 // Which kernels a linear takes.  kSkinny streams weights past operands held in registers: up to 16 rows, anything
 // folded in, one launch.  kWide and kSplit share the activations through LDS (K % 128 == 0, N % 8 == 0): one launch
 // where the rows of the matrix fill the device, partial products plus a finishing pass where they do not.
-// Activations (rows padded by 8 elements) that the skinny kernel's input norm stages in LDS.
-constexpr int64_t kNormStageElements = 24576;
-
 enum class Route { kSkinny, kWide, kSplit };
 
 // From here on the rows of a matrix alone fill the device (64 to a workgroup; 32 of each of the SwiGLU pair).
@@ -609,7 +606,7 @@ Tensor wide(const Tensor& x, const Tensor& w, const Tensor* up, const Tensor* re
 void check_norm_weight(const Tensor& norm, int64_t rows, int64_t K, const char* what) {
     TORCH_CHECK(norm.dim() == 1 && norm.numel() == K && norm.is_contiguous(), what, ": norm_weight ", norm.sizes(),
                 " does not fit K=", K);
-    const int64_t most = K % 512 == 0 ? std::min<int64_t>(16, kNormStageElements / (K + 8)) : 0;
+    const int64_t most = K % 512 == 0 ? std::min<int64_t>(16, L3_LINEAR_NORM_STAGE_ELEMENTS / (K + 8)) : 0;
     TORCH_CHECK(rows <= most, what, ": the input norm takes at most ", most, " rows of width ", K, ", got ", rows);
 }
 

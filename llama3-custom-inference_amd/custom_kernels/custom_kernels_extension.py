@@ -332,9 +332,9 @@ def silu_mul(a, b):
 def linear_decode(x, weight):
     """F.linear(x, weight) for at most 64 activation rows (model.py:95,121,134,225 when T == 1):
     one pass over the weight matrix at HBM speed instead of a GEMM.  x (..., K), weight (N, K)
-    -> (..., N).  Up to 16 rows are one launch whatever the matrix; 17..64 rows (N % 8 == 0,
-    K % 128 == 0) are one launch where the rows of the matrix fill the device (a vocabulary
-    projection), else linear_splitk and linear_splitk_finish.  An extension."""
+    -> (..., N).  17..64 rows need N % 8 == 0 and K % 128 == 0.  One launch up to 16 rows and, whatever the rows, where those of
+    the matrix fill the device (a vocabulary projection); otherwise linear_splitk and linear_splitk_finish, two launches, from 17
+    rows on and for large matrices before (16 M elements from 5 rows on, 32 M from one).  An extension."""
     return _l3lib.native().linear_decode(x, weight)
 
 
@@ -351,8 +351,8 @@ def linear_decode_fused_max_rows(K: int) -> int:
 
 
 def linear_decode_fused(x, weight, norm_weight=None, eps: float = 1e-5, w_up=None, residual=None):
-    """linear_decode with the operators around it folded into the one launch, each optional:
-    rms_norm(x, norm_weight, eps) in front (model.py:70-72), the SwiGLU product with a second
+    """linear_decode with the operators around it folded in, each optional (in the same launches; a norm in front of what is not
+    the one-launch form for up to 16 rows is one of its own): rms_norm(x, norm_weight, eps) in front (model.py:70-72), the SwiGLU product with a second
     matrix w_up (weight is then the gate, model.py:134), and `residual + result` behind
     (model.py:147-148) -- all with the rounding points of the separate operators.  An extension."""
     return _l3lib.native().linear_decode_fused(x, weight, norm_weight, eps, w_up, residual)

@@ -430,3 +430,10 @@ def test_read_stream_argument_checks():
     assert lib.l3_hbm_read_stream(FAKE, 0, FAKE, 0, None) == _l3lib.L3_ERR_SHAPE
     assert lib.l3_hbm_read_stream(FAKE, 1000, FAKE, 0, None) == _l3lib.L3_ERR_SHAPE
     assert lib.l3_hbm_read_stream(FAKE + 8, 1 << 20, FAKE, 0, None) == _l3lib.L3_ERR_ALIGNMENT
+
+
+def test_linear_limits_match_header():
+    text = open(HEADER).read()
+    for define, value in (("L3_LINEAR_SPLITK_MAX_ROWS", _l3lib.L3_LINEAR_SPLITK_MAX_ROWS),
+                          ("L3_LINEAR_NORM_STAGE_ELEMENTS", _l3lib.L3_LINEAR_STAGE_ELEMS)):
+        assert int(re.search(rf"#define {define} (\d+)", text).group(1)) == value

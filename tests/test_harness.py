@@ -300,8 +300,8 @@ def test_full_size_logits_match_cpu_model_on_the_split_k_route(gpu, full_size_mo
 @pytest.mark.gpu
 @pytest.mark.parametrize("batch", [1, 64])
 def test_full_size_graphed_loop_matches_eager(gpu, full_size_model, batch):
-    """128 prompt ids + 128 greedy tokens at batch 1 (fused single-launch linears) and batch 64
-    (library GEMMs, strided gate|up halves): the HIP-graph replay against the eager loop.  The two
+    """128 prompt ids + 128 greedy tokens at batch 1 (all layers of a step in one launch, in both loops) and batch 64
+    (split-K and wide linears): the HIP-graph replay against the eager loop.  At batch 64 the two
     loops plan the attention splits differently (device-side against host-side KV length), so a
     near-tie may fork a stream: a long common prefix and broad agreement are required, not identity."""
     m = full_size_model
