@@ -424,7 +424,8 @@ int l3_rot_embed_append_partials(const void* part, int ksplit, const float* freq
  * one, L3_ERR_SHAPE elsewhere); every workgroup attends for itself, so meant for caches of a few hundred tokens.
  * workspace: l3_decode_layers_workspace_bytes bytes, 256-byte aligned, zeroed once before the first launch and handed
  * to one launch at a time.  The workgroups of a launch wait for each other; all waits are bounded.  If one runs out
- * -- the device did not hold the whole launch at once, because something else occupied part of it -- the first
+ * -- the device did not hold the whole launch at once, because something else occupied part of it, or did not
+ * place its workgroups on the XCDs in turn (handed-over words name the XCD that wrote them) -- the first
  * word of the workspace is non-zero afterwards: results are void then, as are those of later launches with this workspace.
  */
 int l3_decode_layers_supported(int M, int C, int H, int QH, int KVH, int HD);
