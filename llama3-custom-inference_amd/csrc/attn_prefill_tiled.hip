@@ -16,6 +16,7 @@
 // issued before the arithmetic on tile i and land in the other LDS buffer after it.
 //
 // Query i of T sits at absolute position S - T + i and attends to tokens 0 .. S - T + i.
+#include <algorithm>
 #include <type_traits>
 
 #include "attn_mfma_core.hpp"
@@ -23,6 +24,8 @@
 namespace l3 {
 
 namespace {
+
+constexpr int kDeviceScope = 16;   // buffer accesses that go to where all XCDs see them (sc1)
 
 // Maximum that hands a NaN on (v_maximum3_f32): unlike fmaxf it needs no quieting of its inputs, which
 // costs an instruction per value that comes out of a matrix instruction or a lane swap.
@@ -44,9 +47,10 @@ __device__ __forceinline__ float column_maximum(float x) {
 // not padded; instead the 16-byte chunk c of token row r sits at chunk position c ^ key(r), which
 // spreads the rows that an operand read touches together over all banks.  The two stages are separate
 // arrays, so that the compiler can tell a read of one from the load in flight into the other.
-template <int HD, int CB, int NW, int TK, int WPE, bool NOMAX>
+template <int HD, int CB, int NW, int TK, int WPE, bool NOMAX, bool SPLIT = false>
 __global__ void __launch_bounds__(NW * kWaveSize) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
-attn_prefill_tiled_kernel(const PrefillParams p) {
+attn_prefill_tiled_kernel(const PrefillParams p, const std::conditional_t<SPLIT, PrefillItems, NoItems> items) {
+    static_assert(!(SPLIT && NOMAX), "the loop without a maximum takes its reference from the first tile of the row");
     constexpr int NG = TK / 16, KS = TK / 32, KC = HD / 32, NB = HD / 16;
     constexpr int CPR = HD / 8;                  // 16-byte chunks per token row
     constexpr int ROWB = HD * 2;                 // bytes per token row
@@ -80,14 +84,28 @@ attn_prefill_tiled_kernel(const PrefillParams p) {
         const int k = rank / p.snake, j = rank % p.snake;
         if ((k & 1) && (k + 1) * p.snake <= int(gridDim.x)) rank = k * p.snake + (p.snake - 1 - j);
     }
-    const int wg = wgs_per_head - 1 - rank / heads;
+    int wg = wgs_per_head - 1 - rank / heads;
     const int bh = rank % heads;
+    int piece = 0, pieces = 1, first_slot = 0;
+    if constexpr (SPLIT) {
+        const uint32_t item = items.item[rank / heads];
+        wg = int(item & 0x1ff);
+        first_slot = int(item >> 9) & 0x1ff;
+        piece = int(item >> 18) & 0x7f;
+        pieces = int(item >> 25);
+    }
     const int kvh = bh % p.KVH;
     const int b = bh / p.KVH;
 
     const int wg_first_qi = wg * wg_pos;
     const int wg_last_qi = min(p.T, wg_first_qi + wg_pos) - 1;
-    const int wg_t_end = p.S - p.T + wg_last_qi + 1;     // tokens any column of the workgroup may see
+    int wg_t_end = p.S - p.T + wg_last_qi + 1;           // tokens any column of the workgroup may see
+    int wg_t_begin = 0;
+    if constexpr (SPLIT) {   // this piece's whole tiles of them
+        const int tiles = (wg_t_end + TK - 1) / TK;
+        wg_t_begin = tiles * piece / pieces * TK;
+        wg_t_end = min(wg_t_end, tiles * (piece + 1) / pieces * TK);
+    }
     const int wave_first_qi = wg_first_qi + wave * CB * ppw;
     const int wave_last_qi = min(p.T, wave_first_qi + CB * ppw) - 1;
     // tiles at or beyond this are skipped (all of them for a wavefront past the last query)
@@ -167,12 +185,15 @@ attn_prefill_tiled_kernel(const PrefillParams p) {
     // over all four k groups) next to O.  The vector pipe, which bounds this kernel at head size 64, is
     // spared one addition per score; P enters both sums rounded to bf16, so the weights of a column add
     // up to one exactly.
+    // (a piece may begin with a tile that a column sees nothing of: its reference lies above the masked scores, so that
+    // their weights are zeros and not whatever the rounding of a difference of such numbers leaves)
+    constexpr float kNoScore = SPLIT ? 0.99f * kMaskedScore : kMaskedScore;
     f32x4_t O[CB][NB], L[CB];
     float Lsum[CB];    // the hand-laid tile keeps the denominator as one number per column (it looks at a tile's sum first)
     float m_run[CB];
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) {
-        m_run[cb] = kMaskedScore;
+        m_run[cb] = kNoScore;
         Lsum[cb] = 0.f;
         L[cb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -608,9 +629,9 @@ attn_prefill_tiled_kernel(const PrefillParams p) {
         return t0;   // the first tile this loop has not been offered
     };
     if constexpr (PF) {
-        tiles_from(std::false_type{}, 0);
+        tiles_from(std::false_type{}, wg_t_begin);
     } else if constexpr (!NOMAX) {
-        tiles_from(std::true_type{}, 0);
+        tiles_from(std::true_type{}, wg_t_begin);
 #pragma unroll
         for (int cb = 0; cb < CB; ++cb) Lsum[cb] = L[cb][0];
     } else {
@@ -633,6 +654,99 @@ attn_prefill_tiled_kernel(const PrefillParams p) {
         }
     }
 
+    if constexpr (SPLIT) {
+        if (pieces > 1) {   // workgroup-uniform
+            // A piece leaves its accumulators as they lie in the registers, so that every access is whole lines and the
+            // merging thread finds its own columns.  The pieces of a block may run on different XCDs: stores write
+            // through and loads do not stop at the caches (device scope), and the count of arrivals is the device's.
+            constexpr int VECS = CB * NB;
+            constexpr int NT = NW * kWaveSize;
+            constexpr int kSlotBytes = (VECS * 16 + CB * 8) * NT;
+            char* const block = items.part + (int64_t(bh) * items.slots_per_head + first_slot) * kSlotBytes;
+            __shared__ int s_last;
+            {
+                const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(block + int64_t(piece) * kSlotBytes, 0, kSlotBytes, 0x00020000);
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb) {
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb) {
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, O[cb][nb]), to, tid * 16, (cb * NB + nb) * NT * 16, kDeviceScope);
+                    }
+                    const u32x2_t ml = {__builtin_bit_cast(uint32_t, m_run[cb]), __builtin_bit_cast(uint32_t, Lsum[cb])};
+                    __builtin_amdgcn_raw_buffer_store_b64(ml, to, tid * 8, VECS * NT * 16 + cb * NT * 8, kDeviceScope);
+                }
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's part is where every XCD reads it
+            __syncthreads();
+            unsigned* const counter = items.counters + (int64_t(bh) * items.slots_per_head + first_slot) / 2 * kPrefillCounterStride;
+            if (tid == 0) {
+                const unsigned before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                s_last = before == unsigned(pieces - 1);
+                // (nobody else arrives before the next launch, which finds zero again)
+                if (s_last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            __syncthreads();
+            if (!s_last) return;
+            // The pieces in their order, whichever arrived last, so that a result does not depend on who merges it; the
+            // next piece is on its way while one is added.
+            f32x4_t sum[CB][NB];
+            float total[CB], M[CB];
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) {
+                M[cb] = kNoScore;
+                total[cb] = 0.f;
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) sum[cb][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            }
+            u32x4_t part[2][CB][NB];
+            u32x2_t ml[2][CB];
+            auto request = [&](int i, u32x4_t (&o)[CB][NB], u32x2_t (&st)[CB]) __attribute__((always_inline)) {
+                const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc(block + int64_t(min(i, pieces - 1)) * kSlotBytes, 0, kSlotBytes, 0x00020000);
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb) {
+                    st[cb] = __builtin_amdgcn_raw_buffer_load_b64(from, tid * 8, VECS * NT * 16 + cb * NT * 8, kDeviceScope);
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb) {
+                        o[cb][nb] = __builtin_amdgcn_raw_buffer_load_b128(from, tid * 16, (cb * NB + nb) * NT * 16, kDeviceScope);
+                    }
+                }
+            };
+            auto add = [&](const u32x4_t (&o)[CB][NB], const u32x2_t (&st)[CB]) __attribute__((always_inline)) {
+#pragma unroll
+                for (int cb = 0; cb < CB; ++cb) {
+                    const float m = __builtin_bit_cast(float, uint32_t(st[cb][0]));
+                    const float m_new = maximum(M[cb], m);
+                    const float f_old = fast_exp2((M[cb] - m_new) * c), f = fast_exp2((m - m_new) * c);
+                    M[cb] = m_new;
+                    total[cb] = fmaf(__builtin_bit_cast(float, uint32_t(st[cb][1])), f, total[cb] * f_old);
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb) {
+                        const f32x4_t v = __builtin_bit_cast(f32x4_t, o[cb][nb]);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) sum[cb][nb][j] = fmaf(v[j], f, sum[cb][nb][j] * f_old);
+                    }
+                }
+            };
+            request(0, part[0], ml[0]);
+            for (int i = 0; i < pieces; i += 2) {
+                request(i + 1, part[1], ml[1]);
+                asm volatile("" ::: "memory");   // (the compiler would move the loads to where they are used)
+                add(part[0], ml[0]);
+                if (i + 1 < pieces) {
+                    request(i + 2, part[0], ml[0]);
+                    asm volatile("" ::: "memory");
+                    add(part[1], ml[1]);
+                }
+            }
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) {
+                Lsum[cb] = total[cb];
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) O[cb][nb] = sum[cb][nb];
+            }
+        }
+    }
+
 #pragma unroll
     for (int cb = 0; cb < CB; ++cb) {
         if (col_limit[cb] > 0) {
@@ -651,6 +765,20 @@ attn_prefill_tiled_kernel(const PrefillParams p) {
     }
 }
 
+// Pieces of a split launch: a table of (block, piece, pieces, first slot), longest blocks first.
+template <int HD, int CB, int NW, int TK, int WPE>
+int launch_pieces(const PrefillParams& p, const PrefillSplitPlan& plan, void* part, unsigned* counters, hipStream_t stream) {
+    static_assert(prefill_slot_bytes(HD, CB) == (CB * HD + CB * 8) * NW * kWaveSize, "slots");
+    PrefillItems items;
+    items.part = static_cast<char*>(part);
+    items.counters = counters;
+    const int n = prefill_items(plan, p.QH / p.KVH, p.T, p.S, &items);
+    const dim3 grid(unsigned(p.B) * unsigned(p.KVH) * unsigned(n));
+    PrefillParams q = p;
+    q.snake = 0;
+    return enqueue(attn_prefill_tiled_kernel<HD, CB, NW, TK, WPE, false, true>, grid, dim3(NW * kWaveSize), 0, stream, q, items);
+}
+
 template <class Kernel>
 int launch_blocks(Kernel kernel, const PrefillParams& p, int waves, int col_blocks, hipStream_t stream) {
     const int R = p.QH / p.KVH;
@@ -660,10 +788,85 @@ int launch_blocks(Kernel kernel, const PrefillParams& p, int waves, int col_bloc
     PrefillParams q = p;
     const int cus = current_device_cus();
     q.snake = (int64_t(grid.x) <= 4 * int64_t(cus)) ? cus : 0;
-    return enqueue(kernel, grid, dim3(waves * kWaveSize), 0, stream, q);
+    return enqueue(kernel, grid, dim3(waves * kWaveSize), 0, stream, q, NoItems{});
 }
 
 }  // namespace
+
+int prefill_items(const PrefillSplitPlan& plan, int R, int T, int S, PrefillItems* items) {
+    const int pos = kPrefillTiledWaves * plan.col_blocks * (16 / R);
+    int n = 0, slots = 0;
+    for (int wg = (T + pos - 1) / pos - 1; wg >= 0; --wg) {
+        const int t_end = S - T + std::min(T, (wg + 1) * pos);
+        const int tiles = (t_end + kPrefillSplitTile - 1) / kPrefillSplitTile;
+        const int pieces = (tiles + plan.max_tiles - 1) / plan.max_tiles;
+        if (n + pieces > kPrefillMaxItems || pieces > kPrefillMaxPieces) return -1;
+        if (items) {
+            for (int i = 0; i < pieces; ++i) {
+                items->item[n + i] = uint32_t(wg) | uint32_t(slots) << 9 | uint32_t(i) << 18 | uint32_t(pieces) << 25;
+            }
+        }
+        n += pieces;
+        if (pieces > 1) slots += pieces;
+    }
+    if (items) items->slots_per_head = slots;
+    return n;
+}
+
+// Which calls are cut.  A short piece of a prompt behind many cached tokens has few blocks, each with a long range: 64
+// queries behind 4032 tokens are 32 workgroups of 64 tiles.  Cut into pieces of n per block they fill the device; what
+// that costs is the partial results (18 to 66 KB each, written and read past the caches) and the merge, a chain of n reads.
+// Measured (us, uncut / cut; 32 query heads over 8, one sequence): 8 queries of 4096 tokens 54.9 / 10.3, 64 of 4096
+// 37.9 / 11.5, 512 of 7012 64.1 / 43.1, head size 128 105.8 / 66.4.  The lines, from a sweep over B 1 ... 16, R 3, 4, 8:
+//   * n: at most two pieces per compute unit (a 513th starts when a first has ended: 23.6 -> 29 us for 200 of 3200 at head
+//     size 128), pieces of at least 3/4 sqrt(tiles) tiles (8 of 3008: 4 tiles 9.4, 8 tiles 10.5, 1 tile 12 us);
+//   * one column block per wavefront while its blocks do not fill the device (64 of 4096: 11.5 against 14 us), two beyond
+//     and for the longest ranges (512 of 7012 at head size 128: 66 against 80 us);
+//   * below 12 tiles, or where the blocks alone occupy the device, the merge costs what the balance gives (64 of 314: 6.6
+//     uncut, 7.0; 512 x 16 sequences of 572: 37.5, 40.7); the same holds for prompts without a past, whose longest blocks end a
+//     launch that has kept the device busy (2 x 1531: 29.5 uncut, 29.0 ... 36 by the cut; 2048: 27.2, 30.0).
+PrefillSplitPlan prefill_split_plan(int B, int QH, int KVH, int T, int S, int HD, int num_cus) {
+    const PrefillSplitPlan none{0, 0, 0};
+    const int R = QH / KVH;
+    const int tiles = (S + kPrefillSplitTile - 1) / kPrefillSplitTile;
+    if (S / 2 < T || tiles < 12) return none;
+    auto blocks = [&](int col_blocks) { const int pos = kPrefillTiledWaves * col_blocks * (16 / R); return (T + pos - 1) / pos; };
+    const int64_t heads = int64_t(B) * KVH, one = heads * blocks(1), two = heads * blocks(2), cus = num_cus;
+    PrefillSplitPlan plan = none;
+    int64_t room = 2 * cus;
+    if (10 * one <= 9 * cus || (one <= cus && tiles >= 24)) {
+        plan.col_blocks = (tiles >= 64 && 2 * one > cus) ? 2 : 1;
+    } else if (two <= cus && tiles >= 40) {
+        plan.col_blocks = 2;
+    } else if (5 * two <= 8 * cus && tiles >= (HD == 128 ? 64 : 100)) {
+        plan.col_blocks = 2;   // (1500 of 8000: at head size 128 258 / 193 us, at 64 123 / 110: units with one block and with two)
+        room = 5 * cus;
+    } else {
+        return none;
+    }
+    int least = 3;
+    while (16 * least * least < 9 * tiles) ++least;
+    const int per_head = blocks(plan.col_blocks);
+    const int64_t n = std::min({room / (heads * per_head), int64_t((tiles + least - 1) / least), int64_t(kPrefillMaxItems / per_head),
+                                int64_t(kPrefillMaxPieces)});
+    if (n < 2) return none;
+    plan.max_tiles = int((tiles + n - 1) / n);
+    PrefillItems items;
+    if (prefill_items(plan, R, T, S, &items) < 0 || items.slots_per_head == 0) return none;
+    plan.slots = heads * items.slots_per_head;
+    return plan.slots <= kPrefillMaxSlots ? plan : none;
+}
+
+int launch_attn_prefill_split(const PrefillParams& p, int HD, const PrefillSplitPlan& plan, void* part, unsigned* counters,
+                              hipStream_t stream) {
+    constexpr int NW = kPrefillTiledWaves;
+    if (HD == 64) {
+        if (plan.col_blocks == 1) return launch_pieces<64, 1, NW, 64, 4>(p, plan, part, counters, stream);
+        return launch_pieces<64, 2, NW, 64, 4>(p, plan, part, counters, stream);
+    }
+    if (plan.col_blocks == 1) return launch_pieces<128, 1, NW, 64, 2>(p, plan, part, counters, stream);
+    return launch_pieces<128, 2, NW, 64, 2>(p, plan, part, counters, stream);
+}
 
 int launch_attn_prefill_tiled(const PrefillParams& p, int HD, hipStream_t stream) {
     constexpr int CB = kPrefillColBlocks, NW = kPrefillTiledWaves;

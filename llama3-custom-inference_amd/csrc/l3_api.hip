@@ -30,6 +30,12 @@ int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 size_t round_up(size_t n, size_t a) { return (n + a - 1) / a * a; }
 
+// How a prefill call is cut into pieces; a forced form is not.
+PrefillSplitPlan prefill_plan_of(int B, int QH, int KVH, int T, int S, int HD, int flags) {
+    if (flags & L3_ATTN_FLAG_PREFILL_MASK) return PrefillSplitPlan{0, 0, 0};
+    return prefill_split_plan(B, QH, KVH, T, S, HD, current_device_cus());
+}
+
 int check_attn_shape(int B, int QH, int KVH, int S, int HD) {
     if (HD != 64 && HD != 128) return L3_ERR_HEAD_SIZE;
     if (B <= 0 || QH <= 0 || KVH <= 0 || S <= 0) return L3_ERR_SHAPE;
@@ -516,9 +522,23 @@ int l3_attn_decode_devlen(const void* q, const void* k, const void* v, void* out
                             v_strides, out_strides, scale, num_splits, flags, kv_len_dev, stream);
 }
 
+size_t l3_attn_prefill_workspace_bytes(int B, int QH, int KVH, int T, int S, int HD, int flags) {
+    if (check_attn_shape(B, QH, KVH, S, HD) != L3_OK || !attn_flags_ok(flags) || T <= 0 || T > S) return 0;
+    const PrefillSplitPlan plan = prefill_plan_of(B, QH, KVH, T, S, HD, flags);
+    return plan.max_tiles > 0 ? L3_ATTN_COUNTER_BYTES + size_t(plan.slots) * prefill_slot_bytes(HD, plan.col_blocks) : 0;
+}
+
 int l3_attn_prefill(const void* q, const void* k, const void* v, void* out, int B, int QH, int KVH, int T, int S,
                     int HD, const int64_t q_strides[3], const int64_t k_strides[3], const int64_t v_strides[3],
                     const int64_t out_strides[3], float scale, int flags, void* stream) {
+    return l3_attn_prefill_ws(q, k, v, out, nullptr, 0, nullptr, B, QH, KVH, T, S, HD, q_strides, k_strides, v_strides,
+                              out_strides, scale, flags, stream);
+}
+
+int l3_attn_prefill_ws(const void* q, const void* k, const void* v, void* out, void* workspace, size_t workspace_bytes,
+                       void* counters, int B, int QH, int KVH, int T, int S, int HD, const int64_t q_strides[3],
+                       const int64_t k_strides[3], const int64_t v_strides[3], const int64_t out_strides[3], float scale,
+                       int flags, void* stream) {
     if (!q || !k || !v || !out || !q_strides || !k_strides || !v_strides || !out_strides)
         return L3_ERR_NULL_POINTER;
     if (int rc = check_attn_shape(B, QH, KVH, S, HD); rc != L3_OK) return rc;
@@ -550,6 +570,22 @@ int l3_attn_prefill(const void* q, const void* k, const void* v, void* out, int 
     p.snake = 0;
     p.no_max_tiles = (flags & L3_ATTN_FLAG_PREFILL_MASK) == L3_ATTN_FLAG_PREFILL_TILED_NO_MAX;
     p.auto_form = (flags & L3_ATTN_FLAG_PREFILL_MASK) == 0;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (workspace) {
+        const PrefillSplitPlan plan = prefill_plan_of(B, QH, KVH, T, S, HD, flags);
+        if (plan.max_tiles > 0) {
+            if (workspace_bytes < L3_ATTN_COUNTER_BYTES + size_t(plan.slots) * prefill_slot_bytes(HD, plan.col_blocks))
+                return L3_ERR_WORKSPACE;
+            if (!aligned(workspace, kWorkspaceAlign) || !aligned(counters, kWorkspaceAlign)) return L3_ERR_ALIGNMENT;
+            unsigned* arrivals = static_cast<unsigned*>(counters);
+            if (!arrivals) {
+                arrivals = static_cast<unsigned*>(workspace);
+                if (launch_fill_zero_u32(arrivals, L3_ATTN_COUNTER_BYTES / sizeof(unsigned), st) != 0) return L3_ERR_HIP;
+            }
+            const int rc = launch_attn_prefill_split(p, HD, plan, static_cast<char*>(workspace) + L3_ATTN_COUNTER_BYTES, arrivals, st);
+            return rc == 0 ? L3_OK : L3_ERR_HIP;
+        }
+    }
     // Which form (graph-timed sweeps over B 1 ... 256, T 8 ... 8192, head ratios 1, 3, 4 and 8): a prompt
     // that does not exceed one workgroup of the tiled form's small variant (one column block per wavefront) per
     // kv head, with few enough wavefronts for the device to hold them all at once, runs as independent
@@ -562,7 +598,6 @@ int l3_attn_prefill(const void* q, const void* k, const void* v, void* out, int 
         const bool tiny = T <= prefill_tiled_positions_per_wg(R) / 2 && private_waves <= 4 * int64_t(current_device_cus());
         form = tiny ? L3_ATTN_FLAG_PREFILL_WAVE : L3_ATTN_FLAG_PREFILL_TILED;
     }
-    hipStream_t st = static_cast<hipStream_t>(stream);
     const int rc = (form == L3_ATTN_FLAG_PREFILL_WAVE) ? launch_attn_prefill(p, HD, st) : launch_attn_prefill_tiled(p, HD, st);
     return rc == 0 ? L3_OK : L3_ERR_HIP;
 }

@@ -107,6 +107,31 @@ struct PrefillParams {
     int auto_form;      // the form was the library's choice (it may then run one column block per wavefront)
 };
 
+// Prefill blocks (a workgroup's query positions against all their tokens) cut into pieces of whole tiles.
+constexpr int kPrefillMaxItems = 512;        // pieces of a (batch, kv head); their table rides in the kernel arguments
+constexpr int kPrefillMaxPieces = 127;       // of a block
+constexpr int kPrefillSplitTile = 64;        // tokens per tile
+constexpr int kPrefillCounterStride = 8;     // words from one block's arrival counter to the next
+constexpr int64_t kPrefillMaxSlots = 2 * (L3_ATTN_COUNTER_BYTES / 4 / kPrefillCounterStride - 4);   // (two slots a counter at least; the last words are a diagnostic)
+struct PrefillSplitPlan {
+    int col_blocks;   // 16-column blocks per wavefront
+    int max_tiles;    // tiles of a piece at most; 0: the launch is not cut
+    int64_t slots;    // partial results of the whole launch
+};
+struct PrefillItems {
+    char* part;            // slots, each what a workgroup holds in registers
+    unsigned* counters;
+    int slots_per_head;
+    uint32_t item[kPrefillMaxItems];   // block (9 bits), its first slot (9), piece (7), pieces (7)
+};
+struct NoItems {};
+constexpr int prefill_slot_bytes(int HD, int col_blocks) { return col_blocks * (HD + 8) * 4 * 64; }
+// Fills in the table (if given) and its slots; the number of items, or -1 where the table is too small.
+int prefill_items(const PrefillSplitPlan& plan, int R, int T, int S, PrefillItems* items);
+PrefillSplitPlan prefill_split_plan(int B, int QH, int KVH, int T, int S, int HD, int num_cus);
+int launch_attn_prefill_split(const PrefillParams& p, int HD, const PrefillSplitPlan& plan, void* part, unsigned* counters,
+                              hipStream_t stream);
+
 struct LinearParams {
     const uint16_t* x;    // (M, K) activations, row stride x_stride
     const uint16_t* w0;   // (N, K) weights, row stride w_stride

@@ -1,0 +1,137 @@
+"""Causal prefill of a few queries behind many cached tokens: the launch is cut into pieces of rows x tokens, and the
+piece of a block that finishes last adds them up (l3_attn_prefill_ws)."""
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import assert_attn_close, randn_bf16, t2bits, t2f32
+
+
+def cut_bytes(B, QH, KVH, T, S, HD):
+    from custom_kernels import _l3lib
+
+    return _l3lib.load().l3_attn_prefill_workspace_bytes(B, QH, KVH, T, S, HD, 0)
+
+
+def make(B, QH, KVH, T, S, HD, gain=1.0, head_major=False):
+    q = randn_bf16((B, T, QH, HD), 301, scale=gain)
+    k, v = randn_bf16((B, S + 5, KVH, HD), 302), randn_bf16((B, S + 5, KVH, HD), 303)
+
+    def view(t, dev):
+        t = t.to(dev)[:, :S].transpose(1, 2)
+        return t.contiguous() if head_major else t
+
+    return lambda dev: (q.to(dev).transpose(1, 2), view(k, dev), view(v, dev))
+
+
+# 12 tiles are the fewest that are cut; lengths either side of a tile's edge; queries either side of a block's edge, for every
+# head ratio; blocks of one and of two column blocks; pieces that begin where some of a wavefront's columns see nothing
+SHAPES = [(1, 8, 1, 1, 705, 64), (1, 32, 8, 8, 768, 64), (2, 32, 8, 16, 1023, 64), (1, 24, 8, 21, 1025, 64), (1, 8, 8, 65, 1000, 64),
+          (1, 16, 8, 63, 2049, 64), (3, 16, 2, 40, 1500, 64), (1, 32, 8, 200, 1216, 64), (8, 32, 8, 64, 2600, 64),
+          (1, 4, 2, 3, 5000, 64)]
+
+
+def test_which_calls_are_cut():
+    for B, QH, KVH, T, S, HD in SHAPES:
+        assert cut_bytes(B, QH, KVH, T, S, HD) > 0
+        assert cut_bytes(B, QH, KVH, T, S, 128) > 0
+    for B, QH, KVH, T, S, HD in [(1, 32, 8, 8, 704, 64), (1, 32, 8, 512, 1000, 64), (2, 32, 8, 1531, 1531, 64), (64, 32, 8, 128, 128, 64),
+                                 (16, 32, 8, 512, 1100, 128), (1, 32, 8, 8, 4096, 96), (1, 32, 8, 8, 7, 64)]:
+        assert cut_bytes(B, QH, KVH, T, S, HD) == 0
+    from custom_kernels import _l3lib
+
+    for flag in (_l3lib.L3_ATTN_FLAG_PREFILL_WAVE, _l3lib.L3_ATTN_FLAG_PREFILL_TILED):      # a forced form is never cut
+        assert _l3lib.load().l3_attn_prefill_workspace_bytes(1, 32, 8, 8, 4096, 64, flag) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("HD", [64, 128])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s[:5])))
+def test_against_oracle(gpu, shape, HD):
+    from custom_kernels import custom_kernels_extension as cke
+    from oracle import attention_prefill_ref
+
+    B, QH, KVH, T, S, _ = shape
+    print(f"prefill pieces B={B} QH={QH} KVH={KVH} T={T} S={S} HD={HD}", flush=True)
+    inputs = make(B, QH, KVH, T, S, HD)
+    out = cke.flash_attention_prefill(*inputs(gpu))
+    torch.cuda.synchronize()
+    assert_attn_close(out, attention_prefill_ref(*(t2f32(t) for t in inputs("cpu"))), what=f"pieces {shape} HD={HD}")
+    again = cke.flash_attention_prefill(*inputs(gpu))       # whoever merges, and with the counters the first call left
+    np.testing.assert_array_equal(t2bits(out), t2bits(again))
+    dense = cke.flash_attention_prefill(*make(B, QH, KVH, T, S, HD, head_major=True)(gpu))      # other strides
+    np.testing.assert_array_equal(t2bits(out), t2bits(dense))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,T,S,HD", [(1, 512, 7012, 64), (1, 512, 7012, 128), (1, 1400, 8000, 128), (1, 1500, 6600, 64), (16, 64, 6564, 64)])
+def test_against_the_uncut_kernel(gpu, B, T, S, HD):
+    """The largest shapes that are cut, with scores spread over many powers of two: both against the same float64 rows."""
+    from custom_kernels import custom_kernels_extension as cke
+    from oracle import attention_prefill_ref
+
+    assert cut_bytes(B, 32, 8, T, S, HD) > 0
+    print(f"prefill pieces against the uncut kernel B={B} T={T} S={S} HD={HD}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(5)
+    q = torch.empty(B, T, 32, HD, dtype=torch.bfloat16, device=gpu).normal_(0, 3, generator=g).transpose(1, 2)
+    k, v = (torch.empty(B, S, 8, HD, dtype=torch.bfloat16, device=gpu).normal_(0, 1, generator=g).transpose(1, 2) for _ in range(2))
+    out = cke.flash_attention_prefill(q, k, v)
+    with cke.attention_flags(prefill="tiled"):
+        uncut = cke.flash_attention_prefill(q, k, v)
+    torch.cuda.synchronize()
+    for i in (0, 31, 32, 33, T // 2, T - 1):
+        n = S - T + i + 1
+        ref = attention_prefill_ref(t2f32(q[-1:, :, i:i + 1].cpu()), t2f32(k[-1:, :, :n].cpu()), t2f32(v[-1:, :, :n].cpu()))
+        for o, name in ((out, "cut"), (uncut, "uncut")):
+            assert_attn_close(o[-1:, :, i:i + 1], ref, what=f"{name} row {i}", regression=False)
+    # two bf16 roundings of results that differ by float32 sums in another order and bf16 weights against another reference
+    # (2^-9 of the result each): two units in the last place of the largest value
+    assert float((out.float() - uncut.float()).abs().max()) <= 2.0 ** -6 * float(uncut.float().abs().max())
+
+
+@pytest.mark.gpu
+def test_recorded_and_on_streams(gpu):
+    """Under capture the counters are the recording's own; the bits are the eager call's, on every replay and every stream."""
+    from custom_kernels import custom_kernels_extension as cke
+
+    q, k, v = make(1, 32, 8, 40, 3000, 64)(gpu)
+    ref = t2bits(cke.flash_attention_prefill(q, k, v))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = cke.flash_attention_prefill(q, k, v)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(t2bits(out), ref)
+        np.testing.assert_array_equal(t2bits(cke.flash_attention_prefill(q, k, v)), ref)
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    outs = []
+    for _ in range(4):
+        for s in streams:
+            s.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(s):
+                outs.append(cke.flash_attention_prefill(q, k, v))
+                cke.flash_attention_decode(q[:, :, :1], k, v)       # shares the stream's counters
+    torch.cuda.synchronize()
+    for o in outs:
+        np.testing.assert_array_equal(t2bits(o), ref)
+
+
+@pytest.mark.gpu
+def test_values_that_are_not_finite(gpu):
+    """A NaN or an infinite key reaches the rows that see it and no other."""
+    from custom_kernels import custom_kernels_extension as cke
+
+    q, k, v = make(1, 8, 2, 24, 2000, 64)(gpu)
+    clean = cke.flash_attention_prefill(q, k, v)
+    k = k.clone()
+    k[0, 0, 1990] = float("nan")
+    out = cke.flash_attention_prefill(q, k, v)
+    torch.cuda.synchronize()
+    assert torch.equal(out[:, 4:], clean[:, 4:])                    # the other kv head's
+    first = 1990 - (2000 - 24)                                      # the first query that sees it
+    # (columns of a wavefront follow a new maximum together, so a neighbour's may move the last bit)
+    assert float((out[:, :4, :first].float() - clean[:, :4, :first].float()).abs().max()) <= 2.0 ** -7 * float(clean.float().abs().max())
+    assert bool(out[:, :4, first:].isnan().all())
