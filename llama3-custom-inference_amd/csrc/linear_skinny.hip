@@ -54,9 +54,11 @@ constexpr int kXldsMaxElems = L3_LINEAR_NORM_STAGE_ELEMENTS;
 // j % 4 over k range j / 4 -- so one instruction covers 4 weight rows x 128 k, the blocks on the
 // diagonal (i / 4 == j / 4) hold the products and the rest is ignored.  Four times as many
 // wavefronts share a matrix with few rows, and a weight row is read 256 contiguous bytes at a time.
-template <int NW, int CBLK, int U, bool SWIGLU, bool XLDS, int RW>
+// XCH = 16-byte chunks of the activations a thread normalises (0: no norm in front).
+template <int NW, int CBLK, int U, bool SWIGLU, int XCH, int RW>
 __global__ void __launch_bounds__(NW * kWaveSize)
 linear_skinny_kernel(const LinearParams p) {
+    constexpr bool XLDS = XCH > 0;
     static_assert(!XLDS || CBLK == 1, "activations are staged in LDS only for up to 16 rows");
     static_assert(RW == 16 || (RW == 4 && CBLK == 1), "the four-row mapping takes at most four activation rows");
     constexpr int KQ = 16 / RW;                            // k ranges per matrix instruction
@@ -113,55 +115,62 @@ linear_skinny_kernel(const LinearParams p) {
     };
     // RMSNorm of the activations into LDS (XLDS).  The workgroup shares the 16-byte chunks of all
     // rows; K % 512 == 0, so the 64 chunks of a wavefront lie in one row and the row's sum of squares
-    // is a fixed-order sum of per-wavefront parts.  A thread's first chunk stays in registers and
-    // its loads are issued BEFORE the weight ring is filled (loads return in order, and the norm
-    // must not wait behind kilobytes of weights coming from HBM); with more than two rows the
-    // further chunks go through LDS, one at a time, so that the prologue costs few registers.
+    // is a fixed-order sum of per-wavefront parts.  A thread's chunks stay in registers from their load to the scaled
+    // store, and all the loads are issued BEFORE the weight ring is filled (loads return in order, and the norm must
+    // not wait behind kilobytes of weights coming from HBM).  Taken one at a time through LDS, with the norm weights
+    // read again for each, the chunks of three or four rows were a chain of memory round trips in front of every
+    // workgroup's products (us, before / now: 6144 x 4096, 2 / 3 / 4 rows 13.2 / 15.6 / 17.2, now 11.7 / 11.8 / 12.8; 3072 x
+    // 2048, 3 / 8 rows 7.4 / 10.1, now 6.5 / 8.1).
     constexpr int NT = NW * kWaveSize;
     const int KP = p.K + 8;                                // LDS row pitch in elements
     const int cpr = p.K / 8;                               // chunks per row
     const int nchunks = p.M * cpr;
-    uint4 xv0 = make_uint4(0u, 0u, 0u, 0u), gv0 = xv0;
+    uint4 xv[XLDS ? XCH : 1], gv = make_uint4(0u, 0u, 0u, 0u);
     if constexpr (XLDS) {
-        const int c = int(threadIdx.x);
-        if (c < nchunks) {                                 // wave-uniform
-            xv0 = load16(p.x + int64_t(c / cpr) * p.x_stride + (c % cpr) * 8);
-            gv0 = load16(p.norm_w + (c % cpr) * 8);
+#pragma unroll
+        for (int it = 0; it < XCH; ++it) {
+            const int c = int(threadIdx.x) + it * NT;
+            xv[it] = make_uint4(0u, 0u, 0u, 0u);
+            if (c < nchunks) xv[it] = load16(p.x + int64_t(c / cpr) * p.x_stride + (c % cpr) * 8);   // wave-uniform
         }
+        if (int(threadIdx.x) < nchunks) gv = load16(p.norm_w + (int(threadIdx.x) % cpr) * 8);
     }
     auto norm_prologue = [&]() {
         __shared__ float s_part[kXldsMaxElems / 8 / kWaveSize];
         const int parts_per_row = cpr / kWaveSize;
-        for (int c = int(threadIdx.x), it = 0; c < nchunks; c += NT, ++it) {
-            const int r = c / cpr, col = c % cpr;
-            uint4 v = xv0;
-            if (it > 0) {
-                v = load16(p.x + int64_t(r) * p.x_stride + col * 8);
-                *reinterpret_cast<uint4*>(s_x + r * KP + col * 8) = v;   // raw, re-read by this thread below
-            }
-            float f[8];
-            unpack8(v, f);
-            float ss = 0.f;
+        const bool same_columns = NT % cpr == 0;           // of all chunks of a thread
 #pragma unroll
-            for (int i = 0; i < 8; ++i) ss = fmaf(f[i], f[i], ss);
-            ss = wave_sum(ss);
-            if (lane == 0) s_part[c / kWaveSize] = ss;
+        for (int it = 0; it < XCH; ++it) {
+            const int c = int(threadIdx.x) + it * NT;
+            if (c < nchunks) {
+                float f[8];
+                unpack8(xv[it], f);
+                float ss = 0.f;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) ss = fmaf(f[i], f[i], ss);
+                ss = wave_sum(ss);
+                if (lane == 0) s_part[c / kWaveSize] = ss;
+            }
         }
         __syncthreads();
-        for (int c = int(threadIdx.x), it = 0; c < nchunks; c += NT, ++it) {
-            const int r = c / cpr, col = c % cpr;
-            float ss = 0.f;
-            for (int q = 0; q < parts_per_row; ++q) ss += s_part[r * parts_per_row + q];
-            const float inv = rsqrtf(ss / float(p.K) + p.norm_eps);
-            float f[8], g[8];
-            unpack8(it == 0 ? xv0 : *reinterpret_cast<const uint4*>(s_x + r * KP + col * 8), f);
-            unpack8(it == 0 ? gv0 : load16(p.norm_w + col * 8), g);
-            uint4 o;
-            o.x = pack_bf16x2(f[0] * inv * g[0], f[1] * inv * g[1]);
-            o.y = pack_bf16x2(f[2] * inv * g[2], f[3] * inv * g[3]);
-            o.z = pack_bf16x2(f[4] * inv * g[4], f[5] * inv * g[5]);
-            o.w = pack_bf16x2(f[6] * inv * g[6], f[7] * inv * g[7]);
-            *reinterpret_cast<uint4*>(s_x + r * KP + col * 8) = o;
+#pragma unroll
+        for (int it = 0; it < XCH; ++it) {
+            const int c = int(threadIdx.x) + it * NT;
+            if (c < nchunks) {
+                const int r = c / cpr, col = c % cpr;
+                float ss = 0.f;
+                for (int q = 0; q < parts_per_row; ++q) ss += s_part[r * parts_per_row + q];
+                const float inv = rsqrtf(ss / float(p.K) + p.norm_eps);
+                float f[8], g[8];
+                unpack8(xv[it], f);
+                unpack8(it == 0 || same_columns ? gv : load16(p.norm_w + col * 8), g);
+                uint4 o;
+                o.x = pack_bf16x2(f[0] * inv * g[0], f[1] * inv * g[1]);
+                o.y = pack_bf16x2(f[2] * inv * g[2], f[3] * inv * g[3]);
+                o.z = pack_bf16x2(f[4] * inv * g[4], f[5] * inv * g[5]);
+                o.w = pack_bf16x2(f[6] * inv * g[6], f[7] * inv * g[7]);
+                *reinterpret_cast<uint4*>(s_x + r * KP + col * 8) = o;
+            }
         }
         __syncthreads();
     };
@@ -318,14 +327,30 @@ linear_skinny_kernel(const LinearParams p) {
     }
 }
 
-template <int NW, int CBLK, int U, bool SWIGLU, bool XLDS, int RW = 16>
-int launch_variant(const LinearParams& p, hipStream_t stream) {
+template <int NW, int CBLK, int U, bool SWIGLU, int XCH, int RW>
+int launch_chunks(const LinearParams& p, hipStream_t stream) {
     const int row_blocks = (p.N + RW - 1) / RW;
     const int rb_per_wg = NW / p.sk;
     const dim3 grid(unsigned((row_blocks + rb_per_wg - 1) / rb_per_wg));
-    const size_t lds = XLDS ? size_t(p.M) * size_t(p.K + 8) * sizeof(uint16_t) : 0;
-    return enqueue(linear_skinny_kernel<NW, CBLK, U, SWIGLU, XLDS, RW>, grid, dim3(NW * kWaveSize), lds, stream,
+    const size_t lds = XCH > 0 ? size_t(p.M) * size_t(p.K + 8) * sizeof(uint16_t) : 0;
+    return enqueue(linear_skinny_kernel<NW, CBLK, U, SWIGLU, XCH, RW>, grid, dim3(NW * kWaveSize), lds, stream,
                    p);
+}
+
+// One row of up to 4096 (two of 2048) is a chunk per thread and needs few registers; more rows take all a thread can have.
+template <int NW, int CBLK, int U, bool SWIGLU, bool XLDS, int RW = 16>
+int launch_variant(const LinearParams& p, hipStream_t stream) {
+    constexpr int NT = NW * kWaveSize;
+    if constexpr (XLDS) {
+        if (p.M * (p.K / 8) <= NT) return launch_chunks<NW, CBLK, U, SWIGLU, 1, RW>(p, stream);
+        if (p.M * (p.K / 8) <= 2 * NT) return launch_chunks<NW, CBLK, U, SWIGLU, 2, RW>(p, stream);
+        if constexpr (NW == 8) {
+            if (p.M * (p.K / 8) <= 4 * NT) return launch_chunks<NW, CBLK, U, SWIGLU, 4, RW>(p, stream);
+        }
+        return launch_chunks<NW, CBLK, U, SWIGLU, (kXldsMaxElems / 8 + NT - 1) / NT, RW>(p, stream);
+    } else {
+        return launch_chunks<NW, CBLK, U, SWIGLU, 0, RW>(p, stream);
+    }
 }
 
 }  // namespace

@@ -549,11 +549,12 @@ constexpr int64_t kWideRows = 12288, kWidePairRows = 6144;
 // rows 139 / 87; gate|up pair 8192 x 2048, 3 rows 14.0 / 13.2, 4 rows 14.7 / 13.3, 16 rows 21.0 / 12.8; pair 14336 x
 // 4096 (235 MB), 1 row 47.9 / 39.2; 2048 x 8192, 4 rows 10.2 / 10.6, 5 rows 15.4 / 10.7; 4096 x 4096, 5 rows 10.1 / 10.4, 16
 // rows 12.3 / 10.6; 6144 x 4096, 2 rows 11.3 / 12.8, 5 rows 16.2 / 12.9; 4096 x 14336, 1 row 23.2 / 22.9; 2048 x 2048 and
-// 3072 x 2048, 12 rows 6.7 / 6.6 and 6.9 / 7.1.
+// 3072 x 2048, 12 rows 6.7 / 6.6 and 6.9 / 7.1.  With the norm in front (inside the skinny kernel): gate|up pair 8192 x
+// 2048, 4 rows 13.8 / 15.0, 5 rows 22.6 / 15.2; pair 14336 x 4096, 1 row 44.8 / 41.9.
 //
 // Up to 16 rows the skinny kernel says what is taken and what is refused: operands that it takes and the others do not stay
 // with it, and so do those that it refuses.
-Route route_of(const Rows& r, const Tensor& w, bool pair, const Tensor* residual) {
+Route route_of(const Rows& r, const Tensor& w, bool norm, bool pair, const Tensor* residual) {
     const int64_t K = r.K, N = size_at(w, 0);
     const bool near_rows = stride_at(w, 0) <= L3_LINEAR_WIDE_MAX_STRIDE;
     if (r.rows > L3_LINEAR_MAX_ROWS) {
@@ -564,7 +565,7 @@ Route route_of(const Rows& r, const Tensor& w, bool pair, const Tensor* residual
     if (K % 128 != 0 || N % 8 != 0 || !near_rows || misaligned(r.x) || r.stride < K || r.stride % 8 != 0) return Route::kSkinny;
     if (pair) {
         const bool large = N * K >= int64_t(32) << 20;   // each of the two
-        return N >= kWidePairRows && (r.rows >= 4 || large) ? Route::kWide : Route::kSkinny;
+        return N >= kWidePairRows && (r.rows >= (norm ? 5 : 4) || large) ? Route::kWide : Route::kSkinny;
     }
     if (residual && residual->is_contiguous() && misaligned(ptr(*residual))) return Route::kSkinny;
     if (N >= kWideRows) return r.rows >= 4 ? Route::kWide : Route::kSkinny;
@@ -645,7 +646,7 @@ Tensor linear(const Tensor& x, const Tensor& w, const Tensor* norm, double eps, 
     const Rows r = linear_rows(x, L3_LINEAR_SPLITK_MAX_ROWS, false);
     check_weight(w, w, x, r.K);
     if (up) check_weight(*up, w, x, r.K);
-    const Route route = route_of(r, w, up != nullptr, residual);
+    const Route route = route_of(r, w, norm != nullptr, up != nullptr, residual);
     if (route == Route::kSkinny) check_rows(r.rows, L3_LINEAR_MAX_ROWS, x);
     if (norm) check_norm_weight(*norm, r.rows, r.K, "linear_decode_fused");
     if (route != Route::kSkinny) {

@@ -131,6 +131,31 @@ def test_linear_fused_input_norm(gpu, M, N, K):
     assert err.max() <= 2.0 ** -6 * max(1.0, np.abs(ref).max()), f"fused norm vs oracle: max err {err.max()}"
 
 
+# 16-byte chunks per thread of the norm inside the kernel: 1, 2, 4 and as many as LDS holds, widths whose chunks of a
+# thread lie in one column (K a power of two up to 4096) and others, workgroups of eight and of sixteen wavefronts, and the
+# fewest and most rows of each
+@pytest.mark.parametrize("M,K", [(1, 512), (16, 512), (2, 2048), (3, 2048), (4, 2048), (1, 4096), (2, 4096), (4, 4096), (5, 4096),
+                                 (9, 2048), (11, 2048), (3, 1536), (15, 1536), (4, 3072), (7, 3072), (2, 8192), (1, 24064), (3, 7680)])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_linear_norm_chunks(gpu, M, K, swiglu):
+    from custom_kernels import custom_kernels_extension as cke
+    from oracle import rms_norm_ref, round_to_bf16
+
+    N = 44
+    print(f"linear norm chunks M={M} K={K} swiglu={swiglu}", flush=True)
+    x = randn_bf16((M, 1, K), 81, scale=2.0)
+    x[-1] *= 64       # rows of other sizes
+    nw = randn_bf16((K,), 82, scale=0.1, mean=1.0)
+    w, u = randn_bf16((N, K), 83, scale=0.05), randn_bf16((N, K), 84, scale=0.05)
+    y = cke.linear_decode_fused(x.to(gpu), w.to(gpu), norm_weight=nw.to(gpu), eps=1e-5, w_up=u.to(gpu) if swiglu else None)
+    torch.cuda.synchronize()
+    h = round_to_bf16(rms_norm_ref(t2f32(x), t2f32(nw), 1e-5))
+    ref = swiglu_linear_ref(h, t2f32(w), t2f32(u)) if swiglu else linear_ref(h, t2f32(w))
+    err = np.abs(t2f32(y).astype(np.float64) - ref)
+    # (the bounds of the tests around this one, for the same two forms)
+    assert err.max() <= (0.02 if swiglu else 2.0 ** -6) * max(1.0, np.abs(ref).max()), f"max err {err.max()}"
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 8192, 2048), (4, 1024, 512), (11, 8192, 2048), (16, 260, 256)])
 @pytest.mark.parametrize("with_norm", [False, True])
 def test_linear_fused_swiglu_with_residual(gpu, M, N, K, with_norm):
