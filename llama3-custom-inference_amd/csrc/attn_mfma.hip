@@ -31,16 +31,21 @@ namespace {
 // LOADS = 4 (head size 64, cooperative form, at most 512 tokens): half-size tiles of 32 tokens, so
 // that a short sequence still gives every wavefront a tile, and slabs small enough for two
 // workgroups per CU.
-template <int HD, bool COOP, int LOADS = 8>
-__global__ void __launch_bounds__(kMfmaWaves * kWaveSize, 2)
+// NW = 4 (cooperative form, one split, more heads than compute units): half the wavefronts and half the LDS, so that two
+// or three workgroups are resident where one of eight wavefronts was, and a launch of up to three heads per unit needs
+// no second round.  us, eight wavefronts or streaming / this: 64 sequences x 8 heads at head size 128, 16 tokens 6.8 / 4.1, 200
+// tokens 13.1 / 10.7; 80 sequences at head size 64, 200 tokens 11.9 / 8.6, 800 tokens 34.8 / 26.8.
+template <int HD, bool COOP, int LOADS = 8, int NW = kMfmaWaves>
+__global__ void __launch_bounds__(NW * kWaveSize, 2)
 attn_splitkv_mfma_kernel(const int R, const int hpw_log2, const AttnParams p) {
     using T = MfmaTile<HD, LOADS>;
     constexpr int WT = T::WT, KC = T::KC, NB = T::NB, SLAB = T::SLAB;
-    constexpr int STEP = COOP ? kMfmaWaves * WT : WT;  // token stride between a wavefront's tiles
+    constexpr int STEP = COOP ? NW * WT : WT;  // token stride between a wavefront's tiles
     static_assert(LOADS != 8 || WT == attn_tile_tokens(HD, kAttnImplMfma), "host plan and kernel tile disagree");
     static_assert(LOADS == 8 || COOP, "the split plan counts full tiles");
+    static_assert(NW == kMfmaWaves || COOP, "the streaming form lays eight wavefronts over heads and splits");
 
-    __shared__ __align__(16) unsigned char s_slab[kMfmaWaves][SLAB];
+    __shared__ __align__(16) unsigned char s_slab[NW][SLAB];
 
     const int lane = threadIdx.x & (kWaveSize - 1);
     const int wave = wave_uniform(int(threadIdx.x) / kWaveSize);   // scalar: everything derived from it is wave-uniform
@@ -64,7 +69,7 @@ attn_splitkv_mfma_kernel(const int R, const int hpw_log2, const AttnParams p) {
     // Single-launch form (cooperative workgroups with p.arrive set): the workgroup that finishes a (batch,
     // kv head) last merges its partials, and every split of the plan is counted as an arrival -- also one
     // that a device-side KV length leaves without tokens (it streams and writes nothing, the merge skips its row).
-    const bool merge_here = COOP && p.arrive != nullptr;
+    const bool merge_here = COOP && NW == kMfmaWaves && p.arrive != nullptr;
     // A split past the plan (last workgroup of the streaming form: whole wavefront, no barrier follows)
     // or, with a combine launch to follow, past a device-side KV length (whole workgroup when COOP).
     if (split >= p.num_splits || (!merge_here && t_begin >= S)) return;
@@ -104,10 +109,10 @@ attn_splitkv_mfma_kernel(const int R, const int hpw_log2, const AttnParams p) {
     const float m_log2 = (m_run == kMaskedScore) ? kMaskedScore : m_run * c;  // a COOP wave may have had no tile
 
     if constexpr (COOP) {
-        // merge the eight wavefronts through LDS, then write like the streaming form
-        __shared__ float s_m[kMfmaWaves][kAttnMaxRatio];
-        __shared__ float s_l[kMfmaWaves][kAttnMaxRatio];
-        __shared__ __align__(16) float s_o[kMfmaWaves][kAttnMaxRatio][HD];
+        // merge the wavefronts through LDS, then write like the streaming form
+        __shared__ float s_m[NW][kAttnMaxRatio];
+        __shared__ float s_l[NW][kAttnMaxRatio];
+        __shared__ __align__(16) float s_o[NW][kAttnMaxRatio][HD];
         __shared__ int s_last;
         if (fn < R) {
 #pragma unroll
@@ -121,15 +126,15 @@ attn_splitkv_mfma_kernel(const int R, const int hpw_log2, const AttnParams p) {
             }
         }
         __syncthreads();
-        for (int idx = threadIdx.x; idx < R * (HD / 2); idx += kMfmaWaves * kWaveSize) {
+        for (int idx = threadIdx.x; idx < R * (HD / 2); idx += NW * kWaveSize) {
             const int h = idx / (HD / 2);
             const int d = (idx % (HD / 2)) * 2;
             float M = s_m[0][h];
 #pragma unroll
-            for (int w = 1; w < kMfmaWaves; ++w) M = fmaxf(M, s_m[w][h]);
+            for (int w = 1; w < NW; ++w) M = fmaxf(M, s_m[w][h]);
             float L = 0.f, o0 = 0.f, o1 = 0.f;
 #pragma unroll
-            for (int w = 0; w < kMfmaWaves; ++w) {
+            for (int w = 0; w < NW; ++w) {
                 const float e = fast_exp2(s_m[w][h] - M);  // wavefronts without a tile: 0
                 L = fmaf(s_l[w][h], e, L);
                 o0 = fmaf(s_o[w][h][d], e, o0);
@@ -260,7 +265,17 @@ int launch_attn_splitkv_mfma(const AttnParams& params, int HD, int R, bool coop,
         int rc;
         if (coop) {
             const dim3 grid(unsigned(p.KVH), unsigned(p.B), unsigned(p.num_splits));
-            if (HD == 64 && p.tokens_per_split <= 2 * kMfmaWaves * 32) {
+            if (p.num_splits == 1 && int64_t(p.B) * p.KVH > current_device_cus()) {
+                constexpr int NW = 4;
+                const dim3 four(NW * kWaveSize);
+                if (HD == 64 && p.tokens_per_split <= 2 * NW * 32) {
+                    rc = enqueue(attn_splitkv_mfma_kernel<64, true, 4, NW>, grid, four, 0, stream, R, 0, p);
+                } else if (HD == 64) {
+                    rc = enqueue(attn_splitkv_mfma_kernel<64, true, 8, NW>, grid, four, 0, stream, R, 0, p);
+                } else {
+                    rc = enqueue(attn_splitkv_mfma_kernel<128, true, 8, NW>, grid, four, 0, stream, R, 0, p);
+                }
+            } else if (HD == 64 && p.tokens_per_split <= 2 * kMfmaWaves * 32) {
                 rc = enqueue(attn_splitkv_mfma_kernel<64, true, 4>, grid, block, 0, stream, R, 0, p);
             } else if (HD == 64) {
                 rc = enqueue(attn_splitkv_mfma_kernel<64, true>, grid, block, 0, stream, R, 0, p);

@@ -170,6 +170,28 @@ bool attn_merge_in_launch_wanted(int flags) {
     return (flags & L3_ATTN_FLAG_WS_COUNTERS) && !(flags & (L3_ATTN_FLAG_TWO_LAUNCHES | L3_ATTN_FLAG_KERNEL_FMA));
 }
 }  // namespace
+// Tiles of a sequence for which a (batch, kv head) is one workgroup of four wavefronts, where there are more of those
+// than compute units: from a sweep of 272 to 1024 heads and 16 to 2400 tokens against the streaming form (us, streaming / this).
+//   * Up to 5/4 heads per unit some units have twice the work of others, so longer sequences stream in splits (272 heads at
+//     head size 128, 400 tokens 15.5 / 15.0, 512 tokens 17.2 / 18.2; head size 64, 512 tokens 11.2 / 11.6, 800 tokens 14.4 /
+//     16.9); up to 7/4 that is so from 800 tokens on at head size 64 (384 heads, 800: 16.6 / 17.9, 1000: 21.2 / 21.4).
+//   * Up to three heads per unit all of them are resident (640 heads, 1000 tokens: head size 64 42.7 / 31.9, 128 60.3 / 55.7);
+//     a 512-head launch at head size 64, 800 tokens 21.2 / 20.0.  Whole token rows win beyond (640 heads, 1600 tokens at head
+//     size 128: 82.9 / 87.1).
+//   * Up to four heads per unit short sequences only (896 heads, 400 tokens: head size 64 20.6 / 18.7, 128 36.6 / 32.0; 1024
+//     heads, 512 tokens: 24.3 / 25.3 and 45.1 / 46.1).
+//   * At head size 128 a single tile of 640 heads is better streamed (4.9 / 6.0), two tiles of 896 as well (8.4 / 9.0).
+int four_wave_tiles_max(int64_t units, int HD, int64_t cus) {
+    if (4 * units <= 5 * cus) return HD == 64 ? 8 : 12;
+    if (4 * units <= 7 * cus) return HD == 64 ? 13 : 32;
+    if (units <= 3 * cus) return HD == 64 ? 16 : 32;
+    if (units <= 4 * cus) return HD == 64 ? 7 : 12;
+    return 0;
+}
+int four_wave_tiles_min(int64_t units, int HD, int64_t cus) {
+    if (HD == 64 || units <= 2 * cus) return 1;
+    return units <= 3 * cus ? 2 : 3;
+}
 
 AttnPlan attn_make_plan(int B, int KVH, int S, int HD, int requested, int num_cus, int impl, int form,
                         bool merge_in_launch) {
@@ -184,11 +206,18 @@ AttnPlan attn_make_plan(int B, int KVH, int S, int HD, int requested, int num_cu
         plan.coop = impl == kAttnImplMfma && form == L3_ATTN_FLAG_FORM_COOP;
     } else if (impl == kAttnImplMfma) {
         // Short sequences are latency-bound.  With at most one tile per wavefront of a workgroup (or two,
-        // when there are too many heads for each to get a second workgroup) and not already enough
-        // heads to fill the device twice over, one cooperative workgroup per (batch, kv head) finishes
+        // when there are too many heads for each to get a second workgroup), or in workgroups of four
+        // wavefronts where there are more heads than compute units, one cooperative workgroup per (batch, kv head) finishes
         // the row in a single launch.
         const int64_t units = int64_t(B) * KVH;
-        if (units <= 2 * int64_t(num_cus)) {
+        if (units > num_cus) {
+            if (tiles >= four_wave_tiles_min(units, HD, num_cus) && tiles <= four_wave_tiles_max(units, HD, num_cus)) {
+                plan.coop = true;
+                plan.num_splits = 1;
+                plan.tokens_per_split = tiles * tile;
+                return plan;
+            }
+        } else {
             const int wgs = int(std::max<int64_t>(1, num_cus / units));   // workgroups a head can have, one per unit
             // (Head size 64 with at least four workgroups to spare per head: up to six tiles only; its wavefronts
             // work through half tiles one after the other, 4.1 us at 256 tokens but 5.6 / 6.0 us at 448 / 512,
@@ -247,9 +276,11 @@ AttnPlan attn_make_plan(int B, int KVH, int S, int HD, int requested, int num_cu
             // K + V bytes a workgroup streams when there is a single group
             const int64_t stream_bytes = int64_t(kMfmaWaves) * ((S + spg - 1) / spg) * HD * 4;
             const bool short_stream = stream_bytes <= (int64_t(3) << 20);
-            if (short_stream && spg == 1 && wgs_per_split_group * 4 >= num_cus) {
-                groups = 1;   // a quarter of the units busy, but no partials and no second launch
-            } else if (groups == 1 && !short_stream && int64_t(num_cus) / wgs_per_split_group >= 2) {
+            if (short_stream && spg == 1 && (wgs_per_split_group * 2 >= num_cus || (wgs_per_split_group * 4 >= num_cus && tiles <= 2))) {
+                // half of the units busy, but no partials and no second launch (with a quarter of them busy only the
+                // shortest: 64 sequences of 1300 tokens at head size 64 took 53.9 us in one group, 29.6 in three)
+                groups = 1;
+            } else if (groups == 1 && (!short_stream || spg == 1) && int64_t(num_cus) / wgs_per_split_group >= 2) {
                 groups = 2;
             } else if (groups > 1) {
                 // Splits are whole tiles: with few tiles the rounding can halve the workgroup count (16 tiles

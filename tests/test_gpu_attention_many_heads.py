@@ -1,0 +1,72 @@
+"""Decode attention with more (batch, kv head) pairs than compute units: workgroups of four wavefronts, one per pair."""
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import assert_attn_close, make_qkv, t2bits, t2f32
+
+CUS = 256
+
+
+def splits(B, KVH, S, HD):
+    from custom_kernels import custom_kernels_extension as cke
+
+    return cke.attention_num_splits(B, KVH, S, HD, CUS)
+
+
+def test_lengths_that_take_one_workgroup_per_head():
+    """One split up to each line, splits again beyond it (where the streaming form has several)."""
+    for units, last in ((320, {64: 512, 128: 384}), (448, {64: 832, 128: 1024}), (512, {64: 1024, 128: 1024}), (768, {64: 1024, 128: 1024})):
+        for HD in (64, 128):
+            assert splits(units // 8, 8, last[HD], HD) == 1
+            assert splits(units // 8, 8, last[HD] + 1, HD) > 1, (units, HD)
+    # a quarter of the device is not left alone with a long stream
+    assert splits(64, 8, 1300, 64) == 3 and splits(112, 8, 1300, 64) == 2 and splits(128, 8, 1300, 64) == 1
+
+
+# pairs either side of one, 5/4, 2, 3 and 4 per compute unit; lengths of one tile and less, of one and of more rounds of the four
+# wavefronts with a ragged end, and the longest each takes; every head ratio
+CASES = [(257, 1, 1), (33, 8, 16), (33, 8, 129), (33, 8, 384), (40, 8, 512), (41, 8, 257), (64, 8, 63), (64, 8, 255), (64, 8, 1000),
+         (65, 8, 33), (65, 8, 300), (96, 8, 70), (96, 8, 1024), (97, 8, 65), (128, 8, 380), (128, 8, 448), (140, 2, 700), (129, 8, 40)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("HD", [64, 128])
+@pytest.mark.parametrize("B,KVH,S", CASES)
+def test_against_oracle(gpu, B, KVH, S, HD):
+    from custom_kernels import custom_kernels_extension as cke
+    from oracle import attention_decode_ref
+
+    R = (1, 2, 3, 4, 8)[(B + S) % 5]
+    print(f"many heads B={B} KVH={KVH} R={R} S={S} HD={HD} splits={splits(B, KVH, S, HD)}", flush=True)
+    q, k, v = make_qkv(B, R * KVH, KVH, S, HD, seed=91, cache_len=S + 9)
+    qg, kg, vg = make_qkv(B, R * KVH, KVH, S, HD, seed=91, cache_len=S + 9, device=gpu)
+    out = cke.flash_attention_decode(qg, kg, vg)
+    torch.cuda.synchronize()
+    some = [0, 1, B // 2, B - 1]
+    assert_attn_close(out[some], attention_decode_ref(t2f32(q[some]), t2f32(k[some]), t2f32(v[some])), what=f"B={B} S={S} HD={HD}")
+    # every other sequence against the streaming form (partials of three splits and a combine)
+    other = cke.flash_attention_decode(qg, kg, vg, 3)
+    assert_attn_close(out, t2f32(other).astype(np.float64), what=f"against the streaming form B={B} S={S} HD={HD}", regression=False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("HD", [64, 128])
+@pytest.mark.parametrize("length", [1, 31, 64, 200, 256])
+def test_length_on_the_device(gpu, length, HD):
+    """The length of a recorded step: planned for the whole cache, whose other rows are not numbers."""
+    from custom_kernels import custom_kernels_extension as cke
+    from oracle import attention_decode_ref
+
+    B, QH, KVH, S = 64, 32, 8, 256
+    print(f"many heads, device length {length} HD={HD}", flush=True)
+    q, k, v = make_qkv(B, QH, KVH, S, HD, seed=92, cache_len=S)
+    ref = attention_decode_ref(t2f32(q[:2]), t2f32(k[:2, :, :length]), t2f32(v[:2, :, :length]))
+    k[:, :, length:], v[:, :, length:] = float("nan"), float("nan")
+    n = torch.tensor([length], dtype=torch.int32, device=gpu)
+    out = cke.flash_attention_decode_devlen(q.to(gpu), k.to(gpu), v.to(gpu), n)
+    torch.cuda.synchronize()
+    assert_attn_close(out[:2], ref, what=f"device length {length}", regression=False)
+    assert bool(torch.isfinite(out.float()).all())
+    np.testing.assert_array_equal(t2bits(out), t2bits(cke.flash_attention_decode_devlen(q.to(gpu), k.to(gpu), v.to(gpu), n)))
