@@ -16,7 +16,7 @@ namespace {
 constexpr int kRmsThreads = 256;
 
 // One row per group of LANES threads (the launcher uses 256: the whole workgroup on one row,
-// for fewer than 1024 rows and for rows too wide for the streaming kernel further down).  A
+// for as many rows as the device holds and for rows too wide for the streaming kernel further down).  A
 // thread keeps up to MAXV 16-byte vectors of its row in registers; requires C % 8 == 0 and
 // C / 8 <= LANES * MAXV.
 //
@@ -38,13 +38,20 @@ rms_norm_rows_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict_
     const int nvec = C / 8;
     const uint16_t* xr = x + (live ? row : 0) * int64_t(C);
 
-    uint4 xv[MAXV];
+    uint4 xv[MAXV], wv[MAXV];   // (the weights are requested with the row, not behind its reduction)
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < MAXV; ++j) {
         const int vi = t + j * LANES;
         if (vi < nvec) {
             xv[j] = load16(xr + vi * 8);
+            wv[j] = load16(w + vi * 8);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < MAXV; ++j) {
+        const int vi = t + j * LANES;
+        if (vi < nvec) {
             float f[8];
             unpack8(xv[j], f);
             if constexpr (ADD) {
@@ -78,7 +85,7 @@ rms_norm_rows_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict_
         if (vi < nvec) {
             float f[8], g[8];
             unpack8(xv[j], f);
-            unpack8(load16(w + vi * 8), g);
+            unpack8(wv[j], g);
             uint4 o;
             o.x = pack_bf16x2(f[0] * inv * g[0], f[1] * inv * g[1]);
             o.y = pack_bf16x2(f[2] * inv * g[2], f[3] * inv * g[3]);
@@ -280,9 +287,14 @@ int launch_rms_norm_impl(const uint16_t* x, const uint16_t* res, const uint16_t*
                          int64_t rows, int C, float eps, bool vec_ok, hipStream_t stream) {
     const int nvec = C / 8;
     const dim3 block(kRmsThreads);
-    if (vec_ok && rows >= 1024 && nvec <= 64 * 8) {
-        // a thousand rows or more: every wavefront takes several, reads overlapping writes
-        const int64_t waves = std::min<int64_t>(rows / 2, int64_t(current_device_cus()) * 8);
+    // The device holds eight workgroups of a row each per compute unit.  A launch beyond that streams: every wavefront takes
+    // several rows, reads overlapping writes (us, a workgroup per row / streaming; 4096 wide: 1024 rows 4.9 / 5.7, 2048 rows
+    // 7.1 / 8.1, 2600 rows 9.7 / 9.4, 4096 rows 12.9 / 11.8; 1536 wide: 2048 rows 4.0 / 4.7, 2600 rows 4.9 / 4.8).  The line is the
+    // same with and without the residual: the two kernels add the squares in different orders, and add_rms_norm has the bits
+    // of an addition and rms_norm.
+    const int64_t cus = current_device_cus();
+    if (vec_ok && rows > 8 * cus && nvec <= 64 * 8) {
+        const int64_t waves = std::min<int64_t>(rows / 2, cus * 8);
         const dim3 grid(unsigned((waves + 3) / 4));
         if (nvec <= 64 * 4) {
             return enqueue(rms_norm_stream_kernel<4, ADD>, grid, block, 0, stream, x, res, w, sum_out, y, rows, C,

@@ -46,6 +46,25 @@ def test_rms_norm_other_widths(gpu, C, rows):
     assert_within_ulps(out, rms_norm_ref(t2f32(x), t2f32(w), 1e-5), 1, what=f"rms rows{rows} C{C}")
 
 
+# rows either side of what the device holds as a workgroup each (2048); widths either side of 4 and 8 vectors per lane
+@pytest.mark.parametrize("add", [False, True])
+@pytest.mark.parametrize("rows", [2047, 2048, 2049])
+@pytest.mark.parametrize("C", [1536, 2048, 2056, 4096, 4104, 5120])
+def test_norm_of_many_rows(gpu, add, rows, C):
+    from custom_kernels import custom_kernels_extension as cke
+
+    print(f"norm of many rows add={add} rows={rows} C={C}", flush=True)
+    x, res = randn_bf16((1, rows, C), C + 1).to(gpu), randn_bf16((1, rows, C), C + 2).to(gpu)
+    w = randn_bf16((C,), 8, scale=0.5, mean=0.0)
+    if add:
+        total, out = cke.add_rms_norm(x, res, w.to(gpu), 1e-5)
+        assert torch.equal(total, x + res) and torch.equal(out, cke.rms_norm(total, w.to(gpu), 1e-5))
+    else:
+        total, out = x, cke.rms_norm(x, w.to(gpu), 1e-5)
+    torch.cuda.synchronize()
+    assert_within_ulps(out, rms_norm_ref(t2f32(total), t2f32(w), 1e-5), 1, what=f"many rows {rows} C{C} add={add}")
+
+
 def test_rms_norm_adversarial_rows(gpu):
     from custom_kernels import custom_kernels_extension as cke
 
