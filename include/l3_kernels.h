@@ -222,18 +222,14 @@ int l3_attn_prefill(const void* q, const void* k, const void* v, void* out, int 
                     const int64_t out_strides[3], float scale, int flags, void* stream);
 
 /*
- * The same with memory for partial results.  Launches that leave the device waiting for their longest rows (a few
- * prompts of medium length, a short piece of a prompt behind many cached tokens) are then cut into pieces of
- * rows x tokens, and the piece of a row block that finishes last adds them up.
+ * The same with memory for partial results.  Launches of few rows against many tokens (a short piece of a prompt behind
+ * a long cache) are then cut into pieces of rows x tokens, and a second launch adds them up.
  *   workspace : l3_attn_prefill_workspace_bytes() bytes (0: the call is not cut and takes none), aligned to 256; free
  *               to be reused by later work of the stream
- *   counters  : arrival counters that l3_attn_workspace_init prepared and that calls of this stream share, or NULL:
- *               then the call clears some at the head of the workspace with a launch of its own.  The same bits
- *               either way.
  */
 size_t l3_attn_prefill_workspace_bytes(int B, int QH, int KVH, int T, int S, int HD, int flags);
 int l3_attn_prefill_ws(const void* q, const void* k, const void* v, void* out, void* workspace, size_t workspace_bytes,
-                       void* counters, int B, int QH, int KVH, int T, int S, int HD, const int64_t q_strides[3],
+                       int B, int QH, int KVH, int T, int S, int HD, const int64_t q_strides[3],
                        const int64_t k_strides[3], const int64_t v_strides[3], const int64_t out_strides[3], float scale,
                        int flags, void* stream);
 

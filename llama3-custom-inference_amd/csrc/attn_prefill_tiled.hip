@@ -25,8 +25,6 @@ namespace l3 {
 
 namespace {
 
-constexpr int kDeviceScope = 16;   // buffer accesses that go to where all XCDs see them (sc1)
-
 // Maximum that hands a NaN on (v_maximum3_f32): unlike fmaxf it needs no quieting of its inputs, which
 // costs an instruction per value that comes out of a matrix instruction or a lane swap.
 __device__ __forceinline__ float maximum(float a, float b) { return __builtin_elementwise_maximum(a, b); }
@@ -656,94 +654,17 @@ attn_prefill_tiled_kernel(const PrefillParams p, const std::conditional_t<SPLIT,
 
     if constexpr (SPLIT) {
         if (pieces > 1) {   // workgroup-uniform
-            // A piece leaves its accumulators as they lie in the registers, so that every access is whole lines and the
-            // merging thread finds its own columns.  The pieces of a block may run on different XCDs: stores write
-            // through and loads do not stop at the caches (device scope), and the count of arrivals is the device's.
-            constexpr int VECS = CB * NB;
+            // A piece leaves its accumulators as they lie in the registers, so that every access is whole lines; the launch
+            // that follows adds the pieces of a block up.
             constexpr int NT = NW * kWaveSize;
-            constexpr int kSlotBytes = (VECS * 16 + CB * 8) * NT;
-            char* const block = items.part + (int64_t(bh) * items.slots_per_head + first_slot) * kSlotBytes;
-            __shared__ int s_last;
-            {
-                const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(block + int64_t(piece) * kSlotBytes, 0, kSlotBytes, 0x00020000);
-#pragma unroll
-                for (int cb = 0; cb < CB; ++cb) {
-#pragma unroll
-                    for (int nb = 0; nb < NB; ++nb) {
-                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, O[cb][nb]), to, tid * 16, (cb * NB + nb) * NT * 16, kDeviceScope);
-                    }
-                    const u32x2_t ml = {__builtin_bit_cast(uint32_t, m_run[cb]), __builtin_bit_cast(uint32_t, Lsum[cb])};
-                    __builtin_amdgcn_raw_buffer_store_b64(ml, to, tid * 8, VECS * NT * 16 + cb * NT * 8, kDeviceScope);
-                }
-            }
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's part is where every XCD reads it
-            __syncthreads();
-            unsigned* const counter = items.counters + (int64_t(bh) * items.slots_per_head + first_slot) / 2 * kPrefillCounterStride;
-            if (tid == 0) {
-                const unsigned before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                s_last = before == unsigned(pieces - 1);
-                // (nobody else arrives before the next launch, which finds zero again)
-                if (s_last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            __syncthreads();
-            if (!s_last) return;
-            // The pieces in their order, whichever arrived last, so that a result does not depend on who merges it; the
-            // next piece is on its way while one is added.
-            f32x4_t sum[CB][NB];
-            float total[CB], M[CB];
+            char* const slot = items.part + (int64_t(bh) * items.slots_per_head + first_slot + piece) * prefill_slot_bytes(HD, CB);
 #pragma unroll
             for (int cb = 0; cb < CB; ++cb) {
-                M[cb] = kNoScore;
-                total[cb] = 0.f;
 #pragma unroll
-                for (int nb = 0; nb < NB; ++nb) sum[cb][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+                for (int nb = 0; nb < NB; ++nb) *reinterpret_cast<f32x4_t*>(slot + ((cb * NB + nb) * NT + tid) * 16) = O[cb][nb];
+                *reinterpret_cast<float2*>(slot + CB * NB * NT * 16 + (cb * NT + tid) * 8) = make_float2(m_run[cb], Lsum[cb]);
             }
-            u32x4_t part[2][CB][NB];
-            u32x2_t ml[2][CB];
-            auto request = [&](int i, u32x4_t (&o)[CB][NB], u32x2_t (&st)[CB]) __attribute__((always_inline)) {
-                const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc(block + int64_t(min(i, pieces - 1)) * kSlotBytes, 0, kSlotBytes, 0x00020000);
-#pragma unroll
-                for (int cb = 0; cb < CB; ++cb) {
-                    st[cb] = __builtin_amdgcn_raw_buffer_load_b64(from, tid * 8, VECS * NT * 16 + cb * NT * 8, kDeviceScope);
-#pragma unroll
-                    for (int nb = 0; nb < NB; ++nb) {
-                        o[cb][nb] = __builtin_amdgcn_raw_buffer_load_b128(from, tid * 16, (cb * NB + nb) * NT * 16, kDeviceScope);
-                    }
-                }
-            };
-            auto add = [&](const u32x4_t (&o)[CB][NB], const u32x2_t (&st)[CB]) __attribute__((always_inline)) {
-#pragma unroll
-                for (int cb = 0; cb < CB; ++cb) {
-                    const float m = __builtin_bit_cast(float, uint32_t(st[cb][0]));
-                    const float m_new = maximum(M[cb], m);
-                    const float f_old = fast_exp2((M[cb] - m_new) * c), f = fast_exp2((m - m_new) * c);
-                    M[cb] = m_new;
-                    total[cb] = fmaf(__builtin_bit_cast(float, uint32_t(st[cb][1])), f, total[cb] * f_old);
-#pragma unroll
-                    for (int nb = 0; nb < NB; ++nb) {
-                        const f32x4_t v = __builtin_bit_cast(f32x4_t, o[cb][nb]);
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) sum[cb][nb][j] = fmaf(v[j], f, sum[cb][nb][j] * f_old);
-                    }
-                }
-            };
-            request(0, part[0], ml[0]);
-            for (int i = 0; i < pieces; i += 2) {
-                request(i + 1, part[1], ml[1]);
-                asm volatile("" ::: "memory");   // (the compiler would move the loads to where they are used)
-                add(part[0], ml[0]);
-                if (i + 1 < pieces) {
-                    request(i + 2, part[0], ml[0]);
-                    asm volatile("" ::: "memory");
-                    add(part[1], ml[1]);
-                }
-            }
-#pragma unroll
-            for (int cb = 0; cb < CB; ++cb) {
-                Lsum[cb] = total[cb];
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb) O[cb][nb] = sum[cb][nb];
-            }
+            return;
         }
     }
 
@@ -765,18 +686,84 @@ attn_prefill_tiled_kernel(const PrefillParams p, const std::conditional_t<SPLIT,
     }
 }
 
-// Pieces of a split launch: a table of (block, piece, pieces, first slot), longest blocks first.
+// Adds up the pieces of the blocks that were cut, in their order.  A workgroup has one block's four 16-dim groups of one column
+// block, a thread the columns and dims that the same thread of the pieces had.  Bound by latency: the reads of four pieces are in
+// flight together.  (Having the piece that finishes last do it inside the launch was 1 to 2 us faster and is not in the tree:
+// the first results in newly allocated memory were wrong now and then.)
+template <int HD, int CB, int NW>
+__global__ void __launch_bounds__(NW * kWaveSize)
+attn_prefill_merge_kernel(const PrefillParams p, const PrefillItems items) {
+    constexpr int NB = HD / 16, NT = NW * kWaveSize, G = 4;
+    const int tid = threadIdx.x, lane = tid & (kWaveSize - 1), wave = tid / kWaveSize, fn = lane & 15, fg = lane >> 4;
+    const int heads = p.B * p.KVH;
+    const int bh = int(blockIdx.x) % heads, kvh = bh % p.KVH, b = bh / p.KVH;
+    const uint32_t item = items.item[blockIdx.x / heads];
+    const int wg = int(item & 0x1ff), first_slot = int(item >> 9) & 0x1ff, pieces = int(item >> 25);
+    const int cb = int(blockIdx.y) / (NB / 4), nb0 = int(blockIdx.y) % (NB / 4) * 4;
+    const char* const slots = items.part + (int64_t(bh) * items.slots_per_head + first_slot) * prefill_slot_bytes(HD, CB);
+
+    f32x4_t sum[4];
+    float total = 0.f, M = 0.99f * kMaskedScore;   // (what a piece starts from)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sum[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < pieces; s0 += G) {
+        f32x4_t o[G][4];
+        float2 ml[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const char* const slot = slots + int64_t(min(s0 + g, pieces - 1)) * prefill_slot_bytes(HD, CB);
+            ml[g] = *reinterpret_cast<const float2*>(slot + CB * NB * NT * 16 + (cb * NT + tid) * 8);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[g][i] = *reinterpret_cast<const f32x4_t*>(slot + ((cb * NB + nb0 + i) * NT + tid) * 16);
+        }
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            if (s0 + g < pieces) {
+                const float m_new = maximum(M, ml[g].x);
+                const float f_old = fast_exp2((M - m_new) * p.scale_log2e), f = fast_exp2((ml[g].x - m_new) * p.scale_log2e);
+                M = m_new;
+                total = fmaf(ml[g].y, f, total * f_old);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) sum[i][j] = fmaf(o[g][i][j], f, sum[i][j] * f_old);
+                }
+            }
+        }
+    }
+    const int R = p.QH / p.KVH, ppw = 16 / R;
+    const int qi = (wg * NW * CB + wave * CB + cb) * ppw + fn / R, qh = kvh * R + fn % R;
+    if (fn >= ppw * R || qi >= p.T) return;
+    const float inv = 1.0f / total;
+    uint16_t* const orow = p.out + b * p.o_sb + int64_t(qh) * p.o_sh + int64_t(qi) * p.o_st + fg * 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint2 w;
+        w.x = pack_bf16x2(sum[i][0] * inv, sum[i][1] * inv);
+        w.y = pack_bf16x2(sum[i][2] * inv, sum[i][3] * inv);
+        *reinterpret_cast<uint2*>(orow + (nb0 + i) * 16) = w;
+    }
+}
+
+// A launch cut into pieces and the one that adds them up.  Both get a table, longest blocks first: the pieces, or the blocks cut.
 template <int HD, int CB, int NW, int TK, int WPE>
-int launch_pieces(const PrefillParams& p, const PrefillSplitPlan& plan, void* part, unsigned* counters, hipStream_t stream) {
+int launch_pieces(const PrefillParams& p, const PrefillSplitPlan& plan, void* part, hipStream_t stream) {
     static_assert(prefill_slot_bytes(HD, CB) == (CB * HD + CB * 8) * NW * kWaveSize, "slots");
     PrefillItems items;
     items.part = static_cast<char*>(part);
-    items.counters = counters;
     const int n = prefill_items(plan, p.QH / p.KVH, p.T, p.S, &items);
-    const dim3 grid(unsigned(p.B) * unsigned(p.KVH) * unsigned(n));
+    const unsigned heads = unsigned(p.B) * unsigned(p.KVH);
     PrefillParams q = p;
     q.snake = 0;
-    return enqueue(attn_prefill_tiled_kernel<HD, CB, NW, TK, WPE, false, true>, grid, dim3(NW * kWaveSize), 0, stream, q, items);
+    if (int rc = enqueue(attn_prefill_tiled_kernel<HD, CB, NW, TK, WPE, false, true>, dim3(heads * unsigned(n)), dim3(NW * kWaveSize), 0,
+                         stream, q, items); rc != 0)
+        return rc;
+    int cut = 0;
+    for (int i = 0; i < n; ++i) {
+        const uint32_t item = items.item[i];
+        if ((item >> 25) > 1 && ((item >> 18) & 0x7f) == 0) items.item[cut++] = item;
+    }
+    return enqueue(attn_prefill_merge_kernel<HD, CB, NW>, dim3(heads * unsigned(cut), CB * HD / 64), dim3(NW * kWaveSize), 0, stream, q, items);
 }
 
 template <class Kernel>
@@ -815,16 +802,20 @@ int prefill_items(const PrefillSplitPlan& plan, int R, int T, int S, PrefillItem
 
 // Which calls are cut.  A short piece of a prompt behind many cached tokens has few blocks, each with a long range: 64
 // queries behind 4032 tokens are 32 workgroups of 64 tiles.  Cut into pieces of n per block they fill the device; what
-// that costs is the partial results (18 to 66 KB each, written and read past the caches) and the merge, a chain of n reads.
-// Measured (us, uncut / cut; 32 query heads over 8, one sequence): 8 queries of 4096 tokens 54.9 / 10.3, 64 of 4096
-// 37.9 / 11.5, 512 of 7012 64.1 / 43.1, head size 128 105.8 / 66.4.  The lines, from a sweep over B 1 ... 16, R 3, 4, 8:
+// that costs is the partial results (18 to 66 KB each, written and read) and a second launch.
+// Measured (us, uncut / cut; 32 query heads over 8, one sequence): 8 queries of 4096 tokens 54.9 / 12.6, 64 of 4096
+// 37.9 / 14.9, 512 of 7012 64.1 / 46.9, head size 128 105.8 / 67.2.  The lines, from a sweep over B 1 ... 16, R 3, 4, 8:
 //   * n: at most two pieces per compute unit (a 513th starts when a first has ended: 23.6 -> 29 us for 200 of 3200 at head
-//     size 128), pieces of at least 3/4 sqrt(tiles) tiles (8 of 3008: 4 tiles 9.4, 8 tiles 10.5, 1 tile 12 us);
+//     size 128), pieces of at least 3/4 sqrt(tiles) tiles (8 of 3008: 4 tiles 9.4, 8 tiles 10.5, 1 tile 12 us before the merge
+//     was a launch of its own);
 //   * one column block per wavefront while its blocks do not fill the device (64 of 4096: 11.5 against 14 us), two beyond
 //     and for the longest ranges (512 of 7012 at head size 128: 66 against 80 us);
-//   * below 12 tiles, or where the blocks alone occupy the device, the merge costs what the balance gives (64 of 314: 6.6
-//     uncut, 7.0; 512 x 16 sequences of 572: 37.5, 40.7); the same holds for prompts without a past, whose longest blocks end a
-//     launch that has kept the device busy (2 x 1531: 29.5 uncut, 29.0 ... 36 by the cut; 2048: 27.2, 30.0).
+//   * below 12 tiles (64 of 314: 6.6 uncut, 9) or where the blocks alone occupy the device the second launch costs what the
+//     balance gives; at head size 64, whose tiles are half the work, the more blocks the more tiles it takes (200 of 800 and 512 of
+//     1512: 11 / 11.3 and 17.8 / 17.7; 64 heads, 200 of 1200: 14.7 / 15.8; 200 of 1200: 14.4 / 12.8), except for the few queries
+//     that would run as single wavefronts (16 sequences, 8 of 1008: 16.4 / 13.6);
+//   * not prompts without a past, whose longest blocks end a launch that has kept the device busy (2 x 1531, with the merge in
+//     the launch: 29.5 uncut, 29.0 ... 36 by the cut; 2048: 27.2, 30.0).
 PrefillSplitPlan prefill_split_plan(int B, int QH, int KVH, int T, int S, int HD, int num_cus) {
     const PrefillSplitPlan none{0, 0, 0};
     const int R = QH / KVH;
@@ -832,14 +823,15 @@ PrefillSplitPlan prefill_split_plan(int B, int QH, int KVH, int T, int S, int HD
     if (S / 2 < T || tiles < 12) return none;
     auto blocks = [&](int col_blocks) { const int pos = kPrefillTiledWaves * col_blocks * (16 / R); return (T + pos - 1) / pos; };
     const int64_t heads = int64_t(B) * KVH, one = heads * blocks(1), two = heads * blocks(2), cus = num_cus;
+    if (HD == 64 && T * R > 64 && tiles * cus < 12 * cus + 14 * one) return none;
     PrefillSplitPlan plan = none;
     int64_t room = 2 * cus;
     if (10 * one <= 9 * cus || (one <= cus && tiles >= 24)) {
         plan.col_blocks = (tiles >= 64 && 2 * one > cus) ? 2 : 1;
-    } else if (two <= cus && tiles >= 40) {
+    } else if (two <= cus && tiles >= (HD == 128 ? 40 : 64)) {
         plan.col_blocks = 2;
     } else if (5 * two <= 8 * cus && tiles >= (HD == 128 ? 64 : 100)) {
-        plan.col_blocks = 2;   // (1500 of 8000: at head size 128 258 / 193 us, at 64 123 / 110: units with one block and with two)
+        plan.col_blocks = 2;   // (1500 of 8000: at head size 128 258 / 196 us: units with one block and with two)
         room = 5 * cus;
     } else {
         return none;
@@ -854,18 +846,17 @@ PrefillSplitPlan prefill_split_plan(int B, int QH, int KVH, int T, int S, int HD
     PrefillItems items;
     if (prefill_items(plan, R, T, S, &items) < 0 || items.slots_per_head == 0) return none;
     plan.slots = heads * items.slots_per_head;
-    return plan.slots <= kPrefillMaxSlots ? plan : none;
+    return plan;
 }
 
-int launch_attn_prefill_split(const PrefillParams& p, int HD, const PrefillSplitPlan& plan, void* part, unsigned* counters,
-                              hipStream_t stream) {
+int launch_attn_prefill_split(const PrefillParams& p, int HD, const PrefillSplitPlan& plan, void* part, hipStream_t stream) {
     constexpr int NW = kPrefillTiledWaves;
     if (HD == 64) {
-        if (plan.col_blocks == 1) return launch_pieces<64, 1, NW, 64, 4>(p, plan, part, counters, stream);
-        return launch_pieces<64, 2, NW, 64, 4>(p, plan, part, counters, stream);
+        if (plan.col_blocks == 1) return launch_pieces<64, 1, NW, 64, 4>(p, plan, part, stream);
+        return launch_pieces<64, 2, NW, 64, 4>(p, plan, part, stream);
     }
-    if (plan.col_blocks == 1) return launch_pieces<128, 1, NW, 64, 2>(p, plan, part, counters, stream);
-    return launch_pieces<128, 2, NW, 64, 2>(p, plan, part, counters, stream);
+    if (plan.col_blocks == 1) return launch_pieces<128, 1, NW, 64, 2>(p, plan, part, stream);
+    return launch_pieces<128, 2, NW, 64, 2>(p, plan, part, stream);
 }
 
 int launch_attn_prefill_tiled(const PrefillParams& p, int HD, hipStream_t stream) {

@@ -556,18 +556,18 @@ int l3_attn_decode_devlen(const void* q, const void* k, const void* v, void* out
 size_t l3_attn_prefill_workspace_bytes(int B, int QH, int KVH, int T, int S, int HD, int flags) {
     if (check_attn_shape(B, QH, KVH, S, HD) != L3_OK || !attn_flags_ok(flags) || T <= 0 || T > S) return 0;
     const PrefillSplitPlan plan = prefill_plan_of(B, QH, KVH, T, S, HD, flags);
-    return plan.max_tiles > 0 ? L3_ATTN_COUNTER_BYTES + size_t(plan.slots) * prefill_slot_bytes(HD, plan.col_blocks) : 0;
+    return plan.max_tiles > 0 ? size_t(plan.slots) * prefill_slot_bytes(HD, plan.col_blocks) : 0;
 }
 
 int l3_attn_prefill(const void* q, const void* k, const void* v, void* out, int B, int QH, int KVH, int T, int S,
                     int HD, const int64_t q_strides[3], const int64_t k_strides[3], const int64_t v_strides[3],
                     const int64_t out_strides[3], float scale, int flags, void* stream) {
-    return l3_attn_prefill_ws(q, k, v, out, nullptr, 0, nullptr, B, QH, KVH, T, S, HD, q_strides, k_strides, v_strides,
+    return l3_attn_prefill_ws(q, k, v, out, nullptr, 0, B, QH, KVH, T, S, HD, q_strides, k_strides, v_strides,
                               out_strides, scale, flags, stream);
 }
 
 int l3_attn_prefill_ws(const void* q, const void* k, const void* v, void* out, void* workspace, size_t workspace_bytes,
-                       void* counters, int B, int QH, int KVH, int T, int S, int HD, const int64_t q_strides[3],
+                       int B, int QH, int KVH, int T, int S, int HD, const int64_t q_strides[3],
                        const int64_t k_strides[3], const int64_t v_strides[3], const int64_t out_strides[3], float scale,
                        int flags, void* stream) {
     if (!q || !k || !v || !out || !q_strides || !k_strides || !v_strides || !out_strides)
@@ -605,15 +605,9 @@ int l3_attn_prefill_ws(const void* q, const void* k, const void* v, void* out, v
     if (workspace) {
         const PrefillSplitPlan plan = prefill_plan_of(B, QH, KVH, T, S, HD, flags);
         if (plan.max_tiles > 0) {
-            if (workspace_bytes < L3_ATTN_COUNTER_BYTES + size_t(plan.slots) * prefill_slot_bytes(HD, plan.col_blocks))
-                return L3_ERR_WORKSPACE;
-            if (!aligned(workspace, kWorkspaceAlign) || !aligned(counters, kWorkspaceAlign)) return L3_ERR_ALIGNMENT;
-            unsigned* arrivals = static_cast<unsigned*>(counters);
-            if (!arrivals) {
-                arrivals = static_cast<unsigned*>(workspace);
-                if (launch_fill_zero_u32(arrivals, L3_ATTN_COUNTER_BYTES / sizeof(unsigned), st) != 0) return L3_ERR_HIP;
-            }
-            const int rc = launch_attn_prefill_split(p, HD, plan, static_cast<char*>(workspace) + L3_ATTN_COUNTER_BYTES, arrivals, st);
+            if (workspace_bytes < size_t(plan.slots) * prefill_slot_bytes(HD, plan.col_blocks)) return L3_ERR_WORKSPACE;
+            if (!aligned(workspace, kWorkspaceAlign)) return L3_ERR_ALIGNMENT;
+            const int rc = launch_attn_prefill_split(p, HD, plan, workspace, st);
             return rc == 0 ? L3_OK : L3_ERR_HIP;
         }
     }

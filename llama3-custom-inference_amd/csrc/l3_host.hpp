@@ -111,8 +111,6 @@ struct PrefillParams {
 constexpr int kPrefillMaxItems = 512;        // pieces of a (batch, kv head); their table rides in the kernel arguments
 constexpr int kPrefillMaxPieces = 127;       // of a block
 constexpr int kPrefillSplitTile = 64;        // tokens per tile
-constexpr int kPrefillCounterStride = 8;     // words from one block's arrival counter to the next
-constexpr int64_t kPrefillMaxSlots = 2 * (L3_ATTN_COUNTER_BYTES / 4 / kPrefillCounterStride - 4);   // (two slots a counter at least; the last words are a diagnostic)
 struct PrefillSplitPlan {
     int col_blocks;   // 16-column blocks per wavefront
     int max_tiles;    // tiles of a piece at most; 0: the launch is not cut
@@ -120,7 +118,6 @@ struct PrefillSplitPlan {
 };
 struct PrefillItems {
     char* part;            // slots, each what a workgroup holds in registers
-    unsigned* counters;
     int slots_per_head;
     uint32_t item[kPrefillMaxItems];   // block (9 bits), its first slot (9), piece (7), pieces (7)
 };
@@ -129,8 +126,7 @@ constexpr int prefill_slot_bytes(int HD, int col_blocks) { return col_blocks * (
 // Fills in the table (if given) and its slots; the number of items, or -1 where the table is too small.
 int prefill_items(const PrefillSplitPlan& plan, int R, int T, int S, PrefillItems* items);
 PrefillSplitPlan prefill_split_plan(int B, int QH, int KVH, int T, int S, int HD, int num_cus);
-int launch_attn_prefill_split(const PrefillParams& p, int HD, const PrefillSplitPlan& plan, void* part, unsigned* counters,
-                              hipStream_t stream);
+int launch_attn_prefill_split(const PrefillParams& p, int HD, const PrefillSplitPlan& plan, void* part, hipStream_t stream);
 
 struct LinearParams {
     const uint16_t* x;    // (M, K) activations, row stride x_stride

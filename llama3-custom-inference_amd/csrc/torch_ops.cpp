@@ -196,12 +196,6 @@ void* grown(Workspace& w, const Tensor& like, size_t nbytes) {
     return ptr(w.memory);
 }
 
-bool capturing(const OnDevice& on) {
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    TORCH_CHECK(hipStreamIsCapturing(on.stream, &capture) == hipSuccess, "hipStreamIsCapturing failed");
-    return capture != hipStreamCaptureStatusNone;
-}
-
 struct DecodeShape {
     int B, QH, KVH, S, HD;
 };
@@ -230,14 +224,16 @@ void decode(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& out
     // Outside stream capture the workspace is the one kept for the stream.  Preparing a new one synchronises,
     // which a capture does not allow, so a call under capture takes a plain buffer from the graph's memory pool
     // and runs split kernel + combine.
-    const bool recorded = capturing(on);
-    flags = recorded ? flags & ~L3_ATTN_FLAG_WS_COUNTERS : flags | L3_ATTN_FLAG_WS_COUNTERS;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    TORCH_CHECK(hipStreamIsCapturing(on.stream, &capture) == hipSuccess, "hipStreamIsCapturing failed");
+    const bool capturing = capture != hipStreamCaptureStatusNone;
+    flags = capturing ? flags & ~L3_ATTN_FLAG_WS_COUNTERS : flags | L3_ATTN_FLAG_WS_COUNTERS;
     const size_t nbytes = lib.l3_attn_decode_workspace_bytes(s.B, s.QH, s.KVH, s.S, s.HD, num_splits, flags);
     TensorBase own;
     void* ws = nullptr;
     std::shared_ptr<Workspace> kept;
     std::unique_lock<std::mutex> in_use;
-    if (nbytes > 0 && recorded) {
+    if (nbytes > 0 && capturing) {
         own = at::detail::empty_cuda({int64_t(std::max(nbytes, size_t(256)))}, at::kByte, q.device(), std::nullopt);
         ws = ptr(own);
     } else if (nbytes > 0) {
@@ -317,21 +313,11 @@ PyObject* flash_attention_prefill(PyObject* const* a) {
         Tensor out(at::detail::empty_strided_cuda(sizes, strides, at::kBFloat16, q.device()));
         if (out.numel() > 0) {
             const OnDevice on(q);
-            // Partial results live for the call; the arrival counters are the stream's, under capture the call's own.
+            // partial results live for the call
             const size_t nbytes = lib.l3_attn_prefill_workspace_bytes(int(B), int(QH), int(KVH), int(T), int(S), int(HD), flags);
             TensorBase part;
-            std::shared_ptr<Workspace> kept;
-            std::unique_lock<std::mutex> in_use;
-            void* counters = nullptr;
-            if (nbytes > 0) {
-                part = at::detail::empty_cuda({int64_t(nbytes)}, at::kByte, q.device(), std::nullopt);
-                if (!capturing(on)) {
-                    kept = attention_workspace(on);
-                    in_use = std::unique_lock<std::mutex>(kept->in_use);
-                    counters = grown(*kept, q, L3_ATTN_COUNTER_BYTES);
-                }
-            }
-            const int rc = lib.l3_attn_prefill_ws(ptr(q), ptr(k), ptr(v), ptr(out), nbytes > 0 ? ptr(part) : nullptr, nbytes, counters,
+            if (nbytes > 0) part = at::detail::empty_cuda({int64_t(nbytes)}, at::kByte, q.device(), std::nullopt);
+            const int rc = lib.l3_attn_prefill_ws(ptr(q), ptr(k), ptr(v), ptr(out), nbytes > 0 ? ptr(part) : nullptr, nbytes,
                                                   int(B), int(QH), int(KVH), int(T), int(S), int(HD), q.strides().data(),
                                                   k.strides().data(), v.strides().data(), strides,
                                                   float(1.0 / std::sqrt(double(HD))), flags, on.stream);

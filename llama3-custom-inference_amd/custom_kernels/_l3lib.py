@@ -91,7 +91,7 @@ SIGNATURES = {
     "l3_attn_prefill_ws": (
         ctypes.c_int,
         [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,                     # q k v out
-         ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p,                                      # workspace bytes counters
+         ctypes.c_void_p, ctypes.c_size_t,                                                       # workspace bytes
          ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,    # B QH KVH T S HD
          _c_i64p, _c_i64p, _c_i64p, _c_i64p, ctypes.c_float, ctypes.c_int, ctypes.c_void_p],
     ),
