@@ -180,7 +180,8 @@ bool attn_merge_in_launch_wanted(int flags) {
 //     size 128: 82.9 / 87.1).
 //   * Up to four heads per unit short sequences only (896 heads, 400 tokens: head size 64 20.6 / 18.7, 128 36.6 / 32.0; 1024
 //     heads, 512 tokens: 24.3 / 25.3 and 45.1 / 46.1).
-//   * At head size 128 a single tile of 640 heads is better streamed (4.9 / 6.0), two tiles of 896 as well (8.4 / 9.0).
+//   * At head size 128 a single tile of 640 heads is better streamed (4.9 / 6.0), two of 896 and three of
+//     792 as well (8.4 / 9.0, 9.6 / 9.9).
 int four_wave_tiles_max(int64_t units, int HD, int64_t cus) {
     if (4 * units <= 5 * cus) return HD == 64 ? 8 : 12;
     if (4 * units <= 7 * cus) return HD == 64 ? 13 : 32;
@@ -190,7 +191,7 @@ int four_wave_tiles_max(int64_t units, int HD, int64_t cus) {
 }
 int four_wave_tiles_min(int64_t units, int HD, int64_t cus) {
     if (HD == 64 || units <= 2 * cus) return 1;
-    return units <= 3 * cus ? 2 : 3;
+    return units <= 3 * cus ? 2 : 4;
 }
 
 AttnPlan attn_make_plan(int B, int KVH, int S, int HD, int requested, int num_cus, int impl, int form,
@@ -276,9 +277,10 @@ AttnPlan attn_make_plan(int B, int KVH, int S, int HD, int requested, int num_cu
             // K + V bytes a workgroup streams when there is a single group
             const int64_t stream_bytes = int64_t(kMfmaWaves) * ((S + spg - 1) / spg) * HD * 4;
             const bool short_stream = stream_bytes <= (int64_t(3) << 20);
-            if (short_stream && spg == 1 && (wgs_per_split_group * 2 >= num_cus || (wgs_per_split_group * 4 >= num_cus && tiles <= 2))) {
+            if (short_stream && spg == 1 && (wgs_per_split_group * 2 >= num_cus || (wgs_per_split_group * 4 >= num_cus && tiles <= 4))) {
                 // half of the units busy, but no partials and no second launch (with a quarter of them busy only the
-                // shortest: 64 sequences of 1300 tokens at head size 64 took 53.9 us in one group, 29.6 in three)
+                // shortest: 99 sequences of 81 tokens at head size 128 take 9.7 us in one group, 11.5 in two; 64 of 1300 tokens at head
+                // size 64 53.9 in one, 29.6 in three)
                 groups = 1;
             } else if (groups == 1 && (!short_stream || spg == 1) && int64_t(num_cus) / wgs_per_split_group >= 2) {
                 groups = 2;
