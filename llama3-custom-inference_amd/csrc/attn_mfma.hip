@@ -31,19 +31,24 @@ namespace {
 // LOADS = 4 (head size 64, cooperative form, at most 512 tokens): half-size tiles of 32 tokens, so
 // that a short sequence still gives every wavefront a tile, and slabs small enough for two
 // workgroups per CU.
-// NW = 4 (cooperative form, one split, more heads than compute units): half the wavefronts and half the LDS, so that two
-// or three workgroups are resident where one of eight wavefronts was, and a launch of up to three heads per unit needs
-// no second round.  us, eight wavefronts or streaming / this: 64 sequences x 8 heads at head size 128, 16 tokens 6.8 / 4.1, 200
-// tokens 13.1 / 10.7; 80 sequences at head size 64, 200 tokens 11.9 / 8.6, 800 tokens 34.8 / 26.8.
+// NW = 4 (cooperative form, one split, more heads than compute units): half the wavefronts and half the slabs, so that two
+// workgroups are resident where one of eight wavefronts was (registers allow no third: 178 and 192; head size 64 up to 512
+// tokens, 111: four).  A wavefront does the work of two, one after the other, with the softmax states of two, and the eight
+// states are merged as eight wavefronts' are: a sequence has the same bits in a batch of 32 and of 64.  (One state for all tiles of a
+// wavefront took 0.3 to 0.8 us less where a wavefront has several: 64 x 8 heads at head size 128, 200 tokens 11.1 us, at head
+// size 64, 512 tokens 14.7; but a batch's results then hung on its size.)  us, eight wavefronts or streaming / this: 64
+// sequences x 8 heads at head size 128, 16 tokens 6.8 / 4.1, 200 tokens 13.4 / 11.7; at head size 64, 256 tokens 8.8 / 8.6, 512
+// tokens 16.0 / 16.4; 80 sequences at head size 64, 200 tokens 13.5 / 9.3, 400 tokens 22.5 / 15.4.
 template <int HD, bool COOP, int LOADS = 8, int NW = kMfmaWaves>
 __global__ void __launch_bounds__(NW * kWaveSize, 2)
 attn_splitkv_mfma_kernel(const int R, const int hpw_log2, const AttnParams p) {
     using T = MfmaTile<HD, LOADS>;
     constexpr int WT = T::WT, KC = T::KC, NB = T::NB, SLAB = T::SLAB;
-    constexpr int STEP = COOP ? NW * WT : WT;  // token stride between a wavefront's tiles
+    constexpr int STEP = COOP ? kMfmaWaves * WT : WT;  // token stride between a state's tiles
+    constexpr bool TWO = COOP && NW < kMfmaWaves;      // a wavefront has the tiles and the states of two
     static_assert(LOADS != 8 || WT == attn_tile_tokens(HD, kAttnImplMfma), "host plan and kernel tile disagree");
     static_assert(LOADS == 8 || COOP, "the split plan counts full tiles");
-    static_assert(NW == kMfmaWaves || COOP, "the streaming form lays eight wavefronts over heads and splits");
+    static_assert(NW == kMfmaWaves || (COOP && 2 * NW == kMfmaWaves), "eight wavefronts, or four with two states each");
 
     __shared__ __align__(16) unsigned char s_slab[NW][SLAB];
 
@@ -94,36 +99,59 @@ attn_splitkv_mfma_kernel(const int R, const int hpw_log2, const AttnParams p) {
     for (int nb = 0; nb < NB; ++nb) O[nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     float m_run = kMaskedScore;  // running maximum of the raw scores (common to the four k groups of a head)
     float l_part = 0.f;          // this lane's share of the softmax denominator
-    // Cooperative workgroups take their tiles in an order rotated by the split index: the splits of a head
-    // start a power of two apart (1 MiB at 16384 tokens in 32 splits), and 32 workgroups that walk such
-    // ranges in step keep hitting the same memory channels (16384 tokens: 16.3 -> 14.9 us at head size 128,
-    // 12.2 -> 10.0 us at 64).  The streaming form, whose split counts are not powers of two, gains nothing.
-    mfma_tile_loop<HD, LOADS, true, COOP>(p.k, p.v, k_head, v_head, p.k_st, p.v_st, s_slab[wave], qfrag,
-                                          t_begin + (COOP ? wave * WT : 0), t_end, STEP, t_end, t_end, c, O, m_run, l_part,
-                                          t_begin, split);
-
-    // ---- this wavefront's result.  O[nb][r] is dim 16*nb + 4*fg + r of head fn; the softmax
-    //      denominator is still spread over the four k groups.
-    l_part += __shfl_xor(l_part, 16, kWaveSize);
-    l_part += __shfl_xor(l_part, 32, kWaveSize);
-    const float m_log2 = (m_run == kMaskedScore) ? kMaskedScore : m_run * c;  // a COOP wave may have had no tile
-
+    // ---- a state.  O[nb][r] is dim 16*nb + 4*fg + r of head fn; the softmax denominator is still spread over the four k groups.
+    float m_log2;
+    auto finish = [&]() {
+        l_part += __shfl_xor(l_part, 16, kWaveSize);
+        l_part += __shfl_xor(l_part, 32, kWaveSize);
+        m_log2 = (m_run == kMaskedScore) ? kMaskedScore : m_run * c;  // a COOP wave may have had no tile
+    };
     if constexpr (COOP) {
-        // merge the wavefronts through LDS, then write like the streaming form
-        __shared__ float s_m[NW][kAttnMaxRatio];
-        __shared__ float s_l[NW][kAttnMaxRatio];
-        __shared__ __align__(16) float s_o[NW][kAttnMaxRatio][HD];
+        // merge the states through LDS, then write like the streaming form
+        __shared__ float s_m[kMfmaWaves][kAttnMaxRatio];
+        __shared__ float s_l[kMfmaWaves][kAttnMaxRatio];
+        __shared__ __align__(16) float s_o[kMfmaWaves][kAttnMaxRatio][HD];
         __shared__ int s_last;
-        if (fn < R) {
+        auto leave = [&](int state) {
+            finish();
+            if (fn < R) {
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-                *reinterpret_cast<float4*>(&s_o[wave][fn][nb * 16 + fg * 4]) =
-                    make_float4(O[nb][0], O[nb][1], O[nb][2], O[nb][3]);
+                for (int nb = 0; nb < NB; ++nb) {
+                    *reinterpret_cast<float4*>(&s_o[state][fn][nb * 16 + fg * 4]) =
+                        make_float4(O[nb][0], O[nb][1], O[nb][2], O[nb][3]);
+                }
+                if (fg == 0) {
+                    s_m[state][fn] = m_log2;
+                    s_l[state][fn] = l_part;
+                }
             }
-            if (fg == 0) {
-                s_m[wave][fn] = m_log2;
-                s_l[wave][fn] = l_part;
-            }
+        };
+        bool second = true;   // the states from the fourth on are there (otherwise they are empty, which adds nothing)
+        if constexpr (TWO) {
+            second = t_begin + NW * WT < t_end;   // workgroup-uniform
+            int state = wave;
+            auto next_state = [&]() {
+                leave(state);
+                state += NW;
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) O[nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+                m_run = kMaskedScore;
+                l_part = 0.f;
+            };
+            mfma_tile_loop<HD, LOADS, true, false, true>(p.k, p.v, k_head, v_head, p.k_st, p.v_st, s_slab[wave], qfrag,
+                                                         t_begin + wave * WT, t_end, STEP, t_end, t_end, c, O, m_run, l_part,
+                                                         0, 0, next_state);
+            if (second && state == wave) next_state();   // wave-uniform: this one's second state is empty
+            leave(state);
+        } else {
+            // The tiles are taken in an order rotated by the split index: the splits of a head
+            // start a power of two apart (1 MiB at 16384 tokens in 32 splits), and 32 workgroups that walk such
+            // ranges in step keep hitting the same memory channels (16384 tokens: 16.3 -> 14.9 us at head size 128,
+            // 12.2 -> 10.0 us at 64).  The streaming form, whose split counts are not powers of two, gains nothing.
+            mfma_tile_loop<HD, LOADS, true, true>(p.k, p.v, k_head, v_head, p.k_st, p.v_st, s_slab[wave], qfrag,
+                                                  t_begin + wave * WT, t_end, STEP, t_end, t_end, c, O, m_run, l_part,
+                                                  t_begin, split);
+            leave(wave);
         }
         __syncthreads();
         for (int idx = threadIdx.x; idx < R * (HD / 2); idx += NW * kWaveSize) {
@@ -132,13 +160,22 @@ attn_splitkv_mfma_kernel(const int R, const int hpw_log2, const AttnParams p) {
             float M = s_m[0][h];
 #pragma unroll
             for (int w = 1; w < NW; ++w) M = fmaxf(M, s_m[w][h]);
-            float L = 0.f, o0 = 0.f, o1 = 0.f;
+            if (TWO && second) {
 #pragma unroll
-            for (int w = 0; w < NW; ++w) {
-                const float e = fast_exp2(s_m[w][h] - M);  // wavefronts without a tile: 0
+                for (int w = NW; w < kMfmaWaves; ++w) M = fmaxf(M, s_m[w][h]);
+            }
+            float L = 0.f, o0 = 0.f, o1 = 0.f;
+            auto add = [&](int w) {
+                const float e = fast_exp2(s_m[w][h] - M);  // states without a tile: 0
                 L = fmaf(s_l[w][h], e, L);
                 o0 = fmaf(s_o[w][h][d], e, o0);
                 o1 = fmaf(s_o[w][h][d + 1], e, o1);
+            };
+#pragma unroll
+            for (int w = 0; w < NW; ++w) add(w);
+            if (TWO && second) {
+#pragma unroll
+                for (int w = NW; w < kMfmaWaves; ++w) add(w);
             }
             const int qh = kvh * R + h;
             if (p.part_o == nullptr) {
@@ -178,7 +215,11 @@ attn_splitkv_mfma_kernel(const int R, const int hpw_log2, const AttnParams p) {
                 else if (wave < R) merge(std::integral_constant<int, 1>{});   // R = 3
             }
         }
-    } else if (fn < R) {
+    } else {
+        mfma_tile_loop<HD, LOADS, true>(p.k, p.v, k_head, v_head, p.k_st, p.v_st, s_slab[wave], qfrag, t_begin, t_end, STEP,
+                                        t_end, t_end, c, O, m_run, l_part);
+        finish();
+        if (fn >= R) return;
         const int qh = kvh * R + fn;
         if (p.part_o == nullptr) {  // single split: the final output row
             const float inv = 1.0f / l_part;
@@ -268,7 +309,7 @@ int launch_attn_splitkv_mfma(const AttnParams& params, int HD, int R, bool coop,
             if (p.num_splits == 1 && int64_t(p.B) * p.KVH > current_device_cus()) {
                 constexpr int NW = 4;
                 const dim3 four(NW * kWaveSize);
-                if (HD == 64 && p.tokens_per_split <= 2 * NW * 32) {
+                if (HD == 64 && p.tokens_per_split <= 2 * kMfmaWaves * 32) {
                     rc = enqueue(attn_splitkv_mfma_kernel<64, true, 4, NW>, grid, four, 0, stream, R, 0, p);
                 } else if (HD == 64) {
                     rc = enqueue(attn_splitkv_mfma_kernel<64, true, 8, NW>, grid, four, 0, stream, R, 0, p);

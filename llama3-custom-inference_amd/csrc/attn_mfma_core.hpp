@@ -112,14 +112,19 @@ __device__ __forceinline__ float column_max(float x) {
 // t_first = t_first0 + first tiles) and t_end, so that workgroups whose ranges start a power of two apart
 // do not all begin at addresses a power of two apart.  The order does not change the result beyond
 // float32 rounding: the softmax state is order-free.
-template <int HD, int LOADS = 8, bool STREAM = false, bool ROTATE = false>
+// TWO: behind these tiles come those from t_first + step / 2 on, in the same steps, with a state of their own: between the
+// two `next_state` puts the first state away and begins another.  (A wavefront that does the work of two, whose next loads are
+// in flight across the change.)
+struct OneState { __device__ void operator()() const {} };
+template <int HD, int LOADS = 8, bool STREAM = false, bool ROTATE = false, bool TWO = false, class NextState = OneState>
 __device__ __forceinline__ void mfma_tile_loop(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
                                                int64_t k_head, int64_t v_head, int64_t k_st, int64_t v_st,
                                                unsigned char* slab,
                                                const bf16x8_t (&qfrag)[MfmaTile<HD>::KC], int t_first, int t_end,
                                                int step, int col_limit, int col_limit_min, float c,
                                                f32x4_t (&O)[MfmaTile<HD>::NB], float& m_run, float& l_part,
-                                               int t_first0 = 0, int rot = 0) {
+                                               int t_first0 = 0, int rot = 0, NextState next_state = {}) {
+    static_assert(!(ROTATE && TWO), "the tiles of one range are rotated");
     using T = MfmaTile<HD, LOADS>;
     static_assert(T::WT % 32 == 0, "a tile is a whole number of 32-token steps of the second product");
     constexpr int LPR = T::LPR, G = T::G, U = T::U, WT = T::WT, NG = T::NG, KC = T::KC, NB = T::NB, KS = T::KS;
@@ -288,6 +293,24 @@ __device__ __forceinline__ void mfma_tile_loop(const uint16_t* __restrict__ k, c
             if (idx >= tiles) idx -= tiles;
             const int tn = t_first0 + idx * WT;
             tile(t0, tn, std::true_type{});
+            t0 = tn;
+        }
+        tile(t0, t0, std::false_type{});
+    } else if constexpr (TWO) {
+        int t0 = t_first;
+        bool first = true;
+        load_tile(kr, kh, k_pitch, krow, t0);
+        load_tile(vr, vh, v_pitch, vrow, t0);
+        while (true) {   // (all of this is scalar)
+            int tn = t0 + step;
+            const bool change = first && tn >= t_end;
+            if (change) tn = t_first + step / 2;
+            if (tn >= t_end) break;
+            tile(t0, tn, std::true_type{});
+            if (change) {
+                next_state();
+                first = false;
+            }
             t0 = tn;
         }
         tile(t0, t0, std::false_type{});

@@ -70,3 +70,36 @@ def test_length_on_the_device(gpu, length, HD):
     assert_attn_close(out[:2], ref, what=f"device length {length}", regression=False)
     assert bool(torch.isfinite(out.float()).all())
     np.testing.assert_array_equal(t2bits(out), t2bits(cke.flash_attention_decode_devlen(q.to(gpu), k.to(gpu), v.to(gpu), n)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("HD", [64, 128])
+@pytest.mark.parametrize("B,S", [(33, 16), (33, 129), (40, 200), (48, 257), (64, 1), (64, 31), (64, 33), (64, 100), (64, 225), (64, 256),
+                                 (64, 300), (64, 384), (64, 512)])
+def test_bits_do_not_hang_on_the_batch(gpu, B, S, HD):
+    """The sequences of a batch with more (batch, kv head) pairs than compute units have the bits that they have in batches
+    with fewer, whose workgroups have eight wavefronts: a batch generates what its halves generate."""
+    from custom_kernels import custom_kernels_extension as cke
+
+    KVH = 8
+    print(f"many heads, bits B={B} S={S} HD={HD}", flush=True)
+    q, k, v = make_qkv(B, 4 * KVH, KVH, S, HD, seed=93, cache_len=S + 7, device=gpu)
+    out = cke.flash_attention_decode(q, k, v)
+    half = (B + 1) // 2
+    parts = [cke.flash_attention_decode(q[i:i + half], k[i:i + half], v[i:i + half]) for i in range(0, B, half)]
+    assert splits(B, KVH, S, HD) == splits(half, KVH, S, HD) == 1 and B * KVH > CUS >= half * KVH > CUS // 2
+    np.testing.assert_array_equal(t2bits(out), np.concatenate([t2bits(p) for p in parts]))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("HD,cap", [(64, 256), (64, 512), (128, 256), (128, 512)])
+def test_recorded_steps_have_the_bits_of_the_eager_ones(gpu, HD, cap):
+    """A step that is planned for the whole cache and reads its length on the device, and one that is planned for its length."""
+    from custom_kernels import custom_kernels_extension as cke
+
+    q, k, v = make_qkv(64, 32, 8, cap, HD, seed=94, cache_len=cap, device=gpu)
+    for S in (1, 40, 130, 200, cap - 1, cap):
+        print(f"many heads, eager and recorded length {S} of {cap} HD={HD}", flush=True)
+        n = torch.tensor([S], dtype=torch.int32, device=gpu)
+        out = cke.flash_attention_decode_devlen(q, k, v, n)
+        np.testing.assert_array_equal(t2bits(out), t2bits(cke.flash_attention_decode(q, k[:, :, :S], v[:, :, :S])))
