@@ -821,6 +821,7 @@ PrefillSplitPlan prefill_split_plan(int B, int QH, int KVH, int T, int S, int HD
     const int R = QH / KVH;
     const int tiles = (S + kPrefillSplitTile - 1) / kPrefillSplitTile;
     if (S / 2 < T || tiles < 12) return none;
+    if (S > (1 << 30)) return none;   // (tiles x pieces, of which the kernel takes a piece's first tile, would not fit 32 bits)
     auto blocks = [&](int col_blocks) { const int pos = kPrefillTiledWaves * col_blocks * (16 / R); return (T + pos - 1) / pos; };
     const int64_t heads = int64_t(B) * KVH, one = heads * blocks(1), two = heads * blocks(2), cus = num_cus;
     if (HD == 64 && T * R > 64 && tiles * cus < 12 * cus + 14 * one) return none;

@@ -39,6 +39,10 @@ def test_which_calls_are_cut():
     for B, QH, KVH, T, S, HD in [(1, 32, 8, 8, 704, 64), (1, 32, 8, 512, 1000, 64), (2, 32, 8, 1531, 1531, 64), (64, 32, 8, 128, 128, 64),
                                  (16, 32, 8, 512, 1100, 128), (1, 32, 8, 8, 4096, 96), (1, 32, 8, 8, 7, 64)]:
         assert cut_bytes(B, QH, KVH, T, S, HD) == 0
+    # a range (of one token, read over and over through a zero stride, it fits) whose tiles x pieces overflow 32 bits
+    assert cut_bytes(1, 8, 1, 8, 1 << 30, 64) > 0 and 127 * ((1 << 30) // 64) < 2 ** 31
+    for S in ((1 << 30) + 1, 1_200_000_000, 2 ** 31 - 1):
+        assert cut_bytes(1, 8, 1, 8, S, 64) == 0
     from custom_kernels import _l3lib
 
     for flag in (_l3lib.L3_ATTN_FLAG_PREFILL_WAVE, _l3lib.L3_ATTN_FLAG_PREFILL_TILED):      # a forced form is never cut
