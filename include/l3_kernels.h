@@ -143,7 +143,7 @@ int l3_attn_decode(const void* q, const void* k, const void* v, void* out,
  * counters with which the split kernel itself merges the partials of a (batch, kv head) -- the workgroup
  * that finishes a head last does it, out of the L2 of the XCD all workgroups of that head were placed on --
  * so that no combine kernel is launched (the reference always launches two kernels: custom_kernels.cu:274-275).
- *   l3_attn_workspace_init  zeroes the counters on `stream` and, on the first call per device, runs a probe
+ *   l3_attn_workspace_init  zeroes the workspace on `stream` and, on the first call per device, runs a probe
  *       launch that confirms the placement rule the scheme rests on (the workgroups of a grid go to the 8
  *       XCDs in turn, so workgroups whose ids agree modulo 8 share an XCD) and WAITS for it: call it at set-up, outside stream capture.  workspace: 256-byte aligned, at least
  *       L3_ATTN_COUNTER_BYTES.  Every later l3_attn_decode / l3_attn_decode_devlen call on that workspace must

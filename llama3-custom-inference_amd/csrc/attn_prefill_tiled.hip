@@ -688,8 +688,8 @@ attn_prefill_tiled_kernel(const PrefillParams p, const std::conditional_t<SPLIT,
 
 // Adds up the pieces of the blocks that were cut, in their order.  A workgroup has one block's four 16-dim groups of one column
 // block, a thread the columns and dims that the same thread of the pieces had.  Bound by latency: the reads of four pieces are in
-// flight together.  (Having the piece that finishes last do it inside the launch was 1 to 2 us faster and is not in the tree:
-// the first results in newly allocated memory were wrong now and then.)
+// flight together.  (Having the piece that finishes last do it inside the launch was 1 to 2 us faster and is not in the tree: a
+// split-K linear with the same hand-over, stores and loads at device scope, had wrong first results in new memory now and then.)
 template <int HD, int CB, int NW>
 __global__ void __launch_bounds__(NW * kWaveSize)
 attn_prefill_merge_kernel(const PrefillParams p, const PrefillItems items) {

@@ -510,7 +510,9 @@ int l3_attn_workspace_init(void* workspace, size_t workspace_bytes, void* stream
     if (g_xcd_state[dev].load(std::memory_order_acquire) == 0) {
         if (int rc = probe_xcd_mapping(dev, counters, st); rc != L3_OK) return rc;
     }
-    if (launch_fill_zero_u32(counters, L3_ATTN_COUNTER_BYTES / sizeof(unsigned), st) != 0) return L3_ERR_HIP;
+    // The partial rows too, which need no value: nothing that a launch hands over inside itself is the first access to its
+    // memory (2 us for 4 MB, once per workspace).  Such a hand-over between XCDs has returned what was there before on new memory only.
+    if (launch_fill_zero_u32(counters, workspace_bytes / sizeof(unsigned), st) != 0) return L3_ERR_HIP;
     return L3_OK;
 }
 

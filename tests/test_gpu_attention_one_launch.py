@@ -245,3 +245,38 @@ def test_calls_on_two_streams_at_once(l3, gpu):
         assert int(c.bad.item()) == 0
         assert int(c.ws[: l3.L3_ATTN_COUNTER_BYTES - 128].view(torch.int32).count_nonzero().item()) == 0
         assert lib.l3_attn_placement_errors(c.ws.data_ptr()) == 0
+
+
+def test_a_prepared_workspace_has_been_written(l3, gpu):
+    """All of it, up to its last whole word and no further: no launch is the first to touch the rows that it hands over."""
+    lib = l3.load()
+    ws = torch.full((l3.L3_ATTN_COUNTER_BYTES + 4096 + 256,), 0xa5, dtype=torch.uint8, device=gpu)
+    for nbytes in (l3.L3_ATTN_COUNTER_BYTES, l3.L3_ATTN_COUNTER_BYTES + 4, l3.L3_ATTN_COUNTER_BYTES + 4096):
+        ws.fill_(0xa5)
+        assert lib.l3_attn_workspace_init(ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        assert int(ws[:nbytes].count_nonzero()) == 0 and bool((ws[nbytes:] == 0xa5).all())
+
+
+@pytest.mark.parametrize("B,S,HD", [(1, 4096, 128), (1, 8192, 64), (8, 3000, 128)])
+def test_first_calls_on_new_streams(l3, gpu, B, S, HD):
+    """The first call of a stream merges rows in memory that was allocated for it: the bits of a call in a workspace in use,
+    64 times, up to the first that differs."""
+    from custom_kernels import custom_kernels_extension as cke
+    from test_gpu_operator_threads import _new_stream
+
+    q, k, v = make_qkv(B, 32, 8, S, HD, seed=41, device=gpu)
+    assert l3.load().l3_attn_launches(B, 32, 8, S, HD, 0, l3.L3_ATTN_FLAG_WS_COUNTERS) == 1
+    cke.flash_attention_decode(q, k, v)
+    want = cke.flash_attention_decode(q, k, v)
+    with cke.attention_flags(launches="two"):
+        two = cke.flash_attention_decode(q, k, v)
+    assert_attn_close(want, t2f32(two).astype(np.float64), what="one launch against two", min_kv_len=S)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()      # what comes is taken from the driver
+    for i in range(64):
+        print(f"new stream {i} B={B} S={S} HD={HD}", flush=True)
+        with torch.cuda.stream(torch.cuda.ExternalStream(_new_stream())):
+            out = cke.flash_attention_decode(q, k, v)
+            torch.cuda.current_stream().synchronize()
+            assert torch.equal(out, want), f"first call of stream {i}: {int((out != want).sum())} values"
