@@ -224,8 +224,9 @@ int l3_attn_prefill(const void* q, const void* k, const void* v, void* out, int 
 /*
  * The same with memory for partial results.  Launches of few rows against many tokens (a short piece of a prompt behind
  * a long cache) are then cut into pieces of rows x tokens, and a second launch adds them up.
- *   workspace : l3_attn_prefill_workspace_bytes() bytes (0: the call is not cut and takes none), aligned to 256; free
- *               to be reused by later work of the stream
+ *   workspace : l3_attn_prefill_workspace_bytes() bytes (0: the call is not cut and takes none; at most five partial
+ *               results of 69632 bytes per compute unit, 85 MiB on 256), aligned to 256; free to be reused by later work of
+ *               the stream.  NULL: not cut, as l3_attn_prefill
  */
 size_t l3_attn_prefill_workspace_bytes(int B, int QH, int KVH, int T, int S, int HD, int flags);
 int l3_attn_prefill_ws(const void* q, const void* k, const void* v, void* out, void* workspace, size_t workspace_bytes,

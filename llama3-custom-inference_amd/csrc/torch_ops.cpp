@@ -313,10 +313,14 @@ PyObject* flash_attention_prefill(PyObject* const* a) {
         Tensor out(at::detail::empty_strided_cuda(sizes, strides, at::kBFloat16, q.device()));
         if (out.numel() > 0) {
             const OnDevice on(q);
-            // partial results live for the call
-            const size_t nbytes = lib.l3_attn_prefill_workspace_bytes(int(B), int(QH), int(KVH), int(T), int(S), int(HD), flags);
+            // partial results live for the call; where there is no memory for them the call is not cut
+            size_t nbytes = lib.l3_attn_prefill_workspace_bytes(int(B), int(QH), int(KVH), int(T), int(S), int(HD), flags);
             TensorBase part;
-            if (nbytes > 0) part = at::detail::empty_cuda({int64_t(nbytes)}, at::kByte, q.device(), std::nullopt);
+            try {
+                if (nbytes > 0) part = at::detail::empty_cuda({int64_t(nbytes)}, at::kByte, q.device(), std::nullopt);
+            } catch (const c10::OutOfMemoryError&) {
+                nbytes = 0;
+            }
             const int rc = lib.l3_attn_prefill_ws(ptr(q), ptr(k), ptr(v), ptr(out), nbytes > 0 ? ptr(part) : nullptr, nbytes,
                                                   int(B), int(QH), int(KVH), int(T), int(S), int(HD), q.strides().data(),
                                                   k.strides().data(), v.strides().data(), strides,

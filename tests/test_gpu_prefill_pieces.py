@@ -138,3 +138,38 @@ def test_values_that_are_not_finite(gpu):
     # (columns of a wavefront follow a new maximum together, so a neighbour's may move the last bit)
     assert float((out[:, :4, :first].float() - clean[:, :4, :first].float()).abs().max()) <= 2.0 ** -7 * float(clean.float().abs().max())
     assert bool(out[:, :4, first:].isnan().all())
+
+
+@pytest.mark.gpu
+def test_without_memory_for_the_pieces(gpu):
+    """A call that was served without a buffer is still served when there is none to be had: it is not cut."""
+    from custom_kernels import custom_kernels_extension as cke
+
+    q, k, v = make(1, 32, 8, 512, 7000, 64)(gpu)
+    cut = cke.flash_attention_prefill(q, k, v)
+    with cke.attention_flags(prefill="tiled"):
+        want = cke.flash_attention_prefill(q, k, v)
+    torch.cuda.synchronize()
+    room = torch.empty_like(want)
+    torch.cuda.empty_cache()
+    print("prefill with the allocator at its limit", flush=True)
+    held = []
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (64 << 20)) / torch.cuda.get_device_properties(0).total_memory)
+    try:
+        try:
+            while True:
+                held.append(torch.empty(8 << 20, dtype=torch.uint8, device=gpu))
+        except torch.OutOfMemoryError:
+            pass
+        assert cut_bytes(1, 32, 8, 512, 7000, 64) > 8 << 20
+        del room                                       # of the result, and of nothing larger
+        out = cke.flash_attention_prefill(q, k, v)
+        torch.cuda.synchronize()
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(cut_bytes(1, 32, 8, 512, 7000, 64), dtype=torch.uint8, device=gpu)
+    finally:
+        held.clear()
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    np.testing.assert_array_equal(t2bits(out), t2bits(want))
+    np.testing.assert_array_equal(t2bits(cke.flash_attention_prefill(q, k, v)), t2bits(cut))
+    assert not torch.equal(cut, want)                  # (the two forms differ in their last bits, so the test sees which ran)
