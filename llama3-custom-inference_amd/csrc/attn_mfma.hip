@@ -28,12 +28,12 @@ namespace {
 // through LDS at the end; with a single split per head the workgroup writes the final output and
 // no combine kernel runs.  It trades the contiguous-row access of the streaming form for eight
 // times the parallelism per head, which is what a latency-bound call (a few tiles per head) needs.
-// LOADS = 4 (head size 64, cooperative form, at most 512 tokens): half-size tiles of 32 tokens, so
+// LOADS = 4 (head size 64, cooperative form, short sequences): half-size tiles of 32 tokens, so
 // that a short sequence still gives every wavefront a tile, and slabs small enough for two
 // workgroups per CU.
 // NW = 4 (cooperative form, one split, more heads than compute units): half the wavefronts and half the slabs, so that two
-// workgroups are resident where one of eight wavefronts was (registers allow no third: 178 and 192; head size 64 up to 512
-// tokens, 111: four).  A wavefront does the work of two, one after the other, with the softmax states of two, and the eight
+// workgroups are resident where one of eight wavefronts was (registers allow no third: 178 and 192; of half tiles,
+// 111: four).  A wavefront does the work of two, one after the other, with the softmax states of two, and the eight
 // states are merged as eight wavefronts' are: a sequence has the same bits in a batch of 32 and of 64.  (One state for all tiles of a
 // wavefront took 0.3 to 0.8 us less where a wavefront has several: 64 x 8 heads at head size 128, 200 tokens 11.1 us, at head
 // size 64, 512 tokens 14.7; but a batch's results then hung on its size.)  us, eight wavefronts or streaming / this: 64
@@ -309,7 +309,11 @@ int launch_attn_splitkv_mfma(const AttnParams& params, int HD, int R, bool coop,
             if (p.num_splits == 1 && int64_t(p.B) * p.KVH > current_device_cus()) {
                 constexpr int NW = 4;
                 const dim3 four(NW * kWaveSize);
-                if (HD == 64 && p.tokens_per_split <= 2 * kMfmaWaves * 32) {
+                // Half tiles as far as eight wavefronts take them, for the same bits, while all workgroups are resident; beyond,
+                // where it was never eight wavefronts, as far as they are faster (us, half / full tiles, 640 heads: 260 tokens 11.0 /
+                // 13.0, 384 tokens 14.3 / 14.5, 512 tokens 20.2 / 18.6).
+                const int half_tiles = int64_t(p.B) * p.KVH <= 2 * int64_t(current_device_cus()) ? 2 * kMfmaWaves : 3 * NW;
+                if (HD == 64 && p.tokens_per_split <= half_tiles * 32) {
                     rc = enqueue(attn_splitkv_mfma_kernel<64, true, 4, NW>, grid, four, 0, stream, R, 0, p);
                 } else if (HD == 64) {
                     rc = enqueue(attn_splitkv_mfma_kernel<64, true, 8, NW>, grid, four, 0, stream, R, 0, p);

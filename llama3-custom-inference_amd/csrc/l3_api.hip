@@ -171,22 +171,30 @@ bool attn_merge_in_launch_wanted(int flags) {
 }
 }  // namespace
 // Tiles of a sequence for which a (batch, kv head) is one workgroup of four wavefronts, where there are more of those
-// than compute units: from a sweep of 272 to 1024 heads and 16 to 2400 tokens against the streaming form (us, streaming / this).
-//   * Up to 5/4 heads per unit some units have twice the work of others, so longer sequences stream in splits (272 heads at
-//     head size 128, 400 tokens 15.5 / 15.0, 512 tokens 17.2 / 18.2; head size 64, 512 tokens 11.2 / 11.6, 800 tokens 14.4 /
-//     16.9); up to 7/4 that is so from 800 tokens on at head size 64 (384 heads, 800: 16.6 / 17.9, 1000: 21.2 / 21.4).
-//   * Up to three heads per unit all of them are resident (640 heads, 1000 tokens: head size 64 42.7 / 31.9, 128 60.3 / 55.7);
-//     a 512-head launch at head size 64, 800 tokens 21.2 / 20.0.  Whole token rows win beyond (640 heads, 1600 tokens at head
-//     size 128: 82.9 / 87.1).
-//   * Up to four heads per unit short sequences only (896 heads, 400 tokens: head size 64 20.6 / 18.7, 128 36.6 / 32.0; 1024
-//     heads, 512 tokens: 24.3 / 25.3 and 45.1 / 46.1).
-//   * At head size 128 a single tile of 640 heads is better streamed (4.9 / 6.0), two of 896 and three of
-//     792 as well (8.4 / 9.0, 9.6 / 9.9).
+// than compute units.  Two such workgroups are resident per unit, four of half tiles (head size 64, up to 512 tokens).  From
+// a sweep of 264 to 1024 heads and 1 to 34 tiles (us, four wavefronts / streaming):
+//   * Up to 5/4 heads per unit some units have twice the work of others, so longer sequences stream in splits (288 heads at
+//     head size 64, 8 tiles 13.1 / 14.3, 9 tiles 13.2 / 11.9; at 128, 13 tiles 15.9 / 16.2, 14 tiles 16.6 / 16.4).
+//   * Up to two, all of them are resident.  Head size 64: up to 7/4 level around 13 tiles (384 heads 18.5 / 18.2, 448 heads
+//     19.5 / 20.1; 14 tiles 20.0 / 18.4 and 21.1 / 20.8), then around 15 (512 heads, 13 tiles 20.6 / 21.4, 15 tiles 22.8 /
+//     23.0, 18 tiles 27.9 / 27.3).  Head size 128: 448 heads, 20 tiles 25.1 / 27.5, 32 tiles 38.6 / 38.9; 384 heads 23.4 / 23.4
+//     and 36.0 / 34.0.
+//   * Beyond, up to 9/4, a second round that is nearly empty takes as long as a full one, and longer sequences stream (520 heads at
+//     head size 64, 520 tokens 18.2 / 16.4, 1000 tokens 30.2 / 27.3; at 128, 600 tokens 31.8 / 30.7, 1000 tokens 50.0 / 45.4).
+//     Up to three the round is worth it (768 heads at head size 64, 600 tokens 22.8 / 23.9, 1000 tokens 34.1 / 35.5; 640 at
+//     head size 128, 600 tokens 33.9 / 36.5, 1000 tokens 53.7 / 58.6; 1024 tokens, which four wavefronts walk in step
+//     with the memory channels, 34.6 / 32.2 and 55.4 / 56.0).
+//   * Up to four short sequences only (head size 64: 896 heads, 7 tiles 20.6 / 21.1, 8 tiles 25.7 / 23.5; 128: 896 heads,
+//     410 tokens 32.0 / 33.8, 776 heads 30.5 / 30.4, 14 tiles 32.8 / 31.7).
+//   * At head size 128 a single tile of more than two heads per unit is better streamed (640 heads 6.3 / 6.0), and up to three
+//     tiles of more than three (896 heads, 2 tiles 9.1 / 8.5, 3 tiles 10.9 / 11.1, 1024 heads 11.7 / 11.3).
 int four_wave_tiles_max(int64_t units, int HD, int64_t cus) {
-    if (4 * units <= 5 * cus) return HD == 64 ? 8 : 12;
+    if (4 * units <= 5 * cus) return HD == 64 ? 8 : 13;
     if (4 * units <= 7 * cus) return HD == 64 ? 13 : 32;
+    if (units <= 2 * cus) return HD == 64 ? 16 : 32;
+    if (4 * units <= 9 * cus) return HD == 64 ? 8 : 15;
     if (units <= 3 * cus) return HD == 64 ? 16 : 32;
-    if (units <= 4 * cus) return HD == 64 ? 7 : 12;
+    if (units <= 4 * cus) return HD == 64 ? 7 : 13;
     return 0;
 }
 int four_wave_tiles_min(int64_t units, int HD, int64_t cus) {
@@ -277,10 +285,10 @@ AttnPlan attn_make_plan(int B, int KVH, int S, int HD, int requested, int num_cu
             // K + V bytes a workgroup streams when there is a single group
             const int64_t stream_bytes = int64_t(kMfmaWaves) * ((S + spg - 1) / spg) * HD * 4;
             const bool short_stream = stream_bytes <= (int64_t(3) << 20);
-            if (short_stream && spg == 1 && (wgs_per_split_group * 2 >= num_cus || (wgs_per_split_group * 4 >= num_cus && tiles <= 4))) {
+            if (short_stream && spg == 1 && (wgs_per_split_group * 2 >= num_cus || (wgs_per_split_group * 4 >= num_cus && tiles <= 3))) {
                 // half of the units busy, but no partials and no second launch (with a quarter of them busy only the
-                // shortest: 99 sequences of 81 tokens at head size 128 take 9.7 us in one group, 11.5 in two; 64 of 1300 tokens at head
-                // size 64 53.9 in one, 29.6 in three)
+                // shortest, head size 128 below four_wave_tiles_min: 99 sequences of 81 tokens take 9.7 us in one group, 11.5 in
+                // two; 64 of 1300 tokens at head size 64 53.9 in one, 29.6 in three)
                 groups = 1;
             } else if (groups == 1 && (!short_stream || spg == 1) && int64_t(num_cus) / wgs_per_split_group >= 2) {
                 groups = 2;

@@ -17,7 +17,9 @@ def splits(B, KVH, S, HD):
 
 def test_lengths_that_take_one_workgroup_per_head():
     """One split up to each line, splits again beyond it (where the streaming form has several)."""
-    for units, last in ((320, {64: 512, 128: 384}), (448, {64: 832, 128: 1024}), (512, {64: 1024, 128: 1024}), (768, {64: 1024, 128: 1024})):
+    for units, last in ((320, {64: 512, 128: 416}), (448, {64: 832, 128: 1024}), (512, {64: 1024, 128: 1024}), (576, {64: 512, 128: 480}),
+                        (768, {64: 1024, 128: 1024}),
+                        (896, {64: 448, 128: 416})):
         for HD in (64, 128):
             assert splits(units // 8, 8, last[HD], HD) == 1
             assert splits(units // 8, 8, last[HD] + 1, HD) > 1, (units, HD)
@@ -28,7 +30,8 @@ def test_lengths_that_take_one_workgroup_per_head():
 # pairs either side of one, 5/4, 2, 3 and 4 per compute unit; lengths of one tile and less, of one and of more rounds of the four
 # wavefronts with a ragged end, and the longest each takes; every head ratio
 CASES = [(257, 1, 1), (33, 8, 16), (33, 8, 129), (33, 8, 384), (40, 8, 512), (41, 8, 257), (64, 8, 63), (64, 8, 255), (64, 8, 1000),
-         (65, 8, 33), (65, 8, 300), (96, 8, 70), (96, 8, 1024), (97, 8, 65), (97, 8, 97), (128, 8, 380), (128, 8, 448), (140, 2, 700), (129, 8, 40)]
+         (65, 8, 33), (65, 8, 300), (96, 8, 70), (96, 8, 1024), (97, 8, 65), (97, 8, 97), (128, 8, 380), (128, 8, 448), (140, 2, 700), (129, 8, 40),
+         (65, 8, 384), (65, 8, 385)]
 
 
 @pytest.mark.gpu
