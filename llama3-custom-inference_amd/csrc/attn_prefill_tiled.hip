@@ -802,18 +802,19 @@ int prefill_items(const PrefillSplitPlan& plan, int R, int T, int S, PrefillItem
 
 // Which calls are cut.  A short piece of a prompt behind many cached tokens has few blocks, each with a long range: 64
 // queries behind 4032 tokens are 32 workgroups of 64 tiles.  Cut into pieces of n per block they fill the device; what
-// that costs is the partial results (18 to 66 KB each, written and read) and a second launch.
-// Measured (us, uncut / cut; 32 query heads over 8, one sequence): 8 queries of 4096 tokens 54.9 / 12.6, 64 of 4096
-// 37.9 / 14.9, 512 of 7012 64.1 / 46.9, head size 128 105.8 / 67.2.  The lines, from a sweep over B 1 ... 16, R 3, 4, 8:
-//   * n: at most two pieces per compute unit (a 513th starts when a first has ended: 23.6 -> 29 us for 200 of 3200 at head
-//     size 128), pieces of at least 3/4 sqrt(tiles) tiles (8 of 3008: 4 tiles 9.4, 8 tiles 10.5, 1 tile 12 us before the merge
-//     was a launch of its own);
-//   * one column block per wavefront while its blocks do not fill the device (64 of 4096: 11.5 against 14 us), two beyond
-//     and for the longest ranges (512 of 7012 at head size 128: 66 against 80 us);
-//   * below 12 tiles (64 of 314: 6.6 uncut, 9) or where the blocks alone occupy the device the second launch costs what the
+// that costs is the partial results (18 to 68 KiB each, written and read) and a second launch.
+// Measured (us, uncut / cut; 32 query heads over 8, one sequence): 8 queries of 4096 tokens 55.1 / 12.7, 64 of 4096
+// 38.8 / 15.2, 512 of 7012 64.5 / 44.1, head size 128 122.8 / 69.9.  The lines, from a sweep over B 1 ... 16, R 3, 4, 8:
+//   * n: at most two pieces per compute unit (200 of 3200 at head size 128: two 25.3, three 29.1 us; only launches of more
+//     than one two-block workgroup per unit, whose units have one block or two, go up to five: 1500 of 8000 at head
+//     size 128, 256.6 us uncut, is 196.2 in three pieces a block), pieces of at least 3/4 sqrt(tiles) tiles (8 of 3008: 4
+//     tiles 11.6, 6 tiles 11.8, 8 tiles 12.5, 1 tile 19.4 us);
+//   * one column block per wavefront while its blocks do not fill the device (64 of 4096: 15.2 against 16.2 us), two beyond
+//     and for the longest ranges (512 of 7012 at head size 128: 68.4 against 78.3 us);
+//   * below 12 tiles (64 of 314: 6.4 uncut, 8.3) or where the blocks alone occupy the device the second launch costs what the
 //     balance gives; at head size 64, whose tiles are half the work, the more blocks the more tiles it takes (200 of 800 and 512 of
-//     1512: 11 / 11.3 and 17.8 / 17.7; 64 heads, 200 of 1200: 14.7 / 15.8; 200 of 1200: 14.4 / 12.8), except for the few queries
-//     that would run as single wavefronts (16 sequences, 8 of 1008: 16.4 / 13.6);
+//     1512: 11.2 / 11.4 and 17.6 / 16.9; 64 heads, 200 of 1200: 14.6 / 15.8; 200 of 1200: 14.7 / 12.8), except for the few queries
+//     that would run as single wavefronts (16 sequences, 8 of 1008: 17.5 / 15.0);
 //   * not prompts without a past, whose longest blocks end a launch that has kept the device busy (2 x 1531, with the merge in
 //     the launch: 29.5 uncut, 29.0 ... 36 by the cut; 2048: 27.2, 30.0).
 PrefillSplitPlan prefill_split_plan(int B, int QH, int KVH, int T, int S, int HD, int num_cus) {
@@ -832,7 +833,7 @@ PrefillSplitPlan prefill_split_plan(int B, int QH, int KVH, int T, int S, int HD
     } else if (two <= cus && tiles >= (HD == 128 ? 40 : 64)) {
         plan.col_blocks = 2;
     } else if (5 * two <= 8 * cus && tiles >= (HD == 128 ? 64 : 100)) {
-        plan.col_blocks = 2;   // (1500 of 8000: at head size 128 258 / 196 us: units with one block and with two)
+        plan.col_blocks = 2;
         room = 5 * cus;
     } else {
         return none;
@@ -854,7 +855,8 @@ int launch_attn_prefill_split(const PrefillParams& p, int HD, const PrefillSplit
     constexpr int NW = kPrefillTiledWaves;
     if (HD == 64) {
         if (plan.col_blocks == 1) return launch_pieces<64, 1, NW, 64, 4>(p, plan, part, stream);
-        return launch_pieces<64, 2, NW, 64, 4>(p, plan, part, stream);
+        // (three wavefronts per SIMD: four, as the uncut kernel has, would spill eight registers here; 512 of 7012 tokens 45.8 -> 44.1 us)
+        return launch_pieces<64, 2, NW, 64, 3>(p, plan, part, stream);
     }
     if (plan.col_blocks == 1) return launch_pieces<128, 1, NW, 64, 2>(p, plan, part, stream);
     return launch_pieces<128, 2, NW, 64, 2>(p, plan, part, stream);
