@@ -179,7 +179,6 @@ __device__ __forceinline__ void store16(uint16_t* p, const uint4& v) { *reinterp
 // reads it next more (32 MB: 11.5 us instead of 8.4 us) than it saved the writer.
 // (-DL3_STREAM_LOADS=0 turns these back into plain loads, for repeating the comparison.)
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 #ifndef L3_STREAM_LOADS
 #define L3_STREAM_LOADS 1
 #endif
