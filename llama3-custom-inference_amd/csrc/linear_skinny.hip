@@ -120,7 +120,9 @@ linear_skinny_kernel(const LinearParams p) {
     // not wait behind kilobytes of weights coming from HBM).  Taken one at a time through LDS, with the norm weights
     // read again for each, the chunks of three or four rows were a chain of memory round trips in front of every
     // workgroup's products (us, before / now: 6144 x 4096, 2 / 3 / 4 rows 13.2 / 15.6 / 17.2, now 11.7 / 11.8 / 12.8; 3072 x
-    // 2048, 3 / 8 rows 7.4 / 10.1, now 6.5 / 8.1).
+    // 2048, 3 / 8 rows 7.4 / 10.1, now 6.5 / 8.1).  The norm weights come with the activations where one 16-byte chunk of them
+    // serves all of a thread's (K / 8 divides the threads); at other widths those of the further chunks are requested behind
+    // the ring (2048 x 2560, 4 rows 7.6 / 6.8; 2048 x 1536, 8 rows 8.0 / 7.8; 4608 x 3072, 4 rows 13.2 / 12.4).
     constexpr int NT = NW * kWaveSize;
     const int KP = p.K + 8;                                // LDS row pitch in elements
     const int cpr = p.K / 8;                               // chunks per row
