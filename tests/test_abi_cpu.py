@@ -310,6 +310,22 @@ def test_prefill_argument_checks():
     assert call(q_strides=_l3lib.i64_array((131072, 64, 2052))) == _l3lib.L3_ERR_STRIDE
     assert call(k_strides=_l3lib.i64_array((131072, -64, 512))) == _l3lib.L3_ERR_STRIDE
 
+    # with memory for the pieces: refused where it is too small or misaligned, before any launch
+    need = lib.l3_attn_prefill_workspace_bytes(1, 32, 8, 16, 4096, 64, 0)
+    assert need > 0
+    big = _l3lib.i64_array((4096 * 512, 64, 512))
+
+    def with_workspace(ws, nbytes, out=FAKE):
+        return lib.l3_attn_prefill_ws(FAKE, FAKE, FAKE, out, ws, nbytes, 1, 32, 8, 16, 4096, 64, qs, big, big, qs, 0.125, 0, None)
+
+    assert with_workspace(FAKE, need - 1) == _l3lib.L3_ERR_WORKSPACE
+    assert with_workspace(FAKE, 0) == _l3lib.L3_ERR_WORKSPACE
+    assert with_workspace(FAKE + 128, need) == _l3lib.L3_ERR_ALIGNMENT
+    assert with_workspace(FAKE, need, out=None) == _l3lib.L3_ERR_NULL_POINTER
+    for bad in ((0, 32, 8, 16, 4096, 64, 0), (1, 32, 8, 0, 4096, 64, 0), (1, 32, 8, 16, 15, 64, 0), (1, 40, 8, 16, 4096, 64, 0),
+                (1, 32, 8, 16, 4096, 96, 0), (1, 32, 8, 16, 4096, 64, 0x80)):
+        assert lib.l3_attn_prefill_workspace_bytes(*bad) == 0
+
 
 def test_linear_decode_argument_checks():
     lib = _l3lib.load()

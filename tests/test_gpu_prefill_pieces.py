@@ -123,8 +123,8 @@ def test_recorded_and_on_streams(gpu):
 
 
 @pytest.mark.gpu
-def test_values_that_are_not_finite(gpu):
-    """A NaN or an infinite key reaches the rows that see it and no other."""
+def test_a_nan_key(gpu):
+    """It reaches the rows that see it and no other."""
     from custom_kernels import custom_kernels_extension as cke
 
     q, k, v = make(1, 8, 2, 24, 2000, 64)(gpu)
@@ -138,6 +138,61 @@ def test_values_that_are_not_finite(gpu):
     # (columns of a wavefront follow a new maximum together, so a neighbour's may move the last bit)
     assert float((out[:, :4, :first].float() - clean[:, :4, :first].float()).abs().max()) <= 2.0 ** -7 * float(clean.float().abs().max())
     assert bool(out[:, :4, first:].isnan().all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("at", [1, 700, 1990])
+@pytest.mark.parametrize("HD", [64, 128])
+def test_an_infinite_key(gpu, HD, at):
+    """Scores of +inf make their rows NaN, as without pieces; those of -inf weigh nothing, also against the pieces' own reference."""
+    from custom_kernels import custom_kernels_extension as cke
+    from oracle import attention_prefill_ref
+
+    q, k, v = make(1, 8, 2, 24, 2000, HD)(gpu)
+    assert cut_bytes(1, 8, 2, 24, 2000, HD) > 0
+    k = k.clone()
+    k[0, 0, at, 3] = float("inf")
+    out = cke.flash_attention_prefill(q, k, v)
+    with cke.attention_flags(prefill="tiled"):
+        uncut = cke.flash_attention_prefill(q, k, v)
+    sees = torch.arange(24, device=gpu) + 2000 - 24 >= at
+    plus = (q[0, :4, :, 3] > 0) & sees                               # of the kv head's four query heads
+    assert torch.equal(out[0, :4].isnan().all(-1), plus) and torch.equal(out[0, :4].isnan().any(-1), plus)
+    assert torch.equal(uncut.isnan(), out.isnan()) and bool(plus.any()) and not bool(plus.all())
+    k[0, 0, at] = 0.0
+    k[0, 0, at, 3] = -3.0e38                                         # finite, and as good as -inf for the rows that are left
+    q[0, :4, :, 3] = q[0, :4, :, 3].abs()
+    ref = attention_prefill_ref(*(t2f32(t.cpu()) for t in (q, k, v)))
+    low = cke.flash_attention_prefill(q, k, v)
+    assert_attn_close(low, ref, what=f"a key of no weight at {at} HD={HD}", min_kv_len=1976)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,QH,KVH,T,S,HD", [(1, 32, 8, 8, 4096, 64), (1, 24, 8, 21, 1025, 64), (1, 8, 8, 65, 1000, 128), (1, 32, 8, 512, 7012, 64),
+                                             (1, 16, 4, 2016, 4032, 128), (1, 32, 8, 1400, 8000, 128)])
+def test_pieces_stay_in_the_workspace(gpu, B, QH, KVH, T, S, HD):
+    """Through the C ABI on exactly the bytes that it asks for: nothing is written before or behind them, and the bits are the
+    operator's.  Blocks of one and of two column blocks, some blocks cut and others not (2016 of 4032), up to five pieces per
+    compute unit (1400 of 8000)."""
+    from custom_kernels import _l3lib, custom_kernels_extension as cke
+
+    print(f"prefill workspace B={B} QH={QH} KVH={KVH} T={T} S={S} HD={HD}", flush=True)
+    lib, g = _l3lib.load(), torch.Generator(device=gpu).manual_seed(6)
+    q = torch.empty(B, T, QH, HD, dtype=torch.bfloat16, device=gpu).normal_(0, 1, generator=g).transpose(1, 2)
+    k, v = (torch.empty(B, S, KVH, HD, dtype=torch.bfloat16, device=gpu).normal_(0, 1, generator=g).transpose(1, 2) for _ in range(2))
+    want = cke.flash_attention_prefill(q, k, v)
+    n, guard = cut_bytes(B, QH, KVH, T, S, HD), 1 << 20
+    assert n > 0
+    ws = torch.full((guard + n + guard,), 0xa5, dtype=torch.uint8, device=gpu)
+    out = torch.full_like(want, float("nan"))
+    strides = lambda t: _l3lib.i64_array(t.stride()[:3])  # noqa: E731
+    rc = lib.l3_attn_prefill_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), ws.data_ptr() + guard, n, B, QH, KVH, T, S, HD,
+                                strides(q), strides(k), strides(v), strides(out), 1.0 / HD ** 0.5, 0,
+                                torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    torch.cuda.synchronize()
+    assert bool((ws[:guard] == 0xa5).all()) and bool((ws[guard + n:] == 0xa5).all())
+    np.testing.assert_array_equal(t2bits(out), t2bits(want))
 
 
 @pytest.mark.gpu
