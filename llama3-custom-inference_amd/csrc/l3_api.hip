@@ -181,6 +181,8 @@ bool attn_merge_in_launch_wanted(int flags) {
 //     and 36.0 / 34.0.
 //   * Beyond, up to 9/4, a second round that is nearly empty takes as long as a full one, and longer sequences stream (520 heads at
 //     head size 64, 520 tokens 18.2 / 16.4, 1000 tokens 30.2 / 27.3; at 128, 600 tokens 31.8 / 30.7, 1000 tokens 50.0 / 45.4).
+//     Only over whole token rows (a multiple of eight kv heads): others stream in up to 8 splits per group, whose partials
+//     can be more than the static scratch holds (103 x 5 kv heads of 8 query heads: 16.3 MiB).
 //     Up to three the round is worth it (768 heads at head size 64, 600 tokens 22.8 / 23.9, 1000 tokens 34.1 / 35.5; 640 at
 //     head size 128, 600 tokens 33.9 / 36.5, 1000 tokens 53.7 / 58.6; 1024 tokens, which four wavefronts walk in step
 //     with the memory channels, 34.6 / 32.2 and 55.4 / 56.0).
@@ -188,11 +190,11 @@ bool attn_merge_in_launch_wanted(int flags) {
 //     410 tokens 32.0 / 33.8, 776 heads 30.5 / 30.4, 14 tiles 32.8 / 31.7).
 //   * At head size 128 a single tile of more than two heads per unit is better streamed (640 heads 6.3 / 6.0), and up to three
 //     tiles of more than three (896 heads, 2 tiles 9.1 / 8.5, 3 tiles 10.9 / 11.1, 1024 heads 11.7 / 11.3).
-int four_wave_tiles_max(int64_t units, int HD, int64_t cus) {
+int four_wave_tiles_max(int64_t units, int KVH, int HD, int64_t cus) {
     if (4 * units <= 5 * cus) return HD == 64 ? 8 : 13;
     if (4 * units <= 7 * cus) return HD == 64 ? 13 : 32;
     if (units <= 2 * cus) return HD == 64 ? 16 : 32;
-    if (4 * units <= 9 * cus) return HD == 64 ? 8 : 15;
+    if (4 * units <= 9 * cus && KVH % kMfmaWaves == 0) return HD == 64 ? 8 : 15;
     if (units <= 3 * cus) return HD == 64 ? 16 : 32;
     if (units <= 4 * cus) return HD == 64 ? 7 : 13;
     return 0;
@@ -220,7 +222,7 @@ AttnPlan attn_make_plan(int B, int KVH, int S, int HD, int requested, int num_cu
         // the row in a single launch.
         const int64_t units = int64_t(B) * KVH;
         if (units > num_cus) {
-            if (tiles >= four_wave_tiles_min(units, HD, num_cus) && tiles <= four_wave_tiles_max(units, HD, num_cus)) {
+            if (tiles >= four_wave_tiles_min(units, HD, num_cus) && tiles <= four_wave_tiles_max(units, KVH, HD, num_cus)) {
                 plan.coop = true;
                 plan.num_splits = 1;
                 plan.tokens_per_split = tiles * tile;

@@ -23,6 +23,10 @@ def test_lengths_that_take_one_workgroup_per_head():
         for HD in (64, 128):
             assert splits(units // 8, 8, last[HD], HD) == 1
             assert splits(units // 8, 8, last[HD] + 1, HD) > 1, (units, HD)
+    # kv heads that do not fill whole rows stream in more splits: not where their partials would not fit the static scratch
+    for KVH in (3, 5):
+        for HD in (64, 128):
+            assert splits(-(-513 // KVH), KVH, 1024, HD) == splits(575 // KVH, KVH, 1024, HD) == 1
     # a quarter of the device is not left alone with a long stream
     assert splits(64, 8, 1300, 64) == 3 and splits(112, 8, 1300, 64) == 2 and splits(128, 8, 1300, 64) == 1
 
